@@ -9,8 +9,9 @@
 //     unsigned, the latter less 128, which the code sum makes good: the same integers, so the same bits; the others balanced digits.
 //   * Scales apply per 32 elements (Q6_K: per 16, the codes of the other half masked off), and sums join in the per-token
 //     kernels' order: two groups of a lane first (Q6_K: the four 16-groups of a lane), then a binary tree over a block's
-//     four lanes and over blocks (a counter of pending partial sums per level), so a row's result does not depend on the
-//     batch it is in.
+//     four lanes and over blocks (a counter of pending partial sums per level).  So a row has the same bits alone, in a small
+//     batch and here, wherever the per-token kernels of the format contract the same byte planes: all formats but MXFP4
+//     (whose per-token kernel multiplies floats), rows that fit a wavefront.
 //   * Weights come as in the grouped GEMM (k_grouped_gemm.hip): 16-byte chunks of consecutive lanes, two steps ahead
 //     in registers, through a small LDS region of the wave to a row per lane.  Activations are f32 rows in memory and become
 //     planes here, 256 k at a time into alternating LDS buffers: no launch and no buffer for the conversion.
@@ -33,6 +34,9 @@ typedef int int4v __attribute__((ext_vector_type(4)));
 struct PairScale {
     float s0, s1, m0, m1;   // groups 2j, 2j + 1: value = s * code - m
 };
+
+// The two groups of a lane as the per-token kernels of one lane per two groups add them up: acc = 0, then acc += scale * sum twice.
+__device__ __forceinline__ float two_terms(float s0, float f0, float s1, float f1) { return fmaf(s1, f1, fmaf(s0, f0, 0.0f)); }
 
 struct I4K : G4K {
     static constexpr bool kUnsigned = true, kNibble = false, kHalves = false;
@@ -92,7 +96,8 @@ struct I80 : G80 {
     static __device__ __forceinline__ PairScale scales(const Raw& v, int j) {
         return PairScale{f16_bits_to_f32(v.d[2 * j]), f16_bits_to_f32(v.d[2 * j + 1]), 0.0f, 0.0f};
     }
-    static __device__ __forceinline__ float pair(const PairScale& p, float f0, float f1, float, float) { return p.s0 * f0 + p.s1 * f1; }
+    // (a lane per group in the per-token kernel: both products are rounded)
+    static __device__ __forceinline__ float pair(const PairScale& p, float f0, float f1, float, float) { return __fadd_rn(__fmul_rn(p.s0, f0), __fmul_rn(p.s1, f1)); }
 };
 
 struct I40 : G40 {
@@ -105,7 +110,7 @@ struct I40 : G40 {
         return PairScale{f16_bits_to_f32(v.d[2 * j]), f16_bits_to_f32(v.d[2 * j + 1]), 0.0f, 0.0f};
     }
     static __device__ __forceinline__ float pair(const PairScale& p, float f0, float f1, float x0, float x1) {
-        return p.s0 * (f0 - 8.0f * x0) + p.s1 * (f1 - 8.0f * x1);
+        return two_terms(p.s0, f0 - 8.0f * x0, p.s1, f1 - 8.0f * x1);
     }
 };
 
@@ -131,7 +136,7 @@ struct IIX : GIX {
         return f16_bits_to_f32(v.h.x & 0xFFFFu) * (float)(ls - 32);
     }
     static __device__ __forceinline__ PairScale scales(const Raw& v, int j) { return PairScale{scale(v, 2 * j), scale(v, 2 * j + 1), 0.0f, 0.0f}; }
-    static __device__ __forceinline__ float pair(const PairScale& p, float f0, float f1, float x0, float x1) { return I80::pair(p, f0, f1, x0, x1); }
+    static __device__ __forceinline__ float pair(const PairScale& p, float f0, float f1, float, float) { return two_terms(p.s0, f0, p.s1, f1); }
 };
 
 template <class F>
@@ -309,7 +314,7 @@ __device__ __forceinline__ void int_tile(const GroupedParams& p, const Tile& t, 
                 long b[2];
                 PairScale ps;
                 ps = F::scales(raw, j);
-                if (kPartial && 2 * j + 1 >= groups) ps.s1 = 0.0f;
+                if (kPartial && 2 * j + 1 >= groups) ps.s1 = -0.0f;   // its sum is +0: adds -0.0, the identity
                 b[0] = __builtin_bit_cast(long, F::codes(raw, 2 * j));
                 b[1] = __builtin_bit_cast(long, F::codes(raw, 2 * j + 1));
 #pragma unroll

@@ -112,3 +112,34 @@ def test_decode_rows_of_one_to_sixty_four_lanes(be, gdt, ddt, ne, nff, rows):
     assert np.array_equal(r["idx"], ref["idx"])
     for row in range(rows):
         assert H.rel_l2(out.reshape(rows, ne)[row], ref["dst"].reshape(rows, ne)[row]) < 1e-5, row
+
+
+@pytest.mark.parametrize("dt,ne,nff", [
+    (H.Q8_0, 2048, 352), (H.Q8_0, 160, 1056), (H.Q5K, 1280, 768), (H.Q4_0, 1088, 320), (H.Q4_0, 64, 4032), (H.IQ4_XS, 1280, 768),
+    (H.Q4K, 2304, 1280), (H.Q6K, 768, 4096),
+])
+def test_rows_keep_their_bits_in_a_batch_over_buckets(be, dt, ne, nff):
+    """A token row alone and among three (per-token kernels) and among 20 on seven experts (buckets): the same group sums, scaled
+    and added up in the same order, for every format and row width that both families take; MXFP4 is left out, whose per-token
+    kernel multiplies floats."""
+    rng = np.random.default_rng(dt * 43 + ne)
+    E, rows = 7, 20
+    x = rng.standard_normal((rows, ne)).astype(np.float32)
+    router = (rng.standard_normal((E, ne)) * 0.02).astype(np.float32)
+    gate, up, down = (_zero_some_scales(w, dt, rng) for w in _bank_weights(rng, E, nff, ne, dt, dt))
+    sel = rng.integers(0, E, (rows, 1)).astype(np.int32)
+
+    def run(pick):
+        g, ids = moe_graph(len(pick), ne, E, 1, nff, DType(dt), DType(dt), with_expert_ids=True)
+        be.prof_enable(True)
+        out, _ = run_moe(be, g, ids, dict(x=np.ascontiguousarray(x[pick]), router=router, gate=gate, up=up, down=down,
+                                          expert_ids=np.ascontiguousarray(sel[pick])), len(pick), ne)
+        names = set(be.prof_read())
+        be.prof_enable(False)
+        assert ("moe_down_bucketed" in names) == (len(pick) == rows), names
+        return out
+
+    full = run(list(range(rows)))
+    assert np.array_equal(bits(run([0, 9, 19])), bits(full[[0, 9, 19]]))
+    for r in (0, 9, 19):
+        assert np.array_equal(bits(run([r])[0]), bits(full[r])), r
