@@ -903,8 +903,7 @@ extern "C" infr_status infr_hip_compile(infr_hip_backend* be, const infr_graph* 
                                              (dense_neighbour ? 60.0 : 20.0);
                     bucketed = few_distinct || bucket_us < token_us;
                     if (bucketed)
-                        plan->moe[oi].k_parts = infr::grouped_int_parts((int)c.dt(m.down_exps), (int)m.n_ff_exp,
-                                                                        infr::grouped_int_down_parts((int)m.n_ff_exp, (int)m.ne, (int)std::lround(expect_distinct)));
+                        plan->moe[oi].k_parts = infr::grouped_int_parts((int)c.dt(m.down_exps), (int)m.n_ff_exp, infr::grouped_int_down_parts((int)m.n_ff_exp));
                 }
                 // banks without a matrix-core decoder: from the batched threshold on, the unit kernels walk the
                 // expert buckets (weights fetched once per chunk of tokens)

@@ -470,12 +470,10 @@ bool grouped_int_supported(int dt, int k) {
 }
 
 // Rows of many blocks on few columns leave most compute units without a workgroup: the down rows then go in parts of K, whose
-// sums the combine adds (8 experts of 4096 x 14336, 5 rows: 192 workgroups' worth of steps on 256 compute units).  Rows of up to
-// sixteen 256-k steps stay whole: their sums have the per-token kernels' order.
-int grouped_int_down_parts(int k, int n, int tiles) {
-    const int items = tiles * ((n + 63) / 64), want = 1024 / (items > 0 ? items : 1), most = k / 2048;
-    return k <= 4096 ? 1 : want < 2 ? 1 : want < most ? want : most;
-}
+// sums the combine adds.  Rows of up to sixteen 256-k steps stay whole: their sums have the per-token kernels' order.  Longer
+// ones are cut by their length alone, so that a row's bits do not depend on how many others are in the batch (8 experts of
+// 4096 x 14336, Q6_K, four parts: 5 rows 72 us, 31 rows 158; in the one or two parts that the batch alone would ask for 88 and 172).
+int grouped_int_down_parts(int k) { return (k + 4095) / 4096; }
 int grouped_int_parts(int dt, int k, int k_parts) {
     const int step = dt == INFR_Q8_0 ? 128 : 256, steps = (k + step - 1) / step, per = part_steps(steps, k_parts);
     return (steps + per - 1) / per;

@@ -214,7 +214,7 @@ void launch_grouped_down(hipStream_t s, int dt, const GroupedParams& p);
 // The same two stages for decode batches, f32-accurate (k_grouped_int.hip): tiles of kIntTok pairs, activations in p.xf, the
 // results of down f32 in bucket order.
 bool grouped_int_supported(int dt, int k);
-int grouped_int_down_parts(int k, int n, int tiles);   // p.k_parts worth asking for with that many tiles
+int grouped_int_down_parts(int k);                     // p.k_parts to ask for
 int grouped_int_parts(int dt, int k, int k_parts);     // parts written when k_parts are asked for
 void launch_grouped_int_gate_up(hipStream_t s, int dt, const GroupedParams& p);
 void launch_grouped_int_down(hipStream_t s, int dt, const GroupedParams& p);

@@ -143,3 +143,23 @@ def test_rows_keep_their_bits_in_a_batch_over_buckets(be, dt, ne, nff):
     assert np.array_equal(bits(run([0, 9, 19])), bits(full[[0, 9, 19]]))
     for r in (0, 9, 19):
         assert np.array_equal(bits(run([r])[0]), bits(full[r])), r
+
+
+def test_down_rows_in_parts_keep_their_bits_in_any_batch(be):
+    """Down rows of more than sixteen 256-k steps go in parts of K, as many at 16 rows (some 12 of 24 experts) as at 31."""
+    ne, nff, E, rows, dt = 2048, 4352, 24, 31, H.Q4_0
+    rng = np.random.default_rng(5)
+    x = rng.standard_normal((rows, ne)).astype(np.float32)
+    router = (rng.standard_normal((E, ne)) * 0.02).astype(np.float32)
+    gate, up, down = (np.tile(w, E) for w in _bank_weights(rng, 1, nff, ne, dt, dt))
+    sel = rng.integers(0, E, (rows, 1)).astype(np.int32)
+    outs = []
+    for n in (16, rows):
+        g, ids = moe_graph(n, ne, E, 1, nff, DType(dt), DType(dt), with_expert_ids=True)
+        be.prof_enable(True)
+        out, _ = run_moe(be, g, ids, dict(x=np.ascontiguousarray(x[:n]), router=router, gate=gate, up=up, down=down,
+                                          expert_ids=np.ascontiguousarray(sel[:n])), n, ne)
+        assert "moe_down_bucketed" in set(be.prof_read())
+        be.prof_enable(False)
+        outs.append(out)
+    assert np.array_equal(bits(outs[0]), bits(outs[1][:16]))
