@@ -1,12 +1,13 @@
 // Decode batches of Op::MoeFfn (a few to some dozen token rows) whose pairs share experts: the two expert stages over the
 // buckets, every weight row read once for up to 8 tokens of its expert, in the arithmetic of the per-token kernels.
 //
-// Those contract 24-bit fixed-point activations with the weight codes as three byte planes, exact integer sums joined in
-// f32 (k_gemv.hip), with 24 dot instructions per 32 elements and token.  Here the matrix cores take the byte products:
-//   * v_mfma_i32_16x16x32_i8: operand A is four tokens x (plane A, plane B, plane C, ones) by 32 k, operand B the codes of 16
-//     weight rows; a lane receives the three plane sums of one token and weight row, and the plain sum of the codes, in
-//     its four registers.  Formats with unsigned codes take the planes as the per-token kernels do, A signed and B, C
-//     unsigned, the latter less 128, which the code sum makes good: the same integers, so the same bits; the others balanced digits.
+// Those contract fixed-point activations with the weight codes as three or four byte planes, exact integer sums joined in
+// f32 (k_gemv.hip), with 24 or 32 dot instructions per 32 elements and token.  Here the matrix cores take the byte products:
+//   * v_mfma_i32_16x16x32_i8: operand A is four tokens x (plane A, B, C, and D or ones) by 32 k, operand B the codes of 16
+//     weight rows; a lane receives the plane sums of one token and weight row in its four registers, so the fourth plane of
+//     the formats that have one costs no instruction.  Q4_K and Q6_K take three planes as their per-token kernels do, A signed
+//     and B, C unsigned, the latter less 128, which the sum of the codes in the fourth register makes good: the same integers,
+//     so the same bits; the others balanced digits.
 //   * Scales apply per 32 elements (Q6_K: per 16, the codes of the other half masked off), and sums join in the per-token
 //     kernels' order: two groups of a lane first (Q6_K: the four 16-groups of a lane), then a binary tree over a block's
 //     four lanes and over blocks (a counter of pending partial sums per level).  So a row has the same bits alone, in a small
@@ -39,7 +40,8 @@ struct PairScale {
 __device__ __forceinline__ float two_terms(float s0, float f0, float s1, float f1) { return fmaf(s1, f1, fmaf(s0, f0, 0.0f)); }
 
 struct I4K : G4K {
-    static constexpr bool kUnsigned = true, kNibble = false, kHalves = false;
+    static constexpr int kPlanes = 3;
+    static constexpr bool kUnsigned = true, kNibble = false, kHalves = false, kSums = true;
     static __device__ __forceinline__ uint2 codes(const Raw& v, int g) {
         const uint2 q = v.q[g >> 1];
         return g & 1 ? make_uint2((q.x >> 4) & kLo4, (q.y >> 4) & kLo4) : make_uint2(q.x & kLo4, q.y & kLo4);
@@ -59,7 +61,8 @@ struct I4K : G4K {
 };
 
 struct I5K : G5K {
-    static constexpr bool kUnsigned = true, kNibble = false, kHalves = false;
+    static constexpr int kPlanes = 4;
+    static constexpr bool kUnsigned = false, kNibble = false, kHalves = false, kSums = true;
     static __device__ __forceinline__ uint2 codes(const Raw& v, int g) {
         const uint2 q = v.q[g >> 1];
         auto five = [&](uint32_t w, uint32_t h) { return ((g & 1 ? w >> 4 : w) & kLo4) | (((h >> g) & kB0) << 4); };
@@ -70,7 +73,8 @@ struct I5K : G5K {
 };
 
 struct I6K : G6K {
-    static constexpr bool kUnsigned = true, kNibble = false, kHalves = true;
+    static constexpr int kPlanes = 3;
+    static constexpr bool kUnsigned = true, kNibble = false, kHalves = true, kSums = true;
     static __device__ __forceinline__ uint2 codes(const Raw& v, int g) {
         const int hh = g >> 2, w = g & 3;
         const uint2 l = v.l[2 * hh + (w & 1)], h = v.h[hh];
@@ -88,7 +92,8 @@ struct I6K : G6K {
 };
 
 struct I80 : G80 {
-    static constexpr bool kUnsigned = false, kNibble = false, kHalves = false;
+    static constexpr int kPlanes = 3;
+    static constexpr bool kUnsigned = false, kNibble = false, kHalves = false, kSums = false;
     static __device__ __forceinline__ uint2 codes(const Raw& v, int g) {
         if (g & 1) return make_uint2(v.x[g], v.y[g]);
         return make_uint2(__builtin_amdgcn_alignbyte(v.y[g], v.x[g], 2), __builtin_amdgcn_alignbyte(v.z[g >> 1], v.y[g], 2));
@@ -101,21 +106,26 @@ struct I80 : G80 {
 };
 
 struct I40 : G40 {
-    static constexpr bool kUnsigned = true, kNibble = true, kHalves = false;
+    static constexpr int kPlanes = 4;
+    static constexpr bool kUnsigned = false, kNibble = true, kHalves = false, kSums = false;
     static __device__ __forceinline__ uint2 codes(const Raw& v, int g) {
         const uint32_t x = g & 1 ? v.x[g] : __builtin_amdgcn_alignbyte(v.y[g >> 1], v.x[g], 2);
-        return make_uint2(x & kLo4, (x >> 4) & kLo4);
+        return make_uint2(less8(x & kLo4), less8((x >> 4) & kLo4));
+    }
+    // four nibbles less 8, as signed bytes
+    static __device__ __forceinline__ uint32_t less8(uint32_t q) {
+        const uint32_t v = q ^ 0x08080808u, neg = v & 0x08080808u;
+        return v | ((neg << 5) - (neg << 1));
     }
     static __device__ __forceinline__ PairScale scales(const Raw& v, int j) {
         return PairScale{f16_bits_to_f32(v.d[2 * j]), f16_bits_to_f32(v.d[2 * j + 1]), 0.0f, 0.0f};
     }
-    static __device__ __forceinline__ float pair(const PairScale& p, float f0, float f1, float x0, float x1) {
-        return two_terms(p.s0, f0 - 8.0f * x0, p.s1, f1 - 8.0f * x1);
-    }
+    static __device__ __forceinline__ float pair(const PairScale& p, float f0, float f1, float, float) { return two_terms(p.s0, f0, p.s1, f1); }
 };
 
 struct IMX : GMX {
-    static constexpr bool kUnsigned = false, kNibble = true, kHalves = false;
+    static constexpr int kPlanes = 3;
+    static constexpr bool kUnsigned = false, kNibble = true, kHalves = false, kSums = false;
     static __device__ __forceinline__ uint2 codes(const Raw& v, int g) {   // twice the value
         const uint32_t x = (g + 1) & 3 ? __builtin_amdgcn_alignbyte(v.y[g], v.x[g], (g + 1) & 3) : v.x[g];
         return make_uint2(signed_book(x << 4, x, 0x03020100u, 0x0C080604u, 0xFDFEFF00u, 0xF4F8FAFCu),
@@ -126,7 +136,8 @@ struct IMX : GMX {
 };
 
 struct IIX : GIX {
-    static constexpr bool kUnsigned = false, kNibble = true, kHalves = false;
+    static constexpr int kPlanes = 4;
+    static constexpr bool kUnsigned = false, kNibble = true, kHalves = false, kSums = false;
     static __device__ __forceinline__ uint2 codes(const Raw& v, int g) {
         return make_uint2(signed_book(v.x[g] << 4, v.x[g], 0xBFAD9881u, 0xF6EADDCFu, 0x26190D01u, 0x71594535u),
                           signed_book(v.x[g], v.x[g] >> 4, 0xBFAD9881u, 0xF6EADDCFu, 0x26190D01u, 0x71594535u));
@@ -205,7 +216,7 @@ __device__ __forceinline__ void int_tile(const GroupedParams& p, const Tile& t, 
         }
     };
     auto x_store = [&](int buf) {
-        Digits<E> d = digits_of<E, F::kHalves ? 16 : 32, !F::kUnsigned>(xv);
+        const Digits<E, F::kPlanes> d = digits_of<E, F::kHalves ? 16 : 32, !F::kUnsigned, F::kPlanes>(xv);
         const int g = e_x / (32 / E), o = e_x % (32 / E);              // group, place in it
         uint8_t* const row = al + buf * kIPlanes + ((tok_x >> 2) * 8 + g) * kIGroup + 4 * (tok_x & 3) * 32;
 #pragma unroll
@@ -216,9 +227,10 @@ __device__ __forceinline__ void int_tile(const GroupedParams& p, const Tile& t, 
             *reinterpret_cast<uint32_t*>(at) = d.a[i];
             *reinterpret_cast<uint32_t*>(at + 32) = d.b[i] ^ flip;
             *reinterpret_cast<uint32_t*>(at + 64) = d.c[i] ^ flip;
+            if constexpr (F::kPlanes == 4) *reinterpret_cast<uint32_t*>(at + 96) = d.d[i];
         }
         constexpr int kPer = (F::kHalves ? 16 : 32) / E;               // threads of a scale group
-        if (e_x % kPer == 0) sl[buf * kIntTok * GR + tok_x * GR + e_x / kPer] = make_float2(d.scale, d.sum);
+        if (e_x % kPer == 0) sl[buf * kIntTok * GR + tok_x * GR + e_x / kPer] = make_float2(d.scale, F::kSums ? d.sum : 0.0f);
     };
     const int n_pieces = (n_steps + SPP - 1) / SPP;
     x_load(0);
@@ -226,8 +238,8 @@ __device__ __forceinline__ void int_tile(const GroupedParams& p, const Tile& t, 
     if (n_steps > 1) request(1, w[1]);
     x_store(0);
     if (n_pieces > 1) x_load(1);
-    // the fourth row of every token: ones (both buffers, once)
-    for (int i = tid; i < 2 * TQ * 8 * 4 * 8; i += 256) {   // dwords: buffer, token quad and group, token, dword
+    // with unsigned codes the fourth row of every token: ones (both buffers, once)
+    for (int i = F::kUnsigned ? tid : 2 * TQ * 8 * 4 * 8; i < 2 * TQ * 8 * 4 * 8; i += 256) {   // dwords: buffer, token quad and group, token, dword
         const int dw = i & 7, tk = (i >> 3) & 3, tg = (i >> 5) % (TQ * 8), buf = (i >> 5) / (TQ * 8);
         *reinterpret_cast<uint32_t*>(al + buf * kIPlanes + tg * kIGroup + (4 * tk + 3) * 32 + 4 * dw) = kB0;
     }
@@ -241,6 +253,7 @@ __device__ __forceinline__ void int_tile(const GroupedParams& p, const Tile& t, 
     }
     // join3 of the three plane sums; the lower two in integers first (below 2^28), which rounds as its inner fma does
     auto join = [&](const int4v& y) {
+        if constexpr (F::kPlanes == 4) return join4(y[0], y[1], y[2], y[3]);
         int low = y[1] * 256 + y[2];
         if (F::kUnsigned) low += __mul24(y[3], 128 * 256 + 128);
         return fmaf((float)y[0], 65536.0f, (float)low);

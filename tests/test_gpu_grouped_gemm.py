@@ -163,3 +163,74 @@ def test_down_rows_in_parts_keep_their_bits_in_any_batch(be):
         be.prof_enable(False)
         outs.append(out)
     assert np.array_equal(bits(outs[0]), bits(outs[1][:16]))
+
+
+def _small_first_weight(w, dtype, gain_rows=None):
+    """Element 0 of every group of 32 decodes to zero (IQ4_XS: to its smallest magnitude, the book has no zero), so that an
+    outlier there adds nothing to hide behind; the rows of `gain_rows` get sixteen times the scale."""
+    b = np.ascontiguousarray(w).reshape(-1, H.BLOCK[dtype][1]).copy()
+    d_at = 208 if dtype == H.Q6K else 0
+    if dtype in (H.Q4K, H.Q5K):
+        b[:, 8:12] = 0                    # minimums of groups 0..3, and the upper bits of 4..7's
+        b[:, 12:16] &= 0x0F
+        first = 16 if dtype == H.Q4K else 48
+        for g in range(8):
+            b[:, first + 32 * (g >> 1)] &= 0xF0 if g % 2 == 0 else 0x0F
+        if dtype == H.Q5K:
+            b[:, 16] = 0
+        b[:, 2:4] = 0
+    elif dtype == H.Q6K:                  # code 32
+        for h in range(2):
+            b[:, [64 * h, 64 * h + 32]] = 0
+            b[:, 128 + 32 * h] = 0xAA
+    elif dtype == H.Q8_0:
+        b[:, 2] = 0
+    elif dtype == H.MXFP4:
+        b[:, 1] &= 0xF0
+    elif dtype == H.Q4_0:
+        b[:, 2] = (b[:, 2] & 0xF0) | 8
+    else:
+        assert dtype == H.IQ4_XS
+        for g in range(8):
+            b[:, 8 + 16 * g] = (b[:, 8 + 16 * g] & 0xF0) | 8
+    if gain_rows is not None:
+        rows = b.reshape(len(gain_rows), -1, b.shape[1])[gain_rows]
+        if dtype == H.MXFP4:
+            rows[:, :, 0] += 4
+        else:
+            rows[:, :, d_at:d_at + 2] = (rows[:, :, d_at:d_at + 2].copy().view(np.float16) * np.float16(16)).view(np.uint8)
+        b.reshape(len(gain_rows), -1, b.shape[1])[gain_rows] = rows
+    return b.reshape(-1)
+
+
+@pytest.mark.parametrize("dt,ne,nff,rows", [
+    (H.Q5K, 1280, 768, 1), (H.Q5K, 1280, 768, 20), (H.Q4_0, 1088, 320, 1), (H.Q4_0, 1088, 320, 20), (H.IQ4_XS, 1280, 768, 1),
+    (H.IQ4_XS, 1280, 768, 20),
+])
+def test_small_activations_beside_outliers_keep_their_bits(be, dt, ne, nff, rows):
+    """One element of 32 is some 256 times the others, in x and (through sixteen-fold gate and up rows) in the activated row, and
+    meets a weight of zero.  An f32 sum then loses nothing; fixed point of 24 bits relative to the group's largest is off by up
+    to 256 * 2^-24 = 1.5e-5 of the other elements (and of the result: 1.2e-5 to 3.3e-5).  The bar is what f32 arithmetic
+    allows: 2^-24 for each of the some eight roundings of a sum's tree, twice (gate/up, down): 1e-6."""
+    rng = np.random.default_rng(dt * 47 + ne + rows)
+    E = 1 if rows == 1 else 3
+    x = rng.standard_normal((rows, ne)).astype(np.float32)
+    x[:, ::32] *= 256
+    router = np.zeros((E, ne), np.float32)
+    gain = np.arange(E * nff) % 32 == 0
+    raw = _bank_weights(rng, E, nff, ne, dt, dt)
+    gate, up, down = _small_first_weight(raw[0], dt, gain), _small_first_weight(raw[1], dt, gain), _small_first_weight(raw[2], dt)
+    sel = rng.integers(0, E, (rows, 1)).astype(np.int32)
+    g, ids = moe_graph(rows, ne, E, 1, nff, DType(dt), DType(dt), with_expert_ids=True)
+    be.prof_enable(True)
+    out, _ = run_moe(be, g, ids, dict(x=x, router=router, gate=gate, up=up, down=down, expert_ids=sel), rows, ne)
+    names = set(be.prof_read())
+    be.prof_enable(False)
+    assert ("moe_down_bucketed" in names) == (rows > 1), names
+    wg, wu, wd = (np.asarray(H.ggml_dequant(dt, w), np.float64).reshape(s)
+                  for w, s in ((gate, (E, nff, ne)), (up, (E, nff, ne)), (down, (E, ne, nff))))
+    for r in range(rows):
+        e = sel[r, 0]
+        a, u = wg[e] @ x[r].astype(np.float64), wu[e] @ x[r].astype(np.float64)
+        want = wd[e] @ (a / (1 + np.exp(-a)) * u)
+        assert np.linalg.norm(out[r] - want) < 1e-6 * np.linalg.norm(want), r
