@@ -124,7 +124,7 @@ struct I40 : G40 {
 };
 
 struct IMX : GMX {
-    static constexpr int kPlanes = 3;
+    static constexpr int kPlanes = 4;
     static constexpr bool kUnsigned = false, kNibble = true, kHalves = false, kSums = false;
     static __device__ __forceinline__ uint2 codes(const Raw& v, int g) {   // twice the value
         const uint32_t x = (g + 1) & 3 ? __builtin_amdgcn_alignbyte(v.y[g], v.x[g], (g + 1) & 3) : v.x[g];
@@ -148,6 +148,27 @@ struct IIX : GIX {
     }
     static __device__ __forceinline__ PairScale scales(const Raw& v, int j) { return PairScale{scale(v, 2 * j), scale(v, 2 * j + 1), 0.0f, 0.0f}; }
     static __device__ __forceinline__ float pair(const PairScale& p, float f0, float f1, float, float) { return two_terms(p.s0, f0, p.s1, f1); }
+};
+
+// Rows too wide for a wavefront of the per-token kernels are f32 sums when they come alone: four planes here.
+struct W4K : I4K {
+    static constexpr int kPlanes = 4;
+    static constexpr bool kUnsigned = false;
+};
+struct W6K : I6K {
+    static constexpr int kPlanes = 4;
+    static constexpr bool kUnsigned = false, kSums = false;
+    static __device__ __forceinline__ uint2 codes(const Raw& v, int g) {   // less 32
+        const uint2 c = I6K::codes(v, g);
+        auto less32 = [](uint32_t q) {
+            const uint32_t t = q ^ 0x20202020u, neg = t & 0x20202020u;
+            return t | ((neg << 3) - (neg << 1));
+        };
+        return make_uint2(less32(c.x), less32(c.y));
+    }
+};
+struct W80 : I80 {
+    static constexpr int kPlanes = 4;
 };
 
 template <class F>
@@ -307,8 +328,8 @@ __device__ __forceinline__ void int_tile(const GroupedParams& p, const Tile& t, 
                         const float4 ks = *reinterpret_cast<const float4*>(sb + 4 * m * GR + 2 * g);
                         const float f0 = join(__builtin_amdgcn_mfma_i32_16x16x32_i8(a, b[0], int4v{0, 0, 0, 0}, 0, 0, 0)) * ks.x;
                         const float f1 = join(__builtin_amdgcn_mfma_i32_16x16x32_i8(a, b[1], int4v{0, 0, 0, 0}, 0, 0, 0)) * ks.z;
-                        odd0[m] += sc[0] * (f0 - 32.0f * ks.y);
-                        odd1[m] += sc[1] * (f1 - 32.0f * ks.w);
+                        odd0[m] += sc[0] * (F::kSums ? f0 - 32.0f * ks.y : f0);
+                        odd1[m] += sc[1] * (F::kSums ? f1 - 32.0f * ks.w : f1);
                         pin(odd0[m]);
                         pin(odd1[m]);
                     }
@@ -461,10 +482,10 @@ template <bool DOWN>
 void int_any(hipStream_t s, int dt, const GroupedParams& p) {
     auto go = [&](auto f) { int_gemm<decltype(f), DOWN>(s, p); };
     switch (dt) {
-        case INFR_Q4K: go(I4K{}); break;
+        case INFR_Q4K: p.K > 4096 ? go(W4K{}) : go(I4K{}); break;
         case INFR_Q5K: go(I5K{}); break;
-        case INFR_Q6K: go(I6K{}); break;
-        case INFR_Q8_0: go(I80{}); break;
+        case INFR_Q6K: p.K > 4096 ? go(W6K{}) : go(I6K{}); break;
+        case INFR_Q8_0: p.K > 2048 ? go(W80{}) : go(I80{}); break;
         case INFR_Q4_0: go(I40{}); break;
         case INFR_MXFP4: go(IMX{}); break;
         case INFR_IQ4_XS: go(IIX{}); break;

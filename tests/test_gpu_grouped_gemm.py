@@ -203,32 +203,36 @@ def _small_first_weight(w, dtype, gain_rows=None):
     return b.reshape(-1)
 
 
-@pytest.mark.parametrize("dt,ne,nff,rows", [
-    (H.Q5K, 1280, 768, 1), (H.Q5K, 1280, 768, 20), (H.Q4_0, 1088, 320, 1), (H.Q4_0, 1088, 320, 20), (H.IQ4_XS, 1280, 768, 1),
-    (H.IQ4_XS, 1280, 768, 20),
+@pytest.mark.parametrize("dt,ne,nff,rows,where", [
+    (H.Q5K, 1280, 768, 1, "xh"), (H.Q5K, 1280, 768, 20, "xh"), (H.Q4_0, 1088, 320, 1, "xh"), (H.Q4_0, 1088, 320, 20, "xh"),
+    (H.IQ4_XS, 1280, 768, 1, "xh"), (H.IQ4_XS, 1280, 768, 20, "xh"), (H.MXFP4, 1088, 320, 1, "xh"), (H.MXFP4, 1088, 352, 20, "xh"),
+    # rows too wide for a wavefront of the per-token kernels (h: as down banks behind Q4_0 ones)
+    (H.Q8_0, 2080, 320, 20, "x"), (H.Q8_0, 320, 2304, 20, "h"), (H.Q4K, 4352, 256, 20, "x"), (H.Q4K, 256, 4352, 20, "h"),
+    (H.Q6K, 4352, 256, 20, "x"), (H.Q6K, 256, 4352, 20, "h"),
 ])
-def test_small_activations_beside_outliers_keep_their_bits(be, dt, ne, nff, rows):
-    """One element of 32 is some 256 times the others, in x and (through sixteen-fold gate and up rows) in the activated row, and
+def test_small_activations_beside_outliers_keep_their_bits(be, dt, ne, nff, rows, where):
+    """One element of 32 is some 256 times the others, in x and / or (through sixteen-fold gate and up rows) in the activated row, and
     meets a weight of zero.  An f32 sum then loses nothing; fixed point of 24 bits relative to the group's largest is off by up
     to 256 * 2^-24 = 1.5e-5 of the other elements (and of the result: 1.2e-5 to 3.3e-5).  The bar is what f32 arithmetic
     allows: 2^-24 for each of the some eight roundings of a sum's tree, twice (gate/up, down): 1e-6."""
     rng = np.random.default_rng(dt * 47 + ne + rows)
-    E = 1 if rows == 1 else 3
+    E, gdt = 1 if rows == 1 else 3, H.Q4_0 if where == "h" else dt
     x = rng.standard_normal((rows, ne)).astype(np.float32)
-    x[:, ::32] *= 256
+    if "x" in where:
+        x[:, ::32] *= 256
     router = np.zeros((E, ne), np.float32)
-    gain = np.arange(E * nff) % 32 == 0
-    raw = _bank_weights(rng, E, nff, ne, dt, dt)
-    gate, up, down = _small_first_weight(raw[0], dt, gain), _small_first_weight(raw[1], dt, gain), _small_first_weight(raw[2], dt)
+    gain = (np.arange(E * nff) % 32 == 0) & ("h" in where)
+    raw = _bank_weights(rng, E, nff, ne, gdt, dt)
+    gate, up, down = _small_first_weight(raw[0], gdt, gain), _small_first_weight(raw[1], gdt, gain), _small_first_weight(raw[2], dt)
     sel = rng.integers(0, E, (rows, 1)).astype(np.int32)
-    g, ids = moe_graph(rows, ne, E, 1, nff, DType(dt), DType(dt), with_expert_ids=True)
+    g, ids = moe_graph(rows, ne, E, 1, nff, DType(gdt), DType(dt), with_expert_ids=True)
     be.prof_enable(True)
     out, _ = run_moe(be, g, ids, dict(x=x, router=router, gate=gate, up=up, down=down, expert_ids=sel), rows, ne)
     names = set(be.prof_read())
     be.prof_enable(False)
     assert ("moe_down_bucketed" in names) == (rows > 1), names
-    wg, wu, wd = (np.asarray(H.ggml_dequant(dt, w), np.float64).reshape(s)
-                  for w, s in ((gate, (E, nff, ne)), (up, (E, nff, ne)), (down, (E, ne, nff))))
+    wg, wu, wd = (np.asarray(H.ggml_dequant(d, w), np.float64).reshape(s)
+                  for d, w, s in ((gdt, gate, (E, nff, ne)), (gdt, up, (E, nff, ne)), (dt, down, (E, ne, nff))))
     for r in range(rows):
         e = sel[r, 0]
         a, u = wg[e] @ x[r].astype(np.float64), wu[e] @ x[r].astype(np.float64)
