@@ -809,6 +809,23 @@ def test_linear_sweep_over_every_decoded_weight_format(be, m):
             assert H.rel_l2(got, want) < 1e-5, (DType(dt).name, in_f)
 
 
+@pytest.mark.parametrize("m", [1, 3])
+@pytest.mark.parametrize("dt", [H.Q4K, H.Q5K, H.Q6K, H.Q8_0, H.Q4_0, H.IQ4_XS, H.MXFP4])
+def test_linear_on_activations_near_the_smallest_normal_numbers(be, dt, m):
+    """Rows of about 2^-108 are whole multiples of 2^-126 in the fixed-point groups, off by 2^-127 at most: 2^-19 of an element
+    at worst, and as much of the result."""
+    in_f, out_f = 512, 64
+    rng = np.random.default_rng(dt + m)
+    x = (rng.standard_normal((m, in_f)) * 2.0**-108).astype(np.float32)
+    w = H.centred_weight(dt, out_f * in_f, dt)
+    g = M.Graph()
+    tx, tw, ty = g.input(TensorDesc([m, in_f], DType.F32)), g.weight(TensorDesc([out_f, in_f], DType(dt))), g.output(TensorDesc([m, out_f], DType.F32))
+    g.linear(x=tx, weight=tw, dst=ty, m=m, in_f=in_f, out_f=out_f)
+    got = M.run_graph(be, g, [(tx, x), (tw, w)], ty, m * out_f).reshape(m, out_f).astype(np.float64)
+    want = x.astype(np.float64) @ np.asarray(H.ggml_dequant(dt, w), np.float64).reshape(out_f, in_f).T
+    assert np.linalg.norm(got - want) < 2.0**-19 * np.linalg.norm(want)
+
+
 @pytest.mark.parametrize("dt", [H.F32, H.F16, H.BF16])
 @pytest.mark.parametrize("m,in_f,out_f", [(1, 2048, 96), (3, 4096, 37), (6, 264, 8), (1, 100, 5)])
 def test_linear_on_float_weights(be, dt, m, in_f, out_f):
