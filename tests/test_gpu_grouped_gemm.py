@@ -238,3 +238,24 @@ def test_small_activations_beside_outliers_keep_their_bits(be, dt, ne, nff, rows
         a, u = wg[e] @ x[r].astype(np.float64), wu[e] @ x[r].astype(np.float64)
         want = wd[e] @ (a / (1 + np.exp(-a)) * u)
         assert np.linalg.norm(out[r] - want) < 1e-6 * np.linalg.norm(want), r
+
+
+@pytest.mark.parametrize("rows", [1, 3])
+@pytest.mark.parametrize("dt,nff", [(H.MXFP4, 4096), (H.Q4_0, 4096), (H.Q5K, 4096), (H.Q5K, 2560), (H.IQ4_XS, 2816), (H.Q4K, 4096)])
+def test_down_rows_of_eight_ranks_fill_the_lds(be, dt, nff, rows):
+    """The per-token down kernel holds the activated row of every rank: eight of 4096 are 144 KiB (112 with three planes)."""
+    ne, E, K = 256, 9, 8
+    rng = np.random.default_rng(dt * 53 + nff)
+    x = rng.standard_normal((rows, ne)).astype(np.float32)
+    router = (rng.standard_normal((E, ne)) * 0.02).astype(np.float32)
+    gate, up, down = _bank_weights(rng, E, nff, ne, dt, dt)
+    g, ids = moe_graph(rows, ne, E, K, nff, DType(dt), DType(dt))
+    be.prof_enable(True)
+    out, r = run_moe(be, g, ids, dict(x=x, router=router, gate=gate, up=up, down=down), rows, ne)
+    names = set(be.prof_read())
+    be.prof_enable(False)
+    assert not any("bucket" in n for n in names), names
+    ref = O.moe_ffn(x, router, gate, up, down, ne=ne, n_expert=E, n_used=K, n_ff_exp=nff, gate_dtype=dt, down_dtype=dt)
+    assert np.array_equal(r["idx"], ref["idx"])
+    for row in range(rows):
+        assert H.rel_l2(out[row], ref["dst"][row]) < 1e-5, row
