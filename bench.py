@@ -125,10 +125,6 @@ def algorithmic_tables(shape, batch, distinct, prefill):
     }
     # the decode kernel that routes its own token row also reads that row's logits
     alg["moe_route_gate_up"] = alg["moe_gate_up"] + batch * shape.n_expert * 4
-    # banks on the 32-element-unit kernels: per-pair down results, then the rank-ordered sum as its own launch
-    alg["moe_gate_up_units"], alg["moe_route_gate_up_units"] = alg["moe_gate_up"], alg["moe_route_gate_up"]
-    alg["moe_down_units"] = n_sel * down_b + pairs * shape.n_ff * 4 + pairs * shape.ne * 4
-    alg["moe_down_combine_units"] = alg["moe_down_combine"]
     alg["moe_gate_up_bucketed"] = alg["moe_gate_up"]
     if not prefill and batch < 32:
         alg["moe_unbucket_combine"] = pairs * shape.ne * 4 + batch * shape.ne * 4
@@ -150,7 +146,6 @@ def algorithmic_tables(shape, batch, distinct, prefill):
         "moe_grouped_gate_up": 2.0 * pairs * 2 * shape.n_ff * shape.ne,
         "moe_grouped_down": 2.0 * pairs * shape.ne * shape.n_ff,
     }
-    flops["moe_grouped_units_gate_up"], flops["moe_grouped_units_down"] = flops["moe_grouped_gate_up"], flops["moe_grouped_down"]
     return alg, flops
 
 

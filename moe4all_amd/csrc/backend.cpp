@@ -157,7 +157,6 @@ struct MoeScratch {
     bool bucketed = false;   // kBucketedMinRows .. : f32-accurate GEMV per (expert, bucket), weights read once per expert
     int k_parts = 1;          // with bucketed: parts of K the down stage writes its results in
     bool units_batch = false;   // with bucketed: batches of banks in the other affine formats, unit kernels over the buckets
-    bool units_mfma = false;    // with batched: banks other than Q4_K / Q6_K / Q8_0 of whole 256-k steps (the launches' names)
     int32_t* live_ids = nullptr;  // [pairs] ids with the pairs an expert-parallel band dropped set to -1
     int32_t* offsets = nullptr;   // [n_expert + 1]
     int32_t* pair_src = nullptr;  // [rows * n_used]
@@ -186,7 +185,7 @@ struct infr_hip_plan {
     std::vector<MoeScratch> moe;       // per op (valid for MoeFfn ops)
     // Op::Linear with a batch of rows on the matrix cores: the rows are one bucket of the grouped GEMM.
     struct LinearBatch {
-        int mode = 0;                  // 0: GEMV kernels; 1, 2: grouped GEMM (1: Q4_K / Q6_K / Q8_0 of whole 256-k steps)
+        bool on = false;               // the grouped GEMM (else the GEMV kernels)
         size_t offsets_off = 0;        // arena offset of the bucket table {0, m}; the tile table is 256 bytes behind it
     };
     std::vector<LinearBatch> lin;      // per op (valid for Linear ops)
@@ -324,8 +323,11 @@ int moe_logits_once(const infr_hip_backend* be, const infr_op_moe_ffn& m) {
     return 1;   // measured equal or faster on every shape the kernel takes, and the router is read once
 }
 
-// Formats whose launches have no "units" in their names (whichever kernel runs).
 bool k_or_q8(int dt) { return dt == INFR_Q4K || dt == INFR_Q6K || dt == INFR_Q8_0; }
+// The profiler's name of a grouped GEMM on banks of format dt: of its own operands, through the unit decoder, or float weights.
+const char* grouped_name(int dt, const char* own, const char* units, const char* floats) {
+    return dt == INFR_F16 || dt == INFR_BF16 || dt == INFR_F32 ? floats : infr::grouped_reads_units(dt) ? units : own;
+}
 
 // Rates (MB per microsecond) the decode kernels stream expert rows at, measured at 8 to 30 token rows: per pair, where an expert
 // read twice may still be in a cache (fast: the integer-dot kernels take the rows, else the unit kernels), and over buckets.
@@ -358,12 +360,12 @@ void moe_per_token(infr_hip_backend* be, hipStream_t s, infr::MoeGemvParams& gp,
     infr_hip_backend* tb = timed ? be : nullptr;
     // Every block of the gate/up kernel routes its own token row: two of its waves do, while the others turn the row
     // into fixed-point cells, which measured 1 to 3 % faster than a launch of the routing kernel at every batch of the
-    // per-token path.  The unit-format kernel routes on its only four waves and keeps the older rule.
+    // per-token path (8 rows, three layers of 128 experts of 2048 x 768: Q4_0 169 against 177 us, Q5_K 182 against 190).  The kernel of
+    // the other formats routes on its only four waves, while nothing else moves: few rows of few experts only.
     const bool fast_gu = infr::moe_gate_up_routes_inline(gp);
-    const bool units_gu = !fast_gu && !gp.sh_gate && infr::moe_gate_up_units_supported(gp);
-    const bool units = units_gu || !k_or_q8(gp.gate_dt);   // the launch's name
-    gp.route_inline = ((fast_gu && !units) || ((fast_gu || (units_gu && infr::moe_gate_up_units_routes_inline(gp))) &&
-                                   (rows == 1 || (uint64_t)rows * n_expert_total <= 512))) ? 1 : 0;
+    const bool units = !fast_gu && !gp.sh_gate && infr::moe_gate_up_units_supported(gp);
+    gp.route_inline = fast_gu || (units && infr::moe_gate_up_units_routes_inline(gp) &&
+                                  (rows == 1 || (uint64_t)rows * n_expert_total <= 512)) ? 1 : 0;
     if (!gp.route_inline) {
         Timed t(tb, "route_topk");
         infr::launch_route(s, rp);
@@ -393,7 +395,7 @@ void moe_per_token(infr_hip_backend* be, hipStream_t s, infr::MoeGemvParams& gp,
                                       nullptr, gp.addend, gp.skip_zero_w);
         return;
     }
-    Timed t(tb, gp.sh_down ? "moe_down_combine_shared" : k_or_q8(gp.down_dt) ? "moe_down_combine" : rows <= 2 ? "moe_down_combine_units" : "moe_down_units");
+    Timed t(tb, gp.sh_down ? "moe_down_combine_shared" : "moe_down_combine");
     infr::launch_moe_down_combine(s, gp);
 }
 
@@ -861,7 +863,6 @@ extern "C" infr_status infr_hip_compile(infr_hip_backend* be, const infr_graph* 
                                         infr::grouped_supported(c.dt(m.gate_exps), (int)m.ne) &&
                                         infr::grouped_supported(c.dt(m.down_exps), (int)m.n_ff_exp);
                 if (units_mfma) batched = true;
-                plan->moe[oi].units_mfma = units_mfma;
                 if (batched) {
                     arena += round_up(((size_t)m.n_expert + 2) * 4, 256) + 4 * round_up(pairs * 4 + 4, 256) +
                              round_up(((size_t)infr::gemm_max_tiles((int)pairs, (int)m.n_expert) + 1) * sizeof(int4), 256);
@@ -960,13 +961,8 @@ extern "C" infr_status infr_hip_compile(infr_hip_backend* be, const infr_graph* 
                     // GEMV kernels, which spread over the output rows, are faster)
                     const uint32_t min_rows = be->cfg.moe_batched_min_rows ? be->cfg.moe_batched_min_rows : kLinearBatchedMinRows;
                     const int dt = c.dt(l.weight);
-                    int mode = 0;
-                    if (l.m >= min_rows && l.m <= (1u << 24)) {
-                        if (infr::grouped_k256_supported(dt, (int)l.in_f)) mode = 1;
-                        else if (infr::grouped_supported(dt, (int)l.in_f)) mode = 2;
-                    }
-                    plan->lin[oi].mode = mode;
-                    if (mode) {
+                    plan->lin[oi].on = l.m >= min_rows && l.m <= (1u << 24) && infr::grouped_supported(dt, (int)l.in_f);
+                    if (plan->lin[oi].on) {
                         plan->lin[oi].offsets_off = arena;
                         arena += 256 + round_up(((size_t)infr::gemm_max_tiles((int)l.m, 1) + 1) * sizeof(int4), 256);
                         const size_t shared = round_up((size_t)l.m * l.in_f * 2, 256) + round_up((size_t)l.m * 4, 256) +
@@ -1119,7 +1115,7 @@ extern "C" infr_status infr_hip_compile(infr_hip_backend* be, const infr_graph* 
             if (plan->fuse[oi].kind != infr_hip_plan::kPlain || plan->ops[oi].kind != INFR_OP_LINEAR) continue;
             const infr_op_linear& l1 = plan->ops[oi].u.linear;
             if (l1.m == 0) continue;
-            if (plan->lin[oi].mode) continue;   // a batch on the matrix cores: the epilogues there take no second operand
+            if (plan->lin[oi].on) continue;   // a batch on the matrix cores: the epilogues there take no second operand
             // Linear, Linear, GatedAct
             if (oi + 2 < g->n_ops && plan->ops[oi + 1].kind == INFR_OP_LINEAR && plan->ops[oi + 2].kind == INFR_OP_GATED_ACT) {
                 const infr_op_linear& l2 = plan->ops[oi + 1].u.linear;
@@ -1357,7 +1353,7 @@ extern "C" infr_status infr_hip_compile(infr_hip_backend* be, const infr_graph* 
     plan->zero_ids = (int32_t*)((char*)plan->arena + zero_off);   // stays zero: the arena is zero-filled and nothing writes here
     if (plan->arena) infr::launch_fill_zero(be->stream, plan->arena, arena);
     for (uint32_t oi = 0; oi < g->n_ops; oi++) {
-        if (plan->ops[oi].kind != INFR_OP_LINEAR || !plan->lin[oi].mode) continue;
+        if (plan->ops[oi].kind != INFR_OP_LINEAR || !plan->lin[oi].on) continue;
         const infr_op_linear& l = plan->ops[oi].u.linear;
         plan->lin_xh = (_Float16*)((char*)plan->arena + shared_off);
         const int n_tiles = ((int)l.m + infr::kGemmTok - 1) / infr::kGemmTok;
@@ -1694,7 +1690,7 @@ extern "C" infr_status infr_hip_execute(infr_hip_backend* be, infr_hip_plan* pla
                     q.weight_before = (int)m.weight_before;
                     q.a_sum = sc.xm; q.pair_row = sc.pair_row; q.tiles = sc.tiles;
                     {
-                        Timed t(be, sc.units_mfma ? "moe_grouped_units_gate_up" : "moe_grouped_gate_up");
+                        Timed t(be, grouped_name(gp.gate_dt, "moe_grouped_gate_up", "moe_grouped_units_gate_up", "moe_grouped_float_gate_up"));
                         infr::launch_grouped_gate_up(s, gp.gate_dt, q);
                     }
                     {
@@ -1706,7 +1702,7 @@ extern "C" infr_status infr_hip_execute(infr_hip_backend* be, infr_hip_plan* pla
                     q.out_f16 = 1;   // y is written and read once: f16 halves that traffic, hs restores the scale
                     q.a_sum = sc.hm;
                     {
-                        Timed t(be, sc.units_mfma ? "moe_grouped_units_down" : "moe_grouped_down");
+                        Timed t(be, grouped_name(gp.down_dt, "moe_grouped_down", "moe_grouped_units_down", "moe_grouped_float_down"));
                         infr::launch_grouped_down(s, gp.down_dt, q);
                     }
                     {
@@ -1784,8 +1780,8 @@ extern "C" infr_status infr_hip_execute(infr_hip_backend* be, infr_hip_plan* pla
                 geometry(plan->tensors[l.weight].dtype, &we, &wb);
                 size_t row_bytes = (size_t)(l.in_f / we) * wb;
                 const uint8_t* w = (const uint8_t*)ptr[l.weight] + (size_t)(l.w_off / l.in_f) * row_bytes;
-                if (plan->lin[oi].mode) {
-                    const int dt = plan->tensors[l.weight].dtype, mode = plan->lin[oi].mode;
+                if (plan->lin[oi].on) {
+                    const int dt = plan->tensors[l.weight].dtype;
                     _Float16* xh = plan->lin_xh;
                     float* xs = (float*)((char*)xh + round_up((size_t)l.m * l.in_f * 2, 256));
                     {
@@ -1801,7 +1797,7 @@ extern "C" infr_status infr_hip_execute(infr_hip_backend* be, infr_hip_plan* pla
                     q.w0 = w; q.w0_stride = 0;
                     q.out = (float*)ptr[l.dst];
                     q.K = (int)l.in_f; q.N = (int)l.out_f; q.n_expert = 1; q.n_used = 1; q.n_pairs = (int)l.m;
-                    Timed t(be, mode == 2 ? "linear_grouped_units" : "linear_grouped");
+                    Timed t(be, grouped_name(dt, "linear_grouped", "linear_grouped_units", "linear_grouped_float"));
                     infr::launch_grouped_down(s, dt, q);
                     break;
                 }

@@ -348,6 +348,13 @@ bool grouped_supported(int dt, int k) {
 }
 bool grouped_k256_supported(int dt, int k) { return k > 0 && k % 256 == 0 && (dt == INFR_Q4K || dt == INFR_Q6K || dt == INFR_Q8_0); }
 
+bool grouped_reads_units(int dt) {
+    switch (dt) {
+        case INFR_Q4K: case INFR_Q5K: case INFR_Q6K: case INFR_Q8_0: case INFR_Q4_0: case INFR_MXFP4: case INFR_IQ4_XS: return false;
+        default: return unit_format_block(dt) != 0;
+    }
+}
+
 template <bool DOWN>
 static void gemm_any(hipStream_t s, int dt, const GroupedParams& p) {
     switch (dt) {

@@ -190,7 +190,8 @@ struct GroupedParams {
 };
 // Formats and contraction lengths the grouped kernels take.
 bool grouped_supported(int dt, int k);
-bool grouped_k256_supported(int dt, int k);   // the formats the decode kernels read too, in whole 256-k steps
+bool grouped_k256_supported(int dt, int k);   // Q4_K, Q6_K and Q8_0 in whole 256-k steps
+bool grouped_reads_units(int dt);             // block formats that the GEMM decodes in 32-element units
 // rows of f32 -> f16 with a per-row power-of-two scale, in the k order weights of `weight_dt` unpack to.
 // Q4_K, Q5_K: also the sums of the f16 values over groups of 32, as f16 pairs high + low, sums[rows][n / 256][2][8] (n / 32 dwords a row).
 void launch_rows_to_f16(hipStream_t s, int weight_dt, const float* src, int rows, int n, void* dst, float* scale, uint32_t* sums);

@@ -19,6 +19,8 @@ pytestmark = pytest.mark.gpu
 GOLD = os.path.join(os.path.dirname(__file__), "golden")
 
 MAX_ABS, REL_L2 = 2e-3, 1e-3
+# formats with integer-dot or converting decode kernels and GEMM operands of their own; the others go through the unit decoder
+OWN_KERNELS = {H.Q4K, H.Q5K, H.Q6K, H.Q8_0, H.Q4_0, H.MXFP4, H.IQ4_XS}
 
 
 def bits(a):
@@ -301,9 +303,10 @@ def test_moe_ffn_with_grid_iquant_experts_matches_oracle(be, gdt, ddt, rows):
     be.sync()
     names = set(be.prof_read())
     be.prof_enable(False)
-    # the 32-element unit decoders, not the element-wise kernels: GEMV forms for decode, matrix cores for the chunk
-    want_names = {"moe_grouped_units_gate_up", "moe_grouped_units_down"} if rows >= 32 else \
-        {"moe_route_gate_up_units", "moe_down_combine_units"} if rows == 1 else {"moe_route_gate_up_units", "moe_down_units"}
+    # the 32-element unit decoders, not the element-wise kernels: GEMV forms for decode, matrix cores for the chunk (IQ4_XS has
+    # kernels of its own)
+    want_names = {"moe_grouped_units_gate_up", "moe_grouped_down" if ddt in OWN_KERNELS else "moe_grouped_units_down"} if rows >= 32 else \
+        {"moe_route_gate_up_units", "moe_down_combine" if ddt in OWN_KERNELS else "moe_down_combine_units" if rows == 1 else "moe_down_units"}
     assert want_names <= names, names
     ref = O.moe_ffn(x, router, gate, up, down, ne=ne, n_expert=E, n_used=K, n_ff_exp=nff, gate_dtype=gdt, down_dtype=ddt)
     assert np.array_equal(r["idx"], ref["idx"])
@@ -877,7 +880,8 @@ def test_linear_with_a_batch_of_rows_runs_on_the_matrix_cores(be, dt, m, in_f, o
     be.prof_enable(False)
     want = O.linear(x, raw, dt, in_f, out_f)
     mfma = in_f % 64 == 0 and m >= 128
-    assert (("linear_grouped" in names or "linear_grouped_units" in names) and "linear" not in names) if mfma else names == {"linear"}
+    grouped = "linear_grouped_float" if dt in (H.F16, H.BF16, H.F32) else "linear_grouped" if dt in OWN_KERNELS else "linear_grouped_units"
+    assert (grouped in names and "linear" not in names) if mfma else names == {"linear"}
     for r in range(m):
         assert H.rel_l2(got[r], want[r]) < (REL_L2_MFMA if mfma else 1e-5), r
 
@@ -913,10 +917,11 @@ def test_batched_linear_reads_a_row_band_of_a_concatenated_weight(be):
     (H.TQ1_0, H.TQ2_0, 50, 256, 256), (H.Q2_0, H.NVFP4, 35, 192, 320), (H.MXFP4, H.IQ4_NL, 40, 480, 96),
     (H.Q4K, H.Q5K, 48, 512, 256), (H.Q8_0, H.Q5K, 40, 512, 256), (H.Q6K, H.Q4_1, 36, 256, 256)])
 def test_moe_ffn_with_experts_in_the_other_affine_formats(be, gdt, ddt, rows, ne, nff):
-    """Expert banks in formats without an integer-dot kernel.  Up to 31 rows: the 32-element-unit GEMV kernels,
-    one block column per (row, rank) pair (f32, bar 1e-3).  From 32 rows: bucketing + the unit-decoder grouped
-    GEMM on the matrix cores (f16 operands, bar 1e-2) when both contraction lengths are whole 64-k slices,
-    otherwise the unit GEMV over the expert buckets (f32).  Same routing everywhere."""
+    """Expert banks with a format other than Q4_K, Q6_K and Q8_0 in them.  Up to 31 rows: the formats' own decode
+    kernels or the 32-element-unit GEMV kernels, one block column per (row, rank) pair (bar 1e-3).  From 32 rows:
+    bucketing + the grouped GEMM on the matrix cores (f16 operands, bar 1e-2), with the formats' own operands or through
+    the unit decoder, when both contraction lengths are whole 64-k slices, otherwise the unit GEMV over the expert
+    buckets (f32).  The launches' names say which kernel ran.  Same routing everywhere."""
     E, K = 8, 3
     rng = np.random.default_rng(gdt * 17 + ddt + rows)
     x = rng.standard_normal((rows, ne)).astype(np.float32)
@@ -942,15 +947,18 @@ def test_moe_ffn_with_experts_in_the_other_affine_formats(be, gdt, ddt, rows, ne
     for r in range(rows):   # per row: a row scaled by 2e4 must not drown the others
         assert H.rel_l2(got[r], wd[r]) < (REL_L2_MFMA if mfma else REL_L2), r
     if mfma:
-        assert {"moe_grouped_units_gate_up", "moe_grouped_units_down", "moe_unbucket_combine"} <= names
+        assert {"moe_grouped_gate_up" if gdt in OWN_KERNELS else "moe_grouped_units_gate_up",
+                "moe_grouped_down" if ddt in OWN_KERNELS else "moe_grouped_units_down", "moe_unbucket_combine"} <= names
         b = be.moe_bucketing(keep[0], 0)
         _check_bucketing(b, want, E)
     elif rows >= 32:   # batches walk the expert buckets on the f32 unit kernels
         assert {"moe_gate_up_units_bucketed", "moe_down_units_bucketed", "moe_unbucket_combine"} <= names
     else:
-        # routing rides in the gate/up kernel while rows * n_expert <= 512 (as on the integer-dot kernels)
-        assert ("moe_route_gate_up_units" if rows * E <= 512 else "moe_gate_up_units") in names
-        assert ("route_topk" in names) == (rows * E > 512) and (("moe_down_combine_units" if rows <= 2 else "moe_down_units") in names or ddt == H.Q6K)
+        # routing rides in the gate/up kernel, in the unit kernel while rows * n_expert <= 512
+        inline = gdt in OWN_KERNELS or rows * E <= 512
+        assert ("moe_route" if inline else "moe") + ("_gate_up" if gdt in OWN_KERNELS else "_gate_up_units") in names
+        assert ("route_topk" in names) == (not inline)
+        assert ("moe_down_combine" if ddt in OWN_KERNELS else "moe_down_combine_units" if rows <= 2 else "moe_down_units") in names
     keep[0].free()
     for buf in keep[2] + [keep[3]]:
         buf.free()
@@ -977,7 +985,7 @@ def test_sparse_batches_of_unit_formats_stay_on_the_per_pair_gemv(be, rows, grou
     be.prof_enable(False)
     want = O.moe_ffn(x, router, gate, up, down, ne=ne, n_expert=E, n_used=K, n_ff_exp=nff, gate_dtype=H.MXFP4, down_dtype=H.IQ4_XS)
     assert np.array_equal(be.moe_routing(keep[0], 0)["idx"], want["idx"])
-    assert ("moe_grouped_units_gate_up" in names) == grouped and ("moe_gate_up_units" in names) == (not grouped)
+    assert ("moe_grouped_gate_up" in names) == grouped and ("moe_route_gate_up" in names) == (not grouped)
     wd = want["dst"].reshape(rows, ne)
     for r in range(rows):
         assert H.rel_l2(got[r], wd[r]) < (REL_L2_MFMA if grouped else REL_L2), r
