@@ -323,7 +323,6 @@ int moe_logits_once(const infr_hip_backend* be, const infr_op_moe_ffn& m) {
     return 1;   // measured equal or faster on every shape the kernel takes, and the router is read once
 }
 
-bool k_or_q8(int dt) { return dt == INFR_Q4K || dt == INFR_Q6K || dt == INFR_Q8_0; }
 // The profiler's name of a grouped GEMM on banks of format dt: of its own operands, through the unit decoder, or float weights.
 const char* grouped_name(int dt, const char* own, const char* units, const char* floats) {
     return dt == INFR_F16 || dt == INFR_BF16 || dt == INFR_F32 ? floats : infr::grouped_reads_units(dt) ? units : own;
@@ -853,10 +852,10 @@ extern "C" infr_status infr_hip_compile(infr_hip_backend* be, const infr_graph* 
                                infr::grouped_k256_supported(c.dt(m.gate_exps), (int)m.ne) &&
                                infr::grouped_k256_supported(c.dt(m.down_exps), (int)m.n_ff_exp);
                 // a bank in one of the other formats: the same path
-                // ... unless the batch selects each expert one and a half times or less: then no bucket fills a corner
-                // of a 128-token tile, and the per-pair unit GEMV, which streams an expert's rows at full width, is
-                // faster (2880 x 2880 MXFP4 banks, 128 experts, top-4: 32 rows 0.66 ms, 64 rows 1.04 ms, against the
-                // 1.2 ms that one tile pass over every expert costs)
+                // ... unless the batch selects each expert one and a half times or less: such batches have always kept f32
+                // accuracy, and the kernels over buckets below, which read an expert once as well, lose little by it
+                // (128 experts of 2880 x 2880, top-4, 32 and 48 rows: Q4_0 299 and 371 us, the GEMM 279 and 337; MXFP4 356
+                // and 438, 268 and 321; 256 experts of 4096 x 1536 with an always-on expert in Q5_K / Q6_K, 32 rows 605 and 574)
                 const bool sparse_batch = 2 * pairs <= 3 * (size_t)n_local && be->cfg.moe_batched_min_rows == 0;
                 const bool units_mfma = !batched && rows >= min_rows && m.n_used <= 64 && !sparse_batch &&
                                         (m.fused_gate_up || c.dt(m.gate_exps) == c.dt(m.up_exps)) &&
@@ -881,9 +880,7 @@ extern "C" infr_status infr_hip_compile(infr_hip_backend* be, const infr_graph* 
                 const double expect_distinct = (double)n_local * (1.0 - std::pow(1.0 - (double)m.n_used / (double)m.n_expert, (double)rows));
                 const double expect_pairs = (double)pairs * (double)n_local / (double)m.n_expert;
                 const bool few_distinct = rows >= kBucketedMinRows && expect_distinct < kBucketedMaxDistinctRatio * expect_pairs;
-                // (a sparse batch of the other formats: the per-pair kernels at any row count, see sparse_batch)
-                const bool pairs_only = rows >= min_rows && !(k_or_q8((int)c.dt(m.gate_exps)) && k_or_q8((int)c.dt(m.down_exps)));
-                if (!batched && rows >= 2 && !pairs_only && m.n_used <= 64 && (m.fused_gate_up || c.dt(m.gate_exps) == c.dt(m.up_exps)) &&
+                if (!batched && rows >= 2 && m.n_used <= 64 && (m.fused_gate_up || c.dt(m.gate_exps) == c.dt(m.up_exps)) &&
                     infr::grouped_int_supported(c.dt(m.gate_exps), (int)m.ne) && infr::grouped_int_supported(c.dt(m.down_exps), (int)m.n_ff_exp)) {
                     infr::MoeGemvParams probe{};
                     probe.gate_dt = probe.up_dt = c.dt(m.gate_exps);
