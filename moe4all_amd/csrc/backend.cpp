@@ -328,12 +328,16 @@ const char* grouped_name(int dt, const char* own, const char* units, const char*
     return dt == INFR_F16 || dt == INFR_BF16 || dt == INFR_F32 ? floats : infr::grouped_reads_units(dt) ? units : own;
 }
 
-// Rates (MB per microsecond) the decode kernels stream expert rows at, measured at 8 to 30 token rows: per pair, where an expert
-// read twice may still be in a cache (fast: the integer-dot kernels take the rows, else the unit kernels), and over buckets.
+// Rates (MB per microsecond) the decode kernels stream expert rows at, measured at 8 to 30 token rows (large experts: what a
+// launch costs beside its stream is in the rule that compares them): per pair, where an expert read twice may still be in a
+// cache (fast: the integer-dot kernels take the rows, else the unit kernels), and over buckets.  Q4_K and Q6_K, 8 rows, top-8:
+// 64 experts of 4096 x 1536 6.2 and 5.1 per pair, 4.2 and 3.8 over buckets; of 4096 x 3072 6.5 and 5.2, 4.6 and 4.0.
 double token_rate(int dt, bool fast) {
     if (!fast) return dt == INFR_MXFP4 ? 3.0 : 2.6;
     switch (dt) {
-        case INFR_Q4K: case INFR_Q5K: return 5.2;
+        case INFR_Q4K: return 6.2;
+        case INFR_Q5K: return 5.2;
+        case INFR_Q6K: return 5.0;
         case INFR_MXFP4: return 3.7;
         case INFR_IQ4_XS: return 4.1;
         case INFR_Q8_0: return 4.7;
@@ -342,7 +346,8 @@ double token_rate(int dt, bool fast) {
 }
 double bucket_rate(int dt) {
     switch (dt) {
-        case INFR_Q4K: case INFR_Q5K: return 3.8;
+        case INFR_Q4K: return 4.4;
+        case INFR_Q5K: case INFR_Q6K: return 3.8;
         case INFR_MXFP4: return 2.9;
         case INFR_IQ4_XS: return 3.1;
         case INFR_Q8_0: return 4.5;
@@ -873,10 +878,10 @@ extern "C" infr_status infr_hip_compile(infr_hip_backend* be, const infr_graph* 
                 bool bucketed = false;
                 // Bucketing reads an expert's rows once for its tokens: with uniform routing
                 // E * (1 - (1 - K/E)^rows) experts are expected where the per-token kernels read rows * K.  It pays when the bytes
-                // saved take longer than its three more small launches (about 20 us; with an always-on expert behind the op, which
+                // saved take longer than its three more small launches (about 20 us; with an always-on expert behind the op that
                 // the per-token kernels take along, 60): 128 experts of 2048 x 768 in Q8_0, top-8, from 11 rows on, in Q4_K 18; 8
-                // experts of 4096 x 14336, top-2, from 2 (rows too wide for the per-token kernels).  From 16 rows on also where
-                // the share of distinct experts alone is low.
+                // experts of 4096 x 14336, top-2, Q4_K / Q6_K, from 3 (down rows too wide for the per-token kernels).  From 16 rows on
+                // also where the share of distinct experts alone is low.
                 const double expect_distinct = (double)n_local * (1.0 - std::pow(1.0 - (double)m.n_used / (double)m.n_expert, (double)rows));
                 const double expect_pairs = (double)pairs * (double)n_local / (double)m.n_expert;
                 const bool few_distinct = rows >= kBucketedMinRows && expect_distinct < kBucketedMaxDistinctRatio * expect_pairs;
@@ -892,11 +897,16 @@ extern "C" infr_status infr_hip_compile(infr_hip_backend* be, const infr_graph* 
                     geometry(c.dt(m.gate_exps), &ge, &gb);
                     geometry(c.dt(m.down_exps), &de, &db);
                     const double gate_mb = 2e-6 * (double)m.n_ff_exp * (double)(m.ne / ge * gb), down_mb = 1e-6 * (double)m.ne * (double)(m.n_ff_exp / de * db);
-                    bool dense_neighbour = false;   // a Linear on the same rows: an always-on expert's
-                    for (uint32_t oj = 0; oj < g->n_ops; oj++)
-                        if (g->ops[oj].kind == INFR_OP_LINEAR && g->ops[oj].u.linear.x == m.x) dense_neighbour = true;
-                    const double token_us = expect_pairs * (gate_mb / token_rate((int)c.dt(m.gate_exps), infr::moe_gate_up_routes_inline(probe)) +
-                                                            down_mb / token_rate((int)c.dt(m.down_exps), infr::moe_down_is_fast(probe)));
+                    const bool fast_gu = infr::moe_gate_up_routes_inline(probe), fast_down = infr::moe_down_is_fast(probe);
+                    bool dense_neighbour = false;   // an always-on expert that the per-token kernels take as one more slot
+                    for (uint32_t oj = 0; oj < g->n_ops && fast_gu && fast_down; oj++) {
+                        const infr_op_linear& l = g->ops[oj].u.linear;
+                        if (g->ops[oj].kind == INFR_OP_LINEAR && l.x == m.x && l.in_f == m.ne && l.out_f == m.n_ff_exp &&
+                            l.weight < g->n_tensors && c.dt(l.weight) == c.dt(m.gate_exps))
+                            dense_neighbour = true;
+                    }
+                    const double token_us = expect_pairs * (gate_mb / token_rate((int)c.dt(m.gate_exps), fast_gu) +
+                                                            down_mb / token_rate((int)c.dt(m.down_exps), fast_down));
                     const double bucket_us = expect_distinct * (gate_mb / bucket_rate((int)c.dt(m.gate_exps)) + down_mb / bucket_rate((int)c.dt(m.down_exps))) +
                                              (dense_neighbour ? 60.0 : 20.0);
                     bucketed = few_distinct || bucket_us < token_us;

@@ -259,3 +259,28 @@ def test_down_rows_of_eight_ranks_fill_the_lds(be, dt, nff, rows):
     assert np.array_equal(r["idx"], ref["idx"])
     for row in range(rows):
         assert H.rel_l2(out[row], ref["dst"][row]) < 1e-5, row
+
+
+@pytest.mark.parametrize("gdt,ddt,ne,nff,E,rows,beside,bucketed", [
+    (H.Q4K, H.Q6K, 4096, 1536, 64, 8, None, False), (H.Q4K, H.Q6K, 4096, 3072, 64, 8, None, True),
+    # a Linear of one output on the same rows is no always-on expert; neither is one that the per-token kernels cannot take along
+    (H.Q8_0, H.Q8_0, 2048, 768, 128, 14, None, True), (H.Q8_0, H.Q8_0, 2048, 768, 128, 14, 1, True),
+    (H.Q8_0, H.Q8_0, 2048, 768, 128, 14, 768, False), (H.Q8_0, H.Q8_0, 4096, 1536, 64, 2, 1536, True),
+])
+def test_which_decode_batches_go_over_buckets(be, gdt, ddt, ne, nff, E, rows, beside, bucketed):
+    """The plan's choice alone (nothing is allocated for the weights): by the time of the bytes on either side, and 20 or, where
+    an always-on expert leaves the per-token kernels for launches of its own, 60 us."""
+    g, ids = moe_graph(rows, ne, E, 8, nff, DType(gdt), DType(ddt))
+    if beside:
+        w = g.weight(M.TensorDesc([beside, ne], DType(gdt)))
+        y = g.output(M.TensorDesc([rows, beside], DType.F32))
+        g.linear(x=ids["x"], weight=w, dst=y, m=rows, in_f=ne, out_f=beside)
+    plan = be.compile(g)
+    try:
+        if bucketed:
+            assert len(be.moe_bucketing(plan, 0)["offsets"]) == E + 1
+        else:
+            with pytest.raises(M.BackendError):
+                be.moe_bucketing(plan, 0)
+    finally:
+        plan.free()
