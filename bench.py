@@ -345,9 +345,11 @@ def measure(be, stack, config, batch, steps, warmup, *, sublayer=False, kernel_t
         "ms_per_step_min": round(min(group_ms), 4), "ms_per_step_max": round(max(group_ms), 4),
         "spread": f"min / max over {groups} groups of {per_group} steps run after the timed region, a sync after each group",
         "higher_is_better": True, "scaling": "weak", "vs_baseline": None,
-        # decode: exact integer dots (v_dot4 on byte planes) on 23-bit fixed-point activations, scales and sums in f32;
-        # batched path: f16 operands on the matrix cores with f32 accumulation
-        "dtype": "f16-mfma/f32-acc" if batch >= 32 else "i8dot-23bit-act/f32-acc", "data": "synthetic",
+        # decode: exact integer dots (v_dot4, or over expert buckets the i8 matrix cores, on byte planes) on 24-bit fixed-point
+        # activations (MXFP4: f32 activations), scales and sums in f32; batched path: f16 operands on the matrix cores with
+        # f32 accumulation
+        "dtype": "f16-mfma/f32-acc" if batch >= 32 else "f32" if shape.gate_dtype == M.DType.Mxfp4 else "i8dot-24bit-act/f32-acc",
+        "data": "synthetic",
         "config": {"workload": (shape.name if n_layer == shape.n_layer else f"{shape.name}[{n_layer} layers]") +
                                ("+rmsnorm+residual" if sublayer else "") + ("/unfused" if no_fusion else ""),
                    "layers": n_layer, "hidden": shape.ne, "experts": shape.n_expert, "top_k": shape.n_used,

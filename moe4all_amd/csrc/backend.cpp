@@ -81,10 +81,10 @@ constexpr uint64_t kPlanMagic = 0x494e4652504c414eull;     // "INFRPLAN"
 // Token rows from which Op::MoeFfn buckets tokens by expert and runs grouped GEMMs on the matrix
 // cores (f16 operands, f32 accumulation) instead of one GEMV pass per token row.
 constexpr uint32_t kBatchedMinRows = 32;
-// Token rows from which a decode batch is bucketed by expert so that each selected expert's rows are
-// read from HBM once (same f32-accurate inner product as the per-token kernels).
+// A decode batch of that many token rows is bucketed by expert, so that each selected expert's rows are read from HBM once (same
+// f32-accurate inner product as the per-token kernels), where the expected number of distinct experts is below this share of
+// its pairs, and smaller ones and other shares where the bytes say so (see compile).
 constexpr uint32_t kBucketedMinRows = 16;
-// ... and only when the expected number of distinct experts of the batch is below this share of its pairs.
 constexpr double kBucketedMaxDistinctRatio = 0.62;
 // Token rows from which a dense Op::Linear runs as one bucket of the grouped GEMMs.
 constexpr uint32_t kLinearBatchedMinRows = 128;
@@ -154,7 +154,7 @@ struct MoeScratch {
     int rows = 0;
     // batched path (bucketing + grouped GEMMs); the large buffers are shared by all ops of a plan
     bool batched = false;    // >= kBatchedMinRows: grouped GEMMs on the matrix cores
-    bool bucketed = false;   // kBucketedMinRows .. : f32-accurate GEMV per (expert, bucket), weights read once per expert
+    bool bucketed = false;   // below the batched threshold: f32-accurate kernels per (expert, bucket), weights read once per expert
     int k_parts = 1;          // with bucketed: parts of K the down stage writes its results in
     bool units_batch = false;   // with bucketed: batches of banks in the other affine formats, unit kernels over the buckets
     int32_t* live_ids = nullptr;  // [pairs] ids with the pairs an expert-parallel band dropped set to -1
@@ -356,7 +356,8 @@ double bucket_rate(int dt) {
     }
 }
 
-// The per-token path of Op::MoeFfn (1 to 31 token rows; the bucketed path takes batches of 16 or more whose pairs fall on few distinct experts) once logits are in rp.logits and gp / rp are filled in:
+// The per-token path of Op::MoeFfn (batches below the batched threshold that compile does not send over buckets) once logits
+// are in rp.logits and gp / rp are filled in:
 // routing (inside the gate/up kernel where that is cheaper than a launch), gate/up with the gated activation,
 // down with the rank-ordered combine.  timed == false: no profiling events (nothing is created or allocated).
 void moe_per_token(infr_hip_backend* be, hipStream_t s, infr::MoeGemvParams& gp, const infr::RouteParams& rp, int rows,

@@ -1,6 +1,6 @@
 // Shared by the kernels of Op::MoeFfn's batched path (k_grouped.hip: bucketing, conversion, combine; k_grouped_gemm.hip: the
 // GEMMs on block formats; k_grouped_float.hip: float weights): k orders of the f16
-// activations, the units kernel's work item look-up and tile epilogue.
+// activations, the kernels' work item look-ups, the float kernel's tile epilogue.
 #pragma once
 
 #include <type_traits>
@@ -127,18 +127,17 @@ __device__ __forceinline__ bool tile_item(const int4* __restrict__ tiles, int n_
     return true;
 }
 
-// The block's work item: (expert, 128-row tile of its bucket, column tile nt), items ordered by
+// The block's work item of the float kernel: (expert, kBM-row tile of its bucket, column tile nt), items ordered by
 // expert, row tile, column tile.  Workgroups go to the chip's 8 XCDs round-robin by workgroup id
 // and every XCD has its own L2, so each XCD takes a contiguous eighth of the items: the column
 // tiles of one row tile, which read the same activation tile, then sit behind the same L2.
 // Uniform per wave; false when the block has nothing to do (the grid is an upper bound).
-template <int BM = kBM>
 __device__ __forceinline__ bool find_item(const int32_t* __restrict__ offsets, int n_expert, int n_tiles_n, int lane,
                                           Tile& t, int& nt) {
     const int epl = (n_expert + 63) >> 6;
     const int e_lo = lane * epl, e_hi = min(n_expert, e_lo + epl);
     int mine = 0;
-    for (int e = e_lo; e < e_hi; e++) mine += (offsets[e + 1] - offsets[e] + BM - 1) / BM;
+    for (int e = e_lo; e < e_hi; e++) mine += (offsets[e + 1] - offsets[e] + kBM - 1) / kBM;
     int incl = mine;
 #pragma unroll
     for (int d = 1; d < 64; d <<= 1) {
@@ -159,11 +158,11 @@ __device__ __forceinline__ bool find_item(const int32_t* __restrict__ offsets, i
     const int o_lo = owner * epl, o_hi = min(n_expert, o_lo + epl);
     for (int e = o_lo; e < o_hi; e++) {
         const int cnt = offsets[e + 1] - offsets[e];
-        const int ntile = (cnt + BM - 1) / BM;
+        const int ntile = (cnt + kBM - 1) / kBM;
         if (rem < ntile) {
             t.e = e;
-            t.p0 = offsets[e] + rem * BM;
-            t.cnt = min(BM, cnt - rem * BM);
+            t.p0 = offsets[e] + rem * kBM;
+            t.cnt = min(kBM, cnt - rem * kBM);
             return true;
         }
         rem -= ntile;
@@ -173,9 +172,7 @@ __device__ __forceinline__ bool find_item(const int32_t* __restrict__ offsets, i
 
 // Epilogue of a tile whose accumulators are acc0/acc1[M] (column tiles of the wave, M 32-row
 // sub-tiles): SwiGLU of (gate, up) or the scaled down-projection row, stored to p.out.
-// Only the accumulator registers 4 R4LO .. 4 R4HI - 1 of every 32 x 32 tile are stored (all 16 by default): a kernel whose
-// wavefronts share a tile hands each of them a part of its rows.
-template <bool DOWN, int M, int R4LO = 0, int R4HI = 4>
+template <bool DOWN, int M>
 __device__ __forceinline__ void tile_epilogue(const GroupedParams& p, const Tile& t, int n0, int wave, int lane,
                                               const float* s_scale, const float16v (&acc0)[M], const float16v (&acc1)[M]) {
     // accumulator register r of a 32x32 tile: row 8*(r/4) + 4*(lane/32) + r%4, column lane%32.
@@ -188,7 +185,7 @@ __device__ __forceinline__ void tile_epilogue(const GroupedParams& p, const Tile
 #pragma unroll
         for (int mi = 0; mi < M; mi++) {
 #pragma unroll
-            for (int r4 = R4LO; r4 < R4HI; r4++) {
+            for (int r4 = 0; r4 < 4; r4++) {
                 const int m0 = 32 * mi + 8 * r4 + mrow;   // rows m0 .. m0 + 3
                 const float4 sc4 = *reinterpret_cast<const float4*>(s_scale + m0);
                 const float scs[4] = {sc4.x, sc4.y, sc4.z, sc4.w};

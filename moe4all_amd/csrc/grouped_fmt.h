@@ -27,7 +27,7 @@ __device__ __forceinline__ half8 pack8(half2v a, half2v b, half2v c, half2v d) {
 //   Raw: the lane's share of its row for the step (a quarter of every group of 32 k), in registers; St: what is derived
 //   from it once per step; frag(g) = the lane's eight k of group g of the step, in the order of activation chunk
 //   a_lane(kq) | a_group(g) (four groups cover 16 chunks, disjoint bits).
-//   kScale: the sums are kept in units of the block's d; kMin: minimums, see above.
+//   kScale: the sums are kept in units of the block's d; kMin: the format has minimums (St::mins: those of eight groups).
 struct G4K {
     static constexpr int kStep = 256, kChunks = 9;
     static constexpr bool kScale = true, kMin = true, kUnits = false;
@@ -173,8 +173,8 @@ struct G80 {
     }
 };
 
-// (The formats from here on ran in the unit kernel named above GU before: 333 token rows of 128 experts of 2048 x 768 in Q5_K
-// 144 us gate/up, now 70.)
+// (Before they had operands of their own the formats from here on went through the 32-element unit decoder on tiles of 128
+// tokens: 333 token rows of 128 experts of 2048 x 768, gate/up in Q5_K 113 us, 64 here.)
 // Q5_K as Q4_K with a fifth code bit per element (bit g of byte l of the 32 high-bit bytes): scale * code <= 63 * 31 fits a half.
 struct G5K {
     static constexpr int kStep = 256, kChunks = 11;

@@ -18,10 +18,11 @@
 //     256 k), so the sums of a row are always in units of its current d.  Q4_K's minimums are one more matrix
 //     instruction per 256 k, the integer mins against the activations' group sums (f16 pairs high + low).
 // What bounds it: tiles of few tokens the stream of weight rows (64 token rows of a 128-expert layer, 226 MB of Q4_K gate/up
-// and 165 MB of Q6_K down rows: 49 and 41 us; the same launches without unpacking and matrix instructions 46 and 37, a bare
-// read in the same pattern 42 and 34; the kernel before, 128-token tiles on one workgroup per CU, 76 and 69); full tiles
-// the vector instructions (about 1.4 cycles of them per cycle of matrix instructions: 2048 token rows 170 and 112 us, 187
-// and 146 before).  Two workgroups of twice the rows per wave (64 rows, 250 registers) came to 196 and 153 us there, column
+// and 165 MB of Q6_K down rows: 50 and 41 us; the same launches without unpacking and matrix instructions 46 and 37, a bare
+// read in the same pattern 42 and 34; the kernel before, 128-token tiles on one workgroup per CU, 75 and 69); full tiles
+// the vector instructions (about 1.4 cycles of them per cycle of matrix instructions: 2048 token rows of 128 experts of
+// 2048 x 768, Q4_K / Q6_K, 171 and 114 us, the kernel before 187 and 141 in turn on one box; Q8_0 206 and 111, 226 and 138;
+// times of one build differ by some 5 % between boxes).  Two workgroups of twice the rows per wave (64 rows, 250 registers) came to 196 and 153 us there, column
 // tiles in sequence in one workgroup (no start-up between them) to nothing: the stream is continuous anyway.
 // The order of the additions depends on k alone, not on T or on which tile a token is in: a token's result has the same
 // bits wherever it lands.

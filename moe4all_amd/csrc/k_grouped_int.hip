@@ -17,8 +17,8 @@
 //     in registers, through a small LDS region of the wave to a row per lane.  Activations are f32 rows in memory and become
 //     planes here, 256 k at a time into alternating LDS buffers: no launch and no buffer for the conversion.
 // Bound by the stream of weight rows and, with look-up codes (MXFP4, IQ4_XS), by their unpacking: 16 token rows of 128 experts of
-// 2048 x 768 in Q8_0 60 and 33 us (81 distinct experts at 4.5 TB/s; the per-token kernels read 128: 87 and 48); 20 rows of 8
-// experts of 4096 x 14336, Q5_K / Q6_K, 173 and 124 us (the unit kernels 1231 and 551).  Tiles of 16 tokens would need more registers than three workgroups per CU leave
+// 2048 x 768 in Q8_0 60 and 32 us (81 distinct experts at 4.5 TB/s; the per-token kernels read 128: 83 and 45); 20 rows of 8
+// experts of 4096 x 14336, Q5_K / Q6_K, 179 and 123 us (the unit kernels 1240 and 572).  Tiles of 16 tokens would need more registers than three workgroups per CU leave
 // (100 of them spilled) and be bound by the vector instructions.
 #include "grouped_fmt.h"
 #include "gemv_fmt.h"
