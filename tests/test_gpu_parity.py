@@ -1465,7 +1465,8 @@ def test_routing_of_logits_a_few_dozen_ulp_apart_is_the_stable_sort_of_the_proba
 
 
 @pytest.mark.parametrize("rows", [1, 20])
-def test_non_finite_activations_reach_the_output(be, rows):
+@pytest.mark.parametrize("gdt,ddt", [(H.Q4K, H.Q6K), (H.Q5K, H.Q5K), (H.Q8_0, H.Q8_0), (H.Q4_0, H.Q4_0), (H.IQ4_XS, H.IQ4_XS), (H.MXFP4, H.MXFP4)])
+def test_non_finite_activations_reach_the_output(be, gdt, ddt, rows):
     """An f32 dot product over a NaN or an infinity is not finite (the reference's path, crates/infr-cpu/src/moe.rs:142-173);
     the fixed-point staging of the integer-dot kernels must not turn such an activation into zero.  The router reads a
     clean copy of the rows (Op::MoeFfn.router_x), so the routing stays defined and only the expert dots see them."""
@@ -1476,20 +1477,19 @@ def test_non_finite_activations_reach_the_output(be, rows):
     x[0, 37] = np.nan
     x[rows - 1, 300] = np.inf
     router = (rng.standard_normal((E, ne)) * 0.02).astype(np.float32)
-    gate, up = _realistic(rng, E, nff, ne, H.Q4K), _realistic(rng, E, nff, ne, H.Q4K)
-    down = _realistic(rng, E, ne, nff, H.Q6K)
+    gate, up, down = _bank_weights(rng, E, nff, ne, gdt, ddt)
     g = M.Graph()
     tx, trx = g.input(TensorDesc([rows, ne], DType.F32)), g.input(TensorDesc([rows, ne], DType.F32))
     tr = g.weight(TensorDesc([E, ne], DType.F32))
-    tg, tu = g.weight(TensorDesc([E, nff, ne], DType.Q4K)), g.weight(TensorDesc([E, nff, ne], DType.Q4K))
-    td = g.weight(TensorDesc([E, ne, nff], DType.Q6K))
+    tg, tu = g.weight(TensorDesc([E, nff, ne], DType(gdt))), g.weight(TensorDesc([E, nff, ne], DType(gdt)))
+    td = g.weight(TensorDesc([E, ne, nff], DType(ddt)))
     dst = g.output(TensorDesc([rows, ne], DType.F32))
     g.moe_ffn(x=tx, router_x=trx, router=tr, gate_exps=tg, up_exps=tu, down_exps=td, dst=dst, ne=ne, n_expert=E, n_used=K,
               n_ff_exp=nff)
     out = M.run_graph(be, g, [(tx, x), (trx, clean), (tr, router), (tg, gate), (tu, up), (td, down)], dst, rows * ne)
     out = out.reshape(rows, ne)
     with np.errstate(all="ignore"):
-        ref = O.moe_ffn(x, router, gate, up, down, ne=ne, n_expert=E, n_used=K, n_ff_exp=nff, gate_dtype=H.Q4K, down_dtype=H.Q6K,
+        ref = O.moe_ffn(x, router, gate, up, down, ne=ne, n_expert=E, n_used=K, n_ff_exp=nff, gate_dtype=gdt, down_dtype=ddt,
                         router_x=clean)["dst"]
     assert not np.isfinite(ref[0]).any() and not np.isfinite(ref[rows - 1]).any()
     assert not np.isfinite(out[0]).any() and not np.isfinite(out[rows - 1]).any()
