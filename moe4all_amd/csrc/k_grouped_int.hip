@@ -110,15 +110,10 @@ struct I40 : G40 {
     static constexpr bool kUnsigned = false, kNibble = true, kHalves = false, kSums = false;
     static __device__ __forceinline__ uint2 codes(const Raw& v, int g) {
         const uint32_t x = g & 1 ? v.x[g] : __builtin_amdgcn_alignbyte(v.y[g >> 1], v.x[g], 2);
-        return make_uint2(less8(x & kLo4), less8((x >> 4) & kLo4));
-    }
-    // four nibbles less 8, as signed bytes
-    static __device__ __forceinline__ uint32_t less8(uint32_t q) {
-        const uint32_t v = q ^ 0x08080808u, neg = v & 0x08080808u;
-        return v | ((neg << 5) - (neg << 1));
+        return make_uint2(nibbles_less8(x, false), nibbles_less8(x, true));
     }
     static __device__ __forceinline__ PairScale scales(const Raw& v, int j) {
-        return PairScale{f16_bits_to_f32(v.d[2 * j]), f16_bits_to_f32(v.d[2 * j + 1]), 0.0f, 0.0f};
+        return PairScale{0.0625f * f16_bits_to_f32(v.d[2 * j]), 0.0625f * f16_bits_to_f32(v.d[2 * j + 1]), 0.0f, 0.0f};
     }
     static __device__ __forceinline__ float pair(const PairScale& p, float f0, float f1, float, float) { return two_terms(p.s0, f0, p.s1, f1); }
 };
@@ -158,14 +153,11 @@ struct W4K : I4K {
 struct W6K : I6K {
     static constexpr int kPlanes = 4;
     static constexpr bool kUnsigned = false, kSums = false;
-    static __device__ __forceinline__ uint2 codes(const Raw& v, int g) {   // less 32
+    static __device__ __forceinline__ uint2 codes(const Raw& v, int g) {   // less 32, four times
         const uint2 c = I6K::codes(v, g);
-        auto less32 = [](uint32_t q) {
-            const uint32_t t = q ^ 0x20202020u, neg = t & 0x20202020u;
-            return t | ((neg << 3) - (neg << 1));
-        };
-        return make_uint2(less32(c.x), less32(c.y));
+        return make_uint2((c.x << 2) ^ 0x80808080u, (c.y << 2) ^ 0x80808080u);
     }
+    static __device__ __forceinline__ float scale16(const Raw& v, int g, int odd) { return 0.25f * I6K::scale16(v, g, odd); }
 };
 struct W80 : I80 {
     static constexpr int kPlanes = 4;
