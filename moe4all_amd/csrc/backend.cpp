@@ -163,6 +163,7 @@ struct MoeScratch {
     int32_t* slot_pair = nullptr; // [rows * n_used]
     int32_t* pair_row = nullptr;  // [rows * n_used]
     int4* tiles = nullptr;        // tile table of the grouped GEMMs
+    int tile_log2 = 6;            // batched: its tiles hold up to 1 << tile_log2 pairs
     _Float16* xh = nullptr;       // [rows, ne]
     float* xs = nullptr;          // [rows]
     uint32_t* xm = nullptr;       // [rows, ne / 32] group sums of xh (formats with minimums)
@@ -869,8 +870,9 @@ extern "C" infr_status infr_hip_compile(infr_hip_backend* be, const infr_graph* 
                                         infr::grouped_supported(c.dt(m.down_exps), (int)m.n_ff_exp);
                 if (units_mfma) batched = true;
                 if (batched) {
+                    plan->moe[oi].tile_log2 = infr::gemm_tile_log2(c.dt(m.gate_exps), c.dt(m.down_exps), (int)pairs, (int)n_local, (int)m.ne, (int)m.n_ff_exp);
                     arena += round_up(((size_t)m.n_expert + 2) * 4, 256) + 4 * round_up(pairs * 4 + 4, 256) +
-                             round_up(((size_t)infr::gemm_max_tiles((int)pairs, (int)m.n_expert) + 1) * sizeof(int4), 256);
+                             round_up(((size_t)infr::gemm_max_tiles((int)pairs, (int)m.n_expert, 1 << plan->moe[oi].tile_log2) + 1) * sizeof(int4), 256);
                     shared += round_up((size_t)rows * m.ne * 2, 256) + round_up((size_t)rows * 4, 256) +
                               round_up(pairs * m.n_ff_exp * 2, 256) + round_up(pairs * 4, 256) +
                               round_up((size_t)rows * m.ne / 8, 256) + round_up(pairs * m.n_ff_exp / 8, 256) +
@@ -972,7 +974,7 @@ extern "C" infr_status infr_hip_compile(infr_hip_backend* be, const infr_graph* 
                     plan->lin[oi].on = l.m >= min_rows && l.m <= (1u << 24) && infr::grouped_supported(dt, (int)l.in_f);
                     if (plan->lin[oi].on) {
                         plan->lin[oi].offsets_off = arena;
-                        arena += 256 + round_up(((size_t)infr::gemm_max_tiles((int)l.m, 1) + 1) * sizeof(int4), 256);
+                        arena += 256 + round_up(((size_t)infr::gemm_max_tiles((int)l.m, 1, 1 << infr::kLinearTileLog2) + 1) * sizeof(int4), 256);
                         const size_t shared = round_up((size_t)l.m * l.in_f * 2, 256) + round_up((size_t)l.m * 4, 256) +
                                               round_up((size_t)l.m * l.in_f / 8, 256);
                         if (shared > shared_need) shared_need = shared;
@@ -1364,11 +1366,14 @@ extern "C" infr_status infr_hip_compile(infr_hip_backend* be, const infr_graph* 
         if (plan->ops[oi].kind != INFR_OP_LINEAR || !plan->lin[oi].on) continue;
         const infr_op_linear& l = plan->ops[oi].u.linear;
         plan->lin_xh = (_Float16*)((char*)plan->arena + shared_off);
-        const int n_tiles = ((int)l.m + infr::kGemmTok - 1) / infr::kGemmTok;
+        const int tile = 1 << infr::kLinearTileLog2, n_tiles = ((int)l.m + tile - 1) / tile;
         std::vector<int32_t> table(64 + 4 * (1 + (size_t)n_tiles), 0);   // {0, m}, padded to 256 bytes, then the tile table
         table[1] = (int32_t)l.m;
         table[64] = n_tiles;
-        for (int i = 0; i < n_tiles; i++) table[64 + 4 * (1 + i) + 2] = (int32_t)l.m;   // {expert 0, first pair 0, m pairs, first tile 0}
+        for (int i = 0; i < n_tiles; i++) {   // {expert 0, first row, rows, 0}
+            table[64 + 4 * (1 + i) + 1] = i * tile;
+            table[64 + 4 * (1 + i) + 2] = std::min(tile, (int)l.m - i * tile);
+        }
         e = hipMemcpyAsync((char*)plan->arena + plan->lin[oi].offsets_off, table.data(), table.size() * 4, hipMemcpyHostToDevice, be->stream);
         if (e == hipSuccess) e = hipStreamSynchronize(be->stream);   // `table` is on this stack frame
         if (e != hipSuccess)
@@ -1686,7 +1691,7 @@ extern "C" infr_status infr_hip_execute(infr_hip_backend* be, infr_hip_plan* pla
                             bucket_ids = sc.live_ids;
                         }
                         infr::launch_bucket(s, bucket_ids, pairs, (int)n_local, (int)m.n_used, sc.offsets, sc.pair_src, sc.slot_pair,
-                                            sc.pair_row, sc.tiles);
+                                            sc.pair_row, sc.tiles, 1 << sc.tile_log2, 1);
                     }
                     infr::GroupedParams q{};
                     q.loads_only = be->probe_grouped_loads_only.load() ? 1 : 0;
@@ -1696,7 +1701,7 @@ extern "C" infr_status infr_hip_execute(infr_hip_backend* be, infr_hip_plan* pla
                     q.K = (int)m.ne; q.N = (int)m.n_ff_exp; q.n_expert = (int)n_local; q.n_used = (int)m.n_used;
                     q.n_pairs = pairs; q.act = m.act; q.has_clamp = (int)m.has_swiglu_clamp; q.clamp = m.swiglu_clamp;
                     q.weight_before = (int)m.weight_before;
-                    q.a_sum = sc.xm; q.pair_row = sc.pair_row; q.tiles = sc.tiles;
+                    q.a_sum = sc.xm; q.pair_row = sc.pair_row; q.tiles = sc.tiles; q.tile_log2 = sc.tile_log2;
                     {
                         Timed t(be, grouped_name(gp.gate_dt, "moe_grouped_gate_up", "moe_grouped_units_gate_up", "moe_grouped_float_gate_up"));
                         infr::launch_grouped_gate_up(s, gp.gate_dt, q);
@@ -1802,6 +1807,7 @@ extern "C" infr_status infr_hip_execute(infr_hip_backend* be, infr_hip_plan* pla
                     q.a = xh; q.a_scale = xs; q.a_sum = (const uint32_t*)((char*)xs + round_up((size_t)l.m * 4, 256));
                     q.offsets = (const int32_t*)((const char*)plan->arena + plan->lin[oi].offsets_off);
                     q.tiles = (const int4*)(q.offsets + 64);
+                    q.tile_log2 = infr::kLinearTileLog2;
                     q.w0 = w; q.w0_stride = 0;
                     q.out = (float*)ptr[l.dst];
                     q.K = (int)l.in_f; q.N = (int)l.out_f; q.n_expert = 1; q.n_used = 1; q.n_pairs = (int)l.m;

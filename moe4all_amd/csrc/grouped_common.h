@@ -95,7 +95,11 @@ __device__ __forceinline__ float gated_act_fast(int act, bool has_clamp, float c
 // value of the compiler's can be live in it across the statement.  M0 cannot be named as a clobber: the compiler
 // reserves the register and warns that it does not honour such a clobber.
 __device__ __forceinline__ void dma16(const void* gsrc, uint32_t lds_base) {
-    asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" : : "v"(gsrc), "s"(lds_base) : "memory");
+    asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" : : "v"(gsrc), "s"(__builtin_amdgcn_readfirstlane(lds_base)) : "memory");
+}
+// the same from 32-bit offsets behind a uniform address
+__device__ __forceinline__ void dma16(const void* gbase, uint32_t off, uint32_t lds_base) {
+    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" : : "v"(off), "s"(gbase), "s"(__builtin_amdgcn_readfirstlane(lds_base)) : "memory");
 }
 __device__ __forceinline__ uint32_t lds_address(const void* p) {
     return (uint32_t)(uintptr_t)(__attribute__((address_space(3))) const void*)p;
@@ -105,12 +109,11 @@ __device__ __forceinline__ uint32_t lds_address(const void* p) {
 struct Tile {
     int e, p0, cnt;
 };
-// The workgroup's item of the kernels that go by the tile table of launch_bucket: (tile, column tile).  Items are ordered by
+// The workgroup's item of the integer kernels, by the tile table of launch_bucket: (tile, column tile).  Items are ordered by
 // (expert, group of up to kGroupTiles tiles of its bucket, column tile, tile), and each of the 8 XCDs, which workgroups go to
 // round-robin and which have an L2 each, takes a contiguous eighth of them: the tiles of a group run beside each other on
 // the same weights, which then come from memory once per group, while the group's activations stay in the L2 for its
-// columns.  (Column tiles innermost read an expert's weights once per tile: 1500 token rows of 256 experts of
-// 4096 x 1536, gate/up 618 us against 590.)  Uniform; false when there is nothing to do (the grid is an upper bound).
+// columns.  Uniform; false when there is nothing to do (the grid is an upper bound).
 constexpr int kGroupTiles = 4;
 __device__ __forceinline__ bool tile_item(const int4* __restrict__ tiles, int n_cols, uint32_t n_cols_rcp, int tile_pairs, Tile& t, int& col) {
     const int n_items = tiles[0].x * n_cols, per = (n_items + 7) >> 3, k = (int)(blockIdx.x >> 3);

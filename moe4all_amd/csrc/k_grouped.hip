@@ -105,7 +105,7 @@ constexpr int kBucketChunk = 16384;
 __global__ __launch_bounds__(256) void bucket_kernel(const int32_t* __restrict__ ids, int n_pairs, int n_expert,
                                                      int n_used, int32_t* __restrict__ offsets, int32_t* __restrict__ pair_src,
                                                      int32_t* __restrict__ slot_pair, int32_t* __restrict__ pair_row,
-                                                     int4* __restrict__ tiles, int tile) {
+                                                     int4* __restrict__ tiles, int tile, int by_size) {
     __shared__ uint16_t s_ids[kBucketChunk];
     __shared__ uint32_t s_hist[2048];
     __shared__ uint32_t s_cnt[8];
@@ -170,11 +170,13 @@ __global__ __launch_bounds__(256) void bucket_kernel(const int32_t* __restrict__
         }
     }
     __syncthreads();
+    const uint32_t own = e < (uint32_t)n_expert ? s_hist[e] : 0;
+    auto size_class = [](uint32_t pairs) { return pairs <= 16 ? 0 : pairs > 256 ? 5 : 32 - __clz((pairs - 1) >> 4); };
     uint32_t below = 0, tiles_below = 0;
-    for (int i = tid; i < (int)e; i += 256) {
-        const uint32_t c = s_hist[i];
-        below += c;
-        tiles_below += (c + tile - 1) / tile;
+    for (int i = tid; i < n_expert; i += 256) {
+        const uint32_t c = s_hist[i], nt = (c + tile - 1) / tile;
+        if (i < (int)e) below += c;
+        if (by_size && size_class(c) != size_class(own) ? c > own : i < (int)e) tiles_below += nt;
     }
     below = wave_total(below);
     tiles_below = wave_total(tiles_below);
@@ -183,13 +185,14 @@ __global__ __launch_bounds__(256) void bucket_kernel(const int32_t* __restrict__
     below = s_cnt[0] + s_cnt[1] + s_cnt[2] + s_cnt[3];
     tiles_below = s_cnt[4] + s_cnt[5] + s_cnt[6] + s_cnt[7];
     if (tid == 0) offsets[e] = (int32_t)below;
-    if (tiles) {   // slot 0: the number of tiles; then the tiles, experts ascending
+    if (tiles) {   // slot 0: the number of tiles; then the tiles
         if (e == (uint32_t)n_expert) {
             if (tid == 0) tiles[0] = make_int4((int)tiles_below, 0, 0, 0);
         } else {
-            const int cnt = (int)s_hist[e];
+            const int cnt = (int)own;
             for (int i = tid; i * tile < cnt; i += 256)
-                tiles[1 + tiles_below + i] = make_int4((int)e, (int)below, cnt, (int)tiles_below);
+                tiles[1 + tiles_below + i] = by_size ? make_int4((int)e, (int)below + i * tile, min(tile, cnt - i * tile), 0)
+                                                     : make_int4((int)e, (int)below, cnt, (int)tiles_below);
         }
     }
 
@@ -444,9 +447,9 @@ void launch_rows_to_f16(hipStream_t s, int weight_dt, const float* src, int rows
 }
 
 void launch_bucket(hipStream_t s, const int32_t* ids, int n_pairs, int n_expert, int n_used, int32_t* offsets, int32_t* pair_src,
-                   int32_t* slot_pair, int32_t* pair_row, int4* tiles, int tile) {
+                   int32_t* slot_pair, int32_t* pair_row, int4* tiles, int tile, int by_size) {
     INFR_LAUNCH(bucket_kernel, dim3(n_expert + 1), dim3(256), 0, s, ids, n_pairs, n_expert, n_used, offsets, pair_src, slot_pair,
-                pair_row, tiles, tile);
+                pair_row, tiles, tile, by_size);
 }
 
 void launch_unbucket_combine(hipStream_t s, const void* y, const int32_t* slot_pair, const float* weights, int rows,

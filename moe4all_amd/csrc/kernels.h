@@ -181,6 +181,7 @@ struct GroupedParams {
     int n_tiles_n;            // set by the launcher
     uint32_t n_tiles_rcp;     // set by the launcher: ceil(2^32 / n_tiles_n)
     const int4* tiles;        // block formats: the tile table of launch_bucket, up to gemm_max_tiles(n_pairs, n_expert) tiles
+    int tile_log2;            // block formats: the table's tiles hold up to 1 << tile_log2 pairs
     const int32_t* pair_row;  // block formats, gate/up: token row of each pair
     const uint32_t* a_sum;    // formats with minimums: sums of a over groups of 32, see launch_rows_to_f16
     const float* xf;          // integer kernels: [rows, K] (down: [n_pairs, K]) f32, in place of a
@@ -192,6 +193,8 @@ struct GroupedParams {
 bool grouped_supported(int dt, int k);
 bool grouped_k256_supported(int dt, int k);   // Q4_K, Q6_K and Q8_0 in whole 256-k steps
 bool grouped_reads_units(int dt);             // block formats that the GEMM decodes in 32-element units
+// log2 of the pairs of a tile of the table that both GEMMs of a layer go by (6 or 7)
+int gemm_tile_log2(int gate_dt, int down_dt, int n_pairs, int n_expert, int ne, int nff);
 // rows of f32 -> f16 with a per-row power-of-two scale, in the k order weights of `weight_dt` unpack to.
 // Q4_K, Q5_K: also the sums of the f16 values over groups of 32, as f16 pairs high + low, sums[rows][n / 256][2][8] (n / 32 dwords a row).
 void launch_rows_to_f16(hipStream_t s, int weight_dt, const float* src, int rows, int n, void* dst, float* scale, uint32_t* sums);
@@ -203,11 +206,13 @@ void launch_route_rows_to_f16(hipStream_t s, const RouteParams& rp, int weight_d
 void launch_mask_dropped_pairs(hipStream_t s, const int32_t* ids, const float* weights, int n_pairs, int32_t* out);
 // pair_row (or null): token row of the pair at each bucket position.  tiles (or null): the buckets cut into tiles of up to
 // `tile` pairs: slot 0 = {number of tiles}, then per tile {expert, first pair and pairs of its bucket, the bucket's first tile},
-// experts ascending.
-constexpr int kGemmTok = 64, kIntTok = 8;   // pairs of a tile of the grouped GEMM and of the integer kernels
-inline int gemm_max_tiles(int n_pairs, int n_expert, int tile = kGemmTok) { return n_pairs / tile + (n_expert < n_pairs ? n_expert : n_pairs); }
+// experts ascending; by_size: per tile {expert, first pair, pairs of the tile, 0}, experts of more than 256 pairs first, then those of
+// up to 256, 128, 64, 32 and 16, ascending in each class.
+constexpr int kIntTok = 8;   // pairs of a tile of the integer kernels
+constexpr int kLinearTileLog2 = 6;   // tiles of a Linear's rows: 64 (600 rows of 4096 x 1536, three Linears beside a MoeFfn: 965 us, of 128 996)
+inline int gemm_max_tiles(int n_pairs, int n_expert, int tile) { return n_pairs / tile + (n_expert < n_pairs ? n_expert : n_pairs); }
 void launch_bucket(hipStream_t s, const int32_t* ids, int n_pairs, int n_expert, int n_used, int32_t* offsets, int32_t* pair_src,
-                   int32_t* slot_pair, int32_t* pair_row = nullptr, int4* tiles = nullptr, int tile = kGemmTok);
+                   int32_t* slot_pair, int32_t* pair_row = nullptr, int4* tiles = nullptr, int tile = 1, int by_size = 0);
 // The per-expert GEMMs on weights of format dt (block formats: k_grouped_gemm.hip; F16 / BF16 / F32: k_grouped_float.hip).
 // p.a is in the k order launch_rows_to_f16 writes for dt.
 void launch_grouped_gate_up(hipStream_t s, int dt, const GroupedParams& p);

@@ -65,6 +65,42 @@ def test_buckets_at_the_edges_of_the_token_tiles(be, gdt, ddt, ne, nff):
     assert np.array_equal(bits(out2), bits(out[p]))
 
 
+WIDE_COUNTS = [0, 7, 8, 9, 16, 17, 33, 64, 65, 96, 97, 127, 128, 129, 257]
+
+
+@pytest.mark.parametrize("gdt,ddt,ne,nff", [
+    # wide rows, Q8_0, or MXFP4 / Q5_K gate rows take tiles of 128 tokens
+    (H.Q4K, H.Q6K, 4352, 256), (H.Q6K, H.Q4K, 256, 4352), (H.Q5K, H.IQ4_XS, 256, 4352), (H.IQ4_XS, H.Q5K, 4352, 512),
+    (H.Q8_0, H.Q8_0, 448, 192), (H.Q8_0, H.Q8_0, 1024, 384),
+    # rows that end inside a step
+    (H.Q4_0, H.Q4_0, 4416, 192), (H.MXFP4, H.Q4_0, 192, 4160), (H.Q4_0, H.MXFP4, 320, 4288),
+])
+def test_tiles_of_up_to_128_tokens(be, gdt, ddt, ne, nff):
+    """Buckets at the edges of the 8-, 16-, 32-, 64-, 96- and 128-token tiles; the bar is that of the 64-token tiles (f16 operands on
+    both sides), and a row's bits are those it has in a tile of another size."""
+    rng = np.random.default_rng(gdt * 59 + ddt + ne)
+    E, rows = len(WIDE_COUNTS), sum(WIDE_COUNTS)
+    x = rng.standard_normal((rows, ne)).astype(np.float32)
+    router = np.zeros((E, ne), np.float32)
+    gate, up, down = (_zero_some_scales(w, dt, rng) for w, dt in zip(_bank_weights(rng, E, nff, ne, gdt, ddt), (gdt, gdt, ddt)))
+    sel = rng.permutation(np.repeat(np.arange(E), WIDE_COUNTS)).astype(np.int32).reshape(rows, 1)
+    g, ids = moe_graph(rows, ne, E, 1, nff, DType(gdt), DType(ddt), with_expert_ids=True)
+    data = dict(x=x, router=router, gate=gate, up=up, down=down, expert_ids=sel)
+    out, _, b = _run_batched(be, g, ids, data, rows, ne)
+    assert np.array_equal(np.diff(b["offsets"]), WIDE_COUNTS)
+    ref = O.moe_ffn(x, router, gate, up, down, ne=ne, n_expert=E, n_used=1, n_ff_exp=nff, gate_dtype=gdt, down_dtype=ddt,
+                    expert_ids=sel)
+    for e in range(E):
+        m = sel[:, 0] == e
+        if m.any():
+            assert H.rel_l2(out[m], ref["dst"][m]) < REL_L2_MFMA / 4, (e, WIDE_COUNTS[e])
+    # 40 of the rows alone, in tiles of few tokens
+    p = rng.choice(rows, 40, replace=False)
+    g, ids = moe_graph(40, ne, E, 1, nff, DType(gdt), DType(ddt), with_expert_ids=True)
+    out2, _, _ = _run_batched(be, g, ids, dict(data, x=np.ascontiguousarray(x[p]), expert_ids=np.ascontiguousarray(sel[p])), 40, ne)
+    assert np.array_equal(bits(out2), bits(out[p]))
+
+
 INT_COUNTS = [0, 1, 3, 4, 5, 8, 9]   # tiles of up to 4 and up to 8 tokens
 
 
