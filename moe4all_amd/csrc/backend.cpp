@@ -164,6 +164,8 @@ struct MoeScratch {
     int32_t* pair_row = nullptr;  // [rows * n_used]
     int4* tiles = nullptr;        // tile table of the grouped GEMMs
     int tile_log2 = 6;            // batched: its tiles hold up to 1 << tile_log2 pairs
+    bool always_room = false;     // batched: scratch for an always-on expert's rows behind the pairs'
+    float* ysh = nullptr;         // [rows, ne] its results
     _Float16* xh = nullptr;       // [rows, ne]
     float* xs = nullptr;          // [rows]
     uint32_t* xm = nullptr;       // [rows, ne / 32] group sums of xh (formats with minimums)
@@ -871,12 +873,16 @@ extern "C" infr_status infr_hip_compile(infr_hip_backend* be, const infr_graph* 
                 if (units_mfma) batched = true;
                 if (batched) {
                     plan->moe[oi].tile_log2 = infr::gemm_tile_log2(c.dt(m.gate_exps), c.dt(m.down_exps), (int)pairs, (int)n_local, (int)m.ne, (int)m.n_ff_exp);
-                    arena += round_up(((size_t)m.n_expert + 2) * 4, 256) + 4 * round_up(pairs * 4 + 4, 256) +
-                             round_up(((size_t)infr::gemm_max_tiles((int)pairs, (int)m.n_expert, 1 << plan->moe[oi].tile_log2) + 1) * sizeof(int4), 256);
+                    // (an always-on expert behind the op may join its GEMMs: a pair more per row)
+                    const bool room = oi + 1 < g->n_ops && g->ops[oi + 1].kind == INFR_OP_LINEAR && g->ops[oi + 1].u.linear.x == m.x;
+                    plan->moe[oi].always_room = room;
+                    const size_t all = pairs + (room ? rows : 0);
+                    arena += round_up(((size_t)m.n_expert + 2) * 4, 256) + 3 * round_up(pairs * 4 + 4, 256) + round_up(all * 4 + 4, 256) +
+                             round_up(((size_t)infr::gemm_max_tiles((int)all, (int)m.n_expert + 1, 1 << plan->moe[oi].tile_log2) + 1) * sizeof(int4), 256);
                     shared += round_up((size_t)rows * m.ne * 2, 256) + round_up((size_t)rows * 4, 256) +
-                              round_up(pairs * m.n_ff_exp * 2, 256) + round_up(pairs * 4, 256) +
-                              round_up((size_t)rows * m.ne / 8, 256) + round_up(pairs * m.n_ff_exp / 8, 256) +
-                              round_up(pairs * m.ne * 4, 256);
+                              round_up(all * m.n_ff_exp * 2, 256) + round_up(all * 4, 256) +
+                              round_up((size_t)rows * m.ne / 8, 256) + round_up(all * m.n_ff_exp / 8, 256) +
+                              round_up(pairs * m.ne * 4, 256) + (room ? round_up((size_t)rows * m.ne * 4, 256) : 0);
                 }
                 bool bucketed = false;
                 // Bucketing reads an expert's rows once for its tokens: with uniform routing
@@ -1223,6 +1229,41 @@ extern "C" infr_status infr_hip_compile(infr_hip_backend* be, const infr_graph* 
             // (the gate-logit Linear of the gated form is launched by the fused op, ahead of the kernel that reads it)
             for (uint32_t k = oi + 1; k <= b0 + 4; k++) plan->fuse[k].kind = infr_hip_plan::kSkip;
         }
+        // The same pattern on a batch whose Linears would run on the matrix cores too: the always-on expert joins the MoeFfn's two
+        // GEMM launches as one more expert that every row selects (its results stay f32 and are added to the finished sum).
+        // 1500 rows of 256 experts of 4096 x 1536 beside one: the three Linears with their conversions, the activation and the
+        // Add took 143 of 1357 us.
+        for (uint32_t oi = 0; oi + 5 < g->n_ops; oi++) {
+            if (plan->ops[oi].kind != INFR_OP_MOE_FFN || !plan->moe[oi].batched || !plan->moe[oi].always_room) continue;
+            const infr_op_moe_ffn& m = plan->ops[oi].u.moe_ffn;
+            const int rows = plan->moe[oi].rows;
+            static const int32_t kinds[5] = {INFR_OP_LINEAR, INFR_OP_LINEAR, INFR_OP_GATED_ACT, INFR_OP_LINEAR, INFR_OP_ADD};
+            bool fits = !m.has_ep_band && !m.weight_before && infr::gemm_takes_always(c.dt(m.gate_exps)) && infr::gemm_takes_always(c.dt(m.down_exps));
+            for (int k = 0; k < 5; k++) fits = fits && plan->ops[oi + 1 + k].kind == kinds[k] && plan->fuse[oi + 1 + k].kind == infr_hip_plan::kPlain;
+            if (!fits || !plan->lin[oi + 1].on || !plan->lin[oi + 2].on || !plan->lin[oi + 4].on) continue;
+            const infr_op_linear& l1 = plan->ops[oi + 1].u.linear;
+            const infr_op_linear& l2 = plan->ops[oi + 2].u.linear;
+            const infr_op_gated_act& ga = plan->ops[oi + 3].u.gated_act;
+            const infr_op_linear& ld = plan->ops[oi + 4].u.linear;
+            const infr_op_add& ad = plan->ops[oi + 5].u.add;
+            const bool gate_first = ga.gate == l1.dst && ga.up == l2.dst, up_first = ga.gate == l2.dst && ga.up == l1.dst;
+            auto same = [&](const infr_op_linear& l) {
+                return l.x == m.x && (int)l.m == rows && l.in_f == m.ne && l.out_f == m.n_ff_exp && l.w_off == 0 && c.dt(l.weight) == c.dt(m.gate_exps) && temp(l.dst);
+            };
+            if (!(gate_first || up_first) || !same(l1) || !same(l2) || l1.dst == l2.dst) continue;
+            if (!((int)ga.rows == rows && ga.nff == m.n_ff_exp && ga.up_off == 0 && ga.gate_block_width == 0 &&
+                  (ga.up_stride == 0 || ga.up_stride == ga.nff) && (ga.gate_stride == 0 || ga.gate_stride == ga.nff) && temp(ga.dst) &&
+                  ga.act == m.act && ga.has_swiglu_clamp == m.has_swiglu_clamp && (!ga.has_swiglu_clamp || ga.swiglu_clamp == m.swiglu_clamp)))
+                continue;
+            if (!(ld.x == ga.dst && (int)ld.m == rows && ld.in_f == m.n_ff_exp && ld.out_f == m.ne && ld.w_off == 0 &&
+                  c.dt(ld.weight) == c.dt(m.down_exps) && temp(ld.dst)))
+                continue;
+            if (!(((ad.a == m.dst && ad.b == ld.dst) || (ad.b == m.dst && ad.a == ld.dst)) && temp(m.dst) && (uint64_t)ad.n == (uint64_t)rows * m.ne)) continue;
+            plan->fuse[oi].kind = infr_hip_plan::kMoeShared;
+            plan->fuse[oi].a = gate_first ? oi + 1 : oi + 2;   // the gate Linear
+            plan->fuse[oi].b = oi + 4;
+            for (uint32_t k = oi + 1; k <= oi + 5; k++) plan->fuse[k].kind = infr_hip_plan::kSkip;
+        }
         // MoeFfn -> Add (the residual; the reference's moe_add rewrite, crates/infr-core/src/fusion.rs:20-24):
         // every combine kernel ends with "other operand + finished sum", the Add's own rounding.
         // RmsNorm -> MoeFfn on one token row (fusion.rs:15-19 with moe_ok): the logits kernel normalises the
@@ -1341,7 +1382,7 @@ extern "C" infr_status infr_hip_compile(infr_hip_backend* be, const infr_graph* 
             s.pair_src = (int32_t*)p;  p += round_up(pairs * 4 + 4, 256);
             s.slot_pair = (int32_t*)p; p += round_up(pairs * 4 + 4, 256);
             s.live_ids = (int32_t*)p;  p += round_up(pairs * 4 + 4, 256);
-            s.pair_row = (int32_t*)p;  p += round_up(pairs * 4 + 4, 256);
+            s.pair_row = (int32_t*)p;  p += round_up((pairs + (s.always_room ? rows : 0)) * 4 + 4, 256);
             s.tiles = (int4*)p;
         }
         p = (char*)plan->arena + shared_off;
@@ -1350,10 +1391,12 @@ extern "C" infr_status infr_hip_compile(infr_hip_backend* be, const infr_graph* 
             s.xh = (_Float16*)p; p += round_up(rows * m.ne * 2, 256);
             s.xs = (float*)p;    p += round_up(rows * 4, 256);
             s.xm = (uint32_t*)p; p += round_up(rows * m.ne / 8, 256);
-            s.hh = (_Float16*)p; p += round_up(pairs * m.n_ff_exp * 2, 256);
-            s.hs = (float*)p;    p += round_up(pairs * 4, 256);
-            s.hm = (uint32_t*)p; p += round_up(pairs * m.n_ff_exp / 8, 256);
-            s.y = (float*)p;
+            const size_t all = pairs + (s.always_room ? rows : 0);
+            s.hh = (_Float16*)p; p += round_up(all * m.n_ff_exp * 2, 256);
+            s.hs = (float*)p;    p += round_up(all * 4, 256);
+            s.hm = (uint32_t*)p; p += round_up(all * m.n_ff_exp / 8, 256);
+            s.y = (float*)p;     p += round_up(pairs * m.ne * 4, 256);
+            s.ysh = (float*)p;
         } else {
             s.y = (float*)p;
         }
@@ -1576,6 +1619,20 @@ extern "C" infr_status infr_hip_execute(infr_hip_backend* be, infr_hip_plan* pla
                         gp.sh_logit = (const float*)ptr[lq.dst];
                     }
                 }
+                const uint8_t *al_gate = nullptr, *al_up = nullptr, *al_down = nullptr;   // an always-on expert in the batch's GEMMs
+                if (fz.kind == infr_hip_plan::kMoeShared && sc.batched) {
+                    const infr_op_linear& lg = plan->ops[fz.a].u.linear;
+                    const infr_op_linear& lu = plan->ops[fz.a == oi + 1 ? oi + 2 : oi + 1].u.linear;
+                    const infr_op_linear& ld = plan->ops[fz.b].u.linear;
+                    const uint32_t sum_dst = plan->ops[fz.b + 1].u.add.dst;
+                    if (!(need(lg.weight, "Linear.weight") && need(lu.weight, "Linear.weight") && need(ld.weight, "Linear.weight") &&
+                          (fz.res || need(sum_dst, "Add.dst"))))
+                        return INFR_ERR_BACKEND;
+                    al_gate = (const uint8_t*)ptr[lg.weight];
+                    al_up = (const uint8_t*)ptr[lu.weight];
+                    al_down = (const uint8_t*)ptr[ld.weight];
+                    if (!fz.res) gp.dst = (float*)ptr[sum_dst];
+                }
                 auto launch_gate_logit = [&]() {
                     if (!gp.sh_logit) return;
                     const infr_op_linear& lq = plan->ops[oi + 1].u.linear;
@@ -1691,7 +1748,7 @@ extern "C" infr_status infr_hip_execute(infr_hip_backend* be, infr_hip_plan* pla
                             bucket_ids = sc.live_ids;
                         }
                         infr::launch_bucket(s, bucket_ids, pairs, (int)n_local, (int)m.n_used, sc.offsets, sc.pair_src, sc.slot_pair,
-                                            sc.pair_row, sc.tiles, 1 << sc.tile_log2, 1);
+                                            sc.pair_row, sc.tiles, 1 << sc.tile_log2, 1, al_gate ? rows : 0);
                     }
                     infr::GroupedParams q{};
                     q.loads_only = be->probe_grouped_loads_only.load() ? 1 : 0;
@@ -1701,6 +1758,11 @@ extern "C" infr_status infr_hip_execute(infr_hip_backend* be, infr_hip_plan* pla
                     q.K = (int)m.ne; q.N = (int)m.n_ff_exp; q.n_expert = (int)n_local; q.n_used = (int)m.n_used;
                     q.n_pairs = pairs; q.act = m.act; q.has_clamp = (int)m.has_swiglu_clamp; q.clamp = m.swiglu_clamp;
                     q.weight_before = (int)m.weight_before;
+                    q.sh_e = -1;
+                    if (al_gate) {
+                        q.sh_e = (int)n_local; q.sh_p0 = pairs; q.sh0 = al_gate; q.sh1 = al_up; q.sh_out = sc.ysh;
+                        q.n_pairs = pairs + rows; q.n_expert = (int)n_local + 1;
+                    }
                     q.a_sum = sc.xm; q.pair_row = sc.pair_row; q.tiles = sc.tiles; q.tile_log2 = sc.tile_log2;
                     {
                         Timed t(be, grouped_name(gp.gate_dt, "moe_grouped_gate_up", "moe_grouped_units_gate_up", "moe_grouped_float_gate_up"));
@@ -1708,9 +1770,10 @@ extern "C" infr_status infr_hip_execute(infr_hip_backend* be, infr_hip_plan* pla
                     }
                     {
                         Timed t(be, "rows_to_f16");
-                        infr::launch_rows_to_f16(s, gp.down_dt, sc.h, pairs, (int)m.n_ff_exp, sc.hh, sc.hs, sc.hm);
+                        infr::launch_rows_to_f16(s, gp.down_dt, sc.h, q.n_pairs, (int)m.n_ff_exp, sc.hh, sc.hs, sc.hm);
                     }
                     q.a = sc.hh; q.a_scale = sc.hs; q.w0 = gp.down; q.w0_stride = gp.down_stride; q.w1 = nullptr; q.w1_stride = 0;
+                    q.sh0 = al_down; q.sh1 = nullptr;
                     q.down_scale = gp.down_scale; q.out = sc.y; q.K = (int)m.n_ff_exp; q.N = (int)m.ne;
                     q.out_f16 = 1;   // y is written and read once: f16 halves that traffic, hs restores the scale
                     q.a_sum = sc.hm;
@@ -1721,7 +1784,7 @@ extern "C" infr_status infr_hip_execute(infr_hip_backend* be, infr_hip_plan* pla
                     {
                         Timed t(be, "moe_unbucket_combine");
                         infr::launch_unbucket_combine(s, sc.y, sc.slot_pair, sc.weights, rows, (int)m.ne, (int)m.n_used,
-                                                      (int)m.weight_before, gp.dst, 0, sc.hs, gp.addend);
+                                                      (int)m.weight_before, gp.dst, 0, sc.hs, gp.addend, 0, al_gate ? sc.ysh : nullptr);
                     }
                     break;
                 }
@@ -1776,7 +1839,7 @@ extern "C" infr_status infr_hip_execute(infr_hip_backend* be, infr_hip_plan* pla
                     }
                     Timed t(be, "moe_unbucket_combine");
                     infr::launch_unbucket_combine(s, sc.y, sc.slot_pair, sc.weights, rows, (int)m.ne, (int)m.n_used,
-                                                  (int)m.weight_before, gp.dst, 0, nullptr, gp.addend, 0, sc.k_parts, (size_t)pairs * m.ne);
+                                                  (int)m.weight_before, gp.dst, 0, nullptr, gp.addend, 0, nullptr, sc.k_parts, (size_t)pairs * m.ne);
                     break;
                 }
                 gp.route = rp;
@@ -1808,6 +1871,7 @@ extern "C" infr_status infr_hip_execute(infr_hip_backend* be, infr_hip_plan* pla
                     q.offsets = (const int32_t*)((const char*)plan->arena + plan->lin[oi].offsets_off);
                     q.tiles = (const int4*)(q.offsets + 64);
                     q.tile_log2 = infr::kLinearTileLog2;
+                    q.sh_e = -1;
                     q.w0 = w; q.w0_stride = 0;
                     q.out = (float*)ptr[l.dst];
                     q.K = (int)l.in_f; q.N = (int)l.out_f; q.n_expert = 1; q.n_used = 1; q.n_pairs = (int)l.m;

@@ -105,10 +105,10 @@ constexpr int kBucketChunk = 16384;
 __global__ __launch_bounds__(256) void bucket_kernel(const int32_t* __restrict__ ids, int n_pairs, int n_expert,
                                                      int n_used, int32_t* __restrict__ offsets, int32_t* __restrict__ pair_src,
                                                      int32_t* __restrict__ slot_pair, int32_t* __restrict__ pair_row,
-                                                     int4* __restrict__ tiles, int tile, int by_size) {
+                                                     int4* __restrict__ tiles, int tile, int by_size, int always_rows) {
     __shared__ uint16_t s_ids[kBucketChunk];
     __shared__ uint32_t s_hist[2048];
-    __shared__ uint32_t s_cnt[8];
+    __shared__ uint32_t s_cnt[12];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const uint32_t e = blockIdx.x;
     auto narrow = [&](int32_t v) { return (uint32_t)v < (uint32_t)n_expert ? (uint32_t)v : 0xFFFFu; };  // n_expert <= 2048
@@ -170,30 +170,32 @@ __global__ __launch_bounds__(256) void bucket_kernel(const int32_t* __restrict__
         }
     }
     __syncthreads();
-    const uint32_t own = e < (uint32_t)n_expert ? s_hist[e] : 0;
+    const uint32_t own = e < (uint32_t)n_expert ? s_hist[e] : (uint32_t)always_rows;
     auto size_class = [](uint32_t pairs) { return pairs <= 16 ? 0 : pairs > 256 ? 5 : 32 - __clz((pairs - 1) >> 4); };
-    uint32_t below = 0, tiles_below = 0;
-    for (int i = tid; i < n_expert; i += 256) {
-        const uint32_t c = s_hist[i], nt = (c + tile - 1) / tile;
+    uint32_t below = 0, tiles_below = 0, tiles_all = 0;
+    for (int i = tid; i <= n_expert; i += 256) {
+        const uint32_t c = i < n_expert ? s_hist[i] : (uint32_t)always_rows, nt = (c + tile - 1) / tile;
         if (i < (int)e) below += c;
+        tiles_all += nt;
         if (by_size && size_class(c) != size_class(own) ? c > own : i < (int)e) tiles_below += nt;
     }
     below = wave_total(below);
     tiles_below = wave_total(tiles_below);
-    if (lane == 0) { s_cnt[wave] = below; s_cnt[4 + wave] = tiles_below; }
+    tiles_all = wave_total(tiles_all);
+    if (lane == 0) { s_cnt[wave] = below; s_cnt[4 + wave] = tiles_below; s_cnt[8 + wave] = tiles_all; }
     __syncthreads();
     below = s_cnt[0] + s_cnt[1] + s_cnt[2] + s_cnt[3];
     tiles_below = s_cnt[4] + s_cnt[5] + s_cnt[6] + s_cnt[7];
+    tiles_all = s_cnt[8] + s_cnt[9] + s_cnt[10] + s_cnt[11];
     if (tid == 0) offsets[e] = (int32_t)below;
     if (tiles) {   // slot 0: the number of tiles; then the tiles
-        if (e == (uint32_t)n_expert) {
-            if (tid == 0) tiles[0] = make_int4((int)tiles_below, 0, 0, 0);
-        } else {
-            const int cnt = (int)own;
-            for (int i = tid; i * tile < cnt; i += 256)
-                tiles[1 + tiles_below + i] = by_size ? make_int4((int)e, (int)below + i * tile, min(tile, cnt - i * tile), 0)
-                                                     : make_int4((int)e, (int)below, cnt, (int)tiles_below);
-        }
+        if (e == (uint32_t)n_expert && tid == 0) tiles[0] = make_int4((int)tiles_all, 0, 0, 0);
+        const int cnt = (int)own, first = e == (uint32_t)n_expert ? n_pairs : (int)below;
+        for (int i = tid; i * tile < cnt; i += 256)
+            tiles[1 + tiles_below + i] = by_size ? make_int4((int)e, first + i * tile, min(tile, cnt - i * tile), 0)
+                                                 : make_int4((int)e, first, cnt, (int)tiles_below);
+        if (e == (uint32_t)n_expert)
+            for (int i = tid; i < always_rows; i += 256) pair_row[n_pairs + i] = i;
     }
 
     // ---- pass 1: scatter the pairs with id e (the extra block: mark the ids out of range)
@@ -262,7 +264,7 @@ __global__ __launch_bounds__(256) void unbucket_combine_kernel(const Y* __restri
                                                                const float* __restrict__ weights, int ne, int n_used,
                                                                int weight_before, float* dst, int identity,
                                                                const float* __restrict__ pair_scale, const float* addend,
-                                                               int skip_zero_w, int parts, size_t part_stride) {
+                                                               int skip_zero_w, const float* __restrict__ shared, int parts, size_t part_stride) {
     const size_t row = blockIdx.y;
     const int i = (blockIdx.x * 256 + threadIdx.x) * 4;
     if (i >= ne) return;
@@ -299,6 +301,10 @@ __global__ __launch_bounds__(256) void unbucket_combine_kernel(const Y* __restri
         acc.z = __fadd_rn(acc.z, __fmul_rn(w, v[2]));
         acc.w = __fadd_rn(acc.w, __fmul_rn(w, v[3]));
     }
+    if (shared) {   // the always-on expert's row, the Add that closes its ops
+        float* a = &acc.x;
+        for (int q = 0; q < 4 && i + q < ne; q++) a[q] = __fadd_rn(a[q], shared[row * ne + i + q]);
+    }
     float* o = dst + row * ne + i;
     if (addend) {   // a following Op::Add folded in: the finished sum is added to the other operand
         const float* ad = addend + row * ne + i;
@@ -324,7 +330,7 @@ template <int K>
 __global__ __launch_bounds__(256) void unbucket_combine_h8_kernel(const _Float16* __restrict__ y, const int32_t* __restrict__ slot_pair,
                                                                   const float* __restrict__ weights, int ne, int weight_before,
                                                                   float* dst, int identity, const float* __restrict__ pair_scale,
-                                                                  const float* addend, int skip_zero_w) {
+                                                                  const float* addend, int skip_zero_w, const float* __restrict__ shared) {
     const size_t row = blockIdx.y;
     const int i = (blockIdx.x * 256 + threadIdx.x) * 8;
     if (i >= ne) return;
@@ -352,6 +358,12 @@ __global__ __launch_bounds__(256) void unbucket_combine_h8_kernel(const _Float16
             acc[2 * q] = __fadd_rn(acc[2 * q], __fmul_rn(w[k], (float)h[0] * sc[k]));
             acc[2 * q + 1] = __fadd_rn(acc[2 * q + 1], __fmul_rn(w[k], (float)h[1] * sc[k]));
         }
+    }
+    if (shared) {   // the always-on expert's row, the Add that closes its ops
+        const float4 s0 = *reinterpret_cast<const float4*>(shared + row * ne + i), s1 = *reinterpret_cast<const float4*>(shared + row * ne + i + 4);
+        const float sv[8] = {s0.x, s0.y, s0.z, s0.w, s1.x, s1.y, s1.z, s1.w};
+#pragma unroll
+        for (int q = 0; q < 8; q++) acc[q] = __fadd_rn(acc[q], sv[q]);
     }
     float* o = dst + row * ne + i;
     if (addend) {
@@ -447,14 +459,14 @@ void launch_rows_to_f16(hipStream_t s, int weight_dt, const float* src, int rows
 }
 
 void launch_bucket(hipStream_t s, const int32_t* ids, int n_pairs, int n_expert, int n_used, int32_t* offsets, int32_t* pair_src,
-                   int32_t* slot_pair, int32_t* pair_row, int4* tiles, int tile, int by_size) {
+                   int32_t* slot_pair, int32_t* pair_row, int4* tiles, int tile, int by_size, int always_rows) {
     INFR_LAUNCH(bucket_kernel, dim3(n_expert + 1), dim3(256), 0, s, ids, n_pairs, n_expert, n_used, offsets, pair_src, slot_pair,
-                pair_row, tiles, tile, by_size);
+                pair_row, tiles, tile, by_size, always_rows);
 }
 
 void launch_unbucket_combine(hipStream_t s, const void* y, const int32_t* slot_pair, const float* weights, int rows,
                              int ne, int n_used, int weight_before, float* dst, int identity, const float* pair_scale,
-                             const float* addend, int skip_zero_w, int parts, size_t part_stride) {
+                             const float* addend, int skip_zero_w, const float* shared, int parts, size_t part_stride) {
     if (rows <= 0) return;
     const dim3 grid((ne + 1023) / 1024, rows), block(256);
     if (pair_scale && ne % 8 == 0 && (((uintptr_t)y | (uintptr_t)dst | (uintptr_t)addend) & 15) == 0 &&
@@ -462,7 +474,7 @@ void launch_unbucket_combine(hipStream_t s, const void* y, const int32_t* slot_p
         const dim3 g8((ne + 2047) / 2048, rows);
 #define INFR_H8(KK)                                                                                                       \
     INFR_LAUNCH(unbucket_combine_h8_kernel<KK>, g8, block, 0, s, (const _Float16*)y, slot_pair, weights, ne, weight_before, \
-                dst, identity, pair_scale, addend, skip_zero_w)
+                dst, identity, pair_scale, addend, skip_zero_w, shared)
         if (n_used == 8) INFR_H8(8);
         else if (n_used == 6) INFR_H8(6);
         else if (n_used == 4) INFR_H8(4);
@@ -485,10 +497,10 @@ void launch_unbucket_combine(hipStream_t s, const void* y, const int32_t* slot_p
     }
     if (pair_scale)
         INFR_LAUNCH(unbucket_combine_kernel<_Float16>, grid, block, 0, s, (const _Float16*)y, slot_pair, weights, ne, n_used,
-                    weight_before, dst, identity, pair_scale, addend, skip_zero_w, 1, (size_t)0);
+                    weight_before, dst, identity, pair_scale, addend, skip_zero_w, shared, 1, (size_t)0);
     else
         INFR_LAUNCH(unbucket_combine_kernel<float>, grid, block, 0, s, (const float*)y, slot_pair, weights, ne, n_used,
-                    weight_before, dst, identity, pair_scale, addend, skip_zero_w, parts, part_stride);
+                    weight_before, dst, identity, pair_scale, addend, skip_zero_w, shared, parts, part_stride);
 }
 
 }  // namespace infr

@@ -79,8 +79,10 @@ __device__ __forceinline__ void store_tile(const GroupedParams& p, const Tile& t
     float fin[NB];
 #pragma unroll
     for (int n = 0; n < NB; n++) fin[n] = F::kScale ? dcur[n] * kTwo24 : 1.0f;
-    const bool half_out = DOWN && p.out_f16;
-    const float ds = DOWN && p.down_scale ? p.down_scale[t.e] : 1.0f;
+    const bool always = t.e == p.sh_e, half_out = DOWN && p.out_f16 && !always;
+    const float ds = DOWN && p.down_scale && !always ? p.down_scale[t.e] : 1.0f;
+    uint8_t* const out = reinterpret_cast<uint8_t*>(DOWN && always ? p.sh_out : p.out);
+    const int out0 = DOWN && always ? t.p0 - p.sh_p0 : t.p0;
     const int es = half_out ? 2 : 4, vals = 16 / es, fw = n0 + 8 * (DOWN ? 2 : 1) * NB * wave + (lane & 3) * vals;
 #pragma unroll
     for (int m = 0; m < M; m++) {
@@ -116,7 +118,7 @@ __device__ __forceinline__ void store_tile(const GroupedParams& p, const Tile& t
             asm volatile("" ::: "memory");
             const int tok = 16 * m + 4 * ((lane >> 2) & 3) + (lane >> 4), f = fw + 16 * part;
             const uint4v v = *reinterpret_cast<const uint4v*>(wl + 16 * lane);
-            uint8_t* const dst = reinterpret_cast<uint8_t*>(p.out) + ((size_t)(t.p0 + tok) * p.N + f) * es;
+            uint8_t* const dst = out + ((size_t)(out0 + tok) * p.N + f) * es;
             if (tok >= t.cnt) continue;
             if (f + vals <= p.N && p.N % 8 == 0) {
                 *reinterpret_cast<uint4v*>(dst) = v;
@@ -163,7 +165,7 @@ __device__ __forceinline__ void gemm_tile(const GroupedParams& p, const Tile& t,
     if (F::kMin) xsrc = row_of(tid / 2);
     uint32_t srow[2] = {0, 0};
     float row_scale[2] = {1.0f, 1.0f};   // scales of tokens `lane` and 64 + lane
-    if (!DOWN || !p.out_f16) {
+    if (!DOWN || !p.out_f16 || t.e == p.sh_e) {
 #pragma unroll
         for (int j = 0; j < (S::kWide ? 2 : 1); j++) srow[j] = row_of(64 * j + lane);
 #pragma unroll
@@ -174,8 +176,9 @@ __device__ __forceinline__ void gemm_tile(const GroupedParams& p, const Tile& t,
     // ---- weights: the lane's chunks 64 i + lane of the wave's 32 rows x kChunks
     constexpr int kStepBytes = F::kStep / F::kBlock * F::kBlockBytes;
     const uint32_t row_bytes = (uint32_t)(p.K / F::kBlock) * F::kBlockBytes;
-    const uint8_t* const b0 = p.w0 + (size_t)t.e * p.w0_stride;
-    const uint8_t* const b1 = DOWN ? b0 : p.w1 + (size_t)t.e * p.w1_stride;
+    const bool always = t.e == p.sh_e;
+    const uint8_t* const b0 = always ? p.sh0 : p.w0 + (size_t)t.e * p.w0_stride;
+    const uint8_t* const b1 = DOWN ? b0 : always ? p.sh1 : p.w1 + (size_t)t.e * p.w1_stride;
     uint32_t woff[NL];
 #pragma unroll
     for (int i = 0; i < NL; i++) {          // rows beyond the matrix's last one repeat it
@@ -688,6 +691,8 @@ bool grouped_reads_units(int dt) {
         default: return unit_format_block(dt) != 0;
     }
 }
+
+bool gemm_takes_always(int dt) { return unit_format_block(dt) != 0 && !grouped_reads_units(dt); }
 
 // Tiles of 64 pairs on three workgroups per CU, or of 128 on two?  128 tokens share a weight's unpacking, and the kernel of two has
 // the LDS for two steps of weights ahead of a small tile; three hide more of everything else.  us per layer, 64 | 128 (128 experts of

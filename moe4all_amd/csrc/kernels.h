@@ -184,6 +184,9 @@ struct GroupedParams {
     int tile_log2;            // block formats: the table's tiles hold up to 1 << tile_log2 pairs
     const int32_t* pair_row;  // block formats, gate/up: token row of each pair
     const uint32_t* a_sum;    // formats with minimums: sums of a over groups of 32, see launch_rows_to_f16
+    // block formats with an operand of their own: an always-on expert on every token row as expert sh_e of the tile table, pairs
+    // sh_p0 .. (sh_e < 0: none); down: its results f32 to sh_out, without down_scale
+    int sh_e; int sh_p0; const uint8_t* sh0; const uint8_t* sh1; float* sh_out;
     const float* xf;          // integer kernels: [rows, K] (down: [n_pairs, K]) f32, in place of a
     int k_parts;              // integer kernels, down: parts of K asked for, out is [part][n_pairs, N] (0: one)
     int k_part_steps;         // set by the launcher
@@ -193,6 +196,7 @@ struct GroupedParams {
 bool grouped_supported(int dt, int k);
 bool grouped_k256_supported(int dt, int k);   // Q4_K, Q6_K and Q8_0 in whole 256-k steps
 bool grouped_reads_units(int dt);             // block formats that the GEMM decodes in 32-element units
+bool gemm_takes_always(int dt);               // formats whose GEMM takes an always-on expert along
 // log2 of the pairs of a tile of the table that both GEMMs of a layer go by (6 or 7)
 int gemm_tile_log2(int gate_dt, int down_dt, int n_pairs, int n_expert, int ne, int nff);
 // rows of f32 -> f16 with a per-row power-of-two scale, in the k order weights of `weight_dt` unpack to.
@@ -207,12 +211,14 @@ void launch_mask_dropped_pairs(hipStream_t s, const int32_t* ids, const float* w
 // pair_row (or null): token row of the pair at each bucket position.  tiles (or null): the buckets cut into tiles of up to
 // `tile` pairs: slot 0 = {number of tiles}, then per tile {expert, first pair and pairs of its bucket, the bucket's first tile},
 // experts ascending; by_size: per tile {expert, first pair, pairs of the tile, 0}, experts of more than 256 pairs first, then those of
-// up to 256, 128, 64, 32 and 16, ascending in each class.
+// up to 256, 128, 64, 32 and 16, ascending in each class; with always_rows also the tiles of an expert n_expert that has as many
+// pairs n_pairs .., one per token row.
 constexpr int kIntTok = 8;   // pairs of a tile of the integer kernels
 constexpr int kLinearTileLog2 = 6;   // tiles of a Linear's rows: 64 (600 rows of 4096 x 1536, three Linears beside a MoeFfn: 965 us, of 128 996)
 inline int gemm_max_tiles(int n_pairs, int n_expert, int tile) { return n_pairs / tile + (n_expert < n_pairs ? n_expert : n_pairs); }
 void launch_bucket(hipStream_t s, const int32_t* ids, int n_pairs, int n_expert, int n_used, int32_t* offsets, int32_t* pair_src,
-                   int32_t* slot_pair, int32_t* pair_row = nullptr, int4* tiles = nullptr, int tile = 1, int by_size = 0);
+                   int32_t* slot_pair, int32_t* pair_row = nullptr, int4* tiles = nullptr, int tile = 1, int by_size = 0,
+                   int always_rows = 0);
 // The per-expert GEMMs on weights of format dt (block formats: k_grouped_gemm.hip; F16 / BF16 / F32: k_grouped_float.hip).
 // p.a is in the k order launch_rows_to_f16 writes for dt.
 void launch_grouped_gate_up(hipStream_t s, int dt, const GroupedParams& p);
@@ -233,6 +239,7 @@ void launch_unbucket_combine(hipStream_t s, const void* y, const int32_t* slot_p
                              const float* pair_scale = nullptr,   // != null: y is f16, y[pair] * pair_scale[pair]
                              const float* addend = nullptr,       // != null: dst = addend + sum ([rows, ne], may be dst)
                              int skip_zero_w = 0,
+                             const float* shared = nullptr,       // != null: f32 rows added to the sum ([rows, ne]; with pair_scale)
                              int parts = 1, size_t part_stride = 0);   // f32 y: y[pair] = sum of parts, part_stride floats apart
 
 // Dense weights of format dt on several rows of k elements (p.x: p.rows of them; p.gate / p.up / p.down the weights), two rows

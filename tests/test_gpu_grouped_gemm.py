@@ -101,6 +101,72 @@ def test_tiles_of_up_to_128_tokens(be, gdt, ddt, ne, nff):
     assert np.array_equal(bits(out2), bits(out[p]))
 
 
+@pytest.mark.parametrize("gdt,ddt,ne,nff,rows,K,residual,up_first,down_scale", [
+    (H.Q4K, H.Q6K, 512, 256, 130, 2, True, False, False), (H.Q4K, H.Q6K, 512, 256, 300, 8, False, True, True),
+    (H.Q8_0, H.Q8_0, 320, 192, 128, 3, True, True, False), (H.Q5K, H.Q4K, 256, 4352, 333, 1, True, False, True),
+    (H.MXFP4, H.IQ4_XS, 192, 256, 257, 4, False, False, False),
+])
+def test_always_on_expert_in_the_batchs_gemms(be, gdt, ddt, ne, nff, rows, K, residual, up_first, down_scale):
+    """An always-on expert beside a batch's MoeFfn joins its GEMMs: no launch of its own is left, the result is the oracle's, and that
+    of the separate ops up to the activation (both keep it in f32 until its f16 rounding, with an exponential of 1 ulp here;
+    an element in some thousand rounds to the other neighbour, 2^-11 of it)."""
+    rng = np.random.default_rng(gdt * 61 + ddt + rows)
+    E = 9
+    x = rng.standard_normal((rows, ne)).astype(np.float32)
+    router = (rng.standard_normal((E, ne)) * 0.05).astype(np.float32)
+    gate, up, down = (_zero_some_scales(w, dt, rng) for w, dt in zip(_bank_weights(rng, E, nff, ne, gdt, ddt), (gdt, gdt, ddt)))
+    sg, su, sd = _bank_weights(rng, 1, nff, ne, gdt, ddt)
+    ds = (0.5 + rng.random(E)).astype(np.float32) if down_scale else None
+
+    def graph():
+        g = M.Graph()
+        t = lambda kind, shape, dt=DType.F32: getattr(g, kind)(M.TensorDesc(list(shape), dt))  # noqa: E731
+        ids = {k: t("weight", sh, dt) for k, sh, dt in (
+            ("router", (E, ne), DType.F32), ("gate", (E, nff, ne), DType(gdt)), ("up", (E, nff, ne), DType(gdt)),
+            ("down", (E, ne, nff), DType(ddt)), ("sg", (nff, ne), DType(gdt)), ("su", (nff, ne), DType(gdt)), ("sd", (ne, nff), DType(ddt)))}
+        if down_scale:
+            ids["ds"] = t("weight", (E,))
+        ids["x"], ids["y"] = t("input", (rows, ne)), t("output", (rows, ne))
+        moe, tg, tu, ta, ts = (t("internal", (rows, n)) for n in (ne, nff, nff, nff, ne))
+        total = t("internal", (rows, ne)) if residual else ids["y"]
+        g.moe_ffn(x=ids["x"], router=ids["router"], gate_exps=ids["gate"], up_exps=ids["up"], down_exps=ids["down"], dst=moe, ne=ne,
+                  n_expert=E, n_used=K, n_ff_exp=nff, down_scale=ids.get("ds"))
+        for w, dst in [("su", tu), ("sg", tg)] if up_first else [("sg", tg), ("su", tu)]:
+            g.linear(x=ids["x"], weight=ids[w], dst=dst, m=rows, in_f=ne, out_f=nff)
+        g.gated_act(gate=tg, up=tu, dst=ta, rows=rows, nff=nff)
+        g.linear(x=ta, weight=ids["sd"], dst=ts, m=rows, in_f=nff, out_f=ne)
+        g.add(a=ts if residual else moe, b=moe if residual else ts, dst=total, n=rows * ne)
+        if residual:
+            g.add(a=ids["x"], b=total, dst=ids["y"], n=rows * ne)
+        return g, ids
+
+    data = dict(x=x, router=router, gate=gate, up=up, down=down, sg=sg, su=su, sd=sd)
+    if down_scale:
+        data["ds"] = ds
+    outs, names = {}, {}
+    for off in (False, True):
+        b = be if not off else M.Backend(0, disable_op_fusion=True)
+        try:
+            g, ids = graph()
+            b.prof_enable(True)
+            keep = []
+            outs[off] = M.run_graph(b, g, [(ids[k], v) for k, v in data.items()], ids["y"], rows * ne, keep=keep).reshape(rows, ne)
+            names[off] = set(b.prof_read())
+            b.prof_enable(False)
+        finally:
+            if off:
+                b.close()
+    assert not any(n.startswith(("linear", "gated_act", "add")) for n in names[False]), names[False]
+    assert {"linear_grouped", "gated_act", "add"} <= names[True]
+    moe = O.moe_ffn(x, router, gate, up, down, ne=ne, n_expert=E, n_used=K, n_ff_exp=nff, gate_dtype=gdt, down_dtype=ddt, down_scale=ds)["dst"]
+    always = O.linear(O.gated_act_rows(O.linear(x, sg, gdt, ne, nff), O.linear(x, su, gdt, ne, nff)), sd, ddt, nff, ne)
+    want = np.asarray(moe).reshape(rows, ne) + np.asarray(always).reshape(rows, ne)
+    base = x if residual else 0.0
+    assert H.rel_l2(outs[False] - base, want) < REL_L2_MFMA / 4
+    # 2^-11 for one element in 256 of a row's sum: 2^-11 / 16 = 3e-5
+    assert H.rel_l2(outs[False], outs[True]) < 3e-5
+
+
 INT_COUNTS = [0, 1, 3, 4, 5, 8, 9]   # tiles of up to 4 and up to 8 tokens
 
 
