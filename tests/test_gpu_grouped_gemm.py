@@ -386,3 +386,48 @@ def test_which_decode_batches_go_over_buckets(be, gdt, ddt, ne, nff, E, rows, be
                 be.moe_bucketing(plan, 0)
     finally:
         plan.free()
+
+
+@pytest.mark.parametrize("gdt,ddt,ne,nff,rows", [
+    # h rows of 64 to 2048 elements (a wavefront each, one to four chunks per lane) and beyond; group sums behind them (Q4_K, Q5_K down)
+    (H.Q8_0, H.Q8_0, 64, 64, 33), (H.Q8_0, H.Q4K, 256, 512, 34), (H.Q8_0, H.Q5K, 256, 768, 35), (H.Q8_0, H.Q6K, 256, 1280, 33),
+    (H.Q8_0, H.Q4K, 256, 1536, 37), (H.Q8_0, H.Q4_0, 64, 1600, 33), (H.Q8_0, H.Q4K, 256, 2048, 33), (H.Q8_0, H.Q4K, 256, 2304, 33),
+])
+def test_activated_rows_to_f16(be, gdt, ddt, ne, nff, rows):
+    """Rows of h of any length, among them some of zeros and some a million times larger: each has a scale of its own."""
+    rng = np.random.default_rng(ddt * 67 + nff)
+    E = 3
+    x = rng.standard_normal((rows, ne)).astype(np.float32)
+    x[::5] = 0.0
+    x[1::5] *= 1000.0
+    router = np.zeros((E, ne), np.float32)
+    gate, up, down = _bank_weights(rng, E, nff, ne, gdt, ddt)
+    sel = rng.integers(0, E, (rows, 1)).astype(np.int32)
+    g, ids = moe_graph(rows, ne, E, 1, nff, DType(gdt), DType(ddt), with_expert_ids=True)
+    out, _, _ = _run_batched(be, g, ids, dict(x=x, router=router, gate=gate, up=up, down=down, expert_ids=sel), rows, ne)
+    ref = O.moe_ffn(x, router, gate, up, down, ne=ne, n_expert=E, n_used=1, n_ff_exp=nff, gate_dtype=gdt, down_dtype=ddt,
+                    expert_ids=sel)["dst"]
+    for r in range(rows):
+        if r % 5 == 0:
+            assert not out[r].any()
+        else:
+            assert H.rel_l2(out[r], ref[r]) < REL_L2_MFMA, r
+
+
+@pytest.mark.parametrize("rows,K", [(300, 8), (256, 8), (257, 8), (2100, 8), (5000, 4)])
+def test_bucketing_of_many_pairs(be, rows, K):
+    """Up to 2048 pairs on four wavefronts, more on sixteen, more than 16384 in chunks: the reference's order exactly."""
+    ne, nff, E = 64, 64, 61
+    rng = np.random.default_rng(rows + K)
+    sel = np.argsort(rng.random((rows, E)) + 0.6 * np.arange(E) / E, axis=1)[:, :K].astype(np.int32)   # uneven buckets
+    gate, up, down = _bank_weights(rng, E, nff, ne, H.Q8_0, H.Q8_0)
+    g, ids = moe_graph(rows, ne, E, K, nff, DType.Q8_0, DType.Q8_0, with_expert_ids=True)
+    _, _, b = _run_batched(be, g, ids, dict(x=rng.standard_normal((rows, ne)).astype(np.float32), router=np.zeros((E, ne), np.float32),
+                                            gate=gate, up=up, down=down, expert_ids=sel), rows, ne)
+    flat = sel.reshape(-1)
+    order = np.argsort(flat, kind="stable")
+    assert np.array_equal(np.diff(b["offsets"]), np.bincount(flat, minlength=E))
+    assert np.array_equal(b["pair_row"], order // K) and np.array_equal(b["pair_rank"], order % K)
+    slot = np.empty_like(order)
+    slot[order] = np.arange(len(order))
+    assert np.array_equal(b["slot_pair"].reshape(-1), slot)
