@@ -1790,11 +1790,15 @@ extern "C" infr_status infr_hip_execute(infr_hip_backend* be, infr_hip_plan* pla
                 }
                 if (sc.bucketed) {
                     const int pairs = rows * (int)m.n_used;
+                    bool bucketed = false;
                     {
                         Timed t(be, "route_topk");
-                        infr::launch_route(s, rp);
+                        bucketed = !m.has_ep_band &&
+                                   infr::launch_route_bucket(s, rp, sc.offsets, sc.pair_src, sc.slot_pair, sc.units_batch ? nullptr : sc.pair_row,
+                                                             sc.units_batch ? nullptr : sc.tiles);
+                        if (!bucketed) infr::launch_route(s, rp);
                     }
-                    {
+                    if (!bucketed) {
                         Timed t(be, "moe_bucket");
                         const int32_t* bucket_ids = sc.ids;
                         if (m.has_ep_band) {   // pairs of foreign experts (weight 0) are not bucketed at all

@@ -219,6 +219,10 @@ inline int gemm_max_tiles(int n_pairs, int n_expert, int tile) { return n_pairs 
 void launch_bucket(hipStream_t s, const int32_t* ids, int n_pairs, int n_expert, int n_used, int32_t* offsets, int32_t* pair_src,
                    int32_t* slot_pair, int32_t* pair_row = nullptr, int4* tiles = nullptr, int tile = 1, int by_size = 0,
                    int always_rows = 0);
+// launch_route and launch_bucket (tiles of kIntTok pairs, experts ascending) of a few rows in one launch; false, and nothing is
+// launched, where that does not take the shape.  Not for an expert-parallel band, whose dropped pairs have id 0.
+bool launch_route_bucket(hipStream_t s, const RouteParams& rp, int32_t* offsets, int32_t* pair_src, int32_t* slot_pair, int32_t* pair_row,
+                         int4* tiles);
 // The per-expert GEMMs on weights of format dt (block formats: k_grouped_gemm.hip; F16 / BF16 / F32: k_grouped_float.hip).
 // p.a is in the k order launch_rows_to_f16 writes for dt.
 void launch_grouped_gate_up(hipStream_t s, int dt, const GroupedParams& p);

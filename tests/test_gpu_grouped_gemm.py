@@ -431,3 +431,34 @@ def test_bucketing_of_many_pairs(be, rows, K):
     slot = np.empty_like(order)
     slot[order] = np.arange(len(order))
     assert np.array_equal(b["slot_pair"].reshape(-1), slot)
+
+
+@pytest.mark.parametrize("rows,E,K,units", [(16, 8, 2, False), (16, 64, 2, True), (16, 65, 2, True), (16, 9, 3, False), (17, 8, 1, False),
+                                            (16, 1, 1, False), (1, 5, 2, True), (3, 64, 10, True), (3, 64, 11, True), (1, 64, 32, True)])
+def test_routing_and_bucketing_of_a_few_rows(be, rows, E, K, units):
+    """Up to 16 rows, 32 pairs and 64 experts in one launch, more in two: routing and bucket order exactly, with a selection of the
+    router's and with a given one that names experts twice in a row.  (units: the kernels over buckets
+    that take a width of no whole 64, here from any row count.)"""
+    ne, nff = 256, 96 if units else 64
+    rng = np.random.default_rng(100 * rows + E)
+    x = rng.standard_normal((rows, ne)).astype(np.float32)
+    router = (rng.standard_normal((E, ne)) * 0.2).astype(np.float32)
+    gate, up, down = _bank_weights(rng, E, nff, ne, H.Q8_0, H.Q8_0)
+    b2 = M.Backend(0, moe_batched_min_rows=1) if units else be
+    for given in (False, True):
+        sel = rng.integers(0, max(1, E // 2), (rows, K)).astype(np.int32)
+        g, ids = moe_graph(rows, ne, E, K, nff, DType.Q8_0, DType.Q8_0, with_expert_ids=given)
+        out, r, b = _run_batched(b2, g, ids, dict(x=x, router=router, gate=gate, up=up, down=down, **(dict(expert_ids=sel) if given else {})), rows, ne)
+        ref = O.moe_ffn(x, router, gate, up, down, ne=ne, n_expert=E, n_used=K, n_ff_exp=nff, gate_dtype=H.Q8_0, down_dtype=H.Q8_0,
+                        **(dict(expert_ids=sel) if given else {}))
+        idx = np.asarray(r["idx"]).reshape(rows, K)
+        assert np.array_equal(idx, sel if given else ref["idx"]) and np.array_equal(bits(r["w"]), bits(ref["w"]))
+        order = np.argsort(idx.reshape(-1), kind="stable")
+        assert np.array_equal(np.diff(b["offsets"]), np.bincount(idx.reshape(-1), minlength=E))
+        assert np.array_equal(b["pair_row"], order // K) and np.array_equal(b["pair_rank"], order % K)
+        slot = np.empty_like(order)
+        slot[order] = np.arange(len(order))
+        assert np.array_equal(b["slot_pair"].reshape(-1), slot)
+        assert H.rel_l2(out, ref["dst"].reshape(rows, ne)) < 1e-5   # f32 throughout
+    if units:
+        b2.close()
