@@ -568,7 +568,7 @@ void launch_route_rows_to_f16(hipStream_t s, const RouteParams& rp, int weight_d
 void launch_rows_to_f16(hipStream_t s, int weight_dt, const float* src, int rows, int n, void* dst, float* scale, uint32_t* sums) {
     if (rows <= 0) return;
     _Float16* d = reinterpret_cast<_Float16*>(dst);
-    const int nc = (n / 8 + 63) / 64;
+    const int nc = rows < 1024 ? 0 : (n / 8 + 63) / 64;   // few rows: a block each reaches more CUs
     with_order(weight_dt, [&](auto order) {
         typedef decltype(order) F;
         const dim3 quads((rows + 3) / 4);
