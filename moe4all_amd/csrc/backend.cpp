@@ -872,7 +872,7 @@ extern "C" infr_status infr_hip_compile(infr_hip_backend* be, const infr_graph* 
                                         infr::grouped_supported(c.dt(m.down_exps), (int)m.n_ff_exp);
                 if (units_mfma) batched = true;
                 if (batched) {
-                    plan->moe[oi].tile_log2 = infr::gemm_tile_log2(c.dt(m.gate_exps), c.dt(m.down_exps), (int)pairs, (int)n_local, (int)m.ne, (int)m.n_ff_exp);
+                    plan->moe[oi].tile_log2 = infr::gemm_tile_log2(c.dt(m.gate_exps), c.dt(m.down_exps), (int)rows, (int)pairs, (int)n_local, (int)m.ne, (int)m.n_ff_exp);
                     // (an always-on expert behind the op may join its GEMMs: a pair more per row)
                     const bool room = oi + 1 < g->n_ops && g->ops[oi + 1].kind == INFR_OP_LINEAR && g->ops[oi + 1].u.linear.x == m.x;
                     plan->moe[oi].always_room = room;

@@ -703,12 +703,16 @@ bool gemm_takes_always(int dt) { return unit_format_block(dt) != 0 && !grouped_r
 //   Q4_0          512 rows 161 154 | 172 156, 1024 rows 228 232 | 227 228;  IQ4_XS 512 rows 171 169 | 180 166, 1024 rows 244 255 | 231 243
 //   MXFP4          64 rows 109 | 107, 512 rows 148 140 | 157 137, 500 rows of 2880 x 2880, top-4 - 390 | - 365
 //   8 experts of 4096 x 14336, top-2, Q4_K / Q6_K: 40 rows 585 | 498;  32 experts of 1024 x 512, 2000 rows - 155 | - 162
-// So: 128 from 40 pairs per expert on if that leaves three rounds of workgroups, with Q8_0 always, with Q5_K and MXFP4 below 24
-// pairs per expert, and with long rows.
-int gemm_tile_log2(int gate_dt, int down_dt, int n_pairs, int n_expert, int ne, int nff) {
+//   32 experts of 1024 x 512, Q8_0, 110 rows, Zipf(1.1), five layers: 289 | 331
+// So: 128 with long rows, from 40 pairs per expert on if that leaves three rounds of workgroups, with Q8_0, and with Q5_K and MXFP4
+// below 24 pairs per expert.  But launches that do not fill the chip once: 64, so that a large bucket is spread over more
+// workgroups (up to 64 rows both cut alike, and the kernel of two is the faster one).
+int gemm_tile_log2(int gate_dt, int down_dt, int rows, int n_pairs, int n_expert, int ne, int nff) {
     if (grouped_reads_units(gate_dt) || grouped_reads_units(down_dt)) return 6;
     const int mean = n_pairs / n_expert;
-    if (gate_dt == INFR_Q8_0 || ne > 4096 || nff > 4096) return 7;
+    if (ne > 4096 || nff > 4096) return 7;
+    if ((int64_t)gemm_max_tiles(n_pairs, n_expert, 128) * ((nff + 63) / 64) < 512) return rows <= 64 ? 7 : 6;
+    if (gate_dt == INFR_Q8_0) return 7;
     if (mean >= 40) return (int64_t)gemm_max_tiles(n_pairs, n_expert, 128) * ((nff + 63) / 64) >= 3 * 512 ? 7 : 6;
     return (gate_dt == INFR_Q5K || gate_dt == INFR_MXFP4) && mean < 24 ? 7 : 6;
 }

@@ -198,7 +198,7 @@ bool grouped_k256_supported(int dt, int k);   // Q4_K, Q6_K and Q8_0 in whole 25
 bool grouped_reads_units(int dt);             // block formats that the GEMM decodes in 32-element units
 bool gemm_takes_always(int dt);               // formats whose GEMM takes an always-on expert along
 // log2 of the pairs of a tile of the table that both GEMMs of a layer go by (6 or 7)
-int gemm_tile_log2(int gate_dt, int down_dt, int n_pairs, int n_expert, int ne, int nff);
+int gemm_tile_log2(int gate_dt, int down_dt, int rows, int n_pairs, int n_expert, int ne, int nff);
 // rows of f32 -> f16 with a per-row power-of-two scale, in the k order weights of `weight_dt` unpack to.
 // Q4_K, Q5_K: also the sums of the f16 values over groups of 32, as f16 pairs high + low, sums[rows][n / 256][2][8] (n / 32 dwords a row).
 void launch_rows_to_f16(hipStream_t s, int weight_dt, const float* src, int rows, int n, void* dst, float* scale, uint32_t* sums);

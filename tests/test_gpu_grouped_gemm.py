@@ -69,9 +69,9 @@ WIDE_COUNTS = [0, 7, 8, 9, 16, 17, 33, 64, 65, 96, 97, 127, 128, 129, 257]
 
 
 @pytest.mark.parametrize("gdt,ddt,ne,nff", [
-    # wide rows, Q8_0, or MXFP4 / Q5_K gate rows take tiles of 128 tokens
+    # wide rows take tiles of 128 tokens (small launches of others tiles of 64: the same buckets, the other kernel)
     (H.Q4K, H.Q6K, 4352, 256), (H.Q6K, H.Q4K, 256, 4352), (H.Q5K, H.IQ4_XS, 256, 4352), (H.IQ4_XS, H.Q5K, 4352, 512),
-    (H.Q8_0, H.Q8_0, 448, 192), (H.Q8_0, H.Q8_0, 1024, 384),
+    (H.Q8_0, H.Q8_0, 448, 192), (H.Q8_0, H.Q8_0, 1024, 384), (H.Q8_0, H.Q8_0, 4352, 192), (H.Q8_0, H.Q8_0, 448, 4352),
     # rows that end inside a step
     (H.Q4_0, H.Q4_0, 4416, 192), (H.MXFP4, H.Q4_0, 192, 4160), (H.Q4_0, H.MXFP4, 320, 4288),
 ])
