@@ -80,6 +80,12 @@ __device__ __forceinline__ float act_fast(int act, float g) {
     }
     return 1.0f / (1.0f + __expf(-g));
 }
+// silu with the hardware exp2 and reciprocal (1 ulp each).  The product g * log2(e) is rounded, so the exponential is off by up to
+// |g| 2^-24 of itself: 10 ulp at |g| = 20, where the f16 rounding of the result still hides it.  The reciprocal comes first:
+// g * up may overflow where silu(g) is 0 (g < -88), and infinity times 0 is NaN.
+__device__ __forceinline__ float silu_fast(float g) {
+    return g * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(g * -1.4426950408889634f));
+}
 __device__ __forceinline__ float gated_act_fast(int act, bool has_clamp, float clamp, float gate, float up) {
     if (has_clamp) {
         gate = fminf(gate, clamp);
@@ -226,10 +232,9 @@ __device__ __forceinline__ void tile_epilogue(const GroupedParams& p, const Tile
         }
     } else if (fc0 < p.N) {
         if (p.act == INFR_ACT_SILU && !p.has_clamp && !p.weight_before) {
-            // silu(g) * u with the hardware exp2 and reciprocal (1 ulp each; the operands were f16)
             for_each([&](int mi, int r, int, float sc, float* o) {
                 const float g = acc0[mi][r] * sc, u = acc1[mi][r] * sc;
-                o[0] = g * u * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(g * -1.4426950408889634f));
+                o[0] = silu_fast(g) * u;
             });
         } else {
             for_each([&](int mi, int r, int m, float sc, float* o) {

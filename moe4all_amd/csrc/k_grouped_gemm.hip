@@ -102,8 +102,7 @@ __device__ __forceinline__ void store_tile(const GroupedParams& p, const Tile& t
                     const float sc = __shfl(row_scale[m >> 2], tok & 63, 64);
                     float g = acc[0][m][q] * fin[0] * sc, u = acc[1][m][q] * fin[1] * sc;
                     if (p.act == INFR_ACT_SILU && !p.has_clamp && !p.weight_before) {
-                        // silu(g) * u with the hardware exp2 and reciprocal (1 ulp each; the operands were f16)
-                        g = g * u * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(g * -1.4426950408889634f));
+                        g = silu_fast(g) * u;
                     } else {
                         if (p.weight_before) {
                             const float wp = p.route_w[p.pair_src[t.p0 + min(tok, t.cnt - 1)]];

@@ -462,3 +462,26 @@ def test_routing_and_bucketing_of_a_few_rows(be, rows, E, K, units):
         assert H.rel_l2(out, ref["dst"].reshape(rows, ne)) < 1e-5   # f32 throughout
     if units:
         b2.close()
+
+
+@pytest.mark.parametrize("dt", [H.Q8_0, H.F16])
+def test_gate_times_up_beyond_f32_beside_a_closed_gate(be, dt):
+    """silu(g) is 0 for g below -104; that must hold where g * up is beyond f32 too (block formats and the float kernel)."""
+    ne, nff, E, rows = 256, 128, 4, 48
+    rng = np.random.default_rng(dt)
+    x = (np.abs(rng.standard_normal((rows, ne))) * 1e25).astype(np.float32)
+    router = np.zeros((E, ne), np.float32)
+    if dt == H.F16:
+        gate, up, down = ((0.02 * rng.standard_normal(E * nff * ne)).astype(np.float16) for _ in range(3))
+        gate = -np.abs(gate)
+        gate, up, down = gate.view(np.uint8), up.view(np.uint8), down.view(np.uint8)
+    else:
+        gate, up, down = _bank_weights(rng, E, nff, ne, dt, dt)
+        blk = np.ascontiguousarray(gate).reshape(-1, 34)
+        blk[:, 2:] = (-np.abs(blk[:, 2:].view(np.int8).astype(np.int32))).clip(-127, 0).astype(np.int8).view(np.uint8)
+        gate = blk.reshape(-1)
+    sel = rng.integers(0, E, (rows, 1)).astype(np.int32)
+    g, ids = moe_graph(rows, ne, E, 1, nff, DType(dt), DType(dt), with_expert_ids=True)
+    out, _, _ = _run_batched(be, g, ids, dict(x=x, router=router, gate=gate, up=up, down=down, expert_ids=sel), rows, ne)
+    ref = O.moe_ffn(x, router, gate, up, down, ne=ne, n_expert=E, n_used=1, n_ff_exp=nff, gate_dtype=dt, down_dtype=dt, expert_ids=sel)
+    assert not np.asarray(ref["dst"]).any() and not out.any()
