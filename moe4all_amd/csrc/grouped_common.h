@@ -88,8 +88,8 @@ __device__ __forceinline__ float silu_fast(float g) {
 }
 __device__ __forceinline__ float gated_act_fast(int act, bool has_clamp, float clamp, float gate, float up) {
     if (has_clamp) {
-        gate = fminf(gate, clamp);
-        up = fminf(fmaxf(up, -clamp), clamp);
+        gate = gate < clamp ? gate : clamp;
+        up = up < -clamp ? -clamp : up > clamp ? clamp : up;   // (a NaN stays)
     }
     return act_fast(act, gate) * up;
 }

@@ -485,3 +485,29 @@ def test_gate_times_up_beyond_f32_beside_a_closed_gate(be, dt):
     out, _, _ = _run_batched(be, g, ids, dict(x=x, router=router, gate=gate, up=up, down=down, expert_ids=sel), rows, ne)
     ref = O.moe_ffn(x, router, gate, up, down, ne=ne, n_expert=E, n_used=1, n_ff_exp=nff, gate_dtype=dt, down_dtype=dt, expert_ids=sel)
     assert not np.asarray(ref["dst"]).any() and not out.any()
+
+
+@pytest.mark.parametrize("dt,act", [(H.Q8_0, M.Activation.Silu), (H.Q8_0, M.Activation.Gelu), (H.F16, M.Activation.Silu)])
+def test_clamped_activation_keeps_a_nan_of_up(be, dt, act):
+    """A clamp bounds `up` on both sides and lets a NaN through, as the reference's comparisons do: rows of an expert with a NaN in its
+    up matrix are NaN, all others are not."""
+    ne, nff, E, rows = 256, 128, 4, 48
+    rng = np.random.default_rng(dt)
+    x = rng.standard_normal((rows, ne)).astype(np.float32)
+    router = np.zeros((E, ne), np.float32)
+    if dt == H.F16:
+        gate, up, down = ((0.1 * rng.standard_normal(E * nff * ne)).astype(np.float16).view(np.uint8) for _ in range(3))
+    else:
+        gate, up, down = _bank_weights(rng, E, nff, ne, dt, dt)
+    up = np.ascontiguousarray(up).copy()
+    row_bytes = len(up) // (E * nff)
+    up[(nff + 5) * row_bytes:][:2] = (0x00, 0x7E)   # expert 1, feature 5: the first block's scale, or the first element
+    sel = rng.integers(0, E, (rows, 1)).astype(np.int32)
+    g, ids = moe_graph(rows, ne, E, 1, nff, DType(dt), DType(dt), with_expert_ids=True, swiglu_clamp=2.0, act=act)
+    out, _, _ = _run_batched(be, g, ids, dict(x=x, router=router, gate=gate, up=up, down=down, expert_ids=sel), rows, ne)
+    ref = O.moe_ffn(x, router, gate, up, down, ne=ne, n_expert=E, n_used=1, n_ff_exp=nff, gate_dtype=dt, down_dtype=dt, expert_ids=sel,
+                    swiglu_clamp=2.0, act=int(act))["dst"].reshape(rows, ne)
+    hit = sel[:, 0] == 1
+    assert np.isnan(ref[hit]).all() and np.isfinite(ref[~hit]).all()
+    assert np.isnan(out[hit]).all()
+    assert H.rel_l2(out[~hit], ref[~hit]) < REL_L2_MFMA
