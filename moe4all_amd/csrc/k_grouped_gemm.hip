@@ -68,9 +68,13 @@ __device__ __forceinline__ void wait_loads() { asm volatile("s_waitcnt vmcnt(%0)
 template <int N>
 __device__ __forceinline__ void wait_barrier() { asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" : : "n"(N) : "memory"); }
 
-// Results of a tile through the wave's LDS region `wl`, as rows of 64 bytes that leave in 16-byte stores.
-template <class F, bool DOWN, int NB, int M>
-__device__ __forceinline__ void store_tile(const GroupedParams& p, const Tile& t, int n0, int wave, int lane, uint8_t* wl,
+// Results of a tile through the wave's LDS region `wl`, as rows of 64 bytes that leave in 16-byte stores.  The gate/up rows of an
+// always-on expert are activated as Op::GatedAct does it, exponential and division rounded correctly, so that its results have the
+// bits of the separate ops: on the way out, where one copy of the code serves all registers (1500 rows of 256 experts of
+// 4096 x 1536 beside one: 1053 us a layer with it, 1054 with the routed experts' exponential).
+// SILU: gate/up rows of a routed expert under a plain silu, in code of their own (all forms in one loop: 1.2 to 1.9 % slower batches).
+template <class F, bool DOWN, int NB, int M, bool SILU>
+__device__ __forceinline__ void store_rows(const GroupedParams& p, const Tile& t, int n0, int wave, int lane, uint8_t* wl,
                                            const float (&row_scale)[2], const float4v (&acc)[NB][M], const float (&dcur)[NB]) {
     // Accumulator register q of
     // tile m: token 16 m + 4 kq + q, weight row col of operand n; token 16 m + 4 a + b lies in row 4 b + a, so that a
@@ -79,7 +83,7 @@ __device__ __forceinline__ void store_tile(const GroupedParams& p, const Tile& t
     float fin[NB];
 #pragma unroll
     for (int n = 0; n < NB; n++) fin[n] = F::kScale ? dcur[n] * kTwo24 : 1.0f;
-    const bool always = t.e == p.sh_e, half_out = DOWN && p.out_f16 && !always;
+    const bool always = !F::kUnits && !SILU && t.e == p.sh_e, half_out = DOWN && p.out_f16 && !always;
     const float ds = DOWN && p.down_scale && !always ? p.down_scale[t.e] : 1.0f;
     uint8_t* const out = reinterpret_cast<uint8_t*>(DOWN && always ? p.sh_out : p.out);
     const int out0 = DOWN && always ? t.p0 - p.sh_p0 : t.p0;
@@ -101,8 +105,10 @@ __device__ __forceinline__ void store_tile(const GroupedParams& p, const Tile& t
                 } else {
                     const float sc = __shfl(row_scale[m >> 2], tok & 63, 64);
                     float g = acc[0][m][q] * fin[0] * sc, u = acc[1][m][q] * fin[1] * sc;
-                    if (p.act == INFR_ACT_SILU && !p.has_clamp && !p.weight_before) {
+                    if (SILU) {
                         g = silu_fast(g) * u;
+                    } else if (always) {
+                        reinterpret_cast<float*>(o + 1024)[col] = u;
                     } else {
                         if (p.weight_before) {
                             const float wp = p.route_w[p.pair_src[t.p0 + min(tok, t.cnt - 1)]];
@@ -115,6 +121,12 @@ __device__ __forceinline__ void store_tile(const GroupedParams& p, const Tile& t
                 }
             }
             asm volatile("" ::: "memory");
+            if (!DOWN && !SILU && always) {
+                float* const h = reinterpret_cast<float*>(wl) + 4 * lane;
+#pragma unroll 1
+                for (int i = 0; i < 4; i++) h[i] = gated_act_fn(p.act, p.has_clamp, p.clamp, h[i], h[256 + i]);
+                asm volatile("" ::: "memory");
+            }
             const int tok = 16 * m + 4 * ((lane >> 2) & 3) + (lane >> 4), f = fw + 16 * part;
             const uint4v v = *reinterpret_cast<const uint4v*>(wl + 16 * lane);
             uint8_t* const dst = out + ((size_t)(out0 + tok) * p.N + f) * es;
@@ -130,6 +142,15 @@ __device__ __forceinline__ void store_tile(const GroupedParams& p, const Tile& t
             }
         }
     }
+}
+
+template <class F, bool DOWN, int NB, int M>
+__device__ __forceinline__ void store_tile(const GroupedParams& p, const Tile& t, int n0, int wave, int lane, uint8_t* wl,
+                                           const float (&row_scale)[2], const float4v (&acc)[NB][M], const float (&dcur)[NB]) {
+    if (!DOWN && p.act == INFR_ACT_SILU && !p.has_clamp && !p.weight_before && (F::kUnits || t.e != p.sh_e))
+        store_rows<F, DOWN, NB, M, true>(p, t, n0, wave, lane, wl, row_scale, acc, dcur);
+    else
+        store_rows<F, DOWN, NB, M, false>(p, t, n0, wave, lane, wl, row_scale, acc, dcur);
 }
 
 // An item: M 16-token tiles; FEW: one of up to 8 tokens (the rows of the others hold what was there: a token's sums depend on

@@ -511,3 +511,48 @@ def test_clamped_activation_keeps_a_nan_of_up(be, dt, act):
     assert np.isnan(ref[hit]).all() and np.isfinite(ref[~hit]).all()
     assert np.isnan(out[hit]).all()
     assert H.rel_l2(out[~hit], ref[~hit]) < REL_L2_MFMA
+
+
+@pytest.mark.parametrize("gdt,ddt,ne,nff,rows,K,act,clamp", [
+    (H.Q4K, H.Q6K, 512, 256, 300, 2, M.Activation.Silu, None), (H.Q4K, H.Q6K, 256, 4352, 130, 1, M.Activation.Silu, None),
+    (H.Q8_0, H.Q8_0, 320, 192, 131, 3, M.Activation.Gelu, None), (H.Q5K, H.Q4K, 256, 256, 129, 2, M.Activation.Sigmoid, None),
+    (H.MXFP4, H.IQ4_XS, 192, 256, 257, 4, M.Activation.Silu, 0.75), (H.Q4_0, H.Q8_0, 4416, 192, 128, 2, M.Activation.Gelu, 0.5),
+])
+def test_always_on_expert_in_the_gemms_keeps_the_bits_of_the_ops(be, gdt, ddt, ne, nff, rows, K, act, clamp):
+    """The always-on expert's part of a folded batch, activation included, is what Linear, Linear, GatedAct, Linear, Add give: the
+    same bits, on tiles of up to 64 and of up to 128 tokens."""
+    rng = np.random.default_rng(gdt * 71 + ddt + rows)
+    E = 9
+    x = rng.standard_normal((rows, ne)).astype(np.float32)
+    x[1::7] *= 40.0                                   # closed and wide open gates
+    router = (rng.standard_normal((E, ne)) * 0.05).astype(np.float32)
+    gate, up, down = _bank_weights(rng, E, nff, ne, gdt, ddt)
+    sg, su, sd = _bank_weights(rng, 1, nff, ne, gdt, ddt)
+    outs = {}
+    for off in (False, True):
+        g = M.Graph()
+        t = lambda kind, shape, dt=DType.F32: getattr(g, kind)(M.TensorDesc(list(shape), dt))  # noqa: E731
+        xt, out = t("input", (rows, ne)), t("output", (rows, ne))
+        ws = [t("weight", sh, dt) for sh, dt in (((E, ne), DType.F32), ((E, nff, ne), DType(gdt)), ((E, nff, ne), DType(gdt)),
+                                                 ((E, ne, nff), DType(ddt)), ((nff, ne), DType(gdt)), ((nff, ne), DType(gdt)),
+                                                 ((ne, nff), DType(ddt)))]
+        moe, tg, tu, ta, ts = (t("internal", (rows, n)) for n in (ne, nff, nff, nff, ne))
+        g.moe_ffn(x=xt, router=ws[0], gate_exps=ws[1], up_exps=ws[2], down_exps=ws[3], dst=moe, ne=ne, n_expert=E, n_used=K, n_ff_exp=nff,
+                  act=act, swiglu_clamp=clamp)
+        g.linear(x=xt, weight=ws[4], dst=tg, m=rows, in_f=ne, out_f=nff)
+        g.linear(x=xt, weight=ws[5], dst=tu, m=rows, in_f=ne, out_f=nff)
+        g.gated_act(gate=tg, up=tu, dst=ta, rows=rows, nff=nff, act=act, swiglu_clamp=clamp)
+        g.linear(x=ta, weight=ws[6], dst=ts, m=rows, in_f=nff, out_f=ne)
+        g.add(a=moe, b=ts, dst=out, n=rows * ne)
+        b = M.Backend(0, disable_op_fusion=True) if off else be
+        try:
+            b.prof_enable(True)
+            b.prof_read()
+            outs[off] = M.run_graph(b, g, list(zip([xt] + ws, [x, router, gate, up, down, sg, su, sd])), out, rows * ne)
+            assert any(n.startswith("linear") for n in b.prof_read()) == off
+            b.prof_enable(False)
+        finally:
+            if off:
+                b.close()
+    assert np.isfinite(outs[False]).all()
+    assert np.array_equal(bits(outs[False]), bits(outs[True]))
