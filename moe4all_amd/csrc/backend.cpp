@@ -164,8 +164,8 @@ struct MoeScratch {
     int32_t* pair_row = nullptr;  // [rows * n_used]
     int4* tiles = nullptr;        // tile table of the grouped GEMMs
     int tile_log2 = 6;            // batched: its tiles hold up to 1 << tile_log2 pairs
-    bool always_room = false;     // batched: scratch for an always-on expert's rows behind the pairs'
-    float* ysh = nullptr;         // [rows, ne] its results
+    int always_rows = 0;          // batched: rows of an always-on expert behind the pairs' in pair_row, h, hh, hs and hm
+    size_t tables_off = 0;        // batched or bucketed: arena offset of the bucket tables
     _Float16* xh = nullptr;       // [rows, ne]
     float* xs = nullptr;          // [rows]
     uint32_t* xm = nullptr;       // [rows, ne / 32] group sums of xh (formats with minimums)
@@ -873,17 +873,7 @@ extern "C" infr_status infr_hip_compile(infr_hip_backend* be, const infr_graph* 
                 if (units_mfma) batched = true;
                 if (batched) {
                     plan->moe[oi].tile_log2 = infr::gemm_tile_log2(c.dt(m.gate_exps), c.dt(m.down_exps), (int)rows, (int)pairs, (int)n_local, (int)m.ne, (int)m.n_ff_exp);
-                    // (an always-on expert behind the op may join its GEMMs: a pair more per row)
-                    const bool room = oi + 1 < g->n_ops && g->ops[oi + 1].kind == INFR_OP_LINEAR && g->ops[oi + 1].u.linear.x == m.x;
-                    plan->moe[oi].always_room = room;
-                    const size_t all = pairs + (room ? rows : 0);
-                    arena += round_up(((size_t)m.n_expert + 2) * 4, 256) + 3 * round_up(pairs * 4 + 4, 256) + round_up(all * 4 + 4, 256) +
-                             round_up(((size_t)infr::gemm_max_tiles((int)all, (int)m.n_expert + 1, 1 << plan->moe[oi].tile_log2) + 1) * sizeof(int4), 256);
-                    shared += round_up((size_t)rows * m.ne * 2, 256) + round_up((size_t)rows * 4, 256) +
-                              round_up(all * m.n_ff_exp * 2, 256) + round_up(all * 4, 256) +
-                              round_up((size_t)rows * m.ne / 8, 256) + round_up(all * m.n_ff_exp / 8, 256) +
-                              round_up(pairs * m.ne * 4, 256) + (room ? round_up((size_t)rows * m.ne * 4, 256) : 0);
-                }
+                }   // (its scratch: behind the launch fusion, which may add an always-on expert's rows)
                 bool bucketed = false;
                 // Bucketing reads an expert's rows once for its tokens: with uniform routing
                 // E * (1 - (1 - K/E)^rows) experts are expected where the per-token kernels read rows * K.  It pays when the bytes
@@ -931,6 +921,7 @@ extern "C" infr_status infr_hip_compile(infr_hip_backend* be, const infr_graph* 
                 if (units_batch) bucketed = true;
                 plan->moe[oi].units_batch = units_batch;
                 if (bucketed) {
+                    plan->moe[oi].tables_off = arena;
                     arena += round_up(((size_t)m.n_expert + 2) * 4, 256) + 4 * round_up(pairs * 4 + 4, 256) +
                              round_up(((size_t)infr::gemm_max_tiles((int)pairs, (int)m.n_expert, infr::kIntTok) + 1) * sizeof(int4), 256);
                     shared += round_up((size_t)plan->moe[oi].k_parts * pairs * m.ne * 4, 256);
@@ -1084,9 +1075,6 @@ extern "C" infr_status infr_hip_compile(infr_hip_backend* be, const infr_graph* 
         if (c.st != INFR_OK) c.err = "op " + std::to_string(oi) + ": " + c.err;
     }
     if (c.st != INFR_OK) return bail(c.st, c.err);
-    const size_t shared_off = arena;
-    arena += shared_need;
-
     // ---- launch fusion: Linear + Linear + GatedAct on one input -> one gate/up kernel; Linear + Add
     // -> one kernel.  A temporary may disappear only if it is an Internal tensor written once and read
     // once.  The fused kernels run the same inner products and the same rounding sequence, so the
@@ -1234,7 +1222,7 @@ extern "C" infr_status infr_hip_compile(infr_hip_backend* be, const infr_graph* 
         // 1500 rows of 256 experts of 4096 x 1536 beside one: the three Linears with their conversions, the activation and the
         // Add took 143 of 1357 us.
         for (uint32_t oi = 0; oi + 5 < g->n_ops; oi++) {
-            if (plan->ops[oi].kind != INFR_OP_MOE_FFN || !plan->moe[oi].batched || !plan->moe[oi].always_room) continue;
+            if (plan->ops[oi].kind != INFR_OP_MOE_FFN || !plan->moe[oi].batched) continue;
             const infr_op_moe_ffn& m = plan->ops[oi].u.moe_ffn;
             const int rows = plan->moe[oi].rows;
             static const int32_t kinds[5] = {INFR_OP_LINEAR, INFR_OP_LINEAR, INFR_OP_GATED_ACT, INFR_OP_LINEAR, INFR_OP_ADD};
@@ -1262,6 +1250,7 @@ extern "C" infr_status infr_hip_compile(infr_hip_backend* be, const infr_graph* 
             plan->fuse[oi].kind = infr_hip_plan::kMoeShared;
             plan->fuse[oi].a = gate_first ? oi + 1 : oi + 2;   // the gate Linear
             plan->fuse[oi].b = oi + 4;
+            plan->moe[oi].always_rows = rows;
             for (uint32_t k = oi + 1; k <= oi + 5; k++) plan->fuse[k].kind = infr_hip_plan::kSkip;
         }
         // MoeFfn -> Add (the residual; the reference's moe_add rewrite, crates/infr-core/src/fusion.rs:20-24):
@@ -1299,6 +1288,22 @@ extern "C" infr_status infr_hip_compile(infr_hip_backend* be, const infr_graph* 
             }
         }
     }
+    for (uint32_t oi = 0; oi < g->n_ops; oi++) {
+        MoeScratch& s = plan->moe[oi];
+        if (plan->ops[oi].kind != INFR_OP_MOE_FFN || !s.batched) continue;
+        const infr_op_moe_ffn& m = plan->ops[oi].u.moe_ffn;
+        const size_t rows = s.rows, pairs = rows * m.n_used, all = pairs + s.always_rows;
+        s.tables_off = arena;
+        arena += round_up(((size_t)m.n_expert + 2) * 4, 256) + 3 * round_up(pairs * 4 + 4, 256) + round_up(all * 4 + 4, 256) +
+                 round_up(((size_t)infr::gemm_max_tiles((int)all, (int)m.n_expert + (s.always_rows ? 1 : 0), 1 << s.tile_log2) + 1) * sizeof(int4), 256);
+        const size_t shared = round_up((pairs + rows) * m.n_ff_exp * 4 + 4, 256) + round_up(rows * m.ne * 2, 256) + round_up(rows * 4, 256) +
+                              round_up(rows * m.ne / 8, 256) + round_up(all * m.n_ff_exp * 2, 256) + round_up(all * 4, 256) +
+                              round_up(all * m.n_ff_exp / 8, 256) + round_up(pairs * m.ne * 4, 256);
+        if (shared > shared_need) shared_need = shared;
+    }
+    const size_t shared_off = arena;
+    arena += shared_need;
+
     // One token row through a MoeFfn: the whole op (with an always-on expert folded in, if there is one) as one launch
     // when the shape fits one of the two single-launch kernels.  An RmsNorm folded into the logits kernel is unfolded
     // again: it costs one small launch, the single launch saves two large ones.
@@ -1378,11 +1383,12 @@ extern "C" infr_status infr_hip_compile(infr_hip_backend* be, const infr_graph* 
         s.weights = (float*)p; p += round_up(rows * m.n_used * 4 + 4, 256);
         const size_t pairs = rows * m.n_used;
         if (s.batched || s.bucketed) {
+            p = (char*)plan->arena + s.tables_off;
             s.offsets = (int32_t*)p;   p += round_up(((size_t)m.n_expert + 2) * 4, 256);
             s.pair_src = (int32_t*)p;  p += round_up(pairs * 4 + 4, 256);
             s.slot_pair = (int32_t*)p; p += round_up(pairs * 4 + 4, 256);
             s.live_ids = (int32_t*)p;  p += round_up(pairs * 4 + 4, 256);
-            s.pair_row = (int32_t*)p;  p += round_up((pairs + (s.always_room ? rows : 0)) * 4 + 4, 256);
+            s.pair_row = (int32_t*)p;  p += round_up((pairs + s.always_rows) * 4 + 4, 256);
             s.tiles = (int4*)p;
         }
         p = (char*)plan->arena + shared_off;
@@ -1391,15 +1397,12 @@ extern "C" infr_status infr_hip_compile(infr_hip_backend* be, const infr_graph* 
             s.xh = (_Float16*)p; p += round_up(rows * m.ne * 2, 256);
             s.xs = (float*)p;    p += round_up(rows * 4, 256);
             s.xm = (uint32_t*)p; p += round_up(rows * m.ne / 8, 256);
-            const size_t all = pairs + (s.always_room ? rows : 0);
+            const size_t all = pairs + s.always_rows;
             s.hh = (_Float16*)p; p += round_up(all * m.n_ff_exp * 2, 256);
             s.hs = (float*)p;    p += round_up(all * 4, 256);
             s.hm = (uint32_t*)p; p += round_up(all * m.n_ff_exp / 8, 256);
-            s.y = (float*)p;     p += round_up(pairs * m.ne * 4, 256);
-            s.ysh = (float*)p;
-        } else {
-            s.y = (float*)p;
         }
+        s.y = (float*)p;
     }
     plan->layer_ws = layer_ws ? (char*)plan->arena + layer_ws_off : nullptr;
     plan->stream_ws = stream_ws ? (char*)plan->arena + stream_ws_off : nullptr;
@@ -1620,6 +1623,7 @@ extern "C" infr_status infr_hip_execute(infr_hip_backend* be, infr_hip_plan* pla
                     }
                 }
                 const uint8_t *al_gate = nullptr, *al_up = nullptr, *al_down = nullptr;   // an always-on expert in the batch's GEMMs
+                float* al_out = nullptr;   // its results: the down Linear's Internal tensor
                 if (fz.kind == infr_hip_plan::kMoeShared && sc.batched) {
                     const infr_op_linear& lg = plan->ops[fz.a].u.linear;
                     const infr_op_linear& lu = plan->ops[fz.a == oi + 1 ? oi + 2 : oi + 1].u.linear;
@@ -1631,6 +1635,7 @@ extern "C" infr_status infr_hip_execute(infr_hip_backend* be, infr_hip_plan* pla
                     al_gate = (const uint8_t*)ptr[lg.weight];
                     al_up = (const uint8_t*)ptr[lu.weight];
                     al_down = (const uint8_t*)ptr[ld.weight];
+                    al_out = (float*)ptr[ld.dst];
                     if (!fz.res) gp.dst = (float*)ptr[sum_dst];
                 }
                 auto launch_gate_logit = [&]() {
@@ -1760,7 +1765,7 @@ extern "C" infr_status infr_hip_execute(infr_hip_backend* be, infr_hip_plan* pla
                     q.weight_before = (int)m.weight_before;
                     q.sh_e = -1;
                     if (al_gate) {
-                        q.sh_e = (int)n_local; q.sh_p0 = pairs; q.sh0 = al_gate; q.sh1 = al_up; q.sh_out = sc.ysh;
+                        q.sh_e = (int)n_local; q.sh_p0 = pairs; q.sh0 = al_gate; q.sh1 = al_up; q.sh_out = al_out;
                         q.n_pairs = pairs + rows; q.n_expert = (int)n_local + 1;
                     }
                     q.a_sum = sc.xm; q.pair_row = sc.pair_row; q.tiles = sc.tiles; q.tile_log2 = sc.tile_log2;
@@ -1784,7 +1789,7 @@ extern "C" infr_status infr_hip_execute(infr_hip_backend* be, infr_hip_plan* pla
                     {
                         Timed t(be, "moe_unbucket_combine");
                         infr::launch_unbucket_combine(s, sc.y, sc.slot_pair, sc.weights, rows, (int)m.ne, (int)m.n_used,
-                                                      (int)m.weight_before, gp.dst, 0, sc.hs, gp.addend, 0, al_gate ? sc.ysh : nullptr);
+                                                      (int)m.weight_before, gp.dst, 0, sc.hs, gp.addend, 0, al_out);
                     }
                     break;
                 }

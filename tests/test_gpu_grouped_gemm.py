@@ -10,6 +10,7 @@ import oracle as O
 from moe4all_amd import DType
 
 from test_gpu_parity import REL_L2_MFMA, _bank_weights, _run_batched, bits, moe_graph, run_moe
+from test_zz_no_alloc import _free_device_bytes
 
 pytestmark = pytest.mark.gpu
 
@@ -556,3 +557,40 @@ def test_always_on_expert_in_the_gemms_keeps_the_bits_of_the_ops(be, gdt, ddt, n
                 b.close()
     assert np.isfinite(outs[False]).all()
     assert np.array_equal(bits(outs[False]), bits(outs[True]))
+
+
+@pytest.mark.parametrize("follower", ["projection", "gated", "fusion off", "up format"])
+def test_scratch_for_an_always_on_expert_only_where_it_joins(be, follower):
+    """A Linear that reads the op's input is no always-on expert by itself: a projection beside the op, the gate logit of the gated form,
+    fusion switched off, an expert in another format.  Such a plan takes the op's scratch and the other tensors, no room for the expert's
+    rows (512 * (2.125 * 2048 + 4 * 4096) bytes would be 10 MB)."""
+    ne, nff, E, K, rows = 4096, 2048, 8, 2, 512
+
+    def plan_bytes(b, with_linears):
+        g = M.Graph()
+        t = lambda kind, shape, dt=DType.F32: getattr(g, kind)(M.TensorDesc(list(shape), dt))  # noqa: E731
+        xt, out = t("input", (rows, ne)), t("output", (rows, ne))
+        w = lambda *shape: t("weight", shape, DType.Q4K)  # noqa: E731
+        g.moe_ffn(x=xt, router=t("weight", (E, ne)), gate_exps=w(E, nff, ne), up_exps=w(E, nff, ne), down_exps=w(E, ne, nff), dst=out,
+                  ne=ne, n_expert=E, n_used=K, n_ff_exp=nff)
+        if with_linears:
+            wide = 1 if follower == "gated" else nff
+            wt = t("weight", (wide, ne), DType.Q6K if follower == "up format" else DType.Q4K)
+            g.linear(x=xt, weight=wt, dst=t("output", (rows, wide)), m=rows, in_f=ne, out_f=wide)
+        b.sync()
+        before = _free_device_bytes()
+        p = b.compile(g)
+        b.sync()
+        taken = before - _free_device_bytes()
+        p.free()
+        return taken
+
+    b = M.Backend(0, disable_op_fusion=True) if follower == "fusion off" else be
+    try:
+        plan_bytes(b, False)
+        alone, beside = plan_bytes(b, False), plan_bytes(b, True)
+    finally:
+        if b is not be:
+            b.close()
+    assert alone >= 2 * rows * K * nff * 4
+    assert beside - alone <= 4 << 20   # the Linear's table, and the allocator's granule
