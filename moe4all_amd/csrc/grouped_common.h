@@ -121,6 +121,9 @@ struct Tile {
 // the same weights, which then come from memory once per group, while the group's activations stay in the L2 for its
 // columns.  Uniform; false when there is nothing to do (the grid is an upper bound).
 constexpr int kGroupTiles = 4;
+__device__ __forceinline__ int group_column(uint32_t r, int in_group) {   // item r of a group of in_group tiles: r / in_group
+    return (int)(in_group == 1 ? r : in_group == 2 ? r >> 1 : in_group == 3 ? __umulhi(r, 0x55555556u) : r >> 2);
+}
 __device__ __forceinline__ bool tile_item(const int4* __restrict__ tiles, int n_cols, uint32_t n_cols_rcp, int tile_pairs, Tile& t, int& col) {
     const int n_items = tiles[0].x * n_cols, per = (n_items + 7) >> 3, k = (int)(blockIdx.x >> 3);
     const int item = (int)(blockIdx.x & 7) * per + k;
@@ -128,11 +131,10 @@ __device__ __forceinline__ bool tile_item(const int4* __restrict__ tiles, int n_
     const int some = n_cols == 1 ? item : (int)__umulhi((uint32_t)item, n_cols_rcp);   // item / n_cols: exact below 2^32 / n_cols
     const int4 b = tiles[1 + some];   // expert, its first pair, its pairs, its first tile
     const int first = (some - b.w) & ~(kGroupTiles - 1), in_group = min(kGroupTiles, (b.z + tile_pairs - 1) / tile_pairs - first);
-    const uint32_t r = (uint32_t)(item - (b.w + first) * n_cols);
-    const uint32_t c = in_group == 1 ? r : in_group == 2 ? r >> 1 : in_group == 3 ? __umulhi(r, 0x55555556u) : r >> 2;
-    const int at = (first + (int)(r - c * in_group)) * tile_pairs;
+    const int r = item - (b.w + first) * n_cols, c = group_column((uint32_t)r, in_group);
+    const int at = (first + r - c * in_group) * tile_pairs;
     t = Tile{b.x, b.y + at, min(tile_pairs, b.z - at)};
-    col = (int)c;
+    col = c;
     return true;
 }
 

@@ -468,10 +468,11 @@ __device__ __forceinline__ void gemm_tile(const GroupedParams& p, const Tile& t,
 // 60 token rows of 128 experts of 2048 x 768 in Q5_1 79 + 45 us, 71 + 39 this way) and go row by row through 16 rows of LDS;
 // activations in two pieces of 512 / T k in turn, with one barrier per piece.
 template <class F>
-constexpr size_t unit_lds() { return (size_t)kGW * 256 * F::kChunks + 2 * 16 * 1024; }
+constexpr size_t unit_lds() { return (size_t)kGW * 256 * F::kChunks + 2 * 16 * 1024 + 64 * sizeof(float); }
 template <class F, bool DOWN, int T>
 __device__ __forceinline__ void unit_tile(const GroupedParams& p, const Tile& t, int n0, uint8_t* lds) {
     constexpr int NB = 2;                                              // 16-row weight operands of a wave
+    constexpr bool kPartial = F::kBlock < F::kStep;                    // rows need not be whole steps
     constexpr int KC = 512 / T;                                        // k of an activation piece
     constexpr int SPP = KC > F::kStep ? KC / F::kStep : 1, PPS = F::kStep > KC ? F::kStep / KC : 1;   // steps per piece, pieces per step
     constexpr int G = T;                                               // tokens per 1 KB group of a piece
@@ -483,6 +484,7 @@ __device__ __forceinline__ void unit_tile(const GroupedParams& p, const Tile& t,
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     uint8_t* const wl = lds + wave * (256 * F::kChunks);
     uint8_t* const al = lds + kGW * (256 * F::kChunks);
+    float* const s_scale = reinterpret_cast<float*>(al + 2 * kPiece);   // the tokens' row scales
     const uint32_t al0 = lds_address(al);
 
     // the token rows behind the lane's activation loads: requested ahead of the weights, which would hold them up
@@ -517,7 +519,7 @@ __device__ __forceinline__ void unit_tile(const GroupedParams& p, const Tile& t,
             const bool pure0 = DOWN || 64 * i + 63 < kHalf, pure1 = 64 * i >= kHalf;
             const uint8_t* const b = (pure0 ? b0 : pure1 ? b1 : (64 * i + lane < kHalf ? b0 : b1)) + (uint32_t)(kStepBytes * s);
             uint32_t off = woff[i];
-            if (F::kBlock < F::kStep && (s + 1) * F::kStep > p.K) {   // chunks behind the row's end are not read (the step's first one instead)
+            if (kPartial && (s + 1) * F::kStep > p.K) {   // chunks behind the row's end are not read (the step's first one instead)
                 const int idx = min(64 * i + lane, NC - 1), r = idx / F::kChunks, at = F::src(idx - r * F::kChunks, r & 15);
                 if (kStepBytes * s + at >= (int)row_bytes) off -= (uint32_t)at;
             }
@@ -541,6 +543,8 @@ __device__ __forceinline__ void unit_tile(const GroupedParams& p, const Tile& t,
         }
     };
     fetch(0);
+    // (behind the last step, where they are needed, a memory latency per item; in a register until then, more spills)
+    if ((!DOWN || !p.out_f16) && wave == 0) s_scale[lane] = p.a_scale[srow];   // read behind barriers
     asm volatile("" ::: "memory");
 
     float4v acc[NB][T];
@@ -582,8 +586,9 @@ __device__ __forceinline__ void unit_tile(const GroupedParams& p, const Tile& t,
         }
         if (PPS > 1 && more) request(s + 1);
         asm volatile("" ::: "memory");
-        const int groups = min(F::kStep, p.K - s * F::kStep) / 32;   // groups of 32 k from here to the row's end
-        if (groups < F::kStep / 32) {
+        // groups of 32 k from here to the row's end: known where rows are whole steps (tests and cuts left in for those too: Q3_K 2 to 8 %)
+        const int groups = kPartial ? (p.K - s * F::kStep) / 32 : F::kStep / 32;
+        if (kPartial && groups < F::kStep / 32) {
 #pragma unroll
             for (int n = 0; n < NB; n++) F::cut(raw[n], kq, groups);
         }
@@ -612,8 +617,7 @@ __device__ __forceinline__ void unit_tile(const GroupedParams& p, const Tile& t,
             }
         }
     }
-    float row_scale[2] = {1.0f, 1.0f};
-    if (!DOWN || !p.out_f16) row_scale[0] = p.a_scale[srow];
+    const float row_scale[2] = {s_scale[lane], 1.0f};   // (nothing in it where rows leave without their scale)
     const float unit[NB] = {1.0f, 1.0f};
     store_tile<F, DOWN, NB, T>(p, t, n0, wave, lane, wl, row_scale, acc, unit);
 }
@@ -665,12 +669,28 @@ void gemm_launch(hipStream_t s, const GroupedParams& q, dim3 grid) {
     INFR_LAUNCH((grouped_gemm<F, DOWN, W, false>), grid, dim3(kGW * 64), (gemm_lds<F, W>()), s, q);
 }
 
+// The same for a dense matrix in a format of the unit decoder: a contiguous eighth of the items per XCD, in groups of up to kGroupTiles
+// tiles, columns outside.  Every item of such a launch costs about the same, and its weights, decoded by every workgroup that reads them,
+// are the smaller part: the XCDs share out the tiles' rows.  us per Linear, this order and the other: 512 rows of 2048 x 2048 in Q3_K
+// 29.1 and 30.0, IQ3_S 38.8 and 39.7, 2048 rows of 4096 x 4096 in Q5_1 the same.
+__device__ __forceinline__ bool dense_item(const GroupedParams& p, Tile& t, int& col) {
+    const int n_tiles = p.tiles[0].x, n_items = n_tiles * p.n_tiles_n, per = (n_items + 7) >> 3, k = (int)(blockIdx.x >> 3);
+    const int item = (int)(blockIdx.x & 7) * per + k;
+    if (k >= per || item >= n_items) return false;
+    const int some = p.n_tiles_n == 1 ? item : (int)__umulhi((uint32_t)item, p.n_tiles_rcp), first = some & ~(kGroupTiles - 1);
+    const int in_group = min(kGroupTiles, n_tiles - first), r = item - first * p.n_tiles_n;
+    col = group_column((uint32_t)r, in_group);
+    const int4 b = p.tiles[1 + first + r - col * in_group];
+    t = Tile{b.x, b.y, b.z};
+    return true;
+}
+
 template <class F, bool DOWN>
 __global__ __launch_bounds__(kGW * 64, 3) void grouped_gemm_units(GroupedParams p) {
     extern __shared__ __attribute__((aligned(16))) uint8_t lds_gemm[];
     Tile t;
     int n0;
-    if (!gemm_item(p, t, n0)) return;
+    if (!(DOWN && p.n_expert == 1 ? dense_item(p, t, n0) : gemm_item(p, t, n0))) return;
     n0 *= (DOWN ? 32 : 16) * kGW;
     if (t.cnt <= 16) unit_tile<F, DOWN, 1>(p, t, n0, lds_gemm);
     else if (t.cnt <= 32) unit_tile<F, DOWN, 2>(p, t, n0, lds_gemm);
@@ -683,7 +703,7 @@ void gemm(hipStream_t s, const GroupedParams& p) {
     const int width = DOWN ? 32 * kGW : 16 * kGW;
     q.n_tiles_n = (p.N + width - 1) / width;
     q.n_tiles_rcp = (uint32_t)((0x100000000ull + q.n_tiles_n - 1) / q.n_tiles_n);
-    const dim3 grid((unsigned)(gemm_max_tiles(p.n_pairs, p.n_expert, 1 << p.tile_log2) * q.n_tiles_n));
+    const dim3 grid((unsigned)((gemm_max_tiles(p.n_pairs, p.n_expert, 1 << p.tile_log2) * q.n_tiles_n + 7) & ~7));   // whole rounds of the 8 XCDs
     if constexpr (F::kUnits) {
         INFR_LDS_LIMIT((grouped_gemm_units<F, DOWN>), (int)unit_lds<F>());
         INFR_LAUNCH((grouped_gemm_units<F, DOWN>), grid, dim3(kGW * 64), unit_lds<F>(), s, q);

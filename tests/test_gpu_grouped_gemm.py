@@ -594,3 +594,31 @@ def test_scratch_for_an_always_on_expert_only_where_it_joins(be, follower):
             b.close()
     assert alone >= 2 * rows * K * nff * 4
     assert beside - alone <= 4 << 20   # the Linear's table, and the allocator's granule
+
+
+@pytest.mark.parametrize("dt,in_f", [(H.Q3K, 512), (H.Q4_1, 320), (H.IQ3_S, 256)])
+@pytest.mark.parametrize("rows,out_f", [(128, 128), (150, 100), (257, 300), (512, 130), (577, 640), (1100, 129)])
+def test_dense_matrix_of_the_unit_decoder(be, dt, in_f, rows, out_f):
+    """A Linear in a format of the unit decoder, one to eighteen tiles of 64 rows (groups of one to four of them) times one to five columns:
+    every item is worked on once, and a row has the bits it has among fewer rows."""
+    rng = np.random.default_rng(dt * 73 + rows)
+    x = rng.standard_normal((rows, in_f)).astype(np.float32)
+    w = H.centred_weight(dt, out_f * in_f, 5)
+
+    def linear(v):
+        g = M.Graph()
+        xt, wt = g.input(M.TensorDesc([len(v), in_f], DType.F32)), g.weight(M.TensorDesc([out_f, in_f], DType(dt)))
+        y = g.output(M.TensorDesc([len(v), out_f], DType.F32))
+        g.linear(x=xt, weight=wt, dst=y, m=len(v), in_f=in_f, out_f=out_f)
+        be.prof_enable(True)
+        be.prof_read()
+        out = M.run_graph(be, g, [(xt, v), (wt, w)], y, len(v) * out_f).reshape(len(v), out_f)
+        assert "linear_grouped_units" in be.prof_read()
+        be.prof_enable(False)
+        return out
+
+    out = linear(x)
+    ref = O.linear(x, w, dt, in_f, out_f).reshape(rows, out_f)
+    for r in range(rows):
+        assert H.rel_l2(out[r], ref[r]) < REL_L2_MFMA, r
+    assert np.array_equal(bits(linear(np.ascontiguousarray(x[-128:]))), bits(out[-128:]))
