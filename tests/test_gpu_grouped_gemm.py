@@ -389,30 +389,40 @@ def test_which_decode_batches_go_over_buckets(be, gdt, ddt, ne, nff, E, rows, be
         plan.free()
 
 
-@pytest.mark.parametrize("gdt,ddt,ne,nff,rows", [
-    # h rows of 64 to 2048 elements (a wavefront each, one to four chunks per lane) and beyond; group sums behind them (Q4_K, Q5_K down)
-    (H.Q8_0, H.Q8_0, 64, 64, 33), (H.Q8_0, H.Q4K, 256, 512, 34), (H.Q8_0, H.Q5K, 256, 768, 35), (H.Q8_0, H.Q6K, 256, 1280, 33),
-    (H.Q8_0, H.Q4K, 256, 1536, 37), (H.Q8_0, H.Q4_0, 64, 1600, 33), (H.Q8_0, H.Q4K, 256, 2048, 33), (H.Q8_0, H.Q4K, 256, 2304, 33),
+@pytest.mark.parametrize("gdt,ddt,ne,nff,rows,K", [
+    # from 1024 h rows on a wavefront each, with one to four chunks per lane (64 to 2048 elements, the last chunk full or not), with and
+    # without group sums behind them (Q4_K, Q5_K down); row counts that are no multiple of a block's four
+    (H.Q8_0, H.Q8_0, 64, 64, 343, 3), (H.Q8_0, H.Q4K, 256, 512, 256, 4), (H.Q8_0, H.Q5K, 256, 768, 343, 3), (H.Q8_0, H.Q4K, 256, 1024, 343, 3),
+    (H.Q8_0, H.Q5K, 256, 1280, 205, 5), (H.Q8_0, H.Q4K, 256, 1536, 343, 3), (H.Q8_0, H.Q4_0, 64, 1600, 343, 3), (H.Q8_0, H.Q6K, 256, 1792, 342, 3),
+    (H.Q8_0, H.Q4K, 256, 2048, 343, 3),
+    # a block each: fewer rows, longer ones
+    (H.Q8_0, H.Q5K, 256, 768, 341, 3), (H.Q8_0, H.Q4K, 256, 2304, 343, 3),
 ])
-def test_activated_rows_to_f16(be, gdt, ddt, ne, nff, rows):
-    """Rows of h of any length, among them some of zeros and some a million times larger: each has a scale of its own."""
+def test_activated_rows_to_f16(be, gdt, ddt, ne, nff, rows, K):
+    """Rows of h of any length, among them some of zeros and some a thousand times larger: each has a scale of its own, and the bits
+    that it has in a small batch, whose rows take a block each."""
     rng = np.random.default_rng(ddt * 67 + nff)
-    E = 3
+    E = 7
     x = rng.standard_normal((rows, ne)).astype(np.float32)
     x[::5] = 0.0
     x[1::5] *= 1000.0
     router = np.zeros((E, ne), np.float32)
     gate, up, down = _bank_weights(rng, E, nff, ne, gdt, ddt)
-    sel = rng.integers(0, E, (rows, 1)).astype(np.int32)
-    g, ids = moe_graph(rows, ne, E, 1, nff, DType(gdt), DType(ddt), with_expert_ids=True)
-    out, _, _ = _run_batched(be, g, ids, dict(x=x, router=router, gate=gate, up=up, down=down, expert_ids=sel), rows, ne)
-    ref = O.moe_ffn(x, router, gate, up, down, ne=ne, n_expert=E, n_used=1, n_ff_exp=nff, gate_dtype=gdt, down_dtype=ddt,
-                    expert_ids=sel)["dst"]
+    sel = np.argsort(rng.random((rows, E)), axis=1)[:, :K].astype(np.int32)
+    g, ids = moe_graph(rows, ne, E, K, nff, DType(gdt), DType(ddt), with_expert_ids=True)
+    data = dict(x=x, router=router, gate=gate, up=up, down=down, expert_ids=sel)
+    out, _, _ = _run_batched(be, g, ids, data, rows, ne)
+    ref = O.moe_ffn(x, router, gate, up, down, ne=ne, n_expert=E, n_used=K, n_ff_exp=nff, gate_dtype=gdt, down_dtype=ddt,
+                    expert_ids=sel)["dst"].reshape(rows, ne)
     for r in range(rows):
         if r % 5 == 0:
             assert not out[r].any()
         else:
             assert H.rel_l2(out[r], ref[r]) < REL_L2_MFMA, r
+    p = rng.choice(rows, 40, replace=False)
+    g, ids = moe_graph(40, ne, E, K, nff, DType(gdt), DType(ddt), with_expert_ids=True)
+    few, _, _ = _run_batched(be, g, ids, dict(data, x=np.ascontiguousarray(x[p]), expert_ids=np.ascontiguousarray(sel[p])), 40, ne)
+    assert np.array_equal(bits(few), bits(out[p]))
 
 
 @pytest.mark.parametrize("rows,K", [(300, 8), (256, 8), (257, 8), (2100, 8), (5000, 4)])
