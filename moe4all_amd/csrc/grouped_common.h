@@ -107,6 +107,10 @@ __device__ __forceinline__ void dma16(const void* gsrc, uint32_t lds_base) {
 __device__ __forceinline__ void dma16(const void* gbase, uint32_t off, uint32_t lds_base) {
     asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" : : "v"(off), "s"(gbase), "s"(__builtin_amdgcn_readfirstlane(lds_base)) : "memory");
 }
+// 4 bytes per lane, to lds_base + 4 i
+__device__ __forceinline__ void dma4(const void* gbase, uint32_t off, uint32_t lds_base) {
+    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dword %0, %1" : : "v"(off), "s"(gbase), "s"(__builtin_amdgcn_readfirstlane(lds_base)) : "memory");
+}
 __device__ __forceinline__ uint32_t lds_address(const void* p) {
     return (uint32_t)(uintptr_t)(__attribute__((address_space(3))) const void*)p;
 }

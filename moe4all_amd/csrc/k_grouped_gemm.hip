@@ -166,32 +166,13 @@ __device__ __forceinline__ void gemm_tile(const GroupedParams& p, const Tile& t,
     constexpr bool kPartial = F::kBlock < F::kStep;                    // rows need not be whole steps
     constexpr int GPP = KC / 32;                                       // groups of 32 k in a piece
     constexpr int N = GPP * M, R = N < 8 ? N : 8;                                  // activation operands of a piece; those read ahead
-    static_assert(NA > 0 && 4 * M % G == 0 && (PPS == 1 || PPS == 2 || PPS == 4) && (2 * PPS - 1) * NA + NL < 63, "");
+    static_assert(NA > 0 && 4 * M % G == 0 && (PPS == 1 || PPS == 2 || (PPS == 4 && WB == 1)) && (2 * PPS - 1) * NA + NL < 63, "");
     const int tid = threadIdx.x, lane = tid & 63, col = lane & 15, kq = lane >> 4;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     uint8_t* const wl = lds + wave * (1024 * NL * WB);
     uint8_t* const al = lds + kGW * (1024 * NL * WB);
     uint8_t* const xl = al + kABufs * S::kPiece;
     const uint32_t wl0 = lds_address(wl), al0 = lds_address(al), xl0 = lds_address(xl);
-
-    // the token rows behind the lane's activation loads
-    uint32_t asrc[NA], xsrc = 0;
-    auto row_of = [&](int tok) -> uint32_t {
-        const int pr = t.p0 + min(tok, t.cnt - 1);
-        return (uint32_t)(DOWN ? pr : p.pair_row[pr]);
-    };
-#pragma unroll
-    for (int q = 0; q < NA; q++) asrc[q] = row_of((wave + 4 * q) * G + lane / CH);
-    if (F::kMin) xsrc = row_of(tid / 2);
-    uint32_t srow[2] = {0, 0};
-    float row_scale[2] = {1.0f, 1.0f};   // scales of tokens `lane` and 64 + lane
-    if (!DOWN || !p.out_f16 || t.e == p.sh_e) {
-#pragma unroll
-        for (int j = 0; j < (S::kWide ? 2 : 1); j++) srow[j] = row_of(64 * j + lane);
-#pragma unroll
-        for (int j = 0; j < (S::kWide ? 2 : 1); j++) row_scale[j] = p.a_scale[srow[j]];
-    }
-    asm volatile("" ::: "memory");
 
     // ---- weights: the lane's chunks 64 i + lane of the wave's 32 rows x kChunks
     constexpr int kStepBytes = F::kStep / F::kBlock * F::kBlockBytes;
@@ -229,6 +210,30 @@ __device__ __forceinline__ void gemm_tile(const GroupedParams& p, const Tile& t,
         F::load(wl + (WB == 2 ? (s & 1) * (1024 * NL) : 0) + n * 256 * F::kChunks, col, kq, r);
     };
 
+    // ---- The token rows behind the lane's activation loads.  Gate/up looks them up: the table comes through LDS (the place of the
+    // third piece, unused until step 0 is past its first barrier) ahead of the first weights, so that neither waits for the other; a
+    // load to registers would have to be waited for first, as the compiler's wait covers whatever is requested behind it.
+    constexpr int NR = DOWN ? 0 : S::kWide ? 2 : 1;   // loads of the table
+    const uint32_t* const rows = reinterpret_cast<const uint32_t*>(al + 2 * S::kPiece + wave * 512);
+#pragma unroll
+    for (int j = 0; j < NR; j++) dma4(p.pair_row, 4u * (uint32_t)(t.p0 + min(64 * j + lane, t.cnt - 1)), al0 + 2 * S::kPiece + wave * 512 + 256 * j);
+    request(0);
+    if (!DOWN) wait_loads<NL>();
+    auto row_of = [&](int tok) -> uint32_t {
+        const int i = min(tok, t.cnt - 1);
+        return DOWN ? (uint32_t)(t.p0 + i) : rows[i];
+    };
+    uint32_t asrc[NA], xsrc = 0;
+#pragma unroll
+    for (int q = 0; q < NA; q++) asrc[q] = row_of((wave + 4 * q) * G + lane / CH);
+    if (F::kMin) xsrc = row_of(tid / 2);
+    float row_scale[2] = {1.0f, 1.0f};   // scales of tokens `lane` and 64 + lane
+    if (!DOWN || !p.out_f16 || always) {
+#pragma unroll
+        for (int j = 0; j < (S::kWide ? 2 : 1); j++) row_scale[j] = p.a_scale[row_of(64 * j + lane)];
+    }
+    asm volatile("" ::: "memory");
+
     // ---- activations: a wave's groups of a piece are wave, wave + 4, ..; a group is G whole token pieces of 1024 / G bytes;
     // 16-byte chunk c of token t lies at place c ^ turn(t), so that sixteen tokens reading the same chunk hit distinct banks
     auto turn = [](int tok) { return CH >= 16 ? tok & 15 : rot7(tok) & (CH - 1); };
@@ -260,28 +265,12 @@ __device__ __forceinline__ void gemm_tile(const GroupedParams& p, const Tile& t,
     // same order as if two steps had come before.
     const bool two = WB == 2 && n_steps > 1;
     if (PPS != 4) fetch_sums(0);
-    if (PPS == 1) {
-        fetch(0, 0);
-        request(0);
-        fetch(1, 1);
-        if (two) request(1);
-        if (two) wait_loads<NA + NL>();
-        else wait_loads<NA>();
-    } else if (PPS == 2) {
-        request(0);
-        fetch(0, 0);
-        if (two) request(1);
-        fetch(1, 1);
-        if (two) wait_loads<2 * NA + NL>();
-        else wait_loads<2 * NA>();
-    } else {
-        request(0);
-        if (two) request(1);
-        fetch(0, 0);
-        fetch(1, 1);
-        if (two) wait_loads<2 * NA + NL>();
-        else wait_loads<2 * NA>();
-    }
+    fetch(0, 0);
+    if (PPS == 1) fetch(1, 1);
+    if (two) request(1);
+    if (PPS != 1) fetch(1, 1);
+    if (two) wait_loads<(PPS == 1 ? 1 : 2) * NA + NL>();
+    else wait_loads<(PPS == 1 ? 1 : 2) * NA>();
 #pragma unroll
     for (int n = 0; n < NB; n++) read_weights(0, n, raw[n]);
 #pragma unroll
@@ -420,10 +409,9 @@ __device__ __forceinline__ void gemm_tile(const GroupedParams& p, const Tile& t,
                 for (int n = 0; n < NB; n++)
                     if (i < N && gp + 1 < GPP && m == M * (2 * n + 1) / 4) b[(gp + 1) & 1][n] = unpack(gp + 1, n);
                 if (kMore > 0 && PPS == 4 && sub == 3) {
-                    // the next step's weights: landed by the last barrier (WB = 1), or at most what was requested behind them in flight
+                    // the next step's weights, which landed by the last barrier
 #pragma unroll
                     for (int n = 0; n < NB; n++) {
-                        if (WB == 2 && n == 0 && i == 1) wait_loads<(kMore >= WB ? NL : 0) + 5 * NA>();
                         if (i == 1 + n) read_weights(s + 1, n, next[n]);
                         if (i == (N > 8 ? M + 2 : 4) + n) next_st[n] = F::prep(next[n], kq);
                     }
@@ -631,8 +619,11 @@ __device__ __forceinline__ void unit_tile(const GroupedParams& p, const Tile& t,
 // nothing to do (the grid is an upper bound).
 __device__ __forceinline__ bool gemm_item(const GroupedParams& p, Tile& t, int& col) {
     const int item = (int)blockIdx.x, tile = p.n_tiles_n == 1 ? item : (int)__umulhi((uint32_t)item, p.n_tiles_rcp);   // item / n_tiles_n: exact below 2^32 / n_tiles_n
-    if (tile >= p.tiles[0].x) return false;
-    const int4 b = p.tiles[1 + tile];   // expert, first pair, pairs
+    // expert, first pair, pairs: read beside the number of tiles, not behind it (the grid is the table's size times n_tiles_n)
+    const int n_tiles = p.tiles[0].x;
+    const int4 b = p.tiles[1 + tile];
+    asm volatile("" : : "s"(n_tiles), "s"(b.x), "s"(b.y), "s"(b.z));
+    if (tile >= n_tiles) return false;
     t = Tile{b.x, b.y, b.z};
     col = item - tile * p.n_tiles_n;
     return true;
@@ -703,7 +694,8 @@ void gemm(hipStream_t s, const GroupedParams& p) {
     const int width = DOWN ? 32 * kGW : 16 * kGW;
     q.n_tiles_n = (p.N + width - 1) / width;
     q.n_tiles_rcp = (uint32_t)((0x100000000ull + q.n_tiles_n - 1) / q.n_tiles_n);
-    const dim3 grid((unsigned)((gemm_max_tiles(p.n_pairs, p.n_expert, 1 << p.tile_log2) * q.n_tiles_n + 7) & ~7));   // whole rounds of the 8 XCDs
+    const int items = gemm_max_tiles(p.n_pairs, p.n_expert, 1 << p.tile_log2) * q.n_tiles_n;
+    const dim3 grid((unsigned)(F::kUnits && DOWN && p.n_expert == 1 ? (items + 7) & ~7 : items));   // (dense_item: whole rounds of the 8 XCDs)
     if constexpr (F::kUnits) {
         INFR_LDS_LIMIT((grouped_gemm_units<F, DOWN>), (int)unit_lds<F>());
         INFR_LAUNCH((grouped_gemm_units<F, DOWN>), grid, dim3(kGW * 64), unit_lds<F>(), s, q);
