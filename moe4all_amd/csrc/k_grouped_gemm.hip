@@ -62,9 +62,10 @@ constexpr size_t gemm_lds() {
     return a > b ? (a > c ? a : c) : b > c ? b : c;
 }
 
-// Waits until at most N of the wave's loads are in flight, and for its LDS reads.
+// Waits until at most N of the wave's loads are in flight; wait_lds for its LDS reads; wait_barrier for both and the other waves.
 template <int N>
 __device__ __forceinline__ void wait_loads() { asm volatile("s_waitcnt vmcnt(%0)" : : "n"(N) : "memory"); }
+__device__ __forceinline__ void wait_lds() { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); }
 template <int N>
 __device__ __forceinline__ void wait_barrier() { asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" : : "n"(N) : "memory"); }
 
@@ -164,6 +165,12 @@ __device__ __forceinline__ void gemm_tile(const GroupedParams& p, const Tile& t,
     constexpr int NC = 16 * NB * F::kChunks, NL = kWLoads<F>;          // 16-byte chunks of a wave's step, loads of a lane
     constexpr int NA = (FEW ? 2 : 4) * M / G;                          // loads of a lane per piece
     constexpr bool kPartial = F::kBlock < F::kStep;                    // rows need not be whole steps
+    // One step of weights in LDS and a tile bound by their stream: a wave's weights of the next step are requested as soon as this step's
+    // are in registers, ahead of the barrier, not between the matrix instructions.  us per layer, without and with: 34 rows of 256
+    // experts of 4096 x 1536 beside one in Q4_K / Q6_K 532 and 524, in Q8_0 783 and 767; 90 rows of 128 experts of 2048 x 768 in
+    // Q4_K / Q6_K 122.6 and 121.7, in MXFP4 107.1 and 105.3.  (Not where workgroups have a CU each: 64 rows of 32 experts of
+    // 1024 x 512 in Q5_K 46.4 and 47.2; those take the other kernel.)
+    constexpr bool kEarly = WB == 1 && M <= 2;
     constexpr int GPP = KC / 32;                                       // groups of 32 k in a piece
     constexpr int N = GPP * M, R = N < 8 ? N : 8;                                  // activation operands of a piece; those read ahead
     static_assert(NA > 0 && 4 * M % G == 0 && (PPS == 1 || PPS == 2 || (PPS == 4 && WB == 1)) && (2 * PPS - 1) * NA + NL < 63, "");
@@ -261,8 +268,8 @@ __device__ __forceinline__ void gemm_tile(const GroupedParams& p, const Tile& t,
 
     // ---- Transfers land in the order they were requested in; what may be in flight where something is waited for is what was
     // requested behind it.  The order of a step: behind its first barrier group sums, the piece after next, the weights of
-    // the next step (WB = 1) or of the one after it (WB = 2); behind each further barrier the piece after next.  Here the
-    // same order as if two steps had come before.
+    // the next step (WB = 1) or of the one after it (WB = 2); behind each further barrier the piece after next; kEarly: at its end
+    // the weights of the step after next.  Here the same order as if two steps had come before.
     const bool two = WB == 2 && n_steps > 1;
     if (PPS != 4) fetch_sums(0);
     fetch(0, 0);
@@ -273,6 +280,10 @@ __device__ __forceinline__ void gemm_tile(const GroupedParams& p, const Tile& t,
     else wait_loads<(PPS == 1 ? 1 : 2) * NA>();
 #pragma unroll
     for (int n = 0; n < NB; n++) read_weights(0, n, raw[n]);
+    if (kEarly && n_steps > 1) {
+        wait_lds();
+        request(1);
+    }
 #pragma unroll
     for (int n = 0; n < NB; n++) st[n] = F::prep(raw[n], kq);
 
@@ -324,9 +335,9 @@ __device__ __forceinline__ void gemm_tile(const GroupedParams& p, const Tile& t,
                 }
             } else if (PPS == 2) {
                 if (sub == 0) {
-                    if (WB == 2 && more) wait_barrier<NL + NA>();
+                    if ((WB == 2 || kEarly) && more) wait_barrier<NL + NA>();
                     else wait_barrier<NA>();
-                } else if (req) {
+                } else if (kEarly ? more : req) {
                     wait_barrier<NL + NA>();
                 } else if (more) {
                     wait_barrier<NA>();
@@ -341,7 +352,7 @@ __device__ __forceinline__ void gemm_tile(const GroupedParams& p, const Tile& t,
             cur = cur == 2 ? 0 : cur + 1;
             if (sub == 0) fetch_sums(PPS == 4 ? s : s + 1);
             // (no pieces follow those of the last step; where that is not known here, the row's end is fetched again)
-            const int na = kMore == 0 && sub + 2 >= PPS ? 0 : NA, nd = na + (sub == 0 && (kMore < 0 || req) ? NL : 0);
+            const int na = kMore == 0 && sub + 2 >= PPS ? 0 : NA, nd = na + (sub == 0 && !kEarly && (kMore < 0 || req) ? NL : 0);
             const bool mins = F::kMin && !LO && sub == PPS - 1;
             const int ns = mins ? N + M : N;
             auto operand = [&](int i) {
@@ -429,9 +440,13 @@ __device__ __forceinline__ void gemm_tile(const GroupedParams& p, const Tile& t,
         }
         if (more) {
             if (PPS != 4) {
-                wait_loads<WB == 1 ? (PPS - 1) * NA : (2 * PPS - 1) * NA + (kMore >= WB ? NL : 0)>();
+                wait_loads<kEarly ? PPS * NA : WB == 1 ? (PPS - 1) * NA : (2 * PPS - 1) * NA + (kMore >= WB ? NL : 0)>();
 #pragma unroll
                 for (int n = 0; n < NB; n++) read_weights(s + 1, n, next[n]);
+                if (kEarly && s + 2 < n_steps) {
+                    wait_lds();
+                    request(s + 2);
+                }
 #pragma unroll
                 for (int n = 0; n < NB; n++) next_st[n] = F::prep(next[n], kq);
             }
