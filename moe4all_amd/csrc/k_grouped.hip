@@ -139,19 +139,20 @@ __global__ __launch_bounds__(256) void route_rows_to_f16_kernel(RouteParams rp, 
 
 // --------------------------------------------------------------------------------------------
 // One block of four or sixteen wavefronts per expert e in 0..n_expert; the extra one marks pairs whose id is
-// out of range.  The block stages the pair ids in LDS (16-bit, chunks of 16384), counts every expert's pairs (those of the experts below e give the bucket's offset and its
-// tiles' places in the tile table), and then scatters the pairs equal to e: each wavefront takes a contiguous part of the chunk, the parts' hit
-// counts give every wavefront its base, and inside a part a wave-wide prefix keeps the flat
-// (row, rank) order, so buckets come out rows ascending.
-constexpr int kBucketChunk = 16384;
+// out of range.  The block stages the pair ids in LDS (16-bit, in chunks), counts every expert's pairs (those of the experts below e
+// give the bucket's offset and its tiles' places in the tile table), and then scatters the pairs equal to e: each wavefront takes a
+// contiguous part of the chunk, the parts' hit counts give every wavefront its base, and inside a part a wave-wide prefix keeps the
+// flat (row, rank) order, so buckets come out rows ascending.  Four wavefronts take up to kBucketFew pairs, one chunk.
+constexpr int kBucketFew = 2048, kBucketMany = 16384;
 template <int NT>
 __global__ __launch_bounds__(NT) void bucket_kernel(const int32_t* __restrict__ ids, int n_pairs, int n_expert,
                                                      int n_used, int32_t* __restrict__ offsets, int32_t* __restrict__ pair_src,
                                                      int32_t* __restrict__ slot_pair, int32_t* __restrict__ pair_row,
                                                      int4* __restrict__ tiles, int tile, int by_size, int always_rows) {
-    __shared__ uint16_t s_ids[kBucketChunk];
-    __shared__ uint32_t s_hist[2048];
+    constexpr int kBucketChunk = NT == 256 ? kBucketFew : kBucketMany;
     constexpr int NW = NT / 64, NL = kBucketChunk / 4 / NT;
+    __shared__ __attribute__((aligned(16))) uint16_t s_ids[kBucketChunk];
+    __shared__ uint32_t s_hist[2048];
     __shared__ uint32_t s_cnt[3 * NW];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const uint32_t e = blockIdx.x;
@@ -196,7 +197,7 @@ __global__ __launch_bounds__(NT) void bucket_kernel(const int32_t* __restrict__ 
         for (int d = 32; d >= 1; d >>= 1) v += __shfl_xor(v, d, 64);
         return v;
     };
-    const bool single = n_pairs <= kBucketChunk;   // a single chunk stays staged for the second pass
+    const bool single = NT == 256 || n_pairs <= kBucketChunk;   // a single chunk stays staged for the second pass
 
     // ---- pass 0: how many pairs each expert has; from that the bucket's offset and its tiles' places in the tile table
     for (int i = tid; i < n_expert; i += NT) s_hist[i] = 0;
@@ -584,7 +585,7 @@ void launch_bucket(hipStream_t s, const int32_t* ids, int n_pairs, int n_expert,
                    int32_t* slot_pair, int32_t* pair_row, int4* tiles, int tile, int by_size, int always_rows) {
     // sixteen wavefronts where the ids are many: staging, counting and scattering are each a serial chain per wavefront
     // (rows of 128 experts, top-8: 2048 20.3 -> 14.6 us, 512 9.9 -> 8.8, 333 8.2 -> 7.5)
-    if (n_pairs > 2048)
+    if (n_pairs > kBucketFew)
         INFR_LAUNCH(bucket_kernel<1024>, dim3(n_expert + 1), dim3(1024), 0, s, ids, n_pairs, n_expert, n_used, offsets, pair_src,
                     slot_pair, pair_row, tiles, tile, by_size, always_rows);
     else
