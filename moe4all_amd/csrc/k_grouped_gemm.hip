@@ -743,25 +743,37 @@ bool gemm_takes_always(int dt) { return unit_format_block(dt) != 0 && !grouped_r
 
 // Tiles of 64 pairs on three workgroups per CU, or of 128 on two?  128 tokens share a weight's unpacking, and the kernel of two has
 // the LDS for two steps of weights ahead of a small tile; three hide more of everything else.  us per layer, 64 | 128 (128 experts of
-// 2048 x 768 unless said otherwise; uniform routing, then Zipf(1.1)):
-//   Q4_K / Q6_K   200 rows 137 103 | 139 100, 512 rows 167 165 | 175 164, 1024 rows 237 242 | 227 236, 2048 rows 383 372 | 373 355
-//   Q5_K / Q6_K    40 rows 131 | 128, 512 rows 181 179 | 186 174, 1024 rows 256 262 | 238 250
-//   Q8_0           40 rows 165 | 159, 512 rows 214 210 | 208 199, 2048 rows 437 413 | 406 387
-//   Q4_0          512 rows 161 154 | 172 156, 1024 rows 228 232 | 227 228;  IQ4_XS 512 rows 171 169 | 180 166, 1024 rows 244 255 | 231 243
-//   MXFP4          64 rows 109 | 107, 512 rows 148 140 | 157 137, 500 rows of 2880 x 2880, top-4 - 390 | - 365
-//   8 experts of 4096 x 14336, top-2, Q4_K / Q6_K: 40 rows 585 | 498;  32 experts of 1024 x 512, 2000 rows - 155 | - 162
-//   32 experts of 1024 x 512, Q8_0, 110 rows, Zipf(1.1), five layers: 289 | 331
-// So: 128 with long rows, from 40 pairs per expert on if that leaves three rounds of workgroups, with Q8_0, and with Q5_K and MXFP4
-// below 24 pairs per expert.  But launches that do not fill the chip once: 64, so that a large bucket is spread over more
-// workgroups (up to 64 rows both cut alike, and the kernel of two is the faster one).
+// 2048 x 768 unless said otherwise; uniform routing, then Zipf(1.1) where given):
+//   Q4_K / Q6_K   34 rows 114 | 111, 64 rows 119 | 118, 90 rows 122 82 | 121 83, 200 rows 132 105 | 132 100, 300 rows 140 119 | 142 116,
+//                 512 rows 167 165 | 175 164, 1024 rows 237 242 | 227 236, 2048 rows 383 372 | 373 355
+//   Q5_K / Q6_K   34 rows 124 | 121, 64 rows 130 | 128, 130 rows 137 92 | 136 96, 200 rows 143 111 | 143 105, 300 rows 150 124 | 153 122,
+//                 512 rows 181 179 | 186 174, 1024 rows 256 262 | 238 250
+//   Q8_0          34 rows 156 | 152, 90 rows 169 106 | 165 99, 200 rows 178 131 | 176 123, 512 rows 214 210 | 208 199, 2048 rows 437 413 | 406 387
+//   Q4_0          34 rows 110 | 112, 90 rows 115 77 | 119 78, 200 rows 125 99 | 126 96, 300 rows 130 111 | 138 109, 512 rows 161 154 | 172 156
+//   IQ4_XS        34 rows 126 | 127, 90 rows 132 86 | 133 86, 300 rows 143 121 | 151 117, 512 rows 171 169 | 180 166, 1024 rows 244 255 | 231 243
+//   MXFP4         34 rows 99 | 97, 90 rows 108 71 | 105 70, 200 rows 116 92 | 113 86, 300 rows 123 103 | 121 100, 512 rows 148 140 | 157 137
+//   256 experts of 4096 x 1536 beside one: Q4_K / Q6_K 34 rows 524 | 539, 64 rows 689 | 706, 90 rows 797 465 | 810 471;  Q5_K / Q6_K 64 rows
+//                 787 | 797, 90 rows 914 524 | 919 526;  Q4_0 200 rows 670 416 | 697 416;  Q8_0 34 rows 767 | 760, 200 rows 1137 656 | 1102 630;
+//                 MXFP4 34 rows 614 | 614, 200 rows 611 379 | 596 371
+//   32 experts of 1024 x 512: Q8_0 34 rows 48.5 | 43.5, 90 rows 51.8 53.0 | 48.5 55.8, 130 rows 53.4 54.8 | 51.8 58.1, 200 rows 55.0 56.1 |
+//                 54.5 59.6;  Q4_K / Q6_K 34 rows 43.3 | 42.8, 90 rows 46.7 49.8 | 47.6 54.2, 200 rows 52.6 52.0 | 51.9 58.6;  64 rows in Q4_K /
+//                 Q6_K 45.5 | 46.1, Q5_K / Q6_K 47.2 | 47.5, MXFP4 43.4 | 40.9
+//   8 experts of 4096 x 14336, top-2, Q4_K / Q6_K: 34 rows 241 | 230, 100 rows 272 328 | 264 323, 1000 rows 1155 1161 | 1003 1021;  64 of
+//                 4352 x 1024, top-4: 64 rows 164 | 155, 100 rows 167 136 | 158 140, 1000 rows 289 297 | 266 286;  32 of 2048 x 5120, top-4:
+//                 64 rows 178 | 175, 100 rows 182 172 | 182 179, 1000 rows 486 511 | 453 465;  Q8_0 and Q5_K / Q6_K on these shapes alike
+// So with 128: rows beyond 4096; from 40 pairs per expert on if that leaves three rounds of workgroups; Q8_0; below 24 pairs per expert MXFP4 and, in
+// rows of 2048 and less (longer ones hide a workgroup's start by themselves), Q4_K and Q5_K.  Launches that do not fill the chip
+// once: 64, so that a large bucket is spread over more workgroups, but up to 64 rows, which both cut alike, and for Q8_0 below 40 pairs per
+// expert (uniform routing gains what skewed loses) 128.
 int gemm_tile_log2(int gate_dt, int down_dt, int rows, int n_pairs, int n_expert, int ne, int nff) {
     if (grouped_reads_units(gate_dt) || grouped_reads_units(down_dt)) return 6;
     const int mean = n_pairs / n_expert;
+    const bool k_quant = gate_dt == INFR_Q4K || gate_dt == INFR_Q5K;
     if (ne > 4096 || nff > 4096) return 7;
-    if ((int64_t)gemm_max_tiles(n_pairs, n_expert, 128) * ((nff + 63) / 64) < 512) return rows <= 64 ? 7 : 6;
+    if ((int64_t)gemm_max_tiles(n_pairs, n_expert, 128) * ((nff + 63) / 64) < 512) return rows <= 64 || (gate_dt == INFR_Q8_0 && mean < 40) ? 7 : 6;
     if (gate_dt == INFR_Q8_0) return 7;
     if (mean >= 40) return (int64_t)gemm_max_tiles(n_pairs, n_expert, 128) * ((nff + 63) / 64) >= 3 * 512 ? 7 : 6;
-    return (gate_dt == INFR_Q5K || gate_dt == INFR_MXFP4) && mean < 24 ? 7 : 6;
+    return mean < 24 && (gate_dt == INFR_MXFP4 || (k_quant && ne <= 2048)) ? 7 : 6;
 }
 
 template <bool DOWN>
