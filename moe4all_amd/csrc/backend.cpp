@@ -923,7 +923,7 @@ extern "C" infr_status infr_hip_compile(infr_hip_backend* be, const infr_graph* 
                 if (bucketed) {
                     plan->moe[oi].tables_off = arena;
                     arena += round_up(((size_t)m.n_expert + 2) * 4, 256) + 4 * round_up(pairs * 4 + 4, 256) +
-                             round_up(((size_t)infr::gemm_max_tiles((int)pairs, (int)m.n_expert, infr::kIntTok) + 1) * sizeof(int4), 256);
+                             round_up(infr::gemm_table_slots((int)pairs, (int)m.n_expert, infr::kIntTok) * sizeof(int4), 256);
                     shared += round_up((size_t)plan->moe[oi].k_parts * pairs * m.ne * 4, 256);
                 }
                 if (!batched && !bucketed) shared += round_up(pairs * m.ne * 4, 256);   // per-pair down results of the unit kernels
@@ -971,7 +971,7 @@ extern "C" infr_status infr_hip_compile(infr_hip_backend* be, const infr_graph* 
                     plan->lin[oi].on = l.m >= min_rows && l.m <= (1u << 24) && infr::grouped_supported(dt, (int)l.in_f);
                     if (plan->lin[oi].on) {
                         plan->lin[oi].offsets_off = arena;
-                        arena += 256 + round_up(((size_t)infr::gemm_max_tiles((int)l.m, 1, 1 << infr::kLinearTileLog2) + 1) * sizeof(int4), 256);
+                        arena += 256 + round_up(infr::gemm_table_slots((int)l.m, 1, 1 << infr::kLinearTileLog2) * sizeof(int4), 256);
                         const size_t shared = round_up((size_t)l.m * l.in_f * 2, 256) + round_up((size_t)l.m * 4, 256) +
                                               round_up((size_t)l.m * l.in_f / 8, 256);
                         if (shared > shared_need) shared_need = shared;
@@ -1295,7 +1295,7 @@ extern "C" infr_status infr_hip_compile(infr_hip_backend* be, const infr_graph* 
         const size_t rows = s.rows, pairs = rows * m.n_used, all = pairs + s.always_rows;
         s.tables_off = arena;
         arena += round_up(((size_t)m.n_expert + 2) * 4, 256) + 3 * round_up(pairs * 4 + 4, 256) + round_up(all * 4 + 4, 256) +
-                 round_up(((size_t)infr::gemm_max_tiles((int)all, (int)m.n_expert + (s.always_rows ? 1 : 0), 1 << s.tile_log2) + 1) * sizeof(int4), 256);
+                 round_up(infr::gemm_table_slots((int)all, (int)m.n_expert + (s.always_rows ? 1 : 0), 1 << s.tile_log2) * sizeof(int4), 256);
         const size_t shared = round_up((pairs + rows) * m.n_ff_exp * 4 + 4, 256) + round_up(rows * m.ne * 2, 256) + round_up(rows * 4, 256) +
                               round_up(rows * m.ne / 8, 256) + round_up(all * m.n_ff_exp * 2, 256) + round_up(all * 4, 256) +
                               round_up(all * m.n_ff_exp / 8, 256) + round_up(pairs * m.ne * 4, 256);

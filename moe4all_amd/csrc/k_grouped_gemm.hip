@@ -23,7 +23,7 @@
 // 165 MB of Q6_K down rows: 50 and 40 us; a bare read in the same pattern 42 and 34).  Full tiles: a matrix instruction keeps a SIMD's issue
 // of vector instructions busy for 8 of its 16 cycles and each vector instruction for 4 (measured: two are free beside
 // a matrix instruction, every further one costs its own time), so what counts is vector instructions per matrix instruction:
-// 6.2 on 64 tokens per unpacked weight, 2.6 on 128 (4 x 2.6 + 8 = 18.6 cycles for 16).  128 tokens of each of 128 experts
+// 6.2 on 64 tokens per unpacked weight, 2.6 on 128 (4 x 2.6 + 8 = 18.4 cycles for 16).  128 tokens of each of 128 experts
 // of 2048 x 768, gate/up and down, us: Q4_K / Q6_K 130 and 88 against 158 and 107 for tiles of 64 with weights through registers,
 // Q8_0 154 and 93 (198 and 110).  Half of the rest goes to the barriers and transfers of a step (8900 cycles per step of 256 k
 // for two waves per SIMD before the transfers were spread over the matrix instructions, 4600 of them in matrix instructions).
@@ -630,17 +630,19 @@ __device__ __forceinline__ void unit_tile(const GroupedParams& p, const Tile& t,
 // so that none is left running alone at the end.  (A contiguous eighth of the items per XCD, experts ascending, has an expert's
 // tile read from one L2 only, but left the CUs idle for 8 to 39 % of a launch with skewed experts: 1500 token rows of 256
 // experts of 4096 x 1536 1331 us a layer, so 1184, 512 rows of 128 experts of 2048 x 768 in Q8_0 210 and 198; classes without order
-// inside: neighbouring experts' weights read one after the other, 1 to 2 % of a batch of small tiles.)  Uniform; false when there is
-// nothing to do (the grid is an upper bound).
+// inside: neighbouring experts' weights read one after the other, 1 to 2 % of a batch of small tiles.)  deal_log2 = 3, launches with
+// about one item per CU, where there is nothing to balance: tile 8 i + j on XCD j, whose L2 alone reads the tile's rows.  Uniform;
+// false when there is nothing to do (the grid is an upper bound).
 __device__ __forceinline__ bool gemm_item(const GroupedParams& p, Tile& t, int& col) {
-    const int item = (int)blockIdx.x, tile = p.n_tiles_n == 1 ? item : (int)__umulhi((uint32_t)item, p.n_tiles_rcp);   // item / n_tiles_n: exact below 2^32 / n_tiles_n
-    // expert, first pair, pairs: read beside the number of tiles, not behind it (the grid is the table's size times n_tiles_n)
+    const int item = (int)blockIdx.x >> p.deal_log2, group = p.n_tiles_n == 1 ? item : (int)__umulhi((uint32_t)item, p.n_tiles_rcp);   // item / n_tiles_n: exact below 2^32 / n_tiles_n
+    const int tile = (group << p.deal_log2) + ((int)blockIdx.x & ((1 << p.deal_log2) - 1));
+    // expert, first pair, pairs: read beside the number of tiles, not behind it (the grid is within the table)
     const int n_tiles = p.tiles[0].x;
     const int4 b = p.tiles[1 + tile];
     asm volatile("" : : "s"(n_tiles), "s"(b.x), "s"(b.y), "s"(b.z));
     if (tile >= n_tiles) return false;
     t = Tile{b.x, b.y, b.z};
-    col = item - tile * p.n_tiles_n;
+    col = item - group * p.n_tiles_n;
     return true;
 }
 
@@ -703,13 +705,20 @@ __global__ __launch_bounds__(kGW * 64, 3) void grouped_gemm_units(GroupedParams 
     else unit_tile<F, DOWN, 4>(p, t, n0, lds_gemm);
 }
 
+// Where a tile's columns go to one XCD (gemm_item): up to one and a half items per CU by the launch's bound, and four tiles per XCD
+// (of fewer the XCDs' shares would differ).  us, columns side by side and so: 12 layers of 32 experts of 1024 x 512, 48 rows in Q4_K / Q6_K
+// 527 and 519, Q5_K / Q6_K 550 and 537, MXFP4 473 and 462, 90 rows 553 and 543, 561 and 554, 521 and 516; 2048 rows of a dense 4096 x 1024 in Q8_0
+// 52.7 and 48.4.  Larger launches of skewed buckets lose by it (200 rows of the same experts, Zipf(1.1): 621 and 642).
+constexpr int kDealTiles = 32, kDealItems = 384;
 template <class F, bool DOWN>
 void gemm(hipStream_t s, const GroupedParams& p) {
     GroupedParams q = p;
     const int width = DOWN ? 32 * kGW : 16 * kGW;
     q.n_tiles_n = (p.N + width - 1) / width;
     q.n_tiles_rcp = (uint32_t)((0x100000000ull + q.n_tiles_n - 1) / q.n_tiles_n);
-    const int items = gemm_max_tiles(p.n_pairs, p.n_expert, 1 << p.tile_log2) * q.n_tiles_n;
+    const int tiles = gemm_max_tiles(p.n_pairs, p.n_expert, 1 << p.tile_log2);
+    q.deal_log2 = !F::kUnits && tiles >= kDealTiles && tiles * q.n_tiles_n <= kDealItems ? 3 : 0;
+    const int items = (q.deal_log2 ? (tiles + 7) & ~7 : tiles) * q.n_tiles_n;
     const dim3 grid((unsigned)(F::kUnits && DOWN && p.n_expert == 1 ? (items + 7) & ~7 : items));   // (dense_item: whole rounds of the 8 XCDs)
     if constexpr (F::kUnits) {
         INFR_LDS_LIMIT((grouped_gemm_units<F, DOWN>), (int)unit_lds<F>());

@@ -180,7 +180,8 @@ struct GroupedParams {
     int act, has_clamp; float clamp; int weight_before;
     int n_tiles_n;            // set by the launcher
     uint32_t n_tiles_rcp;     // set by the launcher: ceil(2^32 / n_tiles_n)
-    const int4* tiles;        // block formats: the tile table of launch_bucket, up to gemm_max_tiles(n_pairs, n_expert) tiles
+    int deal_log2;            // set by the launcher: see gemm_item
+    const int4* tiles;        // block formats: the tile table of launch_bucket, gemm_table_slots(n_pairs, n_expert, 1 << tile_log2) slots
     int tile_log2;            // block formats: the table's tiles hold up to 1 << tile_log2 pairs
     const int32_t* pair_row;  // block formats, gate/up: token row of each pair
     const uint32_t* a_sum;    // formats with minimums: sums of a over groups of 32, see launch_rows_to_f16
@@ -216,6 +217,7 @@ void launch_mask_dropped_pairs(hipStream_t s, const int32_t* ids, const float* w
 constexpr int kIntTok = 8;   // pairs of a tile of the integer kernels
 constexpr int kLinearTileLog2 = 6;   // tiles of a Linear's rows: 64 (600 rows of 4096 x 1536, three Linears beside a MoeFfn: 965 us, of 128 996)
 inline int gemm_max_tiles(int n_pairs, int n_expert, int tile) { return n_pairs / tile + (n_expert < n_pairs ? n_expert : n_pairs); }
+inline size_t gemm_table_slots(int n_pairs, int n_expert, int tile) { return 1 + (((size_t)gemm_max_tiles(n_pairs, n_expert, tile) + 7) & ~(size_t)7); }   // whole eights
 void launch_bucket(hipStream_t s, const int32_t* ids, int n_pairs, int n_expert, int n_used, int32_t* offsets, int32_t* pair_src,
                    int32_t* slot_pair, int32_t* pair_row = nullptr, int4* tiles = nullptr, int tile = 1, int by_size = 0,
                    int always_rows = 0);

@@ -168,6 +168,29 @@ def test_always_on_expert_in_the_batchs_gemms(be, gdt, ddt, ne, nff, rows, K, re
     assert H.rel_l2(outs[False], outs[True]) < 3e-5
 
 
+@pytest.mark.parametrize("gdt,ddt,ne,nff,rows,used", [
+    (H.Q4K, H.Q6K, 256, 256, 64, 24), (H.Q4K, H.Q6K, 512, 256, 200, 17), (H.Q5K, H.Q4K, 256, 512, 448, 5), (H.Q8_0, H.Q8_0, 320, 192, 448, 24),
+    (H.MXFP4, H.Q4_0, 192, 64, 150, 9), (H.IQ4_XS, H.IQ4_XS, 256, 256, 65, 1),
+])
+def test_tiles_dealt_to_the_xcds_in_small_launches(be, gdt, ddt, ne, nff, rows, used):
+    """From 32 tiles by the launch's bound on, and up to 384 items, the columns of a tile go to one XCD: 40 experts of which some are
+    selected, so that the tiles that there are end anywhere inside an eight, against 24 experts, whose tiles' columns lie side by side."""
+    rng = np.random.default_rng(gdt * 71 + rows)
+    E, few, K = 40, 24, 1
+    assert rows * K // 64 + few < 32 <= rows * K // 128 + E
+    x = rng.standard_normal((rows, ne)).astype(np.float32)
+    gate, up, down = (_zero_some_scales(w, dt, rng) for w, dt in zip(_bank_weights(rng, E, nff, ne, gdt, ddt), (gdt, gdt, ddt)))
+    sel = rng.permutation(few)[:used][rng.integers(0, used, (rows, K))].astype(np.int32)
+    outs = []
+    for n in (E, few):
+        cut = lambda w: w.reshape(E, -1)[:n].reshape(-1)  # noqa: E731
+        g, ids = moe_graph(rows, ne, n, K, nff, DType(gdt), DType(ddt), with_expert_ids=True)
+        outs.append(_run_batched(be, g, ids, dict(x=x, router=np.zeros((n, ne), np.float32), gate=cut(gate), up=cut(up), down=cut(down), expert_ids=sel), rows, ne)[0])
+    assert np.array_equal(bits(outs[0]), bits(outs[1]))
+    ref = O.moe_ffn(x, np.zeros((E, ne), np.float32), gate, up, down, ne=ne, n_expert=E, n_used=K, n_ff_exp=nff, gate_dtype=gdt, down_dtype=ddt, expert_ids=sel)
+    assert H.rel_l2(outs[0], ref["dst"].reshape(rows, ne)) < REL_L2_MFMA / 4
+
+
 INT_COUNTS = [0, 1, 3, 4, 5, 8, 9]   # tiles of up to 4 and up to 8 tokens
 
 
