@@ -964,8 +964,8 @@ extern "C" infr_status infr_hip_compile(infr_hip_backend* be, const infr_graph* 
                     c.set(INFR_ERR_INVALID, "Linear: w_off/out_f select rows outside the weight tensor");
                 if (c.st == INFR_OK) {
                     // a batch of rows (prefill): f16 operands on the matrix cores, as Op::MoeFfn does from the same row count
-                    // (one bucket means ceil(m / 128) x ceil(out_f / 256) tiles in all: below about a tile of rows the
-                    // GEMV kernels, which spread over the output rows, are faster)
+                    // (one bucket means ceil(m / 64) x ceil(out_f / 128) items in all: below kLinearBatchedMinRows the GEMV kernels,
+                    // which spread over the output rows, are faster and keep f32 accuracy)
                     const uint32_t min_rows = be->cfg.moe_batched_min_rows ? be->cfg.moe_batched_min_rows : kLinearBatchedMinRows;
                     const int dt = c.dt(l.weight);
                     plan->lin[oi].on = l.m >= min_rows && l.m <= (1u << 24) && infr::grouped_supported(dt, (int)l.in_f);
@@ -1880,6 +1880,7 @@ extern "C" infr_status infr_hip_execute(infr_hip_backend* be, infr_hip_plan* pla
                     q.offsets = (const int32_t*)((const char*)plan->arena + plan->lin[oi].offsets_off);
                     q.tiles = (const int4*)(q.offsets + 64);
                     q.tile_log2 = infr::kLinearTileLog2;
+                    q.dense = 1;
                     q.sh_e = -1;
                     q.w0 = w; q.w0_stride = 0;
                     q.out = (float*)ptr[l.dst];

@@ -74,9 +74,10 @@ __device__ __forceinline__ void wait_barrier() { asm volatile("s_waitcnt vmcnt(%
 // bits of the separate ops: on the way out, where one copy of the code serves all registers (1500 rows of 256 experts of
 // 4096 x 1536 beside one: 1053 us a layer with it, 1054 with the routed experts' exponential).
 // SILU: gate/up rows of a routed expert under a plain silu, in code of their own (all forms in one loop: 1.2 to 1.9 % slower batches).
+// s_scale: the tokens' row scales in LDS (unit formats; row_scale is then not read).
 template <class F, bool DOWN, int NB, int M, bool SILU>
 __device__ __forceinline__ void store_rows(const GroupedParams& p, const Tile& t, int n0, int wave, int lane, uint8_t* wl,
-                                           const float (&row_scale)[2], const float4v (&acc)[NB][M], const float (&dcur)[NB]) {
+                                           const float (&row_scale)[2], const float4v (&acc)[NB][M], const float (&dcur)[NB], const float* s_scale) {
     // Accumulator register q of
     // tile m: token 16 m + 4 kq + q, weight row col of operand n; token 16 m + 4 a + b lies in row 4 b + a, so that a
     // wave's write covers all banks.
@@ -101,10 +102,10 @@ __device__ __forceinline__ void store_rows(const GroupedParams& p, const Tile& t
 #pragma unroll
                     for (int n = 0; n < NB; n++) reinterpret_cast<_Float16*>(o)[16 * n + col] = (_Float16)(acc[n][m][q] * fin[n] * ds);
                 } else if (DOWN) {
-                    const float sc = __shfl(row_scale[m >> 2], tok & 63, 64) * ds;
+                    const float sc = (F::kUnits ? s_scale[tok] : __shfl(row_scale[m >> 2], tok & 63, 64)) * ds;
                     reinterpret_cast<float*>(o)[col] = (part ? acc[1][m][q] * fin[1] : acc[0][m][q] * fin[0]) * sc;
                 } else {
-                    const float sc = __shfl(row_scale[m >> 2], tok & 63, 64);
+                    const float sc = F::kUnits ? s_scale[tok] : __shfl(row_scale[m >> 2], tok & 63, 64);
                     float g = acc[0][m][q] * fin[0] * sc, u = acc[1][m][q] * fin[1] * sc;
                     if (SILU) {
                         g = silu_fast(g) * u;
@@ -147,11 +148,11 @@ __device__ __forceinline__ void store_rows(const GroupedParams& p, const Tile& t
 
 template <class F, bool DOWN, int NB, int M>
 __device__ __forceinline__ void store_tile(const GroupedParams& p, const Tile& t, int n0, int wave, int lane, uint8_t* wl,
-                                           const float (&row_scale)[2], const float4v (&acc)[NB][M], const float (&dcur)[NB]) {
+                                           const float (&row_scale)[2], const float4v (&acc)[NB][M], const float (&dcur)[NB], const float* s_scale) {
     if (!DOWN && p.act == INFR_ACT_SILU && !p.has_clamp && !p.weight_before && (F::kUnits || t.e != p.sh_e))
-        store_rows<F, DOWN, NB, M, true>(p, t, n0, wave, lane, wl, row_scale, acc, dcur);
+        store_rows<F, DOWN, NB, M, true>(p, t, n0, wave, lane, wl, row_scale, acc, dcur, s_scale);
     else
-        store_rows<F, DOWN, NB, M, false>(p, t, n0, wave, lane, wl, row_scale, acc, dcur);
+        store_rows<F, DOWN, NB, M, false>(p, t, n0, wave, lane, wl, row_scale, acc, dcur, s_scale);
 }
 
 // An item: M 16-token tiles; FEW: one of up to 8 tokens (the rows of the others hold what was there: a token's sums depend on
@@ -463,7 +464,7 @@ __device__ __forceinline__ void gemm_tile(const GroupedParams& p, const Tile& t,
         step(s, std::integral_constant<int, 0>{});
     }
     wait_loads<0>();   // no transfer outlives the item
-    store_tile<F, DOWN, NB, M>(p, t, n0, wave, lane, wl, row_scale, acc, dcur);
+    store_tile<F, DOWN, NB, M>(p, t, n0, wave, lane, wl, row_scale, acc, dcur, nullptr);
 }
 
 // The formats that go through the 32-element unit decoder (units.h), bound by the decoding: tiles of 16 T tokens, T = 1, 2, 4, three
@@ -620,9 +621,9 @@ __device__ __forceinline__ void unit_tile(const GroupedParams& p, const Tile& t,
             }
         }
     }
-    const float row_scale[2] = {s_scale[lane], 1.0f};   // (nothing in it where rows leave without their scale)
+    const float row_scale[2] = {1.0f, 1.0f};
     const float unit[NB] = {1.0f, 1.0f};
-    store_tile<F, DOWN, NB, T>(p, t, n0, wave, lane, wl, row_scale, acc, unit);
+    store_tile<F, DOWN, NB, T>(p, t, n0, wave, lane, wl, row_scale, acc, unit, s_scale);
 }
 
 // The workgroup's item: the tiles in the table's order, a tile's columns side by side.  Workgroups go to the 8 XCDs round-robin, so
@@ -681,15 +682,17 @@ void gemm_launch(hipStream_t s, const GroupedParams& q, dim3 grid) {
 // tiles, columns outside.  Every item of such a launch costs about the same, and its weights, decoded by every workgroup that reads them,
 // are the smaller part: the XCDs share out the tiles' rows.  us per Linear, this order and the other: 512 rows of 2048 x 2048 in Q3_K
 // 29.1 and 30.0, IQ3_S 38.8 and 39.7, 2048 rows of 4096 x 4096 in Q5_1 the same.
+// The tiles are the rows in turn, so no table is read (two memory latencies per workgroup less: 512 rows of 2048 x 2048 in IQ3_S 39.1 and
+// 38.7, 2048 rows of 4096 x 1024 in Q4_1 56.4 and 55.5).
 __device__ __forceinline__ bool dense_item(const GroupedParams& p, Tile& t, int& col) {
-    const int n_tiles = p.tiles[0].x, n_items = n_tiles * p.n_tiles_n, per = (n_items + 7) >> 3, k = (int)(blockIdx.x >> 3);
-    const int item = (int)(blockIdx.x & 7) * per + k;
+    const int tile = 1 << p.tile_log2, n_tiles = (p.n_pairs + tile - 1) >> p.tile_log2, n_items = n_tiles * p.n_tiles_n, per = (n_items + 7) >> 3;
+    const int k = (int)(blockIdx.x >> 3), item = (int)(blockIdx.x & 7) * per + k;
     if (k >= per || item >= n_items) return false;
     const int some = p.n_tiles_n == 1 ? item : (int)__umulhi((uint32_t)item, p.n_tiles_rcp), first = some & ~(kGroupTiles - 1);
     const int in_group = min(kGroupTiles, n_tiles - first), r = item - first * p.n_tiles_n;
     col = group_column((uint32_t)r, in_group);
-    const int4 b = p.tiles[1 + first + r - col * in_group];
-    t = Tile{b.x, b.y, b.z};
+    const int p0 = (first + r - col * in_group) << p.tile_log2;
+    t = Tile{0, p0, min(tile, p.n_pairs - p0)};
     return true;
 }
 
@@ -698,7 +701,12 @@ __global__ __launch_bounds__(kGW * 64, 3) void grouped_gemm_units(GroupedParams 
     extern __shared__ __attribute__((aligned(16))) uint8_t lds_gemm[];
     Tile t;
     int n0;
-    if (!(DOWN && p.n_expert == 1 ? dense_item(p, t, n0) : gemm_item(p, t, n0))) return;
+    if constexpr (DOWN) {
+        asm volatile("" : : "s"(p.dense), "s"(p.n_tiles_n), "s"(p.n_tiles_rcp), "s"(p.n_pairs), "s"(p.tiles));   // in one round trip
+        if (!(p.dense ? dense_item(p, t, n0) : gemm_item(p, t, n0))) return;
+    } else {
+        if (!gemm_item(p, t, n0)) return;
+    }
     n0 *= (DOWN ? 32 : 16) * kGW;
     if (t.cnt <= 16) unit_tile<F, DOWN, 1>(p, t, n0, lds_gemm);
     else if (t.cnt <= 32) unit_tile<F, DOWN, 2>(p, t, n0, lds_gemm);
@@ -719,7 +727,7 @@ void gemm(hipStream_t s, const GroupedParams& p) {
     const int tiles = gemm_max_tiles(p.n_pairs, p.n_expert, 1 << p.tile_log2);
     q.deal_log2 = !F::kUnits && tiles >= kDealTiles && tiles * q.n_tiles_n <= kDealItems ? 3 : 0;
     const int items = (q.deal_log2 ? (tiles + 7) & ~7 : tiles) * q.n_tiles_n;
-    const dim3 grid((unsigned)(F::kUnits && DOWN && p.n_expert == 1 ? (items + 7) & ~7 : items));   // (dense_item: whole rounds of the 8 XCDs)
+    const dim3 grid((unsigned)(F::kUnits && DOWN && p.dense ? (items + 7) & ~7 : items));   // (dense_item: whole rounds of the 8 XCDs)
     if constexpr (F::kUnits) {
         INFR_LDS_LIMIT((grouped_gemm_units<F, DOWN>), (int)unit_lds<F>());
         INFR_LAUNCH((grouped_gemm_units<F, DOWN>), grid, dim3(kGW * 64), unit_lds<F>(), s, q);

@@ -183,6 +183,7 @@ struct GroupedParams {
     int deal_log2;            // set by the launcher: see gemm_item
     const int4* tiles;        // block formats: the tile table of launch_bucket, gemm_table_slots(n_pairs, n_expert, 1 << tile_log2) slots
     int tile_log2;            // block formats: the table's tiles hold up to 1 << tile_log2 pairs
+    int dense;                // down: a Linear, n_pairs rows of one matrix
     const int32_t* pair_row;  // block formats, gate/up: token row of each pair
     const uint32_t* a_sum;    // formats with minimums: sums of a over groups of 32, see launch_rows_to_f16
     // block formats with an operand of their own: an always-on expert on every token row as expert sh_e of the tile table, pairs
