@@ -219,7 +219,7 @@ constexpr int kIntTok = 8;   // pairs of a tile of the integer kernels
 // Tiles of a Linear's rows: 64.  us per Linear, of 64 | of 128: 128 rows of 4096 x 4096 in Q5_K 40 | 56, 512 rows of 2048 x 2048 in Q8_0 26 | 32, 1500
 // rows of 4096 x 1536 in Q4_K 52 | 58 and of 2048 x 4096 in MXFP4 40 | 43, 2048 rows of 2048 x 2048 in Q8_0 38 | 36, 2048 rows of 4096 x 4096 in
 // Q5_K 115 | 101, 3000 rows of 4096 x 8192 in IQ4_XS 307 | 250: where tiles of 128 would fill the chip (512 items) they would be the faster
-// ones, and no build has had them there.  (The unit-decoder formats have none.)
+// ones; that is not taken yet.  (The unit-decoder formats have none.)
 constexpr int kLinearTileLog2 = 6;
 inline int gemm_max_tiles(int n_pairs, int n_expert, int tile) { return n_pairs / tile + (n_expert < n_pairs ? n_expert : n_pairs); }
 inline size_t gemm_table_slots(int n_pairs, int n_expert, int tile) { return 1 + (((size_t)gemm_max_tiles(n_pairs, n_expert, tile) + 7) & ~(size_t)7); }   // whole eights
