@@ -319,11 +319,13 @@ void drain_prof(infr_hip_backend* be) {
 
 // Single-launch kernel with a guessed selection: is every router logit computed once for the whole grid (and handed
 // over across the XCDs), or by every group of 32 workgroups for itself (eight reads of the router)?
-int moe_logits_once(const infr_hip_backend* be, const infr_op_moe_ffn& m) {
+int moe_logits_once(const infr_hip_backend* be, const infr_op_moe_ffn& m, int rows) {
     if (be->cfg.single_launch_logits == 1) return 1;
     if (be->cfg.single_launch_logits == 2) return 0;
-    (void)m;
-    return 1;   // measured equal or faster on every shape the kernel takes, and the router is read once
+    // Once: measured equal or faster at 128 and more experts, and the router is read once.  The 128 KB router of 32 experts of hidden
+    // size 1024 costs little to read eight times, and a hand-over inside the XCD is shorter: 12 layers of one row in Q8_0 146 us (once
+    // 155), in Q4_K / Q6_K 132 (144), two rows 220 and 166 (227 and 174), four 282 and 204 (283 and 211); eight rows only once.
+    return m.ne > 1024 || rows > 4;
 }
 
 // The profiler's name of a grouped GEMM on banks of format dt: of its own operands, through the unit decoder, or float weights.
@@ -1332,7 +1334,7 @@ extern "C" infr_status infr_hip_compile(infr_hip_backend* be, const infr_graph* 
             probe.g.route.expert_ids = m.expert_ids == INFR_NO_TENSOR ? nullptr : (const int32_t*)plan;
             probe.g.route.ep_n = m.has_ep_band ? (int)m.ep_n_local : 0;
             probe.router_row_floats = m.ne;
-            probe.logits_once = moe_logits_once(be, m);
+            probe.logits_once = moe_logits_once(be, m, sc.rows);
             if (kind == infr_hip_plan::kMoeShared) probe.g.sh_gate = probe.g.sh_up = probe.g.sh_down = (const uint8_t*)plan;
             if (!be->cfg.disable_single_launch_guess && infr::moe_layer_stream_supported(probe)) {
                 sc.single_launch = 2;
@@ -1678,7 +1680,7 @@ extern "C" infr_status infr_hip_execute(infr_hip_backend* be, infr_hip_plan* pla
                         lp.xs = lp.xh + nr * 8 * m.n_ff_exp;
                         lp.ypart = lp.xs + nr * m.n_ff_exp;
                         lp.late = be->fault_dev + 1;
-                        lp.logits_once = moe_logits_once(be, m);
+                        lp.logits_once = moe_logits_once(be, m, rows);
                         lp.guess_skew = (int)std::min<uint32_t>(be->cfg.single_launch_guess_skew, 8u);
                         bool norm_ok = true;
                         if (fz.norm) {   // the token row's RmsNorm, folded: the kernel normalises the raw row

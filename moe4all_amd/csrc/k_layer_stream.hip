@@ -46,11 +46,14 @@ bool stream_shape(const MoeLayerParams& q, StreamShape* out) {
     const MoeGemvParams& p = q.g;
     const int ne = p.ne, nff = p.nff, n_expert = p.route.n_expert;
     const bool shared = p.sh_gate != nullptr;
-    if (ne != 2048 && ne != 4096) return false;                      // 256 or 512 octets on 512 threads
-    if (ne % FG::kBlockElems || nff % FD::kBlockElems || nff % 256 || nff % 384 || nff > 1536) return false;   // six gathering wavefronts
+    if (ne != 1024 && ne != 2048 && ne != 4096) return false;        // 128, 256 or 512 octets on 512 threads
+    if (ne % FG::kBlockElems || nff % FD::kBlockElems || nff % 256 || nff > 1536) return false;
+    // (1024 / 512, 32 experts, 12 layers with norm and residual, three launches and this one, us: one row in Q8_0 242 and 146, in Q4_K /
+    // Q6_K 233 and 132; two rows 315 and 220, 290 and 166; four 351 and 282, 316 and 204; eight in Q4_K / Q6_K 351 and 268)
+    if (ne == 1024 ? nff != 512 || n_expert != 32 : nff % 384 || n_expert == 32) return false;   // whole shares of the gathering wavefronts
     const int lpr_g = ne / FG::kBlockElems * FG::kLPB, lpr_d = nff / FD::kBlockElems * FD::kLPB;
     if (lpr_g > 64 || lpr_d > 64) return false;
-    if (n_expert % 64 || n_expert > 256 || n_expert < 64) return false;
+    if (n_expert != 32 && (n_expert % 64 || n_expert > 256 || n_expert < 64)) return false;
     const int rwc_g = 64 / lpr_g, rwc_d = 64 / lpr_d;
     const int rows = p.rows;
     if (rows != 1 && rows != 2 && rows != 4 && rows != 8) return false;   // whole XCDs per token row
@@ -72,7 +75,7 @@ bool stream_shape(const MoeLayerParams& q, StreamShape* out) {
     out->epb = out->once ? (n_expert + bpr - 1) / bpr : n_expert / mpg;
     const int H = kThreads / (ne / 8);
     out->ept = (out->epb + H - 1) / H;
-    out->nsp = n_expert / 64;
+    out->nsp = n_expert / 64;   // 0: half a wavefront's
     // everything in flight at once when a wavefront has few items, rings otherwise
     out->dg = my_gi <= 2 ? 2 : my_gi <= 4 && std::is_same<FG, Q80Fmt>::value ? 4 : 2;
     out->early_down = my_gi <= out->dg ? 1 : 0;
@@ -99,7 +102,7 @@ bool dispatch_stream(hipStream_t s, MoeLayerParams q, bool launch) {
         const bool done = launch_stream_fixed(s, q, sh, launch, &taken);
         if (taken) return done;
     }
-    if (q.norm_w) return false;   // the fold of the token row's RmsNorm exists for the fixed shapes only
+    if (q.norm_w || q.g.ne == 1024) return false;   // the fold of the token row's RmsNorm and this width exist for the fixed shapes only
     if constexpr (std::is_same<FG, Q4KFmt>::value) {
         INFR_STREAM(2, 2, 2, 2)   // ne 2048, nff 768, 128 experts, a copy of the router per group
         INFR_STREAM(2, 2, 1, 2)   // ... every logit once

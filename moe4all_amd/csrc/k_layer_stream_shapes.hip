@@ -27,11 +27,20 @@ bool launch_stream_fixed(hipStream_t s, const MoeLayerParams& q, const StreamSha
         INFR_STREAM_AT_N(Q4KFmt, Q6KFmt, 2, 4, 1, 4, 4096, 1536, 1, 1)
         INFR_STREAM_AT(Q4KFmt, Q6KFmt, 2, 4, 2, 4, 4096, 1536, 2)
         INFR_STREAM_AT(Q4KFmt, Q6KFmt, 2, 4, 4, 4, 4096, 1536, 4)
+        INFR_STREAM_AT(Q4KFmt, Q6KFmt, 2, 2, 1, 0, 1024, 512, 1)    // 32 experts (the only instantiations of this width)
+        INFR_STREAM_AT_N(Q4KFmt, Q6KFmt, 2, 2, 1, 0, 1024, 512, 1, 1)
+        INFR_STREAM_AT(Q4KFmt, Q6KFmt, 2, 2, 1, 0, 1024, 512, 2)
+        INFR_STREAM_AT(Q4KFmt, Q6KFmt, 2, 2, 1, 0, 1024, 512, 4)
+        INFR_STREAM_AT(Q4KFmt, Q6KFmt, 2, 4, 1, 0, 1024, 512, 8)
     } else if (p.gate_dt == INFR_Q8_0 && p.down_dt == INFR_Q8_0) {
         INFR_STREAM_AT(Q80Fmt, Q80Fmt, 4, 5, 1, 2, 2048, 768, 1)
         INFR_STREAM_AT_N(Q80Fmt, Q80Fmt, 4, 5, 1, 2, 2048, 768, 1, 1)
         INFR_STREAM_AT(Q80Fmt, Q80Fmt, 2, 4, 1, 2, 2048, 768, 2)
         INFR_STREAM_AT(Q80Fmt, Q80Fmt, 2, 4, 1, 2, 2048, 768, 4)
+        INFR_STREAM_AT(Q80Fmt, Q80Fmt, 2, 2, 1, 0, 1024, 512, 1)    // 32 experts
+        INFR_STREAM_AT_N(Q80Fmt, Q80Fmt, 2, 2, 1, 0, 1024, 512, 1, 1)
+        INFR_STREAM_AT(Q80Fmt, Q80Fmt, 4, 2, 1, 0, 1024, 512, 2)
+        INFR_STREAM_AT(Q80Fmt, Q80Fmt, 2, 5, 1, 0, 1024, 512, 4)
     }
 #undef INFR_STREAM_AT
 #undef INFR_STREAM_AT_N

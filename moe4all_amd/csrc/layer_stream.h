@@ -83,10 +83,11 @@ __device__ __forceinline__ int gather_activations(const uint64_t* rec, int n, ui
     return state;
 }
 
-template <int N>
+// PART: n < 64 records, on the first n lanes.
+template <int N, bool PART = false>
 __device__ __forceinline__ bool gather_records(const uint64_t* rec, int n, uint32_t tag, float* out, int lane, int spin_limit) {
     uint64_t r[N];
-    const int ns = n >> 6;
+    const int ns = PART ? (lane < n ? 1 : 0) : n >> 6;
     for (int spin = 0;; spin++) {
 #pragma unroll
         for (int s = 0; s < N; s++) r[s] = s < ns ? rec_load(rec + s * kWave + lane) : ((uint64_t)tag << 32);
@@ -122,15 +123,15 @@ __device__ __forceinline__ int lds_flag_wait(volatile int* f) {
 // and counts the lanes whose largest key beats its own; a member of the top K overall lies in one of the K lanes with
 // the largest heads, so those lanes' K * NS keys (<= 64) are ranked among themselves the same way and the ranks
 // [skew, skew + n_sel) are the guess.  skew > 0 (tests only, <= 8) leaves the `skew` largest out, so the guess is wrong
-// on purpose.  scratch: 128 words of LDS.
+// on purpose.  scratch: 128 words of LDS.  n < 64 (NS = 1): the other lanes' keys are 0, behind every index's.
 template <int NS>
-__device__ __forceinline__ void guess_set(const float* vals, int n_sel, int skew, int lane, int32_t* out, uint32_t* scratch) {
+__device__ __forceinline__ void guess_set(const float* vals, int n, int n_sel, int skew, int lane, int32_t* out, uint32_t* scratch) {
     static_assert(NS == 1 || NS == 2 || NS == 4, "sorting network");
     uint32_t key[NS];
 #pragma unroll
     for (int s = 0; s < NS; s++) {
         const int i = s * kWave + lane;
-        key[s] = (order_key(vals[i]) & ~0xFFu) | (uint32_t)(255 - i);
+        key[s] = NS > 1 || i < n ? (order_key(vals[i]) & ~0xFFu) | (uint32_t)(255 - i) : 0u;
     }
     auto order = [&](int a, int b) {
         const uint32_t hi = max(key[a], key[b]), lo = min(key[a], key[b]);
@@ -218,8 +219,11 @@ __device__ __forceinline__ float dot8(const float4& a0, const float4& a1, const 
 // routing first and has nothing to do while the others stream.
 __host__ __device__ constexpr int router_wave_down_items(int n_di) { return n_di % 8 == 0 ? n_di / 8 : 0; }
 
+// Wavefronts that gather a group's activations and turn them into cells: each a whole number of 64 records.
+__host__ __device__ constexpr int gather_waves(int nff) { return nff % 384 == 0 ? 6 : 4; }
+
 // FG / FD: formats of the gate/up and down banks; DG / DD: ring depths (items in flight per streaming wavefront);
-// EPT: router rows a thread holds while staging (rows per workgroup / (512 / (ne / 8))); NSP: n_expert / 64.
+// EPT: router rows a thread holds while staging (rows per workgroup / (512 / (ne / 8))); NSP: n_expert / 64 (0: 32 experts).
 // NE, NFF, ROWS: hidden size, intermediate size and token rows when they are known at compile time (the benchmark
 // shapes), 0 for any shape.  With constants the lane placement, the item counts and every index division below fold;
 // with run-time values they are integer arithmetic on the critical path of a kernel that one wavefront paces.
@@ -241,7 +245,10 @@ __global__ __launch_bounds__(kThreads) void moe_layer_stream(MoeLayerParams q) {
     __shared__ uint32_t s_seq;
     const MoeGemvParams& p = q.g;
     const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;   // wave: uniform, scalar registers
-    const int ne = NE ? NE : p.ne, nff = NFF ? NFF : p.nff, n_expert = 64 * NSP;
+    const int ne = NE ? NE : p.ne, nff = NFF ? NFF : p.nff;
+    constexpr bool kHalf = NSP == 0;
+    constexpr int NS = kHalf ? 1 : NSP, n_expert = kHalf ? 32 : 64 * NSP;   // experts per lane; all of them
+    const int n_gather = gather_waves(nff);
     const bool shared = p.sh_gate != nullptr;
     // One, two or four token rows per launch: a row takes 8 / rows of the XCDs (workgroups are dealt to the XCDs in turn,
     // so workgroup b sits on XCD b & 7 up to a rotation), its eight groups of mpg = 32 / rows members each lie on one XCD
@@ -280,9 +287,9 @@ __global__ __launch_bounds__(kThreads) void moe_layer_stream(MoeLayerParams q) {
     const bool has_rows = row0 < n_expert;
 
     // LDS: [cells of x][chain operands, transposed][estimates][logits][routing scratch][h][cells of h][h, cells: always-on]
-    const int oct_n = ne >> 3;                 // octets of a row: 256 or 512
+    const int oct_n = ne >> 3;                 // octets of a row: 128, 256 or 512
     const int jstride = oct_n + 4;
-    const int hsel = tid / oct_n, o = tid - hsel * oct_n;   // replica (0 or 1 when ne = 2048) and octet of this thread
+    const int hsel = tid / oct_n, o = tid - hsel * oct_n;   // replica (0 or 1 when ne = 2048, 0..3 when 1024) and octet of this thread
     const int H = kThreads / oct_n;
     uint32_t* cells = dyn_lds;
     float* wst = reinterpret_cast<float*>(cells + (size_t)(ne >> 5) * kCellDwords);
@@ -459,7 +466,7 @@ __global__ __launch_bounds__(kThreads) void moe_layer_stream(MoeLayerParams q) {
             }
         }
         STAMP(16);
-        ok = gather_records<NSP>(q.xl + (size_t)area * n_expert, n_expert, tag, s_logits, lane, spin_limit);
+        ok = gather_records<NS, kHalf>(q.xl + (size_t)area * n_expert, n_expert, tag, s_logits, lane, spin_limit);
         STAMP(17);
         if (ok) {
             __builtin_amdgcn_wave_barrier();
@@ -472,8 +479,8 @@ __global__ __launch_bounds__(kThreads) void moe_layer_stream(MoeLayerParams q) {
             const int guess_state = lds_flag_wait(&s_f_spec);
             if (guess_state != 1) ok = false;
             bool routed = false;
-            if (ok && route_duo_ok(rp) && rp.n_expert == 64 * NSP)
-                routed = route_softmax_checked<NSP>(rp, 0, lane, s_spec, route_scratch, s_tab, s_ids, s_w, os == 0);
+            if (ok && route_duo_ok(rp) && rp.n_expert == n_expert)
+                routed = route_softmax_checked<NS, kHalf>(rp, 0, lane, s_spec, route_scratch, s_tab, s_ids, s_w, os == 0);
             if (!routed) {
                 __builtin_amdgcn_wave_barrier();
                 route_row_any(rp, 0, lane, route_scratch, s_tab, s_ids, s_w, os == 0);
@@ -558,11 +565,11 @@ __global__ __launch_bounds__(kThreads) void moe_layer_stream(MoeLayerParams q) {
         if (sh_n && wave != 1) sh_issue();
         if (wave == 1) {
             // the guess of the selected set, from the estimates
-            bool ok = gather_records<NSP>(q.xa + (size_t)area * n_expert, n_expert, tag, s_alog, lane, spin_limit);
+            bool ok = gather_records<NS, kHalf>(q.xa + (size_t)area * n_expert, n_expert, tag, s_alog, lane, spin_limit);
             STAMP(3);
             if (ok) {
                 __builtin_amdgcn_wave_barrier();
-                guess_set<NSP>(s_alog, kGroups, q.guess_skew, lane, s_spec, s_guess);
+                guess_set<NS>(s_alog, n_expert, kGroups, q.guess_skew, lane, s_spec, s_guess);
             } else if (lane == 0) {
                 s_fault = 1;
                 __hip_atomic_store(q.fault, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
@@ -588,7 +595,7 @@ __global__ __launch_bounds__(kThreads) void moe_layer_stream(MoeLayerParams q) {
         // the members of a group meet on the guess, and the down rows' results carry it too, so nobody consumes a
         // result of an expert the routing did not select.  The routing is looked at after the pass (and, without
         // waiting, before the down stage, which is skipped when it is already known to be for nothing).
-        const int chunk = nff / 6;   // records per gathering wavefront: a multiple of 64
+        const int chunk = nff / n_gather;   // records per gathering wavefront: a multiple of 64
         // (two straight-line copies of the pass instead of a loop: a loop's invariant addresses would stay in registers
         // across the whole pass and spill)
         auto run_pass = [&](const int attempt) __attribute__((always_inline)) -> bool {   // true: once more, with e_cur renewed
@@ -643,9 +650,9 @@ __global__ __launch_bounds__(kThreads) void moe_layer_stream(MoeLayerParams q) {
             if (wave == 3) STAMP(7);
             if (wave == 1) STAMP(21);
             if (wave == 7) STAMP(22);
-            // ---- hand-over of the group's activations: six wavefronts gather a sixth each and turn it into cells
+            // ---- hand-over of the group's activations: six (or four) wavefronts gather a share each and turn it into cells
             bool superseded = false;
-            if (sw < 6) {
+            if (sw < n_gather) {
                 const int st = gather_activations<4>(q.xh + (size_t)g * nff + sw * chunk, chunk, seq_tag | (uint32_t)e_cur,
                                                      s_h + sw * chunk, lane, spin_limit, attempt == 0);
                 if (wave == 1) STAMP(9);
@@ -670,7 +677,7 @@ __global__ __launch_bounds__(kThreads) void moe_layer_stream(MoeLayerParams q) {
             if (!q.early_down && alive) ring_prime<DD>(dn_issue);
             {
                 int v;
-                while ((((v = __builtin_amdgcn_readfirstlane(*(volatile int*)&s_h_done)) & 0xFF) < 6 * (attempt + 1)) && !(v >> 8))
+                while ((((v = __builtin_amdgcn_readfirstlane(*(volatile int*)&s_h_done)) & 0xFF) < n_gather * (attempt + 1)) && !(v >> 8))
                     __builtin_amdgcn_s_sleep(1);
                 asm volatile("" ::: "memory");
                 if (v >> 8) alive = false;
@@ -760,7 +767,7 @@ __global__ __launch_bounds__(kThreads) void moe_layer_stream(MoeLayerParams q) {
             // its rows are requested at once and contracted when the pass that gathers that expert's activations is
             // through (the first if the guess was right, the second otherwise)
             const int e_fin = __builtin_amdgcn_readfirstlane(s_final[g]);
-            const int through = 6 * (__builtin_amdgcn_readfirstlane(s_spec[g]) == e_fin ? 1 : 2);
+            const int through = n_gather * (__builtin_amdgcn_readfirstlane(s_spec[g]) == e_fin ? 1 : 2);
             const uint8_t* rows0 = p.down + (size_t)e_fin * p.down_stride + (size_t)m * R * rb_d;
             const int i0 = n_di - n_w0;
             auto wd_issue = [&](int slot, int j) __attribute__((always_inline)) {

@@ -433,17 +433,18 @@ __device__ __forceinline__ bool route_duo_second(const RouteParams& p, int row, 
 // candidates ARE the reference's selection (lib.rs:3847-3850 sorts by probability descending, ties to the lower id,
 // and no tie crosses the boundary), and their ranks follow from comparing the n_used candidates with each other under
 // that same order.  Otherwise (a wrong candidate set, a tie across the boundary, anything not a number) the function
-// returns false and the caller runs the complete routine.  Needs n_expert == 64 * NS and n_used <= 16.
+// returns false and the caller runs the complete routine.  Needs n_expert == 64 * NS (PART: 32) and n_used <= 16.
 // cand: n_used distinct ids in LDS; lds: 2 * n_expert floats, 16-byte aligned.
-template <int NS>
+template <int NS, bool PART = false>
 __device__ __forceinline__ bool route_softmax_checked(const RouteParams& p, int row, int lane, const int32_t* cand, float* lds,
                                                       const uint64_t* tab, int32_t* lds_ids, float* lds_w, bool store_global) {
     const int n = p.n_expert;
     const float* lg = p.logits + (size_t)row * n;
     float* ex = lds;          // [n] exponentials, then probabilities
+    const bool live = !PART || lane < n;
     float pr[NS];
 #pragma unroll
-    for (int s = 0; s < NS; s++) pr[s] = lg[s * kWave + lane];
+    for (int s = 0; s < NS; s++) pr[s] = live ? lg[s * kWave + lane] : -__builtin_huge_valf();
     float m = pr[0];
 #pragma unroll
     for (int s = 1; s < NS; s++) m = fmaxf(m, pr[s]);
@@ -451,7 +452,7 @@ __device__ __forceinline__ bool route_softmax_checked(const RouteParams& p, int 
 #pragma unroll
     for (int s = 0; s < NS; s++) {
         pr[s] = expf_libm(__fsub_rn(pr[s], m), tab);
-        ex[s * kWave + lane] = pr[s];
+        if (live) ex[s * kWave + lane] = pr[s];
     }
     // which of this lane's experts are candidates (beside the sum's dependent adds, which leave issue slots free)
     uint32_t member = 0;
@@ -487,11 +488,11 @@ __device__ __forceinline__ bool route_softmax_checked(const RouteParams& p, int 
 #pragma unroll
     for (int s = 0; s < NS; s++) {
         pr[s] = __fdiv_rn(pr[s], psum);
-        ex[s * kWave + lane] = pr[s];
+        if (live) ex[s * kWave + lane] = pr[s];
         const uint32_t key = order_key(pr[s]);
         const bool in = (member >> s) & 1u;
         lo_in = in ? min(lo_in, key) : lo_in;
-        hi_out = in ? hi_out : max(hi_out, key);
+        hi_out = in || !live ? hi_out : max(hi_out, key);
     }
     lo_in = wave_min_u32(lo_in);
     hi_out = wave_max_u32(hi_out);
@@ -547,7 +548,8 @@ __device__ __forceinline__ bool route_softmax_checked(const RouteParams& p, int 
     }
     if (p.probs && store_global) {
 #pragma unroll
-        for (int s = 0; s < NS; s++) p.probs[(size_t)row * n + s * kWave + lane] = pr[s];
+        for (int s = 0; s < NS; s++)
+            if (live) p.probs[(size_t)row * n + s * kWave + lane] = pr[s];
     }
     return true;
 }

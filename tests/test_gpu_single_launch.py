@@ -526,3 +526,110 @@ def test_single_launch_with_the_rms_norm_and_the_residual_folded_in(be, shared):
     assert np.array_equal(bits(norms[False]), bits(norms[True]))
     assert np.array_equal(bits(outs[False]), bits(outs[True]))
     assert H.rel_l2(norms[False].reshape(1, ne), O.rms_norm(x, nw, eps).reshape(1, ne)) < 1e-5
+
+
+@pytest.mark.parametrize("rows,gdt,ddt,skew,opts", [
+    (1, H.Q8_0, H.Q8_0, 0, {}), (1, H.Q4K, H.Q6K, 0, {}), (1, H.Q8_0, H.Q8_0, 3, {}), (1, H.Q4K, H.Q6K, 8, {}),
+    (8, H.Q4K, H.Q6K, 2, {}),
+    (1, H.Q8_0, H.Q8_0, 0, dict(gating=M.MoeGating.Sigmoid, scale=2.5, norm_w=False)),
+    (1, H.Q4K, H.Q6K, 1, dict(with_down_scale=True, act=M.Activation.Gelu)),
+    (2, H.Q8_0, H.Q8_0, 0, {}), (4, H.Q8_0, H.Q8_0, 2, {}), (2, H.Q4K, H.Q6K, 1, {}), (4, H.Q4K, H.Q6K, 0, {})])
+def test_32_experts_of_hidden_size_1024_in_one_launch(be3, rows, gdt, ddt, skew, opts):
+    """Half a wavefront of experts, four replicas of the token row's octets, four gathering wavefronts: ids, weights,
+    logits, probabilities and output bits of the three-launch path, also when every row's guess misses `skew` experts."""
+    ne, E, K, nff = 1024, 32, 8, 512
+    rng = np.random.default_rng(50 + rows + gdt + skew + len(opts))
+    x = rng.standard_normal((rows, ne)).astype(np.float32)
+    x[rows - 1] *= 30.0
+    router = (rng.standard_normal((E, ne)) * 0.02).astype(np.float32)
+    gate, up, down = _banks(rng, E, nff, ne, gdt, ddt)
+    data = dict(x=x, router=router, gate=gate, up=up, down=down)
+    if opts.get("with_down_scale"):
+        data["down_scale"] = rng.uniform(0.5, 1.5, E).astype(np.float32)
+    b = M.Backend(0, single_launch_guess_skew=skew)
+    try:
+        before = b.late_experts()
+        for rep in range(2):
+            g, ids = moe_graph(rows, ne, E, K, nff, DType(gdt), DType(ddt), **opts)
+            one, r1 = _run(b, g, ids, data, rows * ne, GUESS)
+            g, ids = moe_graph(rows, ne, E, K, nff, DType(gdt), DType(ddt), **opts)
+            three, r3 = _run(be3, g, ids, data, rows * ne, "moe_route_gate_up")
+            assert np.array_equal(r1["idx"], r3["idx"]) and np.array_equal(bits(r1["w"]), bits(r3["w"]))
+            assert np.array_equal(bits(r1["logits"]), bits(r3["logits"])) and np.array_equal(bits(r1["probs"]), bits(r3["probs"]))
+            assert np.array_equal(bits(one), bits(three))
+        assert b.late_experts() - before == 2 * rows * skew
+    finally:
+        b.close()
+
+
+def test_32_experts_of_hidden_size_1024_with_ties_and_infinities(be, be3):
+    """Exact ties across the edge of the selection, and logits of minus infinity or NaN: the half-filled wavefront's idle
+    lanes must not enter the ranking."""
+    ne, E, K, nff = 1024, 32, 8, 512
+    for case in range(4):
+        data = _plain_case(600 + case, E, H.Q8_0, H.Q8_0, ne, nff)
+        x, router = np.zeros((1, ne), np.float32), data["router"]
+        x[0, 0] = 1.0
+        router[:, 0] = np.linspace(2.0, 1.0, E, dtype=np.float32)
+        if case == 0:
+            router[:, 0] = 1.0                       # all equal: ids 0..7
+        if case == 1:
+            router[[7, 8, 9], 0] = router[7, 0]      # a tie across the boundary
+        if case == 2:
+            router[4:, 0] = -3.0e38                  # probabilities of zero inside the selection
+        if case == 3:
+            router[5, 0] = np.float32(np.nan)
+        data["x"] = x
+        g, ids = moe_graph(1, ne, E, K, nff, DType.Q8_0, DType.Q8_0)
+        one, r1 = _run(be, g, ids, data, ne, GUESS)
+        g, ids = moe_graph(1, ne, E, K, nff, DType.Q8_0, DType.Q8_0)
+        three, r3 = _run(be3, g, ids, data, ne, "moe_route_gate_up")
+        assert np.array_equal(r1["idx"], r3["idx"]), case
+        assert np.array_equal(r1["w"], r3["w"], equal_nan=True) and np.array_equal(one, three, equal_nan=True)
+
+
+@pytest.mark.parametrize("gdt,ddt,shared", [(H.Q8_0, H.Q8_0, False), (H.Q4K, H.Q6K, False), (H.Q4K, H.Q6K, True)])
+def test_32_experts_of_hidden_size_1024_with_norm_and_residual(be, gdt, ddt, shared):
+    """y = x + ffn(rmsnorm(x) * w) of one token as one launch, with and without an always-on expert: the bits of one launch per op."""
+    ne, E, K, nff = 1024, 32, 8, 512
+    rng = np.random.default_rng(70 + gdt)
+    T = M.TensorDesc
+    gd, dd = DType(gdt), DType(ddt)
+    x = (rng.standard_normal((1, ne)) * 3.0).astype(np.float32)
+    nw = rng.uniform(0.5, 1.5, ne).astype(np.float32)
+    router = (rng.standard_normal((E, ne)) * 0.02).astype(np.float32)
+    gate, up, down = _banks(rng, E, nff, ne, gdt, ddt)
+    sg, su, sd = (a.reshape(-1) for a in _banks(rng, 1, nff, ne, gdt, ddt))
+    outs = []
+    for plain in (False, True):
+        b = M.Backend(0, disable_op_fusion=True, disable_single_launch_moe=True) if plain else be
+        try:
+            g = M.Graph()
+            xi, nwt, rt = g.input(T([1, ne], DType.F32)), g.weight(T([ne], DType.F32)), g.weight(T([E, ne], DType.F32))
+            gt, ut, dt = g.weight(T([E, nff, ne], gd)), g.weight(T([E, nff, ne], gd)), g.weight(T([E, ne, nff], dd))
+            xn, moe, y = g.internal(T([1, ne], DType.F32)), g.internal(T([1, ne], DType.F32)), g.output(T([1, ne], DType.F32))
+            g.rms_norm(x=xi, weight=nwt, dst=xn, rows=1, dim=ne, eps=1e-6)
+            g.moe_ffn(x=xn, router=rt, gate_exps=gt, up_exps=ut, down_exps=dt, dst=moe, ne=ne, n_expert=E, n_used=K, n_ff_exp=nff)
+            bound, sub = [(xi, x), (nwt, nw), (rt, router), (gt, gate), (ut, up), (dt, down)], moe
+            if shared:
+                wg, wu, wd = g.weight(T([nff, ne], gd)), g.weight(T([nff, ne], gd)), g.weight(T([ne, nff], dd))
+                tg, tu, ta = (g.internal(T([1, nff], DType.F32)) for _ in range(3))
+                ts, sub = g.internal(T([1, ne], DType.F32)), g.internal(T([1, ne], DType.F32))
+                g.linear(x=xn, weight=wg, dst=tg, m=1, in_f=ne, out_f=nff)
+                g.linear(x=xn, weight=wu, dst=tu, m=1, in_f=ne, out_f=nff)
+                g.gated_act(gate=tg, up=tu, dst=ta, rows=1, nff=nff)
+                g.linear(x=ta, weight=wd, dst=ts, m=1, in_f=nff, out_f=ne)
+                g.add(a=moe, b=ts, dst=sub, n=ne)
+                bound += [(wg, sg), (wu, su), (wd, sd)]
+            g.add(a=xi, b=sub, dst=y, n=ne)
+            b.prof_enable(True)
+            outs.append(M.run_graph(b, g, bound, y, ne))
+            b.sync()
+            names = set(b.prof_read())
+            b.prof_enable(False)
+            if not plain:
+                assert names == {"moe_layer_shared" if shared else "moe_layer"}, names
+        finally:
+            if plain:
+                b.close()
+    assert np.array_equal(bits(outs[0]), bits(outs[1])) and np.abs(outs[0] - x.reshape(-1)).max() > 1e-4
