@@ -325,7 +325,7 @@ int moe_logits_once(const infr_hip_backend* be, const infr_op_moe_ffn& m, int ro
     // Once: measured equal or faster at 128 and more experts, and the router is read once.  The 128 KB router of 32 experts of hidden
     // size 1024 costs little to read eight times, and a hand-over inside the XCD is shorter: 12 layers of one row in Q8_0 146 us (once
     // 155), in Q4_K / Q6_K 132 (144), two rows 220 and 166 (227 and 174), four 282 and 204 (283 and 211); eight rows only once.
-    return m.ne > 1024 || rows > 4;
+    return m.ne > 1024 || rows > 4 || m.n_used != 8;
 }
 
 // The profiler's name of a grouped GEMM on banks of format dt: of its own operands, through the unit decoder, or float weights.

@@ -119,10 +119,45 @@ bool dispatch_stream(hipStream_t s, MoeLayerParams q, bool launch) {
     return false;
 }
 
+template <int NSP, int NORM>
+bool launch_stream4(hipStream_t s, const MoeLayerParams& q, size_t lds) {
+    return launch_stream<Mxfp4Fmt, Mxfp4Fmt, 3, 4, 1, NSP, 0, 0, 1, NORM, 4>(s, q, lds);
+}
+
+// Four experts per token, MXFP4 banks (one token row, no always-on expert).  us per layer of 2880 / 2880, 128 experts, with norm and
+// residual: three launches 32 to 37 over boxes, this one 30.  The stream bounds it (10 us of 1530-byte rows for gate/up, 5 for down: a
+// row is 45 lanes' 34 unaligned bytes, whose loads keep the CU's address path busy as long as their 96 instructions a row keep
+// the vector ALUs), then the hand-over of h between 64 workgroups on two XCDs (3 us).
+bool stream_four(hipStream_t s, MoeLayerParams q, bool launch) {
+    const MoeGemvParams& p = q.g;
+    const int ne = p.ne, nff = p.nff, n_expert = p.route.n_expert, rwc = ne <= 1024 ? 4 : ne <= 2048 ? 2 : 1;
+    if (p.rows != 1 || p.sh_gate || !q.logits_once || (n_expert != 64 && n_expert != 128)) return false;
+    if (ne % 64 || ne < 1024 || ne > 4096 || nff % 64 || nff < 512 || nff > 4096) return false;   // 64 elements per lane, 16 to 64 lanes per row
+    const int share = nff / gather_waves(nff);
+    if (nff % gather_waves(nff) || share % 64 || share > 9 * 64) return false;
+    const int n_gi = (nff / 64 + rwc - 1) / rwc;
+    q.epb = 1;   // one logit on each of the first n_expert workgroups
+    q.early_down = (n_gi + kSW - 1) / kSW <= 3;
+    const int jstride = ne / 8 + 4;
+    const size_t floats = (size_t)2 * 8 * jstride + 2 * (size_t)n_expert + ((route_scratch_floats(n_expert, p.route.n_groups) + 3) & ~(size_t)3) +
+                          2 * (size_t)nff;
+    const size_t lds = cells_bytes<Mxfp4Fmt>(ne) + floats * 4 + 2 * cells_bytes<Mxfp4Fmt>(nff);
+    if (lds > 150 * 1024) return false;
+    if (!launch) return true;
+    if (n_expert == 64) return q.norm_w ? launch_stream4<1, 1>(s, q, lds) : launch_stream4<1, 0>(s, q, lds);
+    {   // the benchmark shape with its sizes as constants, ahead of the instantiation for any (4 layers 120 us, 126)
+        bool taken = false;
+        const bool done = launch_stream_fixed(s, q, StreamShape{3, 4, 1, 2, 1, 1, 0, lds}, launch, &taken);
+        if (taken) return done;
+    }
+    return q.norm_w ? launch_stream4<2, 1>(s, q, lds) : launch_stream4<2, 0>(s, q, lds);
+}
+
 bool stream_any(hipStream_t s, const MoeLayerParams& q, bool launch) {
     const MoeGemvParams& p = q.g;
     const RouteParams& r = p.route;
-    if (p.n_used != kGroups || p.n_cu < kBlocks || p.gate_dt != p.up_dt) return false;
+    const bool four = p.n_used == 4 && p.gate_dt == INFR_MXFP4 && p.down_dt == INFR_MXFP4;
+    if ((p.n_used != kGroups && !four) || p.n_cu < kBlocks || p.gate_dt != p.up_dt) return false;
     if ((p.sh_gate != nullptr) != (p.sh_down != nullptr) || (p.sh_gate != nullptr) != (p.sh_up != nullptr)) return false;
     // the guess ranks the experts by their logits: gatings that are monotone in the logit, no bias, no groups, no given
     // ids; options that need the routing weights before the gate/up stage or remap ids stay on the in-order kernels
@@ -131,6 +166,7 @@ bool stream_any(hipStream_t s, const MoeLayerParams& q, bool launch) {
         return false;
     if (launch && ((((uintptr_t)q.router | (uintptr_t)q.router_x | (uintptr_t)p.x) & 15) != 0 || (q.router_row_floats & 3) != 0))
         return false;
+    if (four) return stream_four(s, q, launch);
     if (p.gate_dt == INFR_Q4K && p.down_dt == INFR_Q6K) return dispatch_stream<Q4KFmt, Q6KFmt>(s, q, launch);
     if (p.gate_dt == INFR_Q8_0 && p.down_dt == INFR_Q8_0) return dispatch_stream<Q80Fmt, Q80Fmt>(s, q, launch);
     return false;

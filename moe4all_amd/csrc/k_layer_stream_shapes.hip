@@ -11,6 +11,15 @@ bool launch_stream_fixed(hipStream_t s, const MoeLayerParams& q, const StreamSha
     const MoeGemvParams& p = q.g;
     *taken = true;
     const int norm = q.norm_w ? 1 : 0;
+    if (p.n_used == 4) {   // MXFP4 (stream_four)
+        if (p.ne == 2880 && p.nff == 2880 && p.route.n_expert == 128) {
+            if (!launch) return true;
+            return norm ? launch_stream<Mxfp4Fmt, Mxfp4Fmt, 3, 4, 1, 2, 2880, 2880, 1, 1, 4>(s, q, sh.lds)
+                        : launch_stream<Mxfp4Fmt, Mxfp4Fmt, 3, 4, 1, 2, 2880, 2880, 1, 0, 4>(s, q, sh.lds);
+        }
+        *taken = false;
+        return false;
+    }
 #define INFR_STREAM_AT_N(FGt, FDt, DGv, DDv, EPTv, NSPv, NEv, NFFv, ROWSv, NORMv)                                             \
     if (sh.dg == DGv && sh.dd == DDv && sh.ept == EPTv && sh.nsp == NSPv && p.ne == NEv && p.nff == NFFv && p.rows == ROWSv && \
         norm == NORMv)                                                                                                       \

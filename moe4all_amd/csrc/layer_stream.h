@@ -220,7 +220,7 @@ __device__ __forceinline__ float dot8(const float4& a0, const float4& a1, const 
 __host__ __device__ constexpr int router_wave_down_items(int n_di) { return n_di % 8 == 0 ? n_di / 8 : 0; }
 
 // Wavefronts that gather a group's activations and turn them into cells: each a whole number of 64 records.
-__host__ __device__ constexpr int gather_waves(int nff) { return nff % 384 == 0 ? 6 : 4; }
+__host__ __device__ constexpr int gather_waves(int nff) { return nff % 384 == 0 ? 6 : nff % 320 == 0 ? 5 : 4; }
 
 // FG / FD: formats of the gate/up and down banks; DG / DD: ring depths (items in flight per streaming wavefront);
 // EPT: router rows a thread holds while staging (rows per workgroup / (512 / (ne / 8))); NSP: n_expert / 64 (0: 32 experts).
@@ -229,7 +229,9 @@ __host__ __device__ constexpr int gather_waves(int nff) { return nff % 384 == 0 
 // with run-time values they are integer arithmetic on the critical path of a kernel that one wavefront paces.
 // NORM: 1 with an Op::RmsNorm of the token row folded in (its own instantiations: the branches of a run-time switch cost
 // the plain kernel a microsecond and a half of its operand staging).
-template <class FG, class FD, int DG, int DD, int EPT, int NSP, int NE = 0, int NFF = 0, int ROWS = 0, int NORM = 0>
+// KR: experts per token, 8 or 4.  Four have groups of 64 workgroups on two XCDs, whose activations are handed over through
+// the last-level cache, and take any hidden size of whole 64s (octets of the row on part of the threads).
+template <class FG, class FD, int DG, int DD, int EPT, int NSP, int NE = 0, int NFF = 0, int ROWS = 0, int NORM = 0, int KR = 8>
 __global__ __launch_bounds__(kThreads) void moe_layer_stream(MoeLayerParams q) {
     extern __shared__ __attribute__((aligned(16))) uint32_t dyn_lds[];
     __shared__ uint64_t s_tab[32];
@@ -237,7 +239,7 @@ __global__ __launch_bounds__(kThreads) void moe_layer_stream(MoeLayerParams q) {
     __shared__ float s_w[64];
     __shared__ float s_g[kWaves][64], s_u[kWaves][64];
     __shared__ float s_part[kWaves][8];
-    __shared__ int32_t s_spec[kGroups], s_final[kGroups], s_gor[kGroups];
+    __shared__ int32_t s_spec[KR], s_final[KR], s_gor[KR];
     __shared__ float s_ysh[64];
     __shared__ float s_red[4];
     __shared__ uint32_t s_guess[2 * kWave];
@@ -254,12 +256,15 @@ __global__ __launch_bounds__(kThreads) void moe_layer_stream(MoeLayerParams q) {
     // so workgroup b sits on XCD b & 7 up to a rotation), its eight groups of mpg = 32 / rows members each lie on one XCD
     // as before, and everything below happens per row among the row's 256 / rows workgroups.
     const int b = blockIdx.x;
-    const int n_rows = ROWS ? ROWS : p.rows, xpr = kGroups / n_rows, mpg = kPerGroup / n_rows, bpr = kBlocks / n_rows;
+    const int n_rows = ROWS ? ROWS : p.rows, xpr = 8 / n_rows, bpr = kBlocks / n_rows, mpg = bpr / KR;
     const int xcd = b & 7, jx = b >> 3;
     const int trow = xcd / xpr;                            // this workgroup's token row
-    const int g = (xcd - trow * xpr) * n_rows + jx / mpg;  // its group: the rank slot it works on
-    const int m = jx % mpg;                                // its place in the group
-    const int os = m * kGroups + g;                        // its place among the row's workgroups: output rows, always-on share
+    const bool one_xcd = KR >= xpr;                        // a group lies on one XCD, or on xpr / KR of them
+    // its group, the rank slot it works on, and its place in the group
+    const int xr = xcd - trow * xpr, xpg = one_xcd ? 1 : xpr / KR;
+    const int g = one_xcd ? xr * (KR / xpr) + jx / mpg : xr / xpg;
+    const int m = one_xcd ? jx % mpg : (xr % xpg) * kPerGroup + jx;
+    const int os = m * KR + g;                             // its place among the row's workgroups: output rows, always-on share
     {   // this row's operands and results
         MoeGemvParams& pw = q.g;
         pw.x += (size_t)trow * ne;
@@ -290,16 +295,18 @@ __global__ __launch_bounds__(kThreads) void moe_layer_stream(MoeLayerParams q) {
     const int oct_n = ne >> 3;                 // octets of a row: 128, 256 or 512
     const int jstride = oct_n + 4;
     const int hsel = tid / oct_n, o = tid - hsel * oct_n;   // replica (0 or 1 when ne = 2048, 0..3 when 1024) and octet of this thread
-    const int H = kThreads / oct_n;
+    constexpr bool kRagged = KR == 4;   // octets that are no whole wavefronts: one replica, the threads behind it have none
+    const int H = kRagged ? 1 : kThreads / oct_n;
+    const bool on_row = !kRagged || hsel < H;
     uint32_t* cells = dyn_lds;
-    float* wst = reinterpret_cast<float*>(cells + (size_t)(ne >> 5) * kCellDwords);
+    float* wst = reinterpret_cast<float*>(cells + (size_t)(ne >> 5) * kCellOf<FG>);
     float* xst = wst + (size_t)epb * 8 * jstride;
     float* s_alog = xst + 8 * jstride;
     float* s_logits = s_alog + n_expert;
     float* route_scratch = s_logits + n_expert;
     float* s_h = route_scratch + ((route_scratch_floats(n_expert, p.route.n_groups) + 3) & ~(size_t)3);
     uint32_t* hcells = reinterpret_cast<uint32_t*>(s_h + nff);
-    float* s_hs = reinterpret_cast<float*>(hcells + (size_t)(nff >> 5) * kCellDwords);
+    float* s_hs = reinterpret_cast<float*>(hcells + (size_t)(nff >> 5) * kCellOf<FD>);
     uint32_t* hscells = reinterpret_cast<uint32_t*>(s_hs + nff);
 
     if (tid < 32) s_tab[tid] = kExp2Table[tid];
@@ -362,7 +369,7 @@ __global__ __launch_bounds__(kThreads) void moe_layer_stream(MoeLayerParams q) {
         // the estimate's share of this thread, summed over the wavefront
 #pragma unroll
         for (int i = 0; i < EPT; i++) {
-            const float part = wave_sum(dot8(w0[i], w1[i], rx0, rx1));
+            const float part = wave_sum(on_row ? dot8(w0[i], w1[i], rx0, rx1) : 0.0f);
             if (lane == 0) s_part[wave][i] = part;
         }
         // chain operands: element 8 o + t belongs to chain t, position o
@@ -385,7 +392,7 @@ __global__ __launch_bounds__(kThreads) void moe_layer_stream(MoeLayerParams q) {
     const uint32_t seq_tag = (s_seq & 0x7FFFFFu) << 9;
     if (wave == 0) STAMP(1);
     const uint32_t tag = seq_tag | kCodePlain;
-    const int waves_per_replica = oct_n >> 6;
+    const int waves_per_replica = (oct_n + 63) >> 6;
     if (wave == 1 && has_rows && lane < epb) {
         // the estimate of logit row0 + lane: the shares of the wavefronts that held that row, in a fixed order
         const int hs = lane % H, i = lane / H;
@@ -394,9 +401,9 @@ __global__ __launch_bounds__(kThreads) void moe_layer_stream(MoeLayerParams q) {
         rec_store_xcd(q.xa + (size_t)area * n_expert + row0 + lane, a, tag, group_local);
     }
     // the token row as fixed-point cells, one set for the workgroup; the guessing wavefront takes its share after the guess
-    const int n_conv_waves = oct_n >> 6;
+    const int n_conv_waves = (oct_n + 63) >> 6;
     auto convert_share = [&]() {
-        if (!converts) return;   // whole wavefronts
+        if (!converts) return;   // whole wavefronts (kRagged: the last one in part, its first lane included; its cells need no neighbours)
         octet_to_cell<FG::kGroup, FG::kSigned>(cx0, cx1, o, cells);
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
         if (lane == 0) __hip_atomic_fetch_add(&s_cells_done, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
@@ -442,9 +449,9 @@ __global__ __launch_bounds__(kThreads) void moe_layer_stream(MoeLayerParams q) {
                 // the reference's order: 8 chains over i = j (mod 8), summed 0..7 (crates/infr-cpu/src/kernels.rs:6568-6583)
                 const float4* wp = reinterpret_cast<const float4*>(wst + (e * 8 + j) * jstride);
                 const float4* xp = reinterpret_cast<const float4*>(xst + j * jstride);
-                const int n4 = oct_n >> 2;   // a multiple of 8
+                const int n4 = oct_n >> 2;   // a multiple of 8 unless kRagged
 #pragma unroll 1
-                for (int c = 0; c < n4; c += 8) {
+                for (int c = 0; c + 8 <= n4; c += 8) {
                     float4 a[8], bb[8];
 #pragma unroll
                     for (int k = 0; k < 8; k++) { a[k] = wp[c + k]; bb[k] = xp[c + k]; }
@@ -454,6 +461,15 @@ __global__ __launch_bounds__(kThreads) void moe_layer_stream(MoeLayerParams q) {
                         acc = __fmaf_rn(a[k].y, bb[k].y, acc);
                         acc = __fmaf_rn(a[k].z, bb[k].z, acc);
                         acc = __fmaf_rn(a[k].w, bb[k].w, acc);
+                    }
+                }
+                if (kRagged) {
+                    for (int c = n4 & ~7; c < n4; c++) {
+                        const float4 a = wp[c], bb = xp[c];
+                        acc = __fmaf_rn(a.x, bb.x, acc);
+                        acc = __fmaf_rn(a.y, bb.y, acc);
+                        acc = __fmaf_rn(a.z, bb.z, acc);
+                        acc = __fmaf_rn(a.w, bb.w, acc);
                     }
                 }
             }
@@ -473,7 +489,7 @@ __global__ __launch_bounds__(kThreads) void moe_layer_stream(MoeLayerParams q) {
             RouteParams rp = p.route;
             rp.logits = s_logits;
             rp.n_expert = n_expert;   // compile-time here: the routing code's loops and index arithmetic fold
-            rp.n_used = kGroups;
+            rp.n_used = KR;
             // the guess is the candidate for the selection: when the exact probabilities confirm it, the selection
             // rounds are not needed; else (a missed expert, a tie at the boundary, another gating) the complete routine
             const int guess_state = lds_flag_wait(&s_f_spec);
@@ -491,21 +507,21 @@ __global__ __launch_bounds__(kThreads) void moe_layer_stream(MoeLayerParams q) {
             if (ok) {
                 // lane k < 8 owns rank k: the group whose guess is that expert; ranks the guess missed take the groups
                 // whose guess is outside the exact set, both in ascending order
-                const bool rank = lane < kGroups;
+                const bool rank = lane < KR;
                 const int id = rank ? s_ids[lane] : -1;
                 int gk = -1;
 #pragma unroll
-                for (int gg = 0; gg < kGroups; gg++)
+                for (int gg = 0; gg < KR; gg++)
                     if (s_spec[gg] == id) gk = gg;
                 uint32_t used = 0;
 #pragma unroll
-                for (int gg = 0; gg < kGroups; gg++) used |= (__ballot(rank && gk == gg) ? 1u : 0u) << gg;
-                const uint32_t missed = (uint32_t)__ballot(rank && gk < 0) & 0xFFu;
+                for (int gg = 0; gg < KR; gg++) used |= (__ballot(rank && gk == gg) ? 1u : 0u) << gg;
+                const uint32_t missed = (uint32_t)__ballot(rank && gk < 0) & ((1u << KR) - 1u);
                 if (rank && gk < 0) {
                     const int j = __builtin_popcount(missed & ((1u << lane) - 1u));
                     int seen = 0;
 #pragma unroll
-                    for (int gg = 0; gg < kGroups; gg++) {
+                    for (int gg = 0; gg < KR; gg++) {
                         const bool free_g = !((used >> gg) & 1u);
                         if (free_g && seen == j) gk = gg;
                         seen += free_g ? 1 : 0;
@@ -569,7 +585,7 @@ __global__ __launch_bounds__(kThreads) void moe_layer_stream(MoeLayerParams q) {
             STAMP(3);
             if (ok) {
                 __builtin_amdgcn_wave_barrier();
-                guess_set<NS>(s_alog, n_expert, kGroups, q.guess_skew, lane, s_spec, s_guess);
+                guess_set<NS>(s_alog, n_expert, KR, q.guess_skew, lane, s_spec, s_guess);
             } else if (lane == 0) {
                 s_fault = 1;
                 __hip_atomic_store(q.fault, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
@@ -644,7 +660,7 @@ __global__ __launch_bounds__(kThreads) void moe_layer_stream(MoeLayerParams q) {
                 if (fi < fpb)
                     rec_store_xcd(q.xh + (size_t)g * nff + f0 + fi,
                                   gated_act_fn(p.act, p.has_clamp, p.clamp, s_g[wave][lane], s_u[wave][lane], s_tab),
-                                  seq_tag | (uint32_t)e_cur, true);
+                                  seq_tag | (uint32_t)e_cur, one_xcd);
             }
             __builtin_amdgcn_wave_barrier();
             if (wave == 3) STAMP(7);
@@ -653,17 +669,19 @@ __global__ __launch_bounds__(kThreads) void moe_layer_stream(MoeLayerParams q) {
             // ---- hand-over of the group's activations: six (or four) wavefronts gather a share each and turn it into cells
             bool superseded = false;
             if (sw < n_gather) {
-                const int st = gather_activations<4>(q.xh + (size_t)g * nff + sw * chunk, chunk, seq_tag | (uint32_t)e_cur,
+                const int st = gather_activations<KR == 4 ? 9 : 4>(q.xh + (size_t)g * nff + sw * chunk, chunk, seq_tag | (uint32_t)e_cur,
                                                      s_h + sw * chunk, lane, spin_limit, attempt == 0);
                 if (wave == 1) STAMP(9);
                 superseded = st == kGatherSuperseded;
                 if (st == kGathered) {
                     __builtin_amdgcn_wave_barrier();
-                    if (lane * 8 < chunk) {   // whole groups of four lanes
-                        const int oct = sw * (chunk >> 3) + lane;
+                    auto to_cell = [&](int o8) __attribute__((always_inline)) {
+                        const int oct = sw * (chunk >> 3) + o8;
                         const float4 lo = *reinterpret_cast<const float4*>(s_h + 8 * oct), hi = *reinterpret_cast<const float4*>(s_h + 8 * oct + 4);
                         octet_to_cell<FD::kGroup, FD::kSigned>(lo, hi, oct, hcells);
-                    }
+                    };
+                    if (lane * 8 < chunk) to_cell(lane);   // whole groups of four lanes
+                    if (KR == 4 && (lane + kWave) * 8 < chunk) to_cell(lane + kWave);   // (more than 512 activations)
                 } else if (st == kGatherTimeout && lane == 0) {
                     s_fault = 1;
                     __hip_atomic_store(q.fault, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
@@ -722,7 +740,7 @@ __global__ __launch_bounds__(kThreads) void moe_layer_stream(MoeLayerParams q) {
         // the output, which are also the rows of the always-on expert it has just computed.  out = sum over ranks of
         // w_rank * y_rank as a separate multiply and add (crates/infr-cpu/src/lib.rs:4290-4302), then the always-on
         // expert, then the residual operand.  The partial results are polled while the streaming wavefronts still work.
-        const int R = ne / mpg, SR = R / kGroups;
+        const int R = ne / mpg, SR = KR == 8 ? R / 8 : (R + KR - 1) / KR;   // (KR = 4: the last groups' shares may be shorter)
         const int nblk_d = nff / FD::kBlockElems;
         const size_t rb_d = (size_t)nblk_d * FD::kBlockBytes;
         const Place<FD> pd(nblk_d, lane);
@@ -794,17 +812,17 @@ __global__ __launch_bounds__(kThreads) void moe_layer_stream(MoeLayerParams q) {
                 ring_drain<DD>(n_w0, wd_issue, wd_finish);
             }
         }
-        const bool mine = lane < SR;
+        const bool mine = lane < SR && (KR == 8 || g * SR + lane < R);
         const size_t oi = (size_t)m * R + (size_t)g * SR + (mine ? lane : 0);
-        uint64_t yk[kGroups];
+        uint64_t yk[KR];
         bool ok = *(volatile int*)&s_f_route == 1;
         if (ok) {
             for (int spin = 0;; spin++) {
 #pragma unroll
-                for (int k = 0; k < kGroups; k++) yk[k] = rec_load(q.ypart + (size_t)s_gor[k] * ne + oi);   // rank order
+                for (int k = 0; k < KR; k++) yk[k] = rec_load(q.ypart + (size_t)s_gor[k] * ne + oi);   // rank order
                 bool got = true;
 #pragma unroll
-                for (int k = 0; k < kGroups; k++) got = got && (uint32_t)(yk[k] >> 32) == (seq_tag | (uint32_t)s_ids[k]);
+                for (int k = 0; k < KR; k++) got = got && (uint32_t)(yk[k] >> 32) == (seq_tag | (uint32_t)s_ids[k]);
                 if (__all(got || !mine)) break;
                 if (spin >= spin_limit) {
                     ok = false;
@@ -820,7 +838,7 @@ __global__ __launch_bounds__(kThreads) void moe_layer_stream(MoeLayerParams q) {
         if (ok && mine && !*(volatile int*)&s_fault) {
             float acc = 0.0f;
 #pragma unroll
-            for (int k = 0; k < kGroups; k++) acc = __fadd_rn(acc, __fmul_rn(s_w[k], __uint_as_float((uint32_t)yk[k])));
+            for (int k = 0; k < KR; k++) acc = __fadd_rn(acc, __fmul_rn(s_w[k], __uint_as_float((uint32_t)yk[k])));
             if (shared) {
                 float ws = 1.0f;
                 if (p.sh_logit)   // crates/infr-cpu/src/lib.rs:3336-3356: sigmoid of the row's gate logit
@@ -842,18 +860,18 @@ struct StreamShape {
 
 namespace {
 
-template <class FG, class FD, int DG, int DD, int EPT, int NSP, int NE = 0, int NFF = 0, int ROWS = 0, int NORM = 0>
+template <class FG, class FD, int DG, int DD, int EPT, int NSP, int NE = 0, int NFF = 0, int ROWS = 0, int NORM = 0, int KR = 8>
 bool launch_stream(hipStream_t s, const MoeLayerParams& q, size_t lds) {
     static bool attr_ok[16] = {};
     int dev = 0;
     if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 16) return false;
     if (!attr_ok[dev]) {
-        if (hipFuncSetAttribute((const void*)moe_layer_stream<FG, FD, DG, DD, EPT, NSP, NE, NFF, ROWS, NORM>,
+        if (hipFuncSetAttribute((const void*)moe_layer_stream<FG, FD, DG, DD, EPT, NSP, NE, NFF, ROWS, NORM, KR>,
                                 hipFuncAttributeMaxDynamicSharedMemorySize, 150 * 1024) != hipSuccess)
             return false;
         attr_ok[dev] = true;
     }
-    INFR_LAUNCH((moe_layer_stream<FG, FD, DG, DD, EPT, NSP, NE, NFF, ROWS, NORM>), dim3(kBlocks), dim3(kThreads), lds, s, q);
+    INFR_LAUNCH((moe_layer_stream<FG, FD, DG, DD, EPT, NSP, NE, NFF, ROWS, NORM, KR>), dim3(kBlocks), dim3(kThreads), lds, s, q);
     return true;
 }
 

@@ -9,7 +9,7 @@ import pytest
 import helpers as H
 import moe4all_amd as M
 import oracle as O
-from moe4all_amd import DType
+from moe4all_amd import DType, synth
 from test_gpu_parity import _realistic, bits, moe_graph
 
 pytestmark = pytest.mark.gpu
@@ -629,6 +629,71 @@ def test_32_experts_of_hidden_size_1024_with_norm_and_residual(be, gdt, ddt, sha
             b.prof_enable(False)
             if not plain:
                 assert names == {"moe_layer_shared" if shared else "moe_layer"}, names
+        finally:
+            if plain:
+                b.close()
+    assert np.array_equal(bits(outs[0]), bits(outs[1])) and np.abs(outs[0] - x.reshape(-1)).max() > 1e-4
+
+
+@pytest.mark.parametrize("ne,nff,E,skew,opts", [
+    (2880, 2880, 128, 0, {}), (2880, 2880, 128, 4, dict(with_down_scale=True)), (1024, 512, 64, 0, {}),
+    (1088, 640, 64, 1, {}),                         # rows of 17 lanes, octets that end inside a wavefront, 17 output rows a workgroup
+    (2048, 768, 128, 2, dict(gating=M.MoeGating.Sigmoid)), (3008, 1920, 128, 0, dict(act=M.Activation.Gelu, swiglu_clamp=0.05)),
+    (4096, 1536, 64, 8, {}), (4096, 2880, 128, 0, {})])
+def test_four_experts_per_token_in_one_launch(be3, ne, nff, E, skew, opts):
+    """Groups of 64 workgroups on two XCDs each, MXFP4 banks: ids, weights, logits, probabilities and output bits of the
+    three-launch path, also when the guess misses `skew` experts."""
+    K, dt = 4, M.DType.Mxfp4
+    rng = np.random.default_rng(ne + nff + skew)
+    x = rng.standard_normal((1, ne)).astype(np.float32)
+    router = (rng.standard_normal((E, ne)) * 0.02).astype(np.float32)
+    gate, up, down = (synth.weights_host(dt, ne + i, E * nff * ne) for i in range(3))
+    data = dict(x=x, router=router, gate=gate, up=up, down=down)
+    if opts.get("with_down_scale"):
+        data["down_scale"] = rng.uniform(0.5, 1.5, E).astype(np.float32)
+    b = M.Backend(0, single_launch_guess_skew=skew)
+    try:
+        before = b.late_experts()
+        for rep in range(2):
+            g, ids = moe_graph(1, ne, E, K, nff, dt, dt, **opts)
+            one, r1 = _run(b, g, ids, data, ne, GUESS)
+            g, ids = moe_graph(1, ne, E, K, nff, dt, dt, **opts)
+            three, r3 = _run(be3, g, ids, data, ne, "moe_route_gate_up")
+            assert np.array_equal(r1["idx"], r3["idx"]) and np.array_equal(bits(r1["w"]), bits(r3["w"]))
+            assert np.array_equal(bits(r1["logits"]), bits(r3["logits"])) and np.array_equal(bits(r1["probs"]), bits(r3["probs"]))
+            assert np.array_equal(bits(one), bits(three)) and np.abs(three).max() > 1e-6
+        assert b.late_experts() - before == 2 * min(skew, K)
+    finally:
+        b.close()
+
+
+def test_four_experts_per_token_with_norm_and_residual(be):
+    """y = x + ffn(rmsnorm(x) * w) of one token as one launch: the bits of one launch per op."""
+    ne, E, K, nff, dt = 2880, 64, 4, 960, DType.Mxfp4
+    rng = np.random.default_rng(77)
+    T = M.TensorDesc
+    x = (rng.standard_normal((1, ne)) * 3.0).astype(np.float32)
+    nw = rng.uniform(0.5, 1.5, ne).astype(np.float32)
+    router = (rng.standard_normal((E, ne)) * 0.02).astype(np.float32)
+    gate, up, down = (synth.weights_host(dt, ne + i, E * nff * ne) for i in range(3))
+    outs = []
+    for plain in (False, True):
+        b = M.Backend(0, disable_op_fusion=True, disable_single_launch_moe=True) if plain else be
+        try:
+            g = M.Graph()
+            xi, nwt, rt = g.input(T([1, ne], DType.F32)), g.weight(T([ne], DType.F32)), g.weight(T([E, ne], DType.F32))
+            gt, ut, dw = g.weight(T([E, nff, ne], dt)), g.weight(T([E, nff, ne], dt)), g.weight(T([E, ne, nff], dt))
+            xn, moe, y = g.internal(T([1, ne], DType.F32)), g.internal(T([1, ne], DType.F32)), g.output(T([1, ne], DType.F32))
+            g.rms_norm(x=xi, weight=nwt, dst=xn, rows=1, dim=ne, eps=1e-6)
+            g.moe_ffn(x=xn, router=rt, gate_exps=gt, up_exps=ut, down_exps=dw, dst=moe, ne=ne, n_expert=E, n_used=K, n_ff_exp=nff)
+            g.add(a=xi, b=moe, dst=y, n=ne)
+            b.prof_enable(True)
+            outs.append(M.run_graph(b, g, [(xi, x), (nwt, nw), (rt, router), (gt, gate), (ut, up), (dw, down)], y, ne))
+            b.sync()
+            names = set(b.prof_read())
+            b.prof_enable(False)
+            if not plain:
+                assert names == {"moe_layer"}, names
         finally:
             if plain:
                 b.close()
