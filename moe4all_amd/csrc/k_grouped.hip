@@ -138,18 +138,110 @@ __global__ __launch_bounds__(256) void route_rows_to_f16_kernel(RouteParams rp, 
 }
 
 // --------------------------------------------------------------------------------------------
-// One block of four or sixteen wavefronts per expert e in 0..n_expert; the extra one marks pairs whose id is
-// out of range.  The block stages the pair ids in LDS (16-bit, in chunks), counts every expert's pairs (those of the experts below e
-// give the bucket's offset and its tiles' places in the tile table), and then scatters the pairs equal to e: each wavefront takes a
-// contiguous part of the chunk, the parts' hit counts give every wavefront its base, and inside a part a wave-wide prefix keeps the
-// flat (row, rank) order, so buckets come out rows ascending.  Four wavefronts take up to kBucketFew pairs, one chunk.
+// The size class of an expert's bucket, by which the tile table is ordered.
+__device__ __forceinline__ int size_class(uint32_t pairs) { return pairs <= 16 ? 0 : pairs > 256 ? 5 : 32 - __clz((pairs - 1) >> 4); }
+
+// Up to NT * J pairs: one block of NT / 64 wavefronts per expert e in 0..n_expert; the extra one marks pairs whose id is out of
+// range.  A thread holds the ids of pairs tid, tid + NT, ... in registers; the block counts every expert's pairs (those of the
+// experts below e give the bucket's offset and its tiles' places in the tile table; consecutive lanes hold consecutive pairs, and
+// the ids of one token differ, so few lanes meet on one counter), and then scatters the pairs equal to e: a ballot per 64 pairs
+// gives the places among them, the ballots' counts in flat (row, rank) order the rest, so buckets come out rows ascending.
+// A chain of latencies: the launch, the ids, the counters, two barriers.  What it takes, us a launch against the ids staged in LDS and scanned twice from there, 128 experts, top-8: 16 rows
+// 5.04 and 4.95, 64 rows 5.47 and 5.09, 2048 rows 14.7 and 14.3; us a pass: 3 layers of 16 rows in Q8_0 358.5 and 354.5, two of 64 in
+// Q4_K / Q6_K 241.8 and 239.5, 333 rows in Q5_K 126.5 and 125.2, 512 in Q8_0 166.1 and 164.7.
 constexpr int kBucketFew = 2048, kBucketMany = 16384;
+template <int NT, int J>
+__global__ __launch_bounds__(NT) void bucket_once_kernel(const int32_t* __restrict__ ids, int n_pairs, int n_expert, int n_used,
+                                                         int32_t* __restrict__ offsets, int32_t* __restrict__ pair_src,
+                                                         int32_t* __restrict__ slot_pair, int32_t* __restrict__ pair_row,
+                                                         int4* __restrict__ tiles, int tile, int by_size, int always_rows) {
+    constexpr int NW = NT / 64;
+    static_assert(NW % 4 == 0 && J * NW <= 256, "");
+    __shared__ uint32_t s_hist[2048];                                  // n_expert <= 2048
+    __shared__ __attribute__((aligned(16))) uint32_t s_hits[256];      // pairs of e among 64 j NW + 64 wave ...
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const uint32_t e = blockIdx.x;
+    uint32_t id[J];
+#pragma unroll
+    for (int j = 0; j < J; j++) {
+        id[j] = ~0u;
+        if (j * NT < n_pairs) id[j] = (uint32_t)ids[min(j * NT + tid, n_pairs - 1)];
+    }
+    for (int i = tid; i < n_expert; i += NT) s_hist[i] = 0;
+    if (tid < 256) s_hits[tid] = 0;
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < J; j++) {
+        if (j * NT >= n_pairs) break;
+        if (j * NT + tid >= n_pairs || id[j] >= (uint32_t)n_expert) id[j] = ~0u;
+        else atomicAdd(&s_hist[id[j]], 1u);
+        const uint32_t hits = __builtin_popcountll(__ballot(id[j] == e));
+        if (lane == 0) s_hits[j * NW + wave] = hits;
+    }
+    __syncthreads();
+    // every wavefront for itself: the bucket's offset and its tiles' places, and where its own pairs of e go
+    const uint32_t own = e < (uint32_t)n_expert ? s_hist[e] : (uint32_t)always_rows;
+    uint32_t below = 0, tiles_below = 0, tiles_all = 0;
+    for (int i = lane; i <= n_expert; i += 64) {
+        const uint32_t c = i < n_expert ? s_hist[i] : (uint32_t)always_rows, nt = (c + tile - 1) / tile;
+        if (i < (int)e) below += c;
+        tiles_all += nt;
+        if (by_size && size_class(c) != size_class(own) ? c > own : i < (int)e) tiles_below += nt;
+    }
+    const uint4 h = *reinterpret_cast<const uint4*>(&s_hits[4 * lane]);
+    uint32_t incl = h.x + h.y + h.z + h.w;
+    const uint32_t quad = incl;
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+        below += __shfl_xor(below, d, 64);
+        tiles_below += __shfl_xor(tiles_below, d, 64);
+        tiles_all += __shfl_xor(tiles_all, d, 64);
+        const uint32_t o = __shfl_up(incl, d, 64);
+        if (lane >= d) incl += o;
+    }
+    if (tid == 0) offsets[e] = (int32_t)below;
+    if (tiles) {   // slot 0: the number of tiles; then the tiles
+        if (e == (uint32_t)n_expert && tid == 0) tiles[0] = make_int4((int)tiles_all, 0, 0, 0);
+        const int cnt = (int)own, first = e == (uint32_t)n_expert ? n_pairs : (int)below;
+        for (int i = tid; i * tile < cnt; i += NT)
+            tiles[1 + tiles_below + i] = by_size ? make_int4((int)e, first + i * tile, min(tile, cnt - i * tile), 0)
+                                                 : make_int4((int)e, first, cnt, (int)tiles_below);
+        if (e == (uint32_t)n_expert)
+            for (int i = tid; i < always_rows; i += NT) pair_row[n_pairs + i] = i;
+    }
+    if (e == (uint32_t)n_expert) {
+#pragma unroll
+        for (int j = 0; j < J; j++)
+            if (j * NT + tid < n_pairs && id[j] == ~0u) slot_pair[j * NT + tid] = -1;
+        return;
+    }
+    const int sub = wave & 3;
+    const uint32_t before = below + incl - quad + (sub > 0 ? h.x : 0u) + (sub > 1 ? h.y : 0u) + (sub > 2 ? h.z : 0u);
+#pragma unroll
+    for (int j = 0; j < J; j++) {
+        if (j * NT >= n_pairs) break;
+        const uint32_t base = (uint32_t)__builtin_amdgcn_readlane((int)before, j * (NW / 4) + (wave >> 2));
+        const uint64_t hits = __ballot(id[j] == e);
+        if (id[j] == e) {
+            const int i = j * NT + tid;
+            const uint32_t pos = base + __builtin_popcountll(hits & ((1ull << lane) - 1));
+            pair_src[pos] = i;
+            slot_pair[i] = (int32_t)pos;
+            if (pair_row) pair_row[pos] = i / n_used;
+        }
+    }
+}
+
+// More pairs: one block of sixteen wavefronts per expert e in 0..n_expert as above.  The block stages the pair ids in LDS (16-bit, in
+// chunks), counts every expert's pairs, and then scatters the pairs equal to e: each wavefront takes a
+// contiguous part of the chunk, the parts' hit counts give every wavefront its base, and inside a part a wave-wide prefix keeps the
+// flat (row, rank) order.
 template <int NT>
 __global__ __launch_bounds__(NT) void bucket_kernel(const int32_t* __restrict__ ids, int n_pairs, int n_expert,
                                                      int n_used, int32_t* __restrict__ offsets, int32_t* __restrict__ pair_src,
                                                      int32_t* __restrict__ slot_pair, int32_t* __restrict__ pair_row,
                                                      int4* __restrict__ tiles, int tile, int by_size, int always_rows) {
-    constexpr int kBucketChunk = NT == 256 ? kBucketFew : kBucketMany;
+    constexpr int kBucketChunk = kBucketMany;
     constexpr int NW = NT / 64, NL = kBucketChunk / 4 / NT;
     __shared__ __attribute__((aligned(16))) uint16_t s_ids[kBucketChunk];
     __shared__ uint32_t s_hist[2048];
@@ -197,7 +289,6 @@ __global__ __launch_bounds__(NT) void bucket_kernel(const int32_t* __restrict__ 
         for (int d = 32; d >= 1; d >>= 1) v += __shfl_xor(v, d, 64);
         return v;
     };
-    const bool single = NT == 256 || n_pairs <= kBucketChunk;   // a single chunk stays staged for the second pass
 
     // ---- pass 0: how many pairs each expert has; from that the bucket's offset and its tiles' places in the tile table
     for (int i = tid; i < n_expert; i += NT) s_hist[i] = 0;
@@ -216,7 +307,6 @@ __global__ __launch_bounds__(NT) void bucket_kernel(const int32_t* __restrict__ 
     }
     __syncthreads();
     const uint32_t own = e < (uint32_t)n_expert ? s_hist[e] : (uint32_t)always_rows;
-    auto size_class = [](uint32_t pairs) { return pairs <= 16 ? 0 : pairs > 256 ? 5 : 32 - __clz((pairs - 1) >> 4); };
     uint32_t below = 0, tiles_below = 0, tiles_all = 0;
     for (int i = tid; i <= n_expert; i += NT) {
         const uint32_t c = i < n_expert ? s_hist[i] : (uint32_t)always_rows, nt = (c + tile - 1) / tile;
@@ -247,7 +337,7 @@ __global__ __launch_bounds__(NT) void bucket_kernel(const int32_t* __restrict__ 
     uint32_t run = below;
     for (int c0 = 0; c0 < n_pairs; c0 += kBucketChunk) {
         const int cn = min(kBucketChunk, n_pairs - c0);
-        if (!single) stage(c0, cn);
+        stage(c0, cn);
         if (e == (uint32_t)n_expert) {
             for (int i = tid; i < cn; i += NT)
                 if (s_ids[i] == 0xFFFFu) slot_pair[c0 + i] = -1;
@@ -583,14 +673,14 @@ void launch_rows_to_f16(hipStream_t s, int weight_dt, const float* src, int rows
 
 void launch_bucket(hipStream_t s, const int32_t* ids, int n_pairs, int n_expert, int n_used, int32_t* offsets, int32_t* pair_src,
                    int32_t* slot_pair, int32_t* pair_row, int4* tiles, int tile, int by_size, int always_rows) {
-    // sixteen wavefronts where the ids are many: staging, counting and scattering are each a serial chain per wavefront
-    // (rows of 128 experts, top-8: 2048 20.3 -> 14.6 us, 512 9.9 -> 8.8, 333 8.2 -> 7.5)
-    if (n_pairs > kBucketFew)
-        INFR_LAUNCH(bucket_kernel<1024>, dim3(n_expert + 1), dim3(1024), 0, s, ids, n_pairs, n_expert, n_used, offsets, pair_src,
-                    slot_pair, pair_row, tiles, tile, by_size, always_rows);
-    else
-        INFR_LAUNCH(bucket_kernel<256>, dim3(n_expert + 1), dim3(256), 0, s, ids, n_pairs, n_expert, n_used, offsets, pair_src,
-                    slot_pair, pair_row, tiles, tile, by_size, always_rows);
+    const dim3 grid(n_expert + 1);
+#define INFR_BUCKET(KERNEL, NT)                                                                                               \
+    INFR_LAUNCH(KERNEL, grid, dim3(NT), 0, s, ids, n_pairs, n_expert, n_used, offsets, pair_src, slot_pair, pair_row, tiles, tile, by_size, \
+                always_rows)
+    if (n_pairs <= kBucketFew) INFR_BUCKET((bucket_once_kernel<256, kBucketFew / 256>), 256);
+    else if (n_pairs <= kBucketMany) INFR_BUCKET((bucket_once_kernel<1024, kBucketMany / 1024>), 1024);
+    else INFR_BUCKET(bucket_kernel<1024>, 1024);
+#undef INFR_BUCKET
 }
 
 bool launch_route_bucket(hipStream_t s, const RouteParams& rp, int32_t* offsets, int32_t* pair_src, int32_t* slot_pair, int32_t* pair_row,

@@ -467,6 +467,35 @@ def test_bucketing_of_many_pairs(be, rows, K):
     assert np.array_equal(b["slot_pair"].reshape(-1), slot)
 
 
+@pytest.mark.parametrize("rows,K,E", [
+    (33, 1, 3), (64, 8, 1000),                       # fewer pairs than threads; more experts than pairs
+    (2048, 1, 7), (683, 3, 61),                      # 2048 pairs on four wavefronts, 2049 on sixteen
+    (2048, 8, 61), (3277, 5, 61),                    # 16384 held in registers, 16385 in chunks
+])
+def test_bucketing_at_the_edges_of_its_kernels(be, rows, K, E):
+    """The reference's order exactly, and token rows that have the bits of small batches (33 rows at a time)."""
+    ne, nff = 64, 64
+    rng = np.random.default_rng(rows + K + E)
+    sel = np.argsort(rng.random((rows, E)) + 0.6 * np.arange(E) / E, axis=1)[:, :K].astype(np.int32)   # uneven buckets
+    gate, up, down = _bank_weights(rng, E, nff, ne, H.Q8_0, H.Q8_0)
+    x = rng.standard_normal((rows, ne)).astype(np.float32)
+    data = dict(router=np.zeros((E, ne), np.float32), gate=gate, up=up, down=down)
+    g, ids = moe_graph(rows, ne, E, K, nff, DType.Q8_0, DType.Q8_0, with_expert_ids=True)
+    out, _, b = _run_batched(be, g, ids, dict(data, x=x, expert_ids=sel), rows, ne)
+    flat = sel.reshape(-1)
+    order = np.argsort(flat, kind="stable")
+    assert np.array_equal(np.diff(b["offsets"]), np.bincount(flat, minlength=E))
+    assert np.array_equal(b["pair_row"], order // K) and np.array_equal(b["pair_rank"], order % K)
+    slot = np.empty_like(order)
+    slot[order] = np.arange(len(order))
+    assert np.array_equal(b["slot_pair"].reshape(-1), slot)
+    for first in (0, rows - 33):   # the last rows among them: they may share a workgroup of the conversion with none
+        part = slice(first, first + 33)
+        g, ids = moe_graph(33, ne, E, K, nff, DType.Q8_0, DType.Q8_0, with_expert_ids=True)
+        few, _, _ = _run_batched(be, g, ids, dict(data, x=np.ascontiguousarray(x[part]), expert_ids=np.ascontiguousarray(sel[part])), 33, ne)
+        assert np.array_equal(bits(few), bits(out[part]))
+
+
 @pytest.mark.parametrize("rows,E,K,units", [(16, 8, 2, False), (16, 64, 2, True), (16, 65, 2, True), (16, 9, 3, False), (17, 8, 1, False),
                                             (16, 1, 1, False), (1, 5, 2, True), (3, 64, 10, True), (3, 64, 11, True), (1, 64, 32, True)])
 def test_routing_and_bucketing_of_a_few_rows(be, rows, E, K, units):
