@@ -1743,19 +1743,20 @@ extern "C" infr_status infr_hip_execute(infr_hip_backend* be, infr_hip_plan* pla
                 }
                 if (sc.batched) {
                     const int pairs = rows * (int)m.n_used;
-                    {   // routing, and in the same launch the token rows as f16 for the gate/up GEMM
-                        Timed t(be, "route_topk");
-                        infr::launch_route_rows_to_f16(s, rp, gp.gate_dt, gp.x, (int)m.ne, sc.xh, sc.xs, sc.xm);
-                    }
                     {
+                        Timed t(be, "route_topk");
+                        infr::launch_route(s, rp);
+                    }
+                    {   // bucketing, and in the same launch the token rows as f16 for the gate/up GEMM
                         Timed t(be, "moe_bucket");
+                        const infr::RowsToF16 conv{gp.x, rows, (int)m.ne, gp.gate_dt, sc.xh, sc.xs, sc.xm};
                         const int32_t* bucket_ids = sc.ids;
                         if (m.has_ep_band) {   // pairs of foreign experts (weight 0) are not bucketed at all
                             infr::launch_mask_dropped_pairs(s, sc.ids, sc.weights, pairs, sc.live_ids);
                             bucket_ids = sc.live_ids;
                         }
                         infr::launch_bucket(s, bucket_ids, pairs, (int)n_local, (int)m.n_used, sc.offsets, sc.pair_src, sc.slot_pair,
-                                            sc.pair_row, sc.tiles, 1 << sc.tile_log2, 1, al_gate ? rows : 0);
+                                            sc.pair_row, sc.tiles, 1 << sc.tile_log2, 1, al_gate ? rows : 0, &conv);
                     }
                     infr::GroupedParams q{};
                     q.loads_only = be->probe_grouped_loads_only.load() ? 1 : 0;

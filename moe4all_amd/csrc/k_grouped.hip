@@ -10,7 +10,7 @@
 //                         of a few rows, in one launch.
 //   rows_to_f16_kernel    activation rows -> f16 with one power-of-two scale per row (so any f32
 //                         magnitude fits), laid out in the k order the weight format unpacks to
-//                         (route_rows_to_f16_kernel: the same for the token rows, with the row's routing).
+//                         (the token rows beside the bucketing, in its launch)
 //   grouped_gemm / grouped_float_mfma   the GEMMs (k_grouped_gemm.hip, k_grouped_float.hip)
 //   unbucket_combine      dst[row] = sum over ranks (rank order, separate mul and add,
 //                         lib.rs:4290-4302) of w * y[pair of (row, rank)].
@@ -60,26 +60,63 @@ __device__ __forceinline__ uint4 chunk_to_f16(float4 a, float4 b, float inv, int
     return uint4{as_u32(h0), as_u32(h1), as_u32(h2), as_u32(h3)};
 }
 
-// One block per row: amax -> power-of-two scale -> f16 in the virtual k order of format F.
+// A row by 256 threads (t: the thread's place among them): amax -> power-of-two scale -> f16 in the virtual k order of format F.
+// Rows of up to 2048 kHold wait in registers for their scale, longer ones are read twice.  All threads of the block pass the one barrier.
 template <class F>
-__device__ __forceinline__ void row_to_f16(const float* __restrict__ src, int n, _Float16* __restrict__ dst,
-                                           float* __restrict__ scale, size_t row, float* s_max, uint32_t* __restrict__ sums) {
+__device__ __forceinline__ void row_to_f16(const float* __restrict__ src, int n, _Float16* __restrict__ dst, float* __restrict__ scale,
+                                           size_t row, int t, float* s_max, uint32_t* __restrict__ sums, bool live = true) {
+    constexpr int kHold = 2;   // chunks of 8 elements a thread holds
     const float* x = src + row * n;
+    uint4* out = reinterpret_cast<uint4*>(dst + row * n);
+    uint32_t* row_sums = sums + row * (n / 32);
+    const bool held = n <= 2048 * kHold;
+    float4 a[kHold], b[kHold];
     float m = 0.0f;
-    for (int k = threadIdx.x * 4; k < n; k += 1024) {
-        const float4 v = *reinterpret_cast<const float4*>(x + k);
-        m = fmaxf(fmaxf(m, fmaxf(fabsf(v.x), fabsf(v.y))), fmaxf(fabsf(v.z), fabsf(v.w)));
+    if (held) {
+#pragma unroll
+        for (int i = 0; i < kHold; i++) {   // (threads behind the row's end repeat its last chunk)
+            const int c = min(256 * i + t, n / 8 - 1);
+            a[i] = *reinterpret_cast<const float4*>(x + F::lo(c));
+            b[i] = *reinterpret_cast<const float4*>(x + F::hi(c));
+        }
+#pragma unroll
+        for (int i = 0; i < kHold; i++) {
+            m = fmaxf(fmaxf(m, fmaxf(fabsf(a[i].x), fabsf(a[i].y))), fmaxf(fabsf(a[i].z), fabsf(a[i].w)));
+            m = fmaxf(fmaxf(m, fmaxf(fabsf(b[i].x), fabsf(b[i].y))), fmaxf(fabsf(b[i].z), fabsf(b[i].w)));
+        }
+    } else {
+        for (int k = t * 4; k < n; k += 1024) {
+            const float4 v = *reinterpret_cast<const float4*>(x + k);
+            m = fmaxf(fmaxf(m, fmaxf(fabsf(v.x), fabsf(v.y))), fmaxf(fabsf(v.z), fabsf(v.w)));
+        }
     }
     m = wave_max(m);
-    if ((threadIdx.x & 63) == 0) s_max[threadIdx.x >> 6] = m;
+    if ((t & 63) == 0) s_max[t >> 6] = m;
     __syncthreads();
+    if (!live) return;
     m = fmaxf(fmaxf(s_max[0], s_max[1]), fmaxf(s_max[2], s_max[3]));
     const int e = row_exponent(m);
     const float inv = ldexpf(1.0f, -e);
-    if (threadIdx.x == 0) scale[row] = ldexpf(1.0f, e);
-    uint4* out = reinterpret_cast<uint4*>(dst + row * n);
-    for (int c = threadIdx.x; c < n / 8; c += 256)
-        out[c] = chunk_to_f16<F>(*reinterpret_cast<const float4*>(x + F::lo(c)), *reinterpret_cast<const float4*>(x + F::hi(c)), inv, c, sums + row * (n / 32));
+    if (t == 0) scale[row] = ldexpf(1.0f, e);
+    if (held) {
+#pragma unroll
+        for (int i = 0; i < kHold; i++)
+            if (256 * i + t < n / 8) out[256 * i + t] = chunk_to_f16<F>(a[i], b[i], inv, 256 * i + t, row_sums);
+    } else {
+        for (int c = t; c < n / 8; c += 256)
+            out[c] = chunk_to_f16<F>(*reinterpret_cast<const float4*>(x + F::lo(c)), *reinterpret_cast<const float4*>(x + F::hi(c)), inv, c, row_sums);
+    }
+}
+
+// The f16 conversion of a batch's token rows for the gate/up GEMM, which a bucketing launch takes along: it depends on nothing that the
+// routing made, and the bucketing is a chain of latencies on n_expert + 1 blocks.  The blocks behind those convert a row per 256 threads.
+// In the routing's launch, ahead of a row's routing on the same wavefronts, it took us a pass: two layers of 64 rows 238.2 and here 236.2,
+// 333 rows 127.9 and 126.5, 2048 rows 326.5 and 324.1 (2048 rows, us a launch: routing with conversion 14.9, bucketing 14.3; now 8 and 16).
+template <class F, int NT>
+__device__ __forceinline__ void rows_beside(const RowsToF16& c, int block) {
+    __shared__ float s_max[NT / 64];
+    const int q = threadIdx.x >> 8, row = block * (NT / 256) + q;
+    row_to_f16<F>(c.src, c.n, reinterpret_cast<_Float16*>(c.dst), c.scale, (size_t)min(row, c.rows - 1), threadIdx.x & 255, s_max + 4 * q, c.sums, row < c.rows);
 }
 
 // A wavefront per row of up to 512 NC elements, four rows per block: the row is read once and waits in registers for its scale
@@ -119,22 +156,7 @@ template <class F>
 __global__ __launch_bounds__(256) void rows_to_f16_kernel(const float* __restrict__ src, int n,
                                                           _Float16* __restrict__ dst, float* __restrict__ scale, uint32_t* __restrict__ sums) {
     __shared__ float s_max[4];
-    row_to_f16<F>(src, n, dst, scale, blockIdx.x, s_max, sums);
-}
-
-// The routing of token row b (route_kernel's work, on the block's first wavefront) behind the f16 conversion of the same
-// row for the gate/up GEMM: both are per row and both precede the bucketing, and a launch of either alone is mostly its
-// dispatch (32 to 2048 rows: 5.0-7.8 us and 3.9-4.7 us as two launches).
-template <class F>
-__global__ __launch_bounds__(256) void route_rows_to_f16_kernel(RouteParams rp, const float* __restrict__ src, int n,
-                                                                _Float16* __restrict__ dst, float* __restrict__ scale,
-                                                                uint32_t* __restrict__ sums) {
-    extern __shared__ float lds[];
-    __shared__ float s_max[4];
-    uint64_t* tab = reinterpret_cast<uint64_t*>(lds);
-    if (threadIdx.x < 32) tab[threadIdx.x] = kExp2Table[threadIdx.x];
-    row_to_f16<F>(src, n, dst, scale, blockIdx.x, s_max, sums);   // (its barrier also publishes the table)
-    if (threadIdx.x < 64) route_row_any(rp, blockIdx.x, threadIdx.x, lds + 64, tab);
+    row_to_f16<F>(src, n, dst, scale, blockIdx.x, threadIdx.x, s_max, sums);
 }
 
 // --------------------------------------------------------------------------------------------
@@ -150,11 +172,15 @@ __device__ __forceinline__ int size_class(uint32_t pairs) { return pairs <= 16 ?
 // 5.04 and 4.95, 64 rows 5.47 and 5.09, 2048 rows 14.7 and 14.3; us a pass: 3 layers of 16 rows in Q8_0 358.5 and 354.5, two of 64 in
 // Q4_K / Q6_K 241.8 and 239.5, 333 rows in Q5_K 126.5 and 125.2, 512 in Q8_0 166.1 and 164.7.
 constexpr int kBucketFew = 2048, kBucketMany = 16384;
-template <int NT, int J>
+template <class F, int NT, int J>
 __global__ __launch_bounds__(NT) void bucket_once_kernel(const int32_t* __restrict__ ids, int n_pairs, int n_expert, int n_used,
                                                          int32_t* __restrict__ offsets, int32_t* __restrict__ pair_src,
                                                          int32_t* __restrict__ slot_pair, int32_t* __restrict__ pair_row,
-                                                         int4* __restrict__ tiles, int tile, int by_size, int always_rows) {
+                                                         int4* __restrict__ tiles, int tile, int by_size, int always_rows, RowsToF16 conv) {
+    if ((int)blockIdx.x > n_expert) {
+        rows_beside<F, NT>(conv, blockIdx.x - n_expert - 1);
+        return;
+    }
     constexpr int NW = NT / 64;
     static_assert(NW % 4 == 0 && J * NW <= 256, "");
     __shared__ uint32_t s_hist[2048];                                  // n_expert <= 2048
@@ -236,11 +262,15 @@ __global__ __launch_bounds__(NT) void bucket_once_kernel(const int32_t* __restri
 // chunks), counts every expert's pairs, and then scatters the pairs equal to e: each wavefront takes a
 // contiguous part of the chunk, the parts' hit counts give every wavefront its base, and inside a part a wave-wide prefix keeps the
 // flat (row, rank) order.
-template <int NT>
+template <class F, int NT>
 __global__ __launch_bounds__(NT) void bucket_kernel(const int32_t* __restrict__ ids, int n_pairs, int n_expert,
                                                      int n_used, int32_t* __restrict__ offsets, int32_t* __restrict__ pair_src,
                                                      int32_t* __restrict__ slot_pair, int32_t* __restrict__ pair_row,
-                                                     int4* __restrict__ tiles, int tile, int by_size, int always_rows) {
+                                                     int4* __restrict__ tiles, int tile, int by_size, int always_rows, RowsToF16 conv) {
+    if ((int)blockIdx.x > n_expert) {
+        rows_beside<F, NT>(conv, blockIdx.x - n_expert - 1);
+        return;
+    }
     constexpr int kBucketChunk = kBucketMany;
     constexpr int NW = NT / 64, NL = kBucketChunk / 4 / NT;
     __shared__ __attribute__((aligned(16))) uint16_t s_ids[kBucketChunk];
@@ -647,15 +677,6 @@ void with_order(int dt, Fn&& f) {
 
 }  // namespace
 
-void launch_route_rows_to_f16(hipStream_t s, const RouteParams& rp, int weight_dt, const float* src, int n, void* dst, float* scale, uint32_t* sums) {
-    if (rp.rows <= 0) return;
-    _Float16* d = reinterpret_cast<_Float16*>(dst);
-    const size_t lds = (64 + route_scratch_floats(rp.n_expert, rp.n_groups)) * sizeof(float);
-    with_order(weight_dt, [&](auto order) {
-        INFR_LAUNCH(route_rows_to_f16_kernel<decltype(order)>, dim3(rp.rows), dim3(256), lds, s, rp, src, n, d, scale, sums);
-    });
-}
-
 void launch_rows_to_f16(hipStream_t s, int weight_dt, const float* src, int rows, int n, void* dst, float* scale, uint32_t* sums) {
     if (rows <= 0) return;
     _Float16* d = reinterpret_cast<_Float16*>(dst);
@@ -672,14 +693,19 @@ void launch_rows_to_f16(hipStream_t s, int weight_dt, const float* src, int rows
 }
 
 void launch_bucket(hipStream_t s, const int32_t* ids, int n_pairs, int n_expert, int n_used, int32_t* offsets, int32_t* pair_src,
-                   int32_t* slot_pair, int32_t* pair_row, int4* tiles, int tile, int by_size, int always_rows) {
-    const dim3 grid(n_expert + 1);
-#define INFR_BUCKET(KERNEL, NT)                                                                                               \
-    INFR_LAUNCH(KERNEL, grid, dim3(NT), 0, s, ids, n_pairs, n_expert, n_used, offsets, pair_src, slot_pair, pair_row, tiles, tile, by_size, \
-                always_rows)
-    if (n_pairs <= kBucketFew) INFR_BUCKET((bucket_once_kernel<256, kBucketFew / 256>), 256);
-    else if (n_pairs <= kBucketMany) INFR_BUCKET((bucket_once_kernel<1024, kBucketMany / 1024>), 1024);
-    else INFR_BUCKET(bucket_kernel<1024>, 1024);
+                   int32_t* slot_pair, int32_t* pair_row, int4* tiles, int tile, int by_size, int always_rows, const RowsToF16* conv) {
+    const int nt = n_pairs <= kBucketFew ? 256 : 1024;
+    const RowsToF16 c = conv ? *conv : RowsToF16{};
+    const dim3 grid(n_expert + 1 + (c.rows + nt / 256 - 1) / (nt / 256)), block(nt);
+#define INFR_BUCKET(...)                                                                                                             \
+    INFR_LAUNCH((__VA_ARGS__), grid, block, 0, s, ids, n_pairs, n_expert, n_used, offsets, pair_src, slot_pair, pair_row, tiles, tile, \
+                by_size, always_rows, c)
+    with_order(conv ? conv->weight_dt : INFR_F32, [&](auto order) {
+        typedef decltype(order) F;
+        if (n_pairs <= kBucketFew) INFR_BUCKET(bucket_once_kernel<F, 256, kBucketFew / 256>);
+        else if (n_pairs <= kBucketMany) INFR_BUCKET(bucket_once_kernel<F, 1024, kBucketMany / 1024>);
+        else INFR_BUCKET(bucket_kernel<F, 1024>);
+    });
 #undef INFR_BUCKET
 }
 

@@ -204,9 +204,14 @@ int gemm_tile_log2(int gate_dt, int down_dt, int rows, int n_pairs, int n_expert
 // rows of f32 -> f16 with a per-row power-of-two scale, in the k order weights of `weight_dt` unpack to.
 // Q4_K, Q5_K: also the sums of the f16 values over groups of 32, as f16 pairs high + low, sums[rows][n / 256][2][8] (n / 32 dwords a row).
 void launch_rows_to_f16(hipStream_t s, int weight_dt, const float* src, int rows, int n, void* dst, float* scale, uint32_t* sums);
-// route_kernel and the conversion of the same rows in one launch (rp.rows rows of n floats)
-void launch_route_rows_to_f16(hipStream_t s, const RouteParams& rp, int weight_dt, const float* src, int n, void* dst, float* scale,
-                              uint32_t* sums);
+// The same as a part of another launch: rows of n floats, as rows of weight_dt unpack.
+struct RowsToF16 {
+    const float* src = nullptr;
+    int rows = 0, n = 0, weight_dt = 0;
+    void* dst = nullptr;
+    float* scale = nullptr;
+    uint32_t* sums = nullptr;
+};
 // offsets / pair_src / slot_pair ([n_pairs], -1 for ids outside [0, n_expert)) from ids [n_pairs].
 // ids with the pairs of weight exactly 0 replaced by -1 (pairs an expert-parallel band dropped).
 void launch_mask_dropped_pairs(hipStream_t s, const int32_t* ids, const float* weights, int n_pairs, int32_t* out);
@@ -225,7 +230,7 @@ inline int gemm_max_tiles(int n_pairs, int n_expert, int tile) { return n_pairs 
 inline size_t gemm_table_slots(int n_pairs, int n_expert, int tile) { return 1 + (((size_t)gemm_max_tiles(n_pairs, n_expert, tile) + 7) & ~(size_t)7); }   // whole eights
 void launch_bucket(hipStream_t s, const int32_t* ids, int n_pairs, int n_expert, int n_used, int32_t* offsets, int32_t* pair_src,
                    int32_t* slot_pair, int32_t* pair_row = nullptr, int4* tiles = nullptr, int tile = 1, int by_size = 0,
-                   int always_rows = 0);
+                   int always_rows = 0, const RowsToF16* conv = nullptr);
 // launch_route and launch_bucket (tiles of kIntTok pairs, experts ascending) of a few rows in one launch; false, and nothing is
 // launched, where that does not take the shape.  Not for an expert-parallel band, whose dropped pairs have id 0.
 bool launch_route_bucket(hipStream_t s, const RouteParams& rp, int32_t* offsets, int32_t* pair_src, int32_t* slot_pair, int32_t* pair_row,
