@@ -425,6 +425,21 @@ __device__ __forceinline__ bool route_duo_second(const RouteParams& p, int row, 
     return true;
 }
 
+// The whole routing of a row by waves 0 and 1 of a block, whose other waves pass one __syncthreads() beside it.
+template <int NS>
+__device__ __forceinline__ void route_row_duo(const RouteParams& p, int row, int wave, int lane, float* lds, uint64_t* tab, RouteDuo* duo) {
+    bool done = false;
+    if (NS <= 8 && route_duo_ok(p)) {
+        float pr[NS];
+        route_duo_first<NS>(p, row, wave, lane, lds, tab, duo, pr);
+        __syncthreads();
+        done = wave != 0 || route_duo_second<NS>(p, row, lane, duo, pr, nullptr, nullptr, true);
+    } else {
+        __syncthreads();
+    }
+    if (wave == 0 && !done) route_row<NS>(p, row, lane, lds, tab, nullptr, nullptr, true, tab);
+}
+
 // ---------------------------------------------------------------------------------------------
 // Plain softmax routing of one token row by one wavefront when a CANDIDATE for the selected set is known (the
 // single-launch kernel has guessed it from estimates of the logits).  The probabilities are computed as always

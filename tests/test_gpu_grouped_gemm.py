@@ -468,7 +468,7 @@ def test_bucketing_of_many_pairs(be, rows, K):
 
 
 @pytest.mark.parametrize("rows,K,E", [
-    (33, 1, 3), (64, 8, 1000),                       # fewer pairs than threads; more experts than pairs
+    (33, 1, 3), (64, 8, 150),                        # fewer pairs than threads; fewer than three pairs per expert
     (2048, 1, 7), (683, 3, 61),                      # 2048 pairs on four wavefronts, 2049 on sixteen
     (2048, 8, 61), (3277, 5, 61),                    # 16384 held in registers, 16385 in chunks
 ])
@@ -494,6 +494,25 @@ def test_bucketing_at_the_edges_of_its_kernels(be, rows, K, E):
         g, ids = moe_graph(33, ne, E, K, nff, DType.Q8_0, DType.Q8_0, with_expert_ids=True)
         few, _, _ = _run_batched(be, g, ids, dict(data, x=np.ascontiguousarray(x[part]), expert_ids=np.ascontiguousarray(sel[part])), 33, ne)
         assert np.array_equal(bits(few), bits(out[part]))
+
+
+@pytest.mark.parametrize("rows,E,K", [(40, 32, 8), (40, 64, 4), (33, 128, 8), (40, 129, 15), (33, 256, 16), (40, 257, 15), (70, 512, 15), (90, 600, 12)])
+def test_routing_of_a_batch_by_itself(be, rows, E, K):
+    """The routing launch of a batch, for every number of experts it has code for: ids and weights of the reference, also in rows whose
+    logits are equal in pairs, all equal, or far apart, which the selection on two wavefronts leaves to the complete routine."""
+    ne, nff = 64, 64
+    rng = np.random.default_rng(rows + E + K)
+    x = rng.standard_normal((rows, ne)).astype(np.float32)
+    x[::5] = 0.0
+    x[1::5] *= 300.0
+    router = (rng.standard_normal((E, ne)) * 0.3).astype(np.float32)
+    router[E // 2:E // 2 + E // 4] = router[:E // 4]
+    gate, up, down = _bank_weights(rng, E, nff, ne, H.Q8_0, H.Q8_0)
+    g, ids = moe_graph(rows, ne, E, K, nff, DType.Q8_0, DType.Q8_0)
+    _, r, _ = _run_batched(be, g, ids, dict(x=x, router=router, gate=gate, up=up, down=down), rows, ne)
+    for i in range(rows):
+        probs, idx, w = O.route_row(r["logits"][i], K)
+        assert np.array_equal(r["idx"][i], idx) and np.array_equal(bits(r["w"][i]), bits(w)) and np.array_equal(bits(r["probs"][i]), bits(probs)), i
 
 
 @pytest.mark.parametrize("rows,E,K,units", [(16, 8, 2, False), (16, 64, 2, True), (16, 65, 2, True), (16, 9, 3, False), (17, 8, 1, False),
