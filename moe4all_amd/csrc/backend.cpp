@@ -1257,8 +1257,8 @@ extern "C" infr_status infr_hip_compile(infr_hip_backend* be, const infr_graph* 
         }
         // MoeFfn -> Add (the residual; the reference's moe_add rewrite, crates/infr-core/src/fusion.rs:20-24):
         // every combine kernel ends with "other operand + finished sum", the Add's own rounding.
-        // RmsNorm -> MoeFfn on one token row (fusion.rs:15-19 with moe_ok): the logits kernel normalises the
-        // raw row while staging it and stores the normalised row, which the expert kernels then read.
+        // RmsNorm -> MoeFfn on fewer than 32 token rows (fusion.rs:15-19 with moe_ok): the logits kernel normalises the
+        // raw rows while staging them and stores the normalised rows, which the expert kernels then read.
         for (uint32_t oi = 0; oi < g->n_ops; oi++) {
             if (plan->ops[oi].kind != INFR_OP_MOE_FFN) continue;
             const infr_hip_plan::Fuse kind = plan->fuse[oi].kind;
@@ -1282,8 +1282,8 @@ extern "C" infr_status infr_hip_compile(infr_hip_backend* be, const infr_graph* 
                 const infr_op_rms_norm& nr = plan->ops[oi - 1].u.rms_norm;
                 int re = 1, rb = 4;
                 geometry(c.dt(m.router), &re, &rb);
-                if (nr.rows == 1 && sc.rows == 1 && !sc.batched && !sc.bucketed && nr.dim == m.ne && nr.dst == m.router_x &&
-                    nr.x != nr.dst && infr::router_logits_can_norm(c.dt(m.router), (size_t)(m.ne / re) * rb, (int)m.ne, 1)) {
+                if ((int)nr.rows == sc.rows && !sc.batched && nr.dim == m.ne && nr.dst == m.router_x &&
+                    nr.x != nr.dst && infr::router_logits_can_norm(c.dt(m.router), (size_t)(m.ne / re) * rb, (int)m.ne, sc.rows)) {
                     plan->fuse[oi].norm = oi;   // 1 + (oi - 1)
                     plan->fuse[oi - 1].kind = infr_hip_plan::kSkip;
                 }
@@ -1731,7 +1731,7 @@ extern "C" infr_status infr_hip_execute(infr_hip_backend* be, infr_hip_plan* pla
                     }
                     if (!normed) {   // operands the fold cannot take (alignment): the op on its own
                         Timed t(be, "rms_norm");
-                        infr::launch_rms_norm(s, (const float*)ptr[nr.x], rn.weight, rn.xn_out, 1, (int)nr.dim, nr.eps, 0);
+                        infr::launch_rms_norm(s, (const float*)ptr[nr.x], rn.weight, rn.xn_out, rows, (int)nr.dim, nr.eps, 0);
                     }
                 }
                 if (!normed) {

@@ -64,13 +64,14 @@ void launch_route(hipStream_t s, const RouteParams& p) {
 // XQ: 128-bit loads of activations a thread holds in the one-burst staging (4: up to 1024 per block; 16: four rows of
 // 4096 elements, for small batches of a wide model, whose blocks would otherwise take one token row each and read the
 // router rows once per token row).
-template <int EPB, int XQ = 4>
+// RN > 0: an Op::RmsNorm folded into the staging of a block of RN token rows, XQ / RN loads of a row per thread.
+template <int EPB, int XQ = 4, int RN = 0>
 __global__ __launch_bounds__(256) void router_logits_kernel(const uint8_t* __restrict__ router, int rdt,
                                                             size_t row_bytes, const float* __restrict__ x, int ne,
                                                             int n_expert, int rows, int rpb,
                                                             float* __restrict__ logits, RouterNorm nrm) {
     extern __shared__ float lds[];
-    __shared__ float red[4];
+    __shared__ float red[4 * (RN ? RN : 1)];
     const int nc = ne >> 3;                 // full chunks of 8
     const int ntail = ne & 7;
     const int jstride = ((nc + 63) & ~63) + 4;
@@ -90,20 +91,29 @@ __global__ __launch_bounds__(256) void router_logits_kernel(const uint8_t* __res
     const int rbase = blockIdx.y * rpb;   // first token row of this block's (only) pass when one_shot
     const bool one_shot = rdt == INFR_F32 && (ne & 3) == 0 && (int)gridDim.y * rpb >= rows && EPB * nv <= 8 * 256 &&
                           rpb * nv <= XQ * 256;
-    if (one_shot) {
-        float4 wr[8], xr[XQ], nw[4];
+    if (RN || one_shot) {
+        float4 wr[8], xr[XQ];
+        // the thread's i-th load: vector v of token row rr of the block (folded norm: as the standalone kernel deals a row out)
+        constexpr int NQ = RN ? XQ / RN : 1;
+        auto at = [&](int i, int& rr, int& v) {
+            const int idx = tid + 256 * i;
+            rr = RN ? i / NQ : idx / nv;
+            v = RN ? tid + 256 * (i % NQ) : idx - rr * nv;
+            return v < nv && rr < rpb;
+        };
 #pragma unroll
         for (int i = 0; i < XQ; i++) {
-            const int idx = tid + 256 * i, rr = idx / nv, v = idx - rr * nv;
+            int rr, v;
             xr[i] = make_float4(0.f, 0.f, 0.f, 0.f);
-            if (rr < rpb && rbase + rr < rows) xr[i] = reinterpret_cast<const float4*>(x + (size_t)(rbase + rr) * ne)[v];
+            if (at(i, rr, v) && rbase + rr < rows) xr[i] = reinterpret_cast<const float4*>(x + (size_t)(rbase + rr) * ne)[v];
         }
-        if (nrm.weight) {
+        float4 nw[NQ];
+        if (RN) {
 #pragma unroll
-            for (int i = 0; i < 4; i++) {
-                const int idx = tid + 256 * i;
+            for (int i = 0; i < NQ; i++) {
+                const int v = tid + 256 * i;
                 nw[i] = make_float4(0.f, 0.f, 0.f, 0.f);
-                if (idx < nv) nw[i] = reinterpret_cast<const float4*>(nrm.weight)[idx];
+                if (v < nv) nw[i] = reinterpret_cast<const float4*>(nrm.weight)[v];
             }
         }
 #pragma unroll
@@ -113,30 +123,36 @@ __global__ __launch_bounds__(256) void router_logits_kernel(const uint8_t* __res
             if (e < EPB && e0 + e < n_expert)
                 wr[i] = reinterpret_cast<const float4*>(router + (size_t)(e0 + e) * row_bytes)[v];
         }
-        if (nrm.weight) {
-            // The single token row arrives raw: Op::RmsNorm is applied while it is staged, with the
-            // summation tree of the standalone kernel, and the first block stores the normalised row.
-            float part = 0.0f;
+        if (RN) {
+            // The token rows arrive raw: Op::RmsNorm is applied while they are staged, with the
+            // summation tree of the standalone kernel, and the first block of a row stores it normalised.
 #pragma unroll
-            for (int i = 0; i < 4; i++)
-                if (tid + 256 * i < nv) part = sumsq4(part, xr[i]);
+            for (int r = 0; r < RN; r++) {
+                float part = 0.0f;
+#pragma unroll
+                for (int i = 0; i < NQ; i++)
+                    if (tid + 256 * i < nv) part = sumsq4(part, xr[r * NQ + i]);
+                part = wave_sum(part);
+                if ((tid & 63) == 0) red[4 * r + (tid >> 6)] = part;
+            }
             LOGITS_STAMP(1);
-            const float sc = rms_scale(block256_sum(part, red), ne, nrm.eps);
+            __syncthreads();
             LOGITS_STAMP(2);
 #pragma unroll
-            for (int i = 0; i < 4; i++) {
-                const int idx = tid + 256 * i;
-                if (idx >= nv) continue;
-                xr[i] = rms_apply4(xr[i], sc, nw[i]);
-                if (blockIdx.x == 0 && blockIdx.y == 0) reinterpret_cast<float4*>(nrm.xn_out)[idx] = xr[i];
+            for (int i = 0; i < XQ; i++) {
+                int rr, v;
+                if (!at(i, rr, v)) continue;
+                const float* q = red + 4 * rr;
+                xr[i] = rms_apply4(xr[i], rms_scale((q[0] + q[1]) + (q[2] + q[3]), ne, nrm.eps), nw[i % NQ]);
+                if (blockIdx.x == 0 && rbase + rr < rows) reinterpret_cast<float4*>(nrm.xn_out + (size_t)(rbase + rr) * ne)[v] = xr[i];
             }
         }
         // element 4v + t of a row: chain (4v + t) & 7 = 4 (v & 1) + t, step (4v + t) >> 3 = v >> 1: the four
         // elements of a 128-bit load go to four chains at one step, or all four to the tail
 #pragma unroll
         for (int i = 0; i < XQ; i++) {
-            const int idx = tid + 256 * i, rr = idx / nv, v = idx - rr * nv;
-            if (rr >= rpb) continue;
+            int rr, v;
+            if (!at(i, rr, v)) continue;
             if ((v >> 1) < nc) {
                 float* d = xs + rr * estride + 4 * (v & 1) * jstride + (v >> 1);
                 d[0] = xr[i].x; d[jstride] = xr[i].y; d[2 * jstride] = xr[i].z; d[3 * jstride] = xr[i].w;
@@ -472,9 +488,13 @@ bool router_logits_fits(int rdt, size_t row_bytes, int ne, int rows) {
     return router_logits_tile(rdt, ne, rows, &epb, &rpb);
 }
 
-// The fold needs the one-burst staging of a single row (rows = 1 gives 2 experts x 1 row per block).
+// The fold needs the one-burst staging: decode and small batches.  Each of a row's n_expert / 2 blocks normalises it again, which
+// costs less than a launch: us a pass with norm and residual, the norm by itself and folded: six layers of 3 rows of 128 experts of
+// 2048 x 768 in Q4_K / Q6_K 213.7 and 196.3, two of 20 rows in IQ4_XS 203.7 and 193.3, of 6 rows of 2880 x 2880, top-4, in MXFP4 225.6 and
+// 206.5, of 8 rows of 256 experts of 4096 x 1536 361.4 and 356.1.  (Several rows of less than 2048 elements keep the launch:
+// which launches such a layer makes is pinned by tests.)
 bool router_logits_can_norm(int rdt, size_t row_bytes, int ne, int rows) {
-    return rows == 1 && rdt == INFR_F32 && (ne & 3) == 0 && ne >= 4 && ne <= 4096 && (row_bytes & 15) == 0;
+    return rows >= 1 && (rows == 1 || (rows < 32 && ne >= 2048)) && rdt == INFR_F32 && (ne & 3) == 0 && ne >= 4 && ne <= 4096 && (row_bytes & 15) == 0;
 }
 
 bool launch_router_logits(hipStream_t s, const uint8_t* router, int rdt, size_t row_bytes, const float* x, int ne,
@@ -524,6 +544,22 @@ bool launch_router_logits(hipStream_t s, const uint8_t* router, int rdt, size_t 
         INFR_LAUNCH(router_logits_kernel<E>, grid, block, lds, s, router, rdt, row_bytes, x, ne, n_expert,  \
                            rows, rpb, logits, nrm);                                                   \
     } while (0)
+    if (nrm.weight) {
+#define LAUNCH_RN(E, Q, R)                                                                                         \
+    do {                                                                                                           \
+        INFR_LDS_LIMIT((router_logits_kernel<E, Q, R>), (int)budget);                                              \
+        INFR_LAUNCH((router_logits_kernel<E, Q, R>), grid, block, lds, s, router, rdt, row_bytes, x, ne, n_expert, rows, rpb, logits, nrm); \
+    } while (0)
+        if (epb > 2 || rpb > 4 || gy != passes) return false;
+        if (rpb == 1 && epb == 1) LAUNCH_RN(1, 4, 1);
+        else if (epb == 1) return false;
+        else if (rpb == 1) LAUNCH_RN(2, 4, 1);
+        else if (rpb == 2 && ne <= 2048) LAUNCH_RN(2, 4, 2);
+        else if (rpb == 2) LAUNCH_RN(2, 8, 2);
+        else LAUNCH_RN(2, 16, 4);
+#undef LAUNCH_RN
+        return true;
+    }
     if (small && rpb * (ne >> 2) > 4 * 256 && epb <= 2) {   // the wide one-burst staging
         INFR_LDS_LIMIT((router_logits_kernel<2, 16>), (int)budget);
         if (epb == 2) INFR_LAUNCH((router_logits_kernel<2, 16>), grid, block, lds, s, router, rdt, row_bytes, x, ne, n_expert, rows, rpb, logits, nrm);

@@ -43,12 +43,12 @@ inline void lds_limit(const void* kernel, int bytes, std::atomic<uint32_t>& done
         ::infr::lds_limit((const void*)kernel, (bytes), lds_limit_done_);   \
     } while (0)
 
-// An Op::RmsNorm of the single token row folded into the logits kernel: x is the raw row, every
-// block normalises it while staging and the first block also stores the normalised row to xn_out.
+// An Op::RmsNorm of up to 31 token rows folded into the logits kernel: x are the raw rows, every
+// block normalises its rows while staging and the first block of a row also stores it normalised to xn_out.
 struct RouterNorm {
     const float* weight = nullptr;   // [ne]
     float eps = 0.0f;
-    float* xn_out = nullptr;         // [ne], not x
+    float* xn_out = nullptr;         // [rows, ne], not x
 };
 bool router_logits_can_norm(int rdt, size_t row_bytes, int ne, int rows);
 // False when launch_router_logits would refuse the shape (its staging does not fit the LDS): asked at compile time.
@@ -220,6 +220,7 @@ void launch_mask_dropped_pairs(hipStream_t s, const int32_t* ids, const float* w
 // experts ascending; by_size: per tile {expert, first pair, pairs of the tile, 0}, experts of more than 256 pairs first, then those of
 // up to 256, 128, 64, 32 and 16, ascending in each class; with always_rows also the tiles of an expert n_expert that has as many
 // pairs n_pairs .., one per token row.
+// conv (or null): token rows that the same launch converts to f16.
 constexpr int kIntTok = 8;   // pairs of a tile of the integer kernels
 // Tiles of a Linear's rows: 64.  us per Linear, of 64 | of 128: 128 rows of 4096 x 4096 in Q5_K 40 | 56, 512 rows of 2048 x 2048 in Q8_0 26 | 32, 1500
 // rows of 4096 x 1536 in Q4_K 52 | 58 and of 2048 x 4096 in MXFP4 40 | 43, 2048 rows of 2048 x 2048 in Q8_0 38 | 36, 2048 rows of 4096 x 4096 in

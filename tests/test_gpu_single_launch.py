@@ -698,3 +698,57 @@ def test_four_experts_per_token_with_norm_and_residual(be):
             if plain:
                 b.close()
     assert np.array_equal(bits(outs[0]), bits(outs[1])) and np.abs(outs[0] - x.reshape(-1)).max() > 1e-4
+
+
+FOLDED = "rms_norm_router_logits"
+
+
+@pytest.mark.parametrize("rows,ne,E,K,nff,gdt,ddt,name", [
+    # two rows to a workgroup of the logits (whole and ragged shares of 256 loads), four; rows behind the last whole workgroup
+    (2, 2048, 8, 2, 256, H.Q4K, H.Q6K, FOLDED), (31, 2048, 32, 2, 256, H.Q8_0, H.Q8_0, FOLDED), (3, 2080, 7, 2, 64, H.Q8_0, H.Q8_0, FOLDED),
+    (5, 2880, 9, 3, 64, H.Q8_0, H.Q8_0, FOLDED), (2, 4096, 8, 2, 256, H.Q4K, H.Q6K, FOLDED), (7, 4096, 8, 2, 256, H.Q4K, H.Q6K, FOLDED),
+])
+def test_rms_norm_of_a_few_rows_folded_in(rows, ne, E, K, nff, gdt, ddt, name):
+    """RmsNorm -> MoeFfn -> Add on 2 to 31 token rows: the normalised rows, the routing and the output have the bits of one launch per op."""
+    rng = np.random.default_rng(rows + ne + E)
+    x = (rng.standard_normal((rows, ne)) * 2).astype(np.float32)
+    x[rows - 1] *= 1e-3
+    nw = (1 + 0.1 * rng.standard_normal(ne)).astype(np.float32)
+    router = (rng.standard_normal((E, ne)) * 0.02).astype(np.float32)
+    gate, up, down = _banks(rng, E, nff, ne, gdt, ddt)
+    outs, norms, routes, names = {}, {}, {}, {}
+    for off in (False, True):
+        b = M.Backend(0, disable_op_fusion=off)
+        try:
+            g, T = M.Graph(), M.TensorDesc
+            xi, nwt, rt = g.input(T([rows, ne], DType.F32)), g.weight(T([ne], DType.F32)), g.weight(T([E, ne], DType.F32))
+            gt, ut = g.weight(T([E, nff, ne], DType(gdt))), g.weight(T([E, nff, ne], DType(gdt)))
+            dt = g.weight(T([E, ne, nff], DType(ddt)))
+            xn, moe, yi = g.output(T([rows, ne], DType.F32)), g.internal(T([rows, ne], DType.F32)), g.output(T([rows, ne], DType.F32))
+            g.rms_norm(x=xi, weight=nwt, dst=xn, rows=rows, dim=ne, eps=1e-6)
+            g.moe_ffn(x=xn, router=rt, gate_exps=gt, up_exps=ut, down_exps=dt, dst=moe, ne=ne, n_expert=E, n_used=K, n_ff_exp=nff)
+            g.add(a=xi, b=moe, dst=yi, n=rows * ne)
+            plan, bind, bufs = b.compile(g), M.Bindings(), []
+            for tid, v in [(xi, x), (nwt, nw), (rt, router), (gt, gate), (ut, up), (dt, down)]:
+                bufs.append(b.buffer_from(v))
+                bind.bind(tid, bufs[-1])
+            o_xn, o_y = b.alloc(rows * ne * 4), b.alloc(rows * ne * 4)
+            bind.bind(xn, o_xn)
+            bind.bind(yi, o_y)
+            b.prof_enable(True)
+            for _ in range(2):
+                b.execute(plan, bind)
+            outs[off] = b.download(o_y, rows * ne * 4, np.float32).copy()
+            norms[off] = b.download(o_xn, rows * ne * 4, np.float32).copy()
+            routes[off] = b.moe_routing(plan, 1)
+            names[off] = set(b.prof_read())
+            for buf in bufs + [o_xn, o_y]:
+                buf.free()
+            plan.free()
+        finally:
+            b.close()
+    assert name in names[False] and "rms_norm" not in names[False] and "rms_norm" in names[True]
+    assert np.array_equal(bits(norms[False]), bits(norms[True]))
+    assert np.array_equal(routes[False]["idx"], routes[True]["idx"]) and np.array_equal(bits(routes[False]["logits"]), bits(routes[True]["logits"]))
+    assert np.array_equal(bits(outs[False]), bits(outs[True]))
+    assert H.rel_l2(norms[False].reshape(rows, ne), O.rms_norm(x, nw, 1e-6).reshape(rows, ne)) < 1e-5
