@@ -173,7 +173,7 @@ struct MoeScratch {
     float* hs = nullptr;          // [rows * n_used]
     uint32_t* hm = nullptr;       // [rows * n_used, nff / 32] group sums of hh
     float* y = nullptr;           // [rows * n_used, ne]
-    int single_launch = 0;        // one token row as one launch: 1 = stages in order (k_layer.hip), 2 = guessed selection (k_layer_stream.hip)
+    int single_launch = 0;        // one, two, four or eight token rows as one launch: 1 = stages in order (k_layer.hip), 2 = guessed selection (k_layer_stream.hip)
 };
 
 struct infr_hip_plan {
@@ -1283,7 +1283,7 @@ extern "C" infr_status infr_hip_compile(infr_hip_backend* be, const infr_graph* 
                 int re = 1, rb = 4;
                 geometry(c.dt(m.router), &re, &rb);
                 if ((int)nr.rows == sc.rows && !sc.batched && nr.dim == m.ne && nr.dst == m.router_x &&
-                    nr.x != nr.dst && infr::router_logits_can_norm(c.dt(m.router), (size_t)(m.ne / re) * rb, (int)m.ne, sc.rows)) {
+                    nr.x != nr.dst && infr::router_logits_can_norm(c.dt(m.router), (size_t)(m.ne / re) * rb, (int)m.ne, (int)m.n_expert, sc.rows)) {
                     plan->fuse[oi].norm = oi;   // 1 + (oi - 1)
                     plan->fuse[oi - 1].kind = infr_hip_plan::kSkip;
                 }
@@ -1353,7 +1353,7 @@ extern "C" infr_status infr_hip_compile(infr_hip_backend* be, const infr_graph* 
             if (plan->fuse[oi].norm && sc.single_launch == 2 && !plan->fuse[oi].gated) {
                 const infr_op_rms_norm& nr = plan->ops[plan->fuse[oi].norm - 1].u.rms_norm;
                 probe.norm_w = (const float*)plan;   // non-null: asked for
-                keep_norm = sc.rows == 1 && m.x == nr.dst && infr::moe_layer_stream_supported(probe);
+                keep_norm = m.x == nr.dst && infr::moe_layer_stream_supported(probe);
             }
             if (plan->fuse[oi].norm && !keep_norm) {
                 plan->fuse[plan->fuse[oi].norm - 1].kind = infr_hip_plan::kPlain;
@@ -1683,7 +1683,7 @@ extern "C" infr_status infr_hip_execute(infr_hip_backend* be, infr_hip_plan* pla
                         lp.logits_once = moe_logits_once(be, m, rows);
                         lp.guess_skew = (int)std::min<uint32_t>(be->cfg.single_launch_guess_skew, 8u);
                         bool norm_ok = true;
-                        if (fz.norm) {   // the token row's RmsNorm, folded: the kernel normalises the raw row
+                        if (fz.norm) {   // the token rows' RmsNorm, folded: the kernel normalises the raw rows
                             const infr_op_rms_norm& nr = plan->ops[fz.norm - 1].u.rms_norm;
                             if (!(need(nr.x, "RmsNorm.x") && need(nr.weight, "RmsNorm.weight") && need(nr.dst, "RmsNorm.dst")))
                                 return INFR_ERR_BACKEND;
@@ -1692,7 +1692,7 @@ extern "C" infr_status infr_hip_execute(infr_hip_backend* be, infr_hip_plan* pla
                             lp.norm_out = (float*)ptr[nr.dst];
                             lp.norm_eps = nr.eps;
                             lp.norm_for_x = m.x == nr.dst ? 1 : 0;
-                            norm_ok = nr.x != nr.dst && m.x == nr.dst && rows == 1 && (((uintptr_t)lp.norm_x | (uintptr_t)lp.norm_w | (uintptr_t)lp.norm_out) & 15) == 0;
+                            norm_ok = lp.norm_x != lp.norm_out && m.x == nr.dst && (((uintptr_t)lp.norm_x | (uintptr_t)lp.norm_w | (uintptr_t)lp.norm_out) & 15) == 0;
                         }
                         if (norm_ok && infr::moe_layer_stream_supported(lp) &&
                             (((uintptr_t)lp.router | (uintptr_t)lp.router_x | (uintptr_t)gp.x) & 15) == 0 && (lp.router_row_floats & 3) == 0) {

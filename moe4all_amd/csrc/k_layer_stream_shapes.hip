@@ -25,29 +25,25 @@ bool launch_stream_fixed(hipStream_t s, const MoeLayerParams& q, const StreamSha
         norm == NORMv)                                                                                                       \
         return launch ? launch_stream<FGt, FDt, DGv, DDv, EPTv, NSPv, NEv, NFFv, ROWSv, NORMv>(s, q, sh.lds) : true;
 #define INFR_STREAM_AT(FGt, FDt, DGv, DDv, EPTv, NSPv, NEv, NFFv, ROWSv) \
-    INFR_STREAM_AT_N(FGt, FDt, DGv, DDv, EPTv, NSPv, NEv, NFFv, ROWSv, 0)
+    INFR_STREAM_AT_N(FGt, FDt, DGv, DDv, EPTv, NSPv, NEv, NFFv, ROWSv, 0)   \
+    INFR_STREAM_AT_N(FGt, FDt, DGv, DDv, EPTv, NSPv, NEv, NFFv, ROWSv, 1)   // the token rows' RmsNorm folded in
     if (p.gate_dt == INFR_Q4K && p.down_dt == INFR_Q6K) {
         INFR_STREAM_AT(Q4KFmt, Q6KFmt, 2, 2, 1, 2, 2048, 768, 1)    // 128 experts, one token row
-        INFR_STREAM_AT_N(Q4KFmt, Q6KFmt, 2, 2, 1, 2, 2048, 768, 1, 1)   // ... with the token row's RmsNorm folded in
         INFR_STREAM_AT(Q4KFmt, Q6KFmt, 2, 4, 1, 2, 2048, 768, 2)
         INFR_STREAM_AT(Q4KFmt, Q6KFmt, 2, 4, 1, 2, 2048, 768, 4)
         INFR_STREAM_AT(Q4KFmt, Q6KFmt, 2, 4, 2, 2, 2048, 768, 8)
         INFR_STREAM_AT(Q4KFmt, Q6KFmt, 2, 4, 1, 4, 4096, 1536, 1)   // 256 experts, with or without the always-on expert
-        INFR_STREAM_AT_N(Q4KFmt, Q6KFmt, 2, 4, 1, 4, 4096, 1536, 1, 1)
         INFR_STREAM_AT(Q4KFmt, Q6KFmt, 2, 4, 2, 4, 4096, 1536, 2)
         INFR_STREAM_AT(Q4KFmt, Q6KFmt, 2, 4, 4, 4, 4096, 1536, 4)
         INFR_STREAM_AT(Q4KFmt, Q6KFmt, 2, 2, 1, 0, 1024, 512, 1)    // 32 experts (the only instantiations of this width)
-        INFR_STREAM_AT_N(Q4KFmt, Q6KFmt, 2, 2, 1, 0, 1024, 512, 1, 1)
         INFR_STREAM_AT(Q4KFmt, Q6KFmt, 2, 2, 1, 0, 1024, 512, 2)
         INFR_STREAM_AT(Q4KFmt, Q6KFmt, 2, 2, 1, 0, 1024, 512, 4)
         INFR_STREAM_AT(Q4KFmt, Q6KFmt, 2, 4, 1, 0, 1024, 512, 8)
     } else if (p.gate_dt == INFR_Q8_0 && p.down_dt == INFR_Q8_0) {
         INFR_STREAM_AT(Q80Fmt, Q80Fmt, 4, 5, 1, 2, 2048, 768, 1)
-        INFR_STREAM_AT_N(Q80Fmt, Q80Fmt, 4, 5, 1, 2, 2048, 768, 1, 1)
         INFR_STREAM_AT(Q80Fmt, Q80Fmt, 2, 4, 1, 2, 2048, 768, 2)
         INFR_STREAM_AT(Q80Fmt, Q80Fmt, 2, 4, 1, 2, 2048, 768, 4)
         INFR_STREAM_AT(Q80Fmt, Q80Fmt, 2, 2, 1, 0, 1024, 512, 1)    // 32 experts
-        INFR_STREAM_AT_N(Q80Fmt, Q80Fmt, 2, 2, 1, 0, 1024, 512, 1, 1)
         INFR_STREAM_AT(Q80Fmt, Q80Fmt, 4, 2, 1, 0, 1024, 512, 2)
         INFR_STREAM_AT(Q80Fmt, Q80Fmt, 2, 5, 1, 0, 1024, 512, 4)
     }

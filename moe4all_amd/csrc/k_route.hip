@@ -491,16 +491,17 @@ bool router_logits_fits(int rdt, size_t row_bytes, int ne, int rows) {
 // The fold needs the one-burst staging: decode and small batches.  Each of a row's n_expert / 2 blocks normalises it again, which
 // costs less than a launch: us a pass with norm and residual, the norm by itself and folded: six layers of 3 rows of 128 experts of
 // 2048 x 768 in Q4_K / Q6_K 213.7 and 196.3, two of 20 rows in IQ4_XS 203.7 and 193.3, of 6 rows of 2880 x 2880, top-4, in MXFP4 225.6 and
-// 206.5, of 8 rows of 256 experts of 4096 x 1536 361.4 and 356.1.  (Several rows of less than 2048 elements keep the launch:
-// which launches such a layer makes is pinned by tests.)
-bool router_logits_can_norm(int rdt, size_t row_bytes, int ne, int rows) {
-    return rows >= 1 && (rows == 1 || (rows < 32 && ne >= 2048)) && rdt == INFR_F32 && (ne & 3) == 0 && ne >= 4 && ne <= 4096 && (row_bytes & 15) == 0;
+// 206.5, of 8 rows of 256 experts of 4096 x 1536 361.4 and 356.1.  Ten layers of 5 rows of 32 experts of 1024 x 512 in Q4_0 286.1
+// and 259.2.  (Several rows of less than 2048 elements and less than 32 experts keep the launch: which launches such a layer makes is
+// pinned by tests.)
+bool router_logits_can_norm(int rdt, size_t row_bytes, int ne, int n_expert, int rows) {
+    return rows >= 1 && (rows == 1 || (rows < 32 && (ne >= 2048 || n_expert >= 32))) && rdt == INFR_F32 && (ne & 3) == 0 && ne >= 4 && ne <= 4096 && (row_bytes & 15) == 0;
 }
 
 bool launch_router_logits(hipStream_t s, const uint8_t* router, int rdt, size_t row_bytes, const float* x, int ne,
                           int n_expert, int rows, float* logits, const RouterNorm* norm) {
     const RouterNorm nrm = norm ? *norm : RouterNorm{};
-    if (nrm.weight && (!router_logits_can_norm(rdt, row_bytes, ne, rows) || !nrm.xn_out || nrm.xn_out == x ||
+    if (nrm.weight && (!router_logits_can_norm(rdt, row_bytes, ne, n_expert, rows) || !nrm.xn_out || nrm.xn_out == x ||
                        (((uintptr_t)x | (uintptr_t)nrm.weight | (uintptr_t)nrm.xn_out) & 15) != 0))
         return false;
     if (rows >= 32 && rdt == INFR_F32 && (ne & 31) == 0 && (row_bytes & 15) == 0) {

@@ -50,7 +50,7 @@ struct RouterNorm {
     float eps = 0.0f;
     float* xn_out = nullptr;         // [rows, ne], not x
 };
-bool router_logits_can_norm(int rdt, size_t row_bytes, int ne, int rows);
+bool router_logits_can_norm(int rdt, size_t row_bytes, int ne, int n_expert, int rows);
 // False when launch_router_logits would refuse the shape (its staging does not fit the LDS): asked at compile time.
 bool router_logits_fits(int rdt, size_t row_bytes, int ne, int rows);
 // Router logits with the reference's dot order (8 FMA lanes, lanes summed 0..7).
@@ -149,7 +149,7 @@ struct MoeLayerParams {
     int logits_once;            // every logit computed by one workgroup for the whole grid, not once per group
     int guess_skew;             // tests: the guess leaves out this many of the largest estimates
     int epb, early_down;        // set by the launcher
-    // an Op::RmsNorm of the single token row folded in (null norm_w: none): router_x is then ignored, the routing row is
+    // an Op::RmsNorm of the token rows folded in (null norm_w: none): router_x is then ignored, the routing row is
     // rmsnorm(norm_x) * norm_w, stored to norm_out by one workgroup; norm_for_x: g.x is that row too (and is not read)
     const float* norm_x = nullptr;
     const float* norm_w = nullptr;

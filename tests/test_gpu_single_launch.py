@@ -706,7 +706,11 @@ FOLDED = "rms_norm_router_logits"
 @pytest.mark.parametrize("rows,ne,E,K,nff,gdt,ddt,name", [
     # two rows to a workgroup of the logits (whole and ragged shares of 256 loads), four; rows behind the last whole workgroup
     (2, 2048, 8, 2, 256, H.Q4K, H.Q6K, FOLDED), (31, 2048, 32, 2, 256, H.Q8_0, H.Q8_0, FOLDED), (3, 2080, 7, 2, 64, H.Q8_0, H.Q8_0, FOLDED),
-    (5, 2880, 9, 3, 64, H.Q8_0, H.Q8_0, FOLDED), (2, 4096, 8, 2, 256, H.Q4K, H.Q6K, FOLDED), (7, 4096, 8, 2, 256, H.Q4K, H.Q6K, FOLDED),
+    (6, 1024, 32, 8, 512, H.Q8_0, H.Q8_0, FOLDED), (5, 2880, 9, 3, 64, H.Q8_0, H.Q8_0, FOLDED), (2, 4096, 8, 2, 256, H.Q4K, H.Q6K, FOLDED), (7, 4096, 8, 2, 256, H.Q4K, H.Q6K, FOLDED),
+    # the whole sublayer in one launch
+    (2, 2048, 128, 8, 768, H.Q4K, H.Q6K, "moe_layer"), (4, 2048, 128, 8, 768, H.Q8_0, H.Q8_0, "moe_layer"),
+    (8, 2048, 128, 8, 768, H.Q4K, H.Q6K, "moe_layer"), (2, 1024, 32, 8, 512, H.Q8_0, H.Q8_0, "moe_layer"),
+    (8, 1024, 32, 8, 512, H.Q4K, H.Q6K, "moe_layer"),
 ])
 def test_rms_norm_of_a_few_rows_folded_in(rows, ne, E, K, nff, gdt, ddt, name):
     """RmsNorm -> MoeFfn -> Add on 2 to 31 token rows: the normalised rows, the routing and the output have the bits of one launch per op."""
