@@ -524,8 +524,12 @@ bool launch_router_logits(hipStream_t s, const uint8_t* router, int rdt, size_t 
     }
     int epb = 0, rpb = 0;
     if (!router_logits_tile(rdt, ne, rows, &epb, &rpb)) return false;
-    // one token row and no more experts than compute units: a block per expert halves what a block stages
-    if (rows == 1 && epb == 2 && n_expert <= 256) epb = 1;
+    // where blocks of fewer token rows, or of one expert, still have a compute unit each, they stage less.  us a pass,
+    // larger and smaller blocks: 5 rows of 8 experts of hidden size 4096 189.3 and 185.7, two layers of 6 rows of 128 experts of 2880 206.1
+    // and 202.8, six of 3 rows of 2048 195.5 and 193.0, ten of 5 rows of 32 experts of 1024 259.1 and 256.6.  (More blocks than compute
+    // units only read the router more often: 8 rows of 256 experts stay with four rows to a block.)
+    while (epb == 2 && rpb > 1 && (n_expert + 1) / 2 * ((rows + rpb / 2 - 1) / (rpb / 2)) <= 256) rpb /= 2;
+    if (epb == 2 && rpb == 1 && n_expert * rows <= 256) epb = 1;
     const bool small = rows <= 2 || (rows < 32 && rdt == INFR_F32 && (ne & 3) == 0 && ne <= 4096);
     const size_t budget = kRouterLdsBudget;
     const int nc = ne >> 3;
