@@ -399,8 +399,13 @@ __device__ __forceinline__ float block256_sum(float v, float* red) {
     return (red[0] + red[1]) + (red[2] + red[3]);
 }
 // Op::RmsNorm's row scale 1 / sqrt(sum(x^2) / dim + eps) (crates/infr-cpu/src/lib.rs:1062-1063).
+// The hardware's square root, written out: __fsqrt_rn may become it or a correctly rounded sequence from one kernel to the next, and a
+// row has to have the same bits in all of them.
 __device__ __forceinline__ float rms_scale(float sumsq, int dim, float eps) {
-    return __fdiv_rn(1.0f, __fsqrt_rn(__fadd_rn(__fdiv_rn(sumsq, (float)dim), eps)));
+    const float v = __fadd_rn(__fdiv_rn(sumsq, (float)dim), eps);
+    const bool tiny = v < 0x1p-126f;   // the instruction takes no subnormals
+    const float r = __builtin_amdgcn_sqrtf(tiny ? __fmul_rn(v, 0x1p32f) : v);
+    return __fdiv_rn(1.0f, tiny ? __fmul_rn(r, 0x1p-16f) : r);
 }
 // A thread's share of a row's sum of squares when thread t of 256 owns the float4s t, t + 256, ...
 __device__ __forceinline__ float sumsq4(float acc, const float4& f) {
