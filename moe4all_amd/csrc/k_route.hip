@@ -91,7 +91,7 @@ __global__ __launch_bounds__(256) void router_logits_kernel(const uint8_t* __res
     const int rbase = blockIdx.y * rpb;   // first token row of this block's (only) pass when one_shot
     const bool one_shot = rdt == INFR_F32 && (ne & 3) == 0 && (int)gridDim.y * rpb >= rows && EPB * nv <= 8 * 256 &&
                           rpb * nv <= XQ * 256;
-    if (RN || one_shot) {
+    if constexpr (RN > 0) {
         float4 wr[8], xr[XQ];
         // the thread's i-th load: vector v of token row rr of the block (folded norm: as the standalone kernel deals a row out)
         constexpr int NQ = RN ? XQ / RN : 1;
@@ -153,6 +153,73 @@ __global__ __launch_bounds__(256) void router_logits_kernel(const uint8_t* __res
         for (int i = 0; i < XQ; i++) {
             int rr, v;
             if (!at(i, rr, v)) continue;
+            if ((v >> 1) < nc) {
+                float* d = xs + rr * estride + 4 * (v & 1) * jstride + (v >> 1);
+                d[0] = xr[i].x; d[jstride] = xr[i].y; d[2 * jstride] = xr[i].z; d[3 * jstride] = xr[i].w;
+            } else {
+                float* d = xt + rr * 8;
+                d[0] = xr[i].x; d[1] = xr[i].y; d[2] = xr[i].z; d[3] = xr[i].w;
+            }
+        }
+#pragma unroll
+        for (int i = 0; i < 8; i++) {
+            const int idx = tid + 256 * i, e = idx / nv, v = idx - e * nv;
+            if (e >= EPB) continue;
+            if ((v >> 1) < nc) {
+                float* d = w + e * estride + 4 * (v & 1) * jstride + (v >> 1);
+                d[0] = wr[i].x; d[jstride] = wr[i].y; d[2 * jstride] = wr[i].z; d[3 * jstride] = wr[i].w;
+            } else {
+                float* d = wt + e * 8;
+                d[0] = wr[i].x; d[1] = wr[i].y; d[2] = wr[i].z; d[3] = wr[i].w;
+            }
+        }
+    } else if (one_shot) {   // (a form of its own: without the run-time fold between them the compiler sinks the loads to their stores, 0.5 us)
+        float4 wr[8], xr[XQ], nw[4];
+#pragma unroll
+        for (int i = 0; i < XQ; i++) {
+            const int idx = tid + 256 * i, rr = idx / nv, v = idx - rr * nv;
+            xr[i] = make_float4(0.f, 0.f, 0.f, 0.f);
+            if (rr < rpb && rbase + rr < rows) xr[i] = reinterpret_cast<const float4*>(x + (size_t)(rbase + rr) * ne)[v];
+        }
+        if (nrm.weight) {
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                const int idx = tid + 256 * i;
+                nw[i] = make_float4(0.f, 0.f, 0.f, 0.f);
+                if (idx < nv) nw[i] = reinterpret_cast<const float4*>(nrm.weight)[idx];
+            }
+        }
+#pragma unroll
+        for (int i = 0; i < 8; i++) {
+            const int idx = tid + 256 * i, e = idx / nv, v = idx - e * nv;
+            wr[i] = make_float4(0.f, 0.f, 0.f, 0.f);
+            if (e < EPB && e0 + e < n_expert)
+                wr[i] = reinterpret_cast<const float4*>(router + (size_t)(e0 + e) * row_bytes)[v];
+        }
+        if (nrm.weight) {
+            // The single token row arrives raw: Op::RmsNorm is applied while it is staged, with the
+            // summation tree of the standalone kernel, and the first block stores the normalised row.
+            float part = 0.0f;
+#pragma unroll
+            for (int i = 0; i < 4; i++)
+                if (tid + 256 * i < nv) part = sumsq4(part, xr[i]);
+            LOGITS_STAMP(1);
+            const float sc = rms_scale(block256_sum(part, red), ne, nrm.eps);
+            LOGITS_STAMP(2);
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                const int idx = tid + 256 * i;
+                if (idx >= nv) continue;
+                xr[i] = rms_apply4(xr[i], sc, nw[i]);
+                if (blockIdx.x == 0 && blockIdx.y == 0) reinterpret_cast<float4*>(nrm.xn_out)[idx] = xr[i];
+            }
+        }
+        // element 4v + t of a row: chain (4v + t) & 7 = 4 (v & 1) + t, step (4v + t) >> 3 = v >> 1: the four
+        // elements of a 128-bit load go to four chains at one step, or all four to the tail
+#pragma unroll
+        for (int i = 0; i < XQ; i++) {
+            const int idx = tid + 256 * i, rr = idx / nv, v = idx - rr * nv;
+            if (rr >= rpb) continue;
             if ((v >> 1) < nc) {
                 float* d = xs + rr * estride + 4 * (v & 1) * jstride + (v >> 1);
                 d[0] = xr[i].x; d[jstride] = xr[i].y; d[2 * jstride] = xr[i].z; d[3 * jstride] = xr[i].w;
