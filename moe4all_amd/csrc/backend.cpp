@@ -1651,6 +1651,24 @@ extern "C" infr_status infr_hip_execute(infr_hip_backend* be, infr_hip_plan* pla
                                         plan->tensors[lq.weight].dtype, rb, (int)lq.m, (int)lq.in_f, (int)lq.out_f,
                                         (float*)ptr[lq.dst], n_cu);
                 };
+                // An RmsNorm folded into the op.  Where the operands are none that a fold can take, it is a launch of its own ahead of
+                // whatever runs the op, and norm_x is null from there on.
+                infr::RouterNorm rn;
+                const float* norm_x = nullptr;
+                auto launch_norm = [&]() {
+                    Timed t(be, "rms_norm");
+                    infr::launch_rms_norm(s, norm_x, rn.weight, rn.xn_out, rows, (int)m.ne, rn.eps, 0);
+                    norm_x = nullptr;
+                };
+                if (fz.norm) {
+                    const infr_op_rms_norm& nr = plan->ops[fz.norm - 1].u.rms_norm;
+                    if (!(need(nr.x, "RmsNorm.x") && need(nr.weight, "RmsNorm.weight") && need(nr.dst, "RmsNorm.dst")))
+                        return INFR_ERR_BACKEND;
+                    norm_x = (const float*)ptr[nr.x];
+                    rn.weight = (const float*)ptr[nr.weight]; rn.eps = nr.eps; rn.xn_out = (float*)ptr[nr.dst];
+                    // (in place, every workgroup but the first would read rows that the first has normalised already)
+                    if (norm_x == rn.xn_out || (((uintptr_t)norm_x | (uintptr_t)rn.weight | (uintptr_t)rn.xn_out) & 15) != 0) launch_norm();
+                }
                 bool single = sc.single_launch != 0;
                 if (single && sc.single_launch == 1 && be->inorder_off.load(std::memory_order_relaxed)) single = false;
                 if (single) {
@@ -1682,19 +1700,17 @@ extern "C" infr_status infr_hip_execute(infr_hip_backend* be, infr_hip_plan* pla
                         lp.late = be->fault_dev + 1;
                         lp.logits_once = moe_logits_once(be, m, rows);
                         lp.guess_skew = (int)std::min<uint32_t>(be->cfg.single_launch_guess_skew, 8u);
-                        bool norm_ok = true;
-                        if (fz.norm) {   // the token rows' RmsNorm, folded: the kernel normalises the raw rows
-                            const infr_op_rms_norm& nr = plan->ops[fz.norm - 1].u.rms_norm;
-                            if (!(need(nr.x, "RmsNorm.x") && need(nr.weight, "RmsNorm.weight") && need(nr.dst, "RmsNorm.dst")))
-                                return INFR_ERR_BACKEND;
-                            lp.norm_x = (const float*)ptr[nr.x];
-                            lp.norm_w = (const float*)ptr[nr.weight];
-                            lp.norm_out = (float*)ptr[nr.dst];
-                            lp.norm_eps = nr.eps;
-                            lp.norm_for_x = m.x == nr.dst ? 1 : 0;
-                            norm_ok = lp.norm_x != lp.norm_out && m.x == nr.dst && (((uintptr_t)lp.norm_x | (uintptr_t)lp.norm_w | (uintptr_t)lp.norm_out) & 15) == 0;
+                        // One workgroup of a row stores it normalised, others read the residual operand and store the result, on other
+                        // XCDs and in no order with that store: neither may be the normalised row's memory (y = h + ffn(h) of
+                        // h = rmsnorm(x) * w, or the norm's dst bound to the op's).
+                        if (norm_x && (rn.xn_out == gp.addend || rn.xn_out == gp.dst)) launch_norm();
+                        if (norm_x) {   // the kernel normalises the raw rows
+                            lp.norm_x = norm_x;
+                            lp.norm_w = rn.weight;
+                            lp.norm_out = rn.xn_out;
+                            lp.norm_eps = rn.eps;
                         }
-                        if (norm_ok && infr::moe_layer_stream_supported(lp) &&
+                        if (infr::moe_layer_stream_supported(lp) &&
                             (((uintptr_t)lp.router | (uintptr_t)lp.router_x | (uintptr_t)gp.x) & 15) == 0 && (lp.router_row_floats & 3) == 0) {
                             launch_gate_logit();   // (a gated always-on expert keeps its norm as an op: the row this reads is there)
                             Timed t(be, gp.sh_gate ? "moe_layer_shared" : "moe_layer");
@@ -1716,29 +1732,11 @@ extern "C" infr_status infr_hip_execute(infr_hip_backend* be, infr_hip_plan* pla
                         }
                     }
                 }
-                bool normed = false;
-                if (fz.norm) {
-                    const infr_op_rms_norm& nr = plan->ops[fz.norm - 1].u.rms_norm;
-                    if (!(need(nr.x, "RmsNorm.x") && need(nr.weight, "RmsNorm.weight") && need(nr.dst, "RmsNorm.dst")))
-                        return INFR_ERR_BACKEND;
-                    infr::RouterNorm rn;
-                    rn.weight = (const float*)ptr[nr.weight]; rn.eps = nr.eps; rn.xn_out = (float*)ptr[nr.dst];
-                    {
-                        Timed t(be, "rms_norm_router_logits");
-                        normed = infr::launch_router_logits(s, (const uint8_t*)ptr[m.router], plan->tensors[m.router].dtype,
-                                                            router_row_bytes, (const float*)ptr[nr.x], (int)m.ne,
-                                                            (int)m.n_expert, rows, sc.logits, &rn);
-                    }
-                    if (!normed) {   // operands the fold cannot take (alignment): the op on its own
-                        Timed t(be, "rms_norm");
-                        infr::launch_rms_norm(s, (const float*)ptr[nr.x], rn.weight, rn.xn_out, rows, (int)nr.dim, nr.eps, 0);
-                    }
-                }
-                if (!normed) {
-                    Timed t(be, "router_logits");
-                    if (!infr::launch_router_logits(s, (const uint8_t*)ptr[m.router], plan->tensors[m.router].dtype,
-                                                    router_row_bytes, (const float*)ptr[m.router_x], (int)m.ne,
-                                                    (int)m.n_expert, rows, sc.logits))
+                {
+                    Timed t(be, norm_x ? "rms_norm_router_logits" : "router_logits");
+                    if (!infr::launch_router_logits(s, (const uint8_t*)ptr[m.router], plan->tensors[m.router].dtype, router_row_bytes,
+                                                    norm_x ? norm_x : (const float*)ptr[m.router_x], (int)m.ne, (int)m.n_expert, rows,
+                                                    sc.logits, norm_x ? &rn : nullptr))
                         return fail(INFR_ERR_UNSUPPORTED, "MoeFfn: ne=%u does not fit the router kernel's LDS budget", m.ne);
                 }
                 if (sc.batched) {

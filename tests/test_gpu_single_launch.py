@@ -756,3 +756,66 @@ def test_rms_norm_of_a_few_rows_folded_in(rows, ne, E, K, nff, gdt, ddt, name):
     assert np.array_equal(routes[False]["idx"], routes[True]["idx"]) and np.array_equal(bits(routes[False]["logits"]), bits(routes[True]["logits"]))
     assert np.array_equal(bits(outs[False]), bits(outs[True]))
     assert H.rel_l2(norms[False].reshape(rows, ne), O.rms_norm(x, nw, 1e-6).reshape(rows, ne)) < 1e-5
+
+
+_SUBLAYERS = {"mid": (2048, 128, 8, 768, DType.Q4K, DType.Q6K), "large": (4096, 256, 8, 1536, DType.Q4K, DType.Q6K),
+              "small": (1024, 32, 8, 512, DType.Q8_0, DType.Q8_0), "small K": (1024, 32, 8, 512, DType.Q4K, DType.Q6K),
+              "square": (2880, 64, 4, 960, DType.Mxfp4, DType.Mxfp4)}
+
+
+@pytest.mark.parametrize("shared", ["the residual", "the result", "the raw rows"])
+@pytest.mark.parametrize("shape,rows", [("mid", 1), ("mid", 2), ("mid", 3), ("mid", 4), ("mid", 8), ("large", 1), ("large", 2), ("large", 4),
+                                        ("small", 1), ("small", 2), ("small", 4), ("small K", 8), ("square", 1)])
+def test_the_normalised_rows_memory_is_an_operand_or_the_result(shape, rows, shared):
+    """h = rmsnorm(x) * w whose memory is also the residual of y = h + ffn(h), or where y goes, or x's own: every pass over one binding,
+    each with another x, has the bits of one launch per op, and the layer stays one launch (three rows: the per-token launches)."""
+    ne, E, K, nff, gd, dd = _SUBLAYERS[shape]
+    T = M.TensorDesc
+    rng = np.random.default_rng(rows + ne)
+    passes = [(rng.standard_normal((rows, ne)) * s).astype(np.float32) for s in (1.0, 5.0, 0.2)]
+    nw = rng.uniform(0.5, 1.5, ne).astype(np.float32)
+    router = (rng.standard_normal((E, ne)) * 0.02).astype(np.float32)
+    outs, names = {}, {}
+    for plain in (False, True):
+        b = M.Backend(0, disable_op_fusion=plain, disable_single_launch_moe=plain)
+        try:
+            g = M.Graph()
+            xi, nwt, rt = g.input(T([rows, ne], DType.F32)), g.weight(T([ne], DType.F32)), g.weight(T([E, ne], DType.F32))
+            banks = [(g.weight(T(dims, dt)), dt, int(np.prod(dims))) for dims, dt in (([E, nff, ne], gd), ([E, nff, ne], gd), ([E, ne, nff], dd))]
+            h, y = g.output(T([rows, ne], DType.F32)), g.output(T([rows, ne], DType.F32))
+            g.rms_norm(x=xi, weight=nwt, dst=h, rows=rows, dim=ne, eps=1e-6)
+            residual = {"the residual": h, "the result": xi, "the raw rows": None}[shared]
+            moe = y if residual is None else g.internal(T([rows, ne], DType.F32))
+            g.moe_ffn(x=h, router=rt, gate_exps=banks[0][0], up_exps=banks[1][0], down_exps=banks[2][0], dst=moe, ne=ne, n_expert=E,
+                      n_used=K, n_ff_exp=nff)
+            if residual is not None:
+                g.add(a=residual, b=moe, dst=y, n=rows * ne)
+            plan, bind, bufs = b.compile(g), M.Bindings(), {}
+            for tid, v in ((xi, passes[0]), (nwt, nw), (rt, router)):
+                bufs[tid] = b.buffer_from(v)
+            for i, (tid, dt, n) in enumerate(banks):
+                bufs[tid] = b.alloc_uninit(M.backend.bytes_for(dt, n))
+                synth.weights_device(b, bufs[tid], dt, ne + i, n)
+            bufs[y] = b.alloc(rows * ne * 4)
+            bufs[h] = {"the residual": None, "the result": bufs[y], "the raw rows": bufs[xi]}[shared] or b.alloc(rows * ne * 4)
+            for tid, buf in bufs.items():
+                bind.bind(tid, buf)
+            b.prof_enable(True)
+            outs[plain] = []
+            for x in passes:
+                b.upload(bufs[xi], x)
+                b.execute(plan, bind)
+                outs[plain] += [b.download(bufs[y], rows * ne * 4, np.float32).copy(), b.download(bufs[h], rows * ne * 4, np.float32).copy()]
+            names[plain] = set(b.prof_read())
+            for buf in {id(v): v for v in bufs.values()}.values():
+                buf.free()
+            plan.free()
+        finally:
+            b.close()
+    if rows == 3:
+        assert ("rms_norm" if shared == "the raw rows" else FOLDED) in names[False] and GUESS not in names[False], names
+    else:
+        assert names[False] == {"rms_norm", GUESS}, names
+    assert "rms_norm" in names[True] and GUESS not in names[True], names
+    assert all(np.array_equal(bits(a), bits(c)) for a, c in zip(outs[False], outs[True]))
+    assert not np.array_equal(outs[True][0], outs[True][2])
