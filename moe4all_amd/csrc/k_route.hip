@@ -555,14 +555,31 @@ bool router_logits_fits(int rdt, size_t row_bytes, int ne, int rows) {
     return router_logits_tile(rdt, ne, rows, &epb, &rpb);
 }
 
-// The fold needs the one-burst staging: decode and small batches.  Each of a row's n_expert / 2 blocks normalises it again, which
-// costs less than a launch: us a pass with norm and residual, the norm by itself and folded: six layers of 3 rows of 128 experts of
-// 2048 x 768 in Q4_K / Q6_K 213.7 and 196.3, two of 20 rows in IQ4_XS 203.7 and 193.3, of 6 rows of 2880 x 2880, top-4, in MXFP4 225.6 and
-// 206.5, of 8 rows of 256 experts of 4096 x 1536 361.4 and 356.1.  Ten layers of 5 rows of 32 experts of 1024 x 512 in Q4_0 286.1
-// and 259.2.  (Several rows of less than 2048 elements and less than 32 experts keep the launch: which launches such a layer makes is
-// pinned by tests.)
+// Experts and token rows per block of a launch: where blocks of fewer token rows, or of one expert, still have a compute unit each,
+// they stage less.  us a pass, larger and smaller blocks: 5 rows of 8 experts of hidden size 4096 189.3 and 185.7, two layers of 6 rows of
+// 128 experts of 2880 206.1 and 202.8, six of 3 rows of 2048 195.5 and 193.0, ten of 5 rows of 32 experts of 1024 259.1 and 256.6.
+// (More blocks than compute units only read the router more often: 8 rows of 256 experts stay with four rows to a block.)
+static bool router_logits_blocks(int rdt, int ne, int n_expert, int rows, int* epb, int* rpb) {
+    if (!router_logits_tile(rdt, ne, rows, epb, rpb)) return false;
+    while (*epb == 2 && *rpb > 1 && (n_expert + 1) / 2 * ((rows + *rpb / 2 - 1) / (*rpb / 2)) <= 256) *rpb /= 2;
+    if (*epb == 2 && *rpb == 1 && n_expert * rows <= 256) *epb = 1;
+    return true;
+}
+
+// The fold needs the one-burst staging: decode and small batches.  Every block normalises its token rows again, so the fold pays while
+// the blocks' rows together are few.  us a layer that it saves over the norm as a launch, by elements normalised (blocks x rows of a block x
+// ne): 1.05 M 1.9 (8 rows of 128 experts of 2048) and 2.4 (of 64 of 4096), 2.1 M 1.8 (16 rows of 128 experts of 2048) and 1.9 (8 of 128 of 4096),
+// 4.2 M 0.03 to 1.3 (16 rows of 128 experts of 4096, 8 rows of 512 of 2048; 8 rows of 256 of 4096 0.1); beyond, 5.9 M -0.3 (16 rows of 256
+// of 2880), 8.4 M -2.6 (of 256 of 4096) and -0.5 (of 512 of 2048), 16.8 M -7.5 (31 rows of 256 of 4096), 33.6 M -19 (of 512).  (6.3 M still saves
+// 0.2 to 0.5 at 2048 and 1024, and loses 2.8 at 4096.)
+// Several rows of less than 2048 elements and less than 32 experts keep the launch, although the fold would save 1.4 to 2.3 us a layer there
+// (5 and 31 rows of 8 experts of 256 to 1024, of 16 of 1024 and 1536): that these are launches of their own is part of what is tested.
 bool router_logits_can_norm(int rdt, size_t row_bytes, int ne, int n_expert, int rows) {
-    return rows >= 1 && (rows == 1 || (rows < 32 && (ne >= 2048 || n_expert >= 32))) && rdt == INFR_F32 && (ne & 3) == 0 && ne >= 4 && ne <= 4096 && (row_bytes & 15) == 0;
+    if (rows < 1 || rows >= 32 || rdt != INFR_F32 || (ne & 3) != 0 || ne < 4 || ne > 4096 || (row_bytes & 15) != 0) return false;
+    if (rows > 1 && ne < 2048 && n_expert < 32) return false;
+    int epb, rpb;
+    if (!router_logits_blocks(rdt, ne, n_expert, rows, &epb, &rpb)) return false;
+    return (size_t)((n_expert + epb - 1) / epb) * ((rows + rpb - 1) / rpb) * rpb * ne <= (size_t)1 << 22;
 }
 
 bool launch_router_logits(hipStream_t s, const uint8_t* router, int rdt, size_t row_bytes, const float* x, int ne,
@@ -590,13 +607,7 @@ bool launch_router_logits(hipStream_t s, const uint8_t* router, int rdt, size_t 
         return true;
     }
     int epb = 0, rpb = 0;
-    if (!router_logits_tile(rdt, ne, rows, &epb, &rpb)) return false;
-    // where blocks of fewer token rows, or of one expert, still have a compute unit each, they stage less.  us a pass,
-    // larger and smaller blocks: 5 rows of 8 experts of hidden size 4096 189.3 and 185.7, two layers of 6 rows of 128 experts of 2880 206.1
-    // and 202.8, six of 3 rows of 2048 195.5 and 193.0, ten of 5 rows of 32 experts of 1024 259.1 and 256.6.  (More blocks than compute
-    // units only read the router more often: 8 rows of 256 experts stay with four rows to a block.)
-    while (epb == 2 && rpb > 1 && (n_expert + 1) / 2 * ((rows + rpb / 2 - 1) / (rpb / 2)) <= 256) rpb /= 2;
-    if (epb == 2 && rpb == 1 && n_expert * rows <= 256) epb = 1;
+    if (!router_logits_blocks(rdt, ne, n_expert, rows, &epb, &rpb)) return false;
     const bool small = rows <= 2 || (rows < 32 && rdt == INFR_F32 && (ne & 3) == 0 && ne <= 4096);
     const size_t budget = kRouterLdsBudget;
     const int nc = ne >> 3;

@@ -819,3 +819,65 @@ def test_the_normalised_rows_memory_is_an_operand_or_the_result(shape, rows, sha
     assert "rms_norm" in names[True] and GUESS not in names[True], names
     assert all(np.array_equal(bits(a), bits(c)) for a, c in zip(outs[False], outs[True]))
     assert not np.array_equal(outs[True][0], outs[True][2])
+
+
+def _sublayer(b, rows, ne, E, K, nff, x, nw, router, eps=1e-6, norm=True):
+    """y = x + ffn(rmsnorm(x) * nw), or x + ffn(x), on generated Q8_0 banks, run twice: (y, the normalised rows, routing, launch names)."""
+    T, dt = M.TensorDesc, DType.Q8_0
+    g, bind, bufs = M.Graph(), M.Bindings(), []
+
+    def bound(tid, buf):
+        bufs.append(buf)
+        bind.bind(tid, buf)
+        return tid
+    xi, rt = bound(g.input(T([rows, ne], DType.F32)), b.buffer_from(x)), bound(g.weight(T([E, ne], DType.F32)), b.buffer_from(router))
+    banks = []
+    for role, dims in enumerate(([E, nff, ne], [E, nff, ne], [E, ne, nff])):
+        n = int(np.prod(dims))
+        banks.append(bound(g.weight(T(dims, dt)), b.alloc_uninit(M.backend.bytes_for(dt, n))))
+        synth.weights_device(b, bufs[-1], dt, role, n)
+    h = xi
+    if norm:
+        nwt, h = bound(g.weight(T([ne], DType.F32)), b.buffer_from(nw)), bound(g.output(T([rows, ne], DType.F32)), b.alloc(rows * ne * 4))
+        g.rms_norm(x=xi, weight=nwt, dst=h, rows=rows, dim=ne, eps=eps)
+    h_buf = bufs[-1]
+    moe, y = g.internal(T([rows, ne], DType.F32)), bound(g.output(T([rows, ne], DType.F32)), b.alloc(rows * ne * 4))
+    g.moe_ffn(x=h, router=rt, gate_exps=banks[0], up_exps=banks[1], down_exps=banks[2], dst=moe, ne=ne, n_expert=E, n_used=K, n_ff_exp=nff)
+    g.add(a=xi, b=moe, dst=y, n=rows * ne)
+    plan = b.compile(g)
+    b.prof_enable(True)
+    for _ in range(2):
+        b.execute(plan, bind)
+    out = b.download(bufs[-1], rows * ne * 4, np.float32).copy()
+    normed = b.download(h_buf, rows * ne * 4, np.float32).copy() if norm else None
+    names = set(b.prof_read())
+    b.prof_enable(False)
+    routing = b.moe_routing(plan, 1 if norm else 0)
+    for buf in bufs:
+        buf.free()
+    plan.free()
+    return out, normed, routing, names
+
+
+def _fold_case(rows, ne, E):
+    rng = np.random.default_rng(rows + ne + E)
+    x = (rng.standard_normal((rows, ne)) * 2).astype(np.float32)
+    x[rows - 1] *= 1e-3
+    return x, (1 + 0.1 * rng.standard_normal(ne)).astype(np.float32), (rng.standard_normal((E, ne)) * 0.02).astype(np.float32)
+
+
+@pytest.mark.parametrize("rows,ne,E,folds", [
+    (16, 4096, 128, True), (8, 2048, 512, True), (31, 2048, 128, True), (8, 1024, 512, True),        # 2^22 elements normalised, and less
+    (17, 4096, 128, False), (9, 2048, 512, False), (31, 4096, 256, False), (31, 1024, 512, False)])  # more: a launch of its own is less work
+def test_rms_norm_ahead_of_many_logits_blocks_keeps_its_launch(be, rows, ne, E, folds):
+    K, nff = 2, 32
+    x, nw, router = _fold_case(rows, ne, E)
+    out, normed, r, names = _sublayer(be, rows, ne, E, K, nff, x, nw, router)
+    assert (FOLDED in names) == folds and ("rms_norm" in names) == (not folds), names
+    b = M.Backend(0, disable_op_fusion=True)
+    try:
+        out1, normed1, r1, _ = _sublayer(b, rows, ne, E, K, nff, x, nw, router)
+    finally:
+        b.close()
+    assert np.array_equal(bits(normed), bits(normed1)) and np.array_equal(bits(out), bits(out1))
+    assert np.array_equal(r["idx"], r1["idx"]) and np.array_equal(bits(r["logits"]), bits(r1["logits"]))
