@@ -128,11 +128,21 @@ bool launch_stream4(hipStream_t s, const MoeLayerParams& q, size_t lds) {
 // residual: three launches 32 to 37 over boxes, this one 30.  The stream bounds it (10 us of 1530-byte rows for gate/up, 5 for down: a
 // row is 45 lanes' 34 unaligned bytes, whose loads keep the CU's address path busy as long as their 96 instructions a row keep
 // the vector ALUs), then the hand-over of h between 64 workgroups on two XCDs (3 us).
+// Where three launches are as fast they stay: with narrow rows and many of them the hand-overs cost more than the launches.  us a layer that
+// one launch saves, with norm and residual | the op alone, at 64 experts: nff 512 1024 / 1280 / 2048 / 2880 / 4096 wide 0.7 0.3 0.9 1.5 3.3 |
+// -0.2 0.1 0.4 1.1 2.4; 1536 -0.5 -0.7 -0.9 0.7 2.0 | -2.0 -0.9 0.3 0.4 1.9; 2880 -1.8 -1.8 -0.2 0.6 1.7 | -1.5 -1.1 -0.1 0.6 2.1; 3456 -1.2 -0.9 -0.8
+// -1.1 0.6 | -1.9 -1.7 -0.4 -1.1 1.0.  At 128: 512 0.9 1.1 1.3 2.3 5.2 | 0.4 0.5 1.4 1.6 2.2; 1024 0.6 1.2 0.7 0.0 2.4 | -0.5 0.0 0.2 0.6 0.2; 2048 0.3 -0.4 0.3
+// 0.2 3.5 | -0.9 -0.7 -0.5 0.2 0.6.  (2304 to 3328 wide at 64 experts and nff 768 to 3072 lies within 1.3 us of either side and stays here.)
+bool four_pays(int ne, int nff, int n_expert) {
+    if (nff <= 640 || ne >= 4096) return true;
+    return n_expert == 128 ? ne >= 2048 || nff <= 1024 : ne >= 2304 && nff <= 3072;
+}
 bool stream_four(hipStream_t s, MoeLayerParams q, bool launch) {
     const MoeGemvParams& p = q.g;
     const int ne = p.ne, nff = p.nff, n_expert = p.route.n_expert, rwc = ne <= 1024 ? 4 : ne <= 2048 ? 2 : 1;
     if (p.rows != 1 || p.sh_gate || !q.logits_once || (n_expert != 64 && n_expert != 128)) return false;
-    if (ne % 64 || ne < 1024 || ne > 4096 || nff % 64 || nff < 512 || nff > 4096) return false;   // 64 elements per lane, 16 to 64 lanes per row
+    if (ne % 64 || ne < 1024 || ne > 4096 || nff % 64 || nff < 512 || nff > 4096) return false;   // 64 elements per lane, 8 to 64 lanes per row
+    if (!four_pays(ne, nff, n_expert)) return false;
     const int share = nff / gather_waves(nff);
     if (nff % gather_waves(nff) || share % 64 || share > 9 * 64) return false;
     const int n_gi = (nff / 64 + rwc - 1) / rwc;

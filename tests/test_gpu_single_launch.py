@@ -881,3 +881,39 @@ def test_rms_norm_ahead_of_many_logits_blocks_keeps_its_launch(be, rows, ne, E, 
         b.close()
     assert np.array_equal(bits(normed), bits(normed1)) and np.array_equal(bits(out), bits(out1))
     assert np.array_equal(r["idx"], r1["idx"]) and np.array_equal(bits(r["logits"]), bits(r1["logits"]))
+
+
+@pytest.mark.parametrize("ne,nff,E,one", [
+    (1280, 640, 64, True), (1024, 768, 64, False), (1024, 3072, 64, False), (2048, 2048, 64, False),
+    (2304, 3072, 64, True), (3328, 3456, 64, False), (4096, 3456, 64, True), (1536, 1024, 128, True), (1536, 1152, 128, False),
+    (2048, 2048, 128, True)])
+def test_four_experts_per_token_where_three_launches_are_faster(be, be3, ne, nff, E, one):
+    """Both sides of each line: the launches that run, and the bits of three launches."""
+    K, dt, T = 4, DType.Mxfp4, M.TensorDesc
+    rng = np.random.default_rng(ne + nff + E)
+    x, router = rng.standard_normal((1, ne)).astype(np.float32), (rng.standard_normal((E, ne)) * 0.02).astype(np.float32)
+    outs = []
+    for b in (be, be3):
+        g, bind, bufs = M.Graph(), M.Bindings(), []
+        xi, rt, y = g.input(T([1, ne], DType.F32)), g.weight(T([E, ne], DType.F32)), g.output(T([1, ne], DType.F32))
+        banks = [g.weight(T([E, nff, ne], dt)), g.weight(T([E, nff, ne], dt)), g.weight(T([E, ne, nff], dt))]
+        for tid, buf in ((xi, b.buffer_from(x)), (rt, b.buffer_from(router)), (y, b.alloc(ne * 4))):
+            bufs.append(buf)
+            bind.bind(tid, buf)
+        for i, tid in enumerate(banks):
+            buf = b.alloc_uninit(M.backend.bytes_for(dt, E * nff * ne))
+            synth.weights_device(b, buf, dt, i, E * nff * ne)
+            bufs.append(buf)
+            bind.bind(tid, buf)
+        g.moe_ffn(x=xi, router=rt, gate_exps=banks[0], up_exps=banks[1], down_exps=banks[2], dst=y, ne=ne, n_expert=E, n_used=K, n_ff_exp=nff)
+        plan = b.compile(g)
+        b.prof_enable(True)
+        b.execute(plan, bind)
+        outs.append(b.download(bufs[2], ne * 4, np.float32).copy())
+        names = set(b.prof_read())
+        b.prof_enable(False)
+        for buf in bufs:
+            buf.free()
+        plan.free()
+        assert (GUESS in names) == (one and b is be), names
+    assert np.array_equal(bits(outs[0]), bits(outs[1])) and np.abs(outs[0]).max() > 1e-6
