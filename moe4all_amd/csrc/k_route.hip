@@ -61,17 +61,19 @@ void launch_route(hipStream_t s, const RouteParams& p) {
 // chain j of a row holds elements j, j+8, j+16, ... contiguously, so a chain thread streams
 // its operands with 128-bit LDS reads.  Strides are padded so the 16 lanes of a read phase
 // (2 experts x 8 chains) hit disjoint banks.
-// XQ: 128-bit loads of activations a thread holds in the one-burst staging (4: up to 1024 per block; 16: four rows of
-// 4096 elements, for small batches of a wide model, whose blocks would otherwise take one token row each and read the
-// router rows once per token row).
-// RN > 0: an Op::RmsNorm folded into the staging of a block of RN token rows, XQ / RN loads of a row per thread.
-template <int EPB, int XQ = 4, int RN = 0>
+// RN > 0: the one-burst staging of a block of RN token rows (its only ones) and EPB router rows, all f32 and of whole 128-bit vectors: every
+// global load of the block is issued before the first LDS store, so it pays the memory latency once.  A thread holds XQ vectors of activations,
+// XQ / RN of each row: up to 1024 per block, or 2048 or 4096 for small batches of a wide model, whose blocks would otherwise take one token
+// row each and read the router rows once per token row.  (Dealt out row by row: in one sequence over the block, with a division for every
+// vector, six layers of 3 rows of 128 experts of 2048 in Q5_K took 205.9 us a pass with norm and residual, and now 202.2; two of 8 of 256 of 4096
+// in Q4_K / Q6_K 348.0 and 346.6, without a norm 358.2 and 356.7.)
+// NORM: an Op::RmsNorm folded into that staging.
+template <int EPB, int XQ = 0, int RN = 0, bool NORM = false>
 __global__ __launch_bounds__(256) void router_logits_kernel(const uint8_t* __restrict__ router, int rdt,
                                                             size_t row_bytes, const float* __restrict__ x, int ne,
                                                             int n_expert, int rows, int rpb,
                                                             float* __restrict__ logits, RouterNorm nrm) {
     extern __shared__ float lds[];
-    __shared__ float red[4 * (RN ? RN : 1)];
     const int nc = ne >> 3;                 // full chunks of 8
     const int ntail = ne & 7;
     const int jstride = ((nc + 63) & ~63) + 4;
@@ -83,49 +85,44 @@ __global__ __launch_bounds__(256) void router_logits_kernel(const uint8_t* __res
     const int tid = threadIdx.x;
     const int e0 = blockIdx.x * EPB;
 
-    // Decode-sized launch (one pass over <= 2 token rows, f32 router): every global load of the
-    // block, activations included, is issued before the first LDS store, so the block pays the
-    // memory latency once.
     LOGITS_STAMP(0);
     const int nv = ne >> 2;
-    const int rbase = blockIdx.y * rpb;   // first token row of this block's (only) pass when one_shot
-    const bool one_shot = rdt == INFR_F32 && (ne & 3) == 0 && (int)gridDim.y * rpb >= rows && EPB * nv <= 8 * 256 &&
-                          rpb * nv <= XQ * 256;
+    // element 4v + t of a row: chain (4v + t) & 7 = 4 (v & 1) + t, step (4v + t) >> 3 = v >> 1: the four
+    // elements of a 128-bit load go to four chains at one step, or all four to the tail
+    auto stage = [&](float* row, float* tail, int v, const float4& f) __attribute__((always_inline)) {
+        if ((v >> 1) < nc) {
+            float* d = row + 4 * (v & 1) * jstride + (v >> 1);
+            d[0] = f.x; d[jstride] = f.y; d[2 * jstride] = f.z; d[3 * jstride] = f.w;
+        } else {
+            tail[0] = f.x; tail[1] = f.y; tail[2] = f.z; tail[3] = f.w;
+        }
+    };
     if constexpr (RN > 0) {
-        float4 wr[8], xr[XQ];
-        // the thread's i-th load: vector v of token row rr of the block (folded norm: as the standalone kernel deals a row out)
-        constexpr int NQ = RN ? XQ / RN : 1;
-        auto at = [&](int i, int& rr, int& v) {
-            const int idx = tid + 256 * i;
-            rr = RN ? i / NQ : idx / nv;
-            v = RN ? tid + 256 * (i % NQ) : idx - rr * nv;
-            return v < nv && rr < rpb;
-        };
+        constexpr int NQ = XQ / RN;
+        const int rbase = blockIdx.y * RN;
+        float4 wr[8], xr[XQ], nw[NORM ? NQ : 1];
+        // (rows behind the last token and expert repeat it: their logits are not stored)
 #pragma unroll
         for (int i = 0; i < XQ; i++) {
-            int rr, v;
-            xr[i] = make_float4(0.f, 0.f, 0.f, 0.f);
-            if (at(i, rr, v) && rbase + rr < rows) xr[i] = reinterpret_cast<const float4*>(x + (size_t)(rbase + rr) * ne)[v];
+            const int v = tid + 256 * (i % NQ);
+            if (v < nv) xr[i] = reinterpret_cast<const float4*>(x + (size_t)min(rbase + i / NQ, rows - 1) * ne)[v];
         }
-        float4 nw[NQ];
-        if (RN) {
+        if constexpr (NORM) {
 #pragma unroll
             for (int i = 0; i < NQ; i++) {
                 const int v = tid + 256 * i;
-                nw[i] = make_float4(0.f, 0.f, 0.f, 0.f);
                 if (v < nv) nw[i] = reinterpret_cast<const float4*>(nrm.weight)[v];
             }
         }
 #pragma unroll
         for (int i = 0; i < 8; i++) {
             const int idx = tid + 256 * i, e = idx / nv, v = idx - e * nv;
-            wr[i] = make_float4(0.f, 0.f, 0.f, 0.f);
-            if (e < EPB && e0 + e < n_expert)
-                wr[i] = reinterpret_cast<const float4*>(router + (size_t)(e0 + e) * row_bytes)[v];
+            if (e < EPB) wr[i] = reinterpret_cast<const float4*>(router + (size_t)min(e0 + e, n_expert - 1) * row_bytes)[v];
         }
-        if (RN) {
-            // The token rows arrive raw: Op::RmsNorm is applied while they are staged, with the
-            // summation tree of the standalone kernel, and the first block of a row stores it normalised.
+        if constexpr (NORM) {
+            // The token rows arrive raw: Op::RmsNorm is applied while they are staged, dealt out to the threads and summed as in
+            // the standalone kernel, and the first block of a row stores it normalised.
+            __shared__ float red[4 * RN];
 #pragma unroll
             for (int r = 0; r < RN; r++) {
                 float part = 0.0f;
@@ -140,105 +137,22 @@ __global__ __launch_bounds__(256) void router_logits_kernel(const uint8_t* __res
             LOGITS_STAMP(2);
 #pragma unroll
             for (int i = 0; i < XQ; i++) {
-                int rr, v;
-                if (!at(i, rr, v)) continue;
+                const int rr = i / NQ, v = tid + 256 * (i % NQ);
+                if (v >= nv) continue;
                 const float* q = red + 4 * rr;
                 xr[i] = rms_apply4(xr[i], rms_scale((q[0] + q[1]) + (q[2] + q[3]), ne, nrm.eps), nw[i % NQ]);
                 if (blockIdx.x == 0 && rbase + rr < rows) reinterpret_cast<float4*>(nrm.xn_out + (size_t)(rbase + rr) * ne)[v] = xr[i];
             }
         }
-        // element 4v + t of a row: chain (4v + t) & 7 = 4 (v & 1) + t, step (4v + t) >> 3 = v >> 1: the four
-        // elements of a 128-bit load go to four chains at one step, or all four to the tail
 #pragma unroll
         for (int i = 0; i < XQ; i++) {
-            int rr, v;
-            if (!at(i, rr, v)) continue;
-            if ((v >> 1) < nc) {
-                float* d = xs + rr * estride + 4 * (v & 1) * jstride + (v >> 1);
-                d[0] = xr[i].x; d[jstride] = xr[i].y; d[2 * jstride] = xr[i].z; d[3 * jstride] = xr[i].w;
-            } else {
-                float* d = xt + rr * 8;
-                d[0] = xr[i].x; d[1] = xr[i].y; d[2] = xr[i].z; d[3] = xr[i].w;
-            }
+            const int rr = i / NQ, v = tid + 256 * (i % NQ);
+            if (v < nv) stage(xs + rr * estride, xt + rr * 8, v, xr[i]);
         }
 #pragma unroll
         for (int i = 0; i < 8; i++) {
-            const int idx = tid + 256 * i, e = idx / nv, v = idx - e * nv;
-            if (e >= EPB) continue;
-            if ((v >> 1) < nc) {
-                float* d = w + e * estride + 4 * (v & 1) * jstride + (v >> 1);
-                d[0] = wr[i].x; d[jstride] = wr[i].y; d[2 * jstride] = wr[i].z; d[3 * jstride] = wr[i].w;
-            } else {
-                float* d = wt + e * 8;
-                d[0] = wr[i].x; d[1] = wr[i].y; d[2] = wr[i].z; d[3] = wr[i].w;
-            }
-        }
-    } else if (one_shot) {   // (a form of its own: without the run-time fold between them the compiler sinks the loads to their stores, 0.5 us)
-        float4 wr[8], xr[XQ], nw[4];
-#pragma unroll
-        for (int i = 0; i < XQ; i++) {
-            const int idx = tid + 256 * i, rr = idx / nv, v = idx - rr * nv;
-            xr[i] = make_float4(0.f, 0.f, 0.f, 0.f);
-            if (rr < rpb && rbase + rr < rows) xr[i] = reinterpret_cast<const float4*>(x + (size_t)(rbase + rr) * ne)[v];
-        }
-        if (nrm.weight) {
-#pragma unroll
-            for (int i = 0; i < 4; i++) {
-                const int idx = tid + 256 * i;
-                nw[i] = make_float4(0.f, 0.f, 0.f, 0.f);
-                if (idx < nv) nw[i] = reinterpret_cast<const float4*>(nrm.weight)[idx];
-            }
-        }
-#pragma unroll
-        for (int i = 0; i < 8; i++) {
-            const int idx = tid + 256 * i, e = idx / nv, v = idx - e * nv;
-            wr[i] = make_float4(0.f, 0.f, 0.f, 0.f);
-            if (e < EPB && e0 + e < n_expert)
-                wr[i] = reinterpret_cast<const float4*>(router + (size_t)(e0 + e) * row_bytes)[v];
-        }
-        if (nrm.weight) {
-            // The single token row arrives raw: Op::RmsNorm is applied while it is staged, with the
-            // summation tree of the standalone kernel, and the first block stores the normalised row.
-            float part = 0.0f;
-#pragma unroll
-            for (int i = 0; i < 4; i++)
-                if (tid + 256 * i < nv) part = sumsq4(part, xr[i]);
-            LOGITS_STAMP(1);
-            const float sc = rms_scale(block256_sum(part, red), ne, nrm.eps);
-            LOGITS_STAMP(2);
-#pragma unroll
-            for (int i = 0; i < 4; i++) {
-                const int idx = tid + 256 * i;
-                if (idx >= nv) continue;
-                xr[i] = rms_apply4(xr[i], sc, nw[i]);
-                if (blockIdx.x == 0 && blockIdx.y == 0) reinterpret_cast<float4*>(nrm.xn_out)[idx] = xr[i];
-            }
-        }
-        // element 4v + t of a row: chain (4v + t) & 7 = 4 (v & 1) + t, step (4v + t) >> 3 = v >> 1: the four
-        // elements of a 128-bit load go to four chains at one step, or all four to the tail
-#pragma unroll
-        for (int i = 0; i < XQ; i++) {
-            const int idx = tid + 256 * i, rr = idx / nv, v = idx - rr * nv;
-            if (rr >= rpb) continue;
-            if ((v >> 1) < nc) {
-                float* d = xs + rr * estride + 4 * (v & 1) * jstride + (v >> 1);
-                d[0] = xr[i].x; d[jstride] = xr[i].y; d[2 * jstride] = xr[i].z; d[3 * jstride] = xr[i].w;
-            } else {
-                float* d = xt + rr * 8;
-                d[0] = xr[i].x; d[1] = xr[i].y; d[2] = xr[i].z; d[3] = xr[i].w;
-            }
-        }
-#pragma unroll
-        for (int i = 0; i < 8; i++) {
-            const int idx = tid + 256 * i, e = idx / nv, v = idx - e * nv;
-            if (e >= EPB) continue;
-            if ((v >> 1) < nc) {
-                float* d = w + e * estride + 4 * (v & 1) * jstride + (v >> 1);
-                d[0] = wr[i].x; d[jstride] = wr[i].y; d[2 * jstride] = wr[i].z; d[3 * jstride] = wr[i].w;
-            } else {
-                float* d = wt + e * 8;
-                d[0] = wr[i].x; d[1] = wr[i].y; d[2] = wr[i].z; d[3] = wr[i].w;
-            }
+            const int idx = tid + 256 * i, e = idx / nv;
+            if (e < EPB) stage(w + e * estride, wt + e * 8, idx - e * nv, wr[i]);
         }
     } else if (rdt == INFR_F32 && (ne & 3) == 0) {
         for (int idx = tid; idx < EPB * nv; idx += 256) {
@@ -269,8 +183,8 @@ __global__ __launch_bounds__(256) void router_logits_kernel(const uint8_t* __res
     const int j = tid & 7;
     const int lane = tid & 63;
     for (int r0 = blockIdx.y * rpb; r0 < rows; r0 += gridDim.y * rpb) {
-        if (!one_shot) __syncthreads();
-        for (int rr = 0; rr < (one_shot ? 0 : rpb); rr++) {
+        if (RN == 0) __syncthreads();
+        for (int rr = 0; rr < (RN ? 0 : rpb); rr++) {
             const bool row_ok = r0 + rr < rows;
             const float* xr = x + (size_t)(row_ok ? r0 + rr : 0) * ne;
             for (int k = tid; k < ne; k += 256) {
@@ -621,45 +535,35 @@ bool launch_router_logits(hipStream_t s, const uint8_t* router, int rdt, size_t 
     if (gy > cap) gy = cap;
     if (gy < 1) gy = 1;
     dim3 grid(gx, gy), block(256);
-#define LAUNCH_RL(E)                                                                                               \
-    do {                                                                                                           \
-        INFR_LDS_LIMIT((router_logits_kernel<E>), (int)budget); \
-        INFR_LAUNCH(router_logits_kernel<E>, grid, block, lds, s, router, rdt, row_bytes, x, ne, n_expert,  \
-                           rows, rpb, logits, nrm);                                                   \
+#define LAUNCH_RL(...)                                                                                              \
+    do {                                                                                                            \
+        INFR_LDS_LIMIT((router_logits_kernel<__VA_ARGS__>), (int)budget);                                           \
+        INFR_LAUNCH((router_logits_kernel<__VA_ARGS__>), grid, block, lds, s, router, rdt, row_bytes, x, ne, n_expert, rows, rpb, logits, nrm); \
+        return true;                                                                                                \
     } while (0)
-    if (nrm.weight) {
-#define LAUNCH_RN(E, Q, R)                                                                                         \
-    do {                                                                                                           \
-        INFR_LDS_LIMIT((router_logits_kernel<E, Q, R>), (int)budget);                                              \
-        INFR_LAUNCH((router_logits_kernel<E, Q, R>), grid, block, lds, s, router, rdt, row_bytes, x, ne, n_expert, rows, rpb, logits, nrm); \
+    // the one-burst staging: a single pass over rows that fit its registers
+#define LAUNCH_RN(E, Q, R)                         \
+    do {                                           \
+        if (nrm.weight) LAUNCH_RL(E, Q, R, true);  \
+        else LAUNCH_RL(E, Q, R);                   \
     } while (0)
-        if (epb > 2 || rpb > 4 || gy != passes) return false;
-        if (rpb == 1 && epb == 1) LAUNCH_RN(1, 4, 1);
-        else if (epb == 1) return false;
-        else if (rpb == 1) LAUNCH_RN(2, 4, 1);
-        else if (rpb == 2 && ne <= 2048) LAUNCH_RN(2, 4, 2);
-        else if (rpb == 2) LAUNCH_RN(2, 8, 2);
-        else LAUNCH_RN(2, 16, 4);
+    if (rdt == INFR_F32 && (ne & 3) == 0 && gy == passes) {
+        if (rpb == 1 && epb == 1 && ne <= 4096) LAUNCH_RN(1, 4, 1);
+        if (rpb == 1 && epb == 2 && ne <= 4096) LAUNCH_RN(2, 4, 1);
+        if (rpb == 2 && epb == 2 && ne <= 2048) LAUNCH_RN(2, 4, 2);
+        if (rpb == 2 && epb == 2 && ne <= 4096) LAUNCH_RN(2, 8, 2);
+        if (rpb == 4 && epb == 2 && ne <= 4096) LAUNCH_RN(2, 16, 4);
+    }
 #undef LAUNCH_RN
-        return true;
-    }
-    if (small && rpb * (ne >> 2) > 4 * 256 && epb <= 2) {   // the wide one-burst staging
-        INFR_LDS_LIMIT((router_logits_kernel<2, 16>), (int)budget);
-        if (epb == 2) INFR_LAUNCH((router_logits_kernel<2, 16>), grid, block, lds, s, router, rdt, row_bytes, x, ne, n_expert, rows, rpb, logits, nrm);
-        else {
-            INFR_LDS_LIMIT((router_logits_kernel<1, 16>), (int)budget);
-            INFR_LAUNCH((router_logits_kernel<1, 16>), grid, block, lds, s, router, rdt, row_bytes, x, ne, n_expert, rows, rpb, logits, nrm);
-        }
-        return true;
-    }
+    if (nrm.weight) return false;
+    if (rdt == INFR_F32 && (ne & 3) == 0 && gy == passes && rpb == 4 && epb == 8 && ne <= 1024) LAUNCH_RL(8, 4, 4);
     switch (epb) {
-        case 8: LAUNCH_RL(8); break;
-        case 4: LAUNCH_RL(4); break;
-        case 2: LAUNCH_RL(2); break;
-        default: LAUNCH_RL(1); break;
+        case 8: LAUNCH_RL(8);
+        case 4: LAUNCH_RL(4);
+        case 2: LAUNCH_RL(2);
+        default: LAUNCH_RL(1);
     }
 #undef LAUNCH_RL
-    return true;
 }
 
 }  // namespace infr

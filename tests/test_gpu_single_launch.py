@@ -917,3 +917,70 @@ def test_four_experts_per_token_where_three_launches_are_faster(be, be3, ne, nff
         plan.free()
         assert (GUESS in names) == (one and b is be), names
     assert np.array_equal(bits(outs[0]), bits(outs[1])) and np.abs(outs[0]).max() > 1e-6
+
+
+@pytest.mark.parametrize("rows,ne,E", [   # experts x token rows of a workgroup of the logits, loads of a row:
+    (1, 2048, 64), (5, 2048, 32), (7, 4096, 8), (5, 2880, 9),   # 1 x 1
+    (1, 2048, 257), (3, 2048, 128), (3, 2048, 127), (4, 4096, 65),   # 2 x 1
+    (16, 2048, 64), (31, 2048, 32), (9, 1024, 65),   # 2 x 2, up to 2048 wide: whole, a row behind the end, and an expert
+    (4, 4096, 256), (6, 2880, 128), (5, 2880, 128), (6, 2080, 127),   # 2 x 2 above: whole and ragged shares of 256 loads
+    (8, 4096, 256), (9, 4096, 128), (15, 2880, 128), (25, 2080, 65),   # 2 x 4
+])
+@pytest.mark.parametrize("norm", [True, False])
+def test_every_form_of_the_logits_of_a_few_rows(be, norm, rows, ne, E):
+    """The normalised rows have the bits of the launch by itself, the logits those of the oracle on these rows (8 chains, summed in order),
+    with the norm folded into the launch and without one."""
+    x, nw, router = _fold_case(rows, ne, E)
+    out, normed, r, names = _sublayer(be, rows, ne, E, 2, 32, x, nw, router, norm=norm)
+    assert (FOLDED if norm else "router_logits") in names and "rms_norm" not in names and GUESS not in names, names
+    b = M.Backend(0, disable_op_fusion=True)
+    try:
+        out1, normed1, r1, names1 = _sublayer(b, rows, ne, E, 2, 32, x, nw, router, norm=norm)
+    finally:
+        b.close()
+    assert ("rms_norm" in names1) == norm
+    if norm:
+        assert np.array_equal(bits(normed), bits(normed1))
+    h = normed.reshape(rows, ne) if norm else x
+    experts = sorted({0, 1, E // 2, E - 2, E - 1})
+    want = np.array([[O.dot(h[i], router[e]) for e in experts] for i in range(rows)], np.float32)
+    assert np.array_equal(bits(r["logits"][:, experts]), bits(want))
+    assert np.array_equal(bits(r["logits"]), bits(r1["logits"])) and np.array_equal(r["idx"], r1["idx"]) and np.array_equal(bits(out), bits(out1))
+
+
+@pytest.mark.parametrize("rows,ne,E", [(32, 100, 10), (41, 1020, 17), (41, 1028, 17), (41, 100, 2048)])   # one burst (last tile ragged), too wide, several passes
+def test_logits_of_batches_the_matrix_cores_do_not_take(be, rows, ne, E):
+    K, nff = 2, 4
+    rng = np.random.default_rng(rows + ne + E)
+    x, router = rng.standard_normal((rows, ne)).astype(np.float32), (rng.standard_normal((E, ne)) * 0.02).astype(np.float32)
+    z = np.zeros(E * nff * ne, np.float32)
+    g, ids = moe_graph(rows, ne, E, K, nff, DType.F32, DType.F32)
+    _, r = _run(be, g, ids, dict(x=x, router=router, gate=z, up=z, down=z), rows * ne, "router_logits")
+    ref = O.moe_ffn(x, router, z, z, z, ne=ne, n_expert=E, n_used=K, n_ff_exp=nff)
+    assert np.array_equal(bits(r["logits"]), bits(ref["logits"])) and np.array_equal(r["idx"], ref["idx"])
+
+
+@pytest.mark.parametrize("rows,ne,E,K,nff,dt,name", [
+    (1, 2048, 64, 2, 32, DType.Q8_0, FOLDED), (3, 2048, 128, 2, 32, DType.Q8_0, FOLDED), (6, 2880, 128, 2, 32, DType.Q8_0, FOLDED),
+    (8, 4096, 256, 2, 32, DType.Q8_0, FOLDED), (40, 2048, 8, 2, 32, DType.Q8_0, "rms_norm"), (1, 2048, 128, 8, 768, DType.Q8_0, GUESS),
+    (2, 2048, 128, 8, 768, DType.Q8_0, GUESS), (4, 1024, 32, 8, 512, DType.Q8_0, GUESS)])
+def test_rms_norm_of_rows_whose_mean_square_is_subnormal(be, rows, ne, E, K, nff, dt, name):
+    """eps = 0 and elements about 2^-66, so that the mean of their squares lies below 2^-126: every kernel that normalises gives the same
+    bits.  A square is rounded by up to 2^-150 at 2^-132, 2^-18 of it; the mean by up to 2^-150 at 1.5 x 2^-132, 2^-18.6; the root halves
+    both to less than 2^-18.2.  The sum's roundings (8 to 24 additions deep, halved too), the root, the quotient and two products add at most
+    2^-19.  2^-17 holds all of it."""
+    rng = np.random.default_rng(rows + ne)
+    x = (rng.choice([-1.0, 1.0], (rows, ne)) * rng.uniform(1.0, 1.5, (rows, ne)) * 2.0 ** -66).astype(np.float32)
+    _, nw, router = _fold_case(rows, ne, E)
+    _, normed, r, names = _sublayer(be, rows, ne, E, K, nff, x, nw, router, eps=0.0)
+    assert name in names, names
+    b = M.Backend(0, disable_op_fusion=True, disable_single_launch_moe=True)
+    try:
+        _, normed1, r1, names1 = _sublayer(b, rows, ne, E, K, nff, x, nw, router, eps=0.0)
+    finally:
+        b.close()
+    assert "rms_norm" in names1
+    assert np.array_equal(bits(normed), bits(normed1)) and np.array_equal(bits(r["logits"]), bits(r1["logits"]))
+    x64 = x.astype(np.float64)
+    want = x64 / np.sqrt((x64 ** 2).mean(axis=1, keepdims=True)) * nw
+    assert (np.abs(normed.reshape(rows, ne) - want) <= np.abs(want) * 2.0 ** -17).all()
