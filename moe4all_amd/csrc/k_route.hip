@@ -65,8 +65,8 @@ void launch_route(hipStream_t s, const RouteParams& p) {
 // global load of the block is issued before the first LDS store, so it pays the memory latency once.  A thread holds XQ vectors of activations,
 // XQ / RN of each row: up to 1024 per block, or 2048 or 4096 for small batches of a wide model, whose blocks would otherwise take one token
 // row each and read the router rows once per token row.  (Dealt out row by row: in one sequence over the block, with a division for every
-// vector, six layers of 3 rows of 128 experts of 2048 in Q5_K took 205.9 us a pass with norm and residual, and now 202.2; two of 8 of 256 of 4096
-// in Q4_K / Q6_K 348.0 and 346.6, without a norm 358.2 and 356.7.)
+// vector, six layers of 3 rows of 128 experts of 2048 in Q5_K took 205.9 us a pass with norm and residual, and now 202.2; two of 3 of
+// 256 of 4096 without a norm 183.7 and 180.7.)
 // NORM: an Op::RmsNorm folded into that staging.
 template <int EPB, int XQ = 0, int RN = 0, bool NORM = false>
 __global__ __launch_bounds__(256) void router_logits_kernel(const uint8_t* __restrict__ router, int rdt,
@@ -480,20 +480,20 @@ static bool router_logits_blocks(int rdt, int ne, int n_expert, int rows, int* e
     return true;
 }
 
-// The fold needs the one-burst staging: decode and small batches.  Every block normalises its token rows again, so the fold pays while
-// the blocks' rows together are few.  us a layer that it saves over the norm as a launch, by elements normalised (blocks x rows of a block x
-// ne): 1.05 M 1.9 (8 rows of 128 experts of 2048) and 2.4 (of 64 of 4096), 2.1 M 1.8 (16 rows of 128 experts of 2048) and 1.9 (8 of 128 of 4096),
-// 4.2 M 0.03 to 1.3 (16 rows of 128 experts of 4096, 8 rows of 512 of 2048; 8 rows of 256 of 4096 0.1); beyond, 5.9 M -0.3 (16 rows of 256
-// of 2880), 8.4 M -2.6 (of 256 of 4096) and -0.5 (of 512 of 2048), 16.8 M -7.5 (31 rows of 256 of 4096), 33.6 M -19 (of 512).  (6.3 M still saves
-// 0.2 to 0.5 at 2048 and 1024, and loses 2.8 at 4096.)
+// The fold needs the one-burst staging: decode and small batches.  Every block normalises its token rows again, so it pays where a block has one
+// or two and the blocks are few.  us a layer that it saves over the norm as a launch: 8 rows of 64 experts of 4096 (256 blocks) 3.5, of 128
+// of 2048 2.5, of 128 of 4096 0.9; 31 rows of 128 experts of 2048 (1024 blocks) 1.6, 24 of 256 (1536) 1.7, 16 of 512 and 8 of 1024 (2048) 0.9 and 1.5,
+// 16 rows of 512 experts of 1024 (2048) 0.6; beyond, 24 of 512 of 1024 (3072) -0.6, 31 (4096) -1.6, 31 of 512 and 16 of 1024 of 2048 (4096) 0.6 and 0.1.
+// Blocks of four rows (wider than 2048, more than 256 blocks of two): 31 rows of 64 experts of 2304 0.3, 10 of 128 of 2880 -0.2, 8 of 256 of 2880 and
+// of 4096 -0.5 and -1.1, 16 of 128 of 4096 -1.1, 31 of 256 of 4096 -12, of 512 -25.
 // Several rows of less than 2048 elements and less than 32 experts keep the launch, although the fold would save 1.4 to 2.3 us a layer there
-// (5 and 31 rows of 8 experts of 256 to 1024, of 16 of 1024 and 1536): that these are launches of their own is part of what is tested.
+// (5 and 31 rows of 8 experts of 256 to 1024, of 16 of 1024 and 1536): tests of the launches rely on it.
 bool router_logits_can_norm(int rdt, size_t row_bytes, int ne, int n_expert, int rows) {
     if (rows < 1 || rows >= 32 || rdt != INFR_F32 || (ne & 3) != 0 || ne < 4 || ne > 4096 || (row_bytes & 15) != 0) return false;
     if (rows > 1 && ne < 2048 && n_expert < 32) return false;
     int epb, rpb;
     if (!router_logits_blocks(rdt, ne, n_expert, rows, &epb, &rpb)) return false;
-    return (size_t)((n_expert + epb - 1) / epb) * ((rows + rpb - 1) / rpb) * rpb * ne <= (size_t)1 << 22;
+    return rpb <= 2 && (n_expert + epb - 1) / epb * ((rows + rpb - 1) / rpb) <= 2048;
 }
 
 bool launch_router_logits(hipStream_t s, const uint8_t* router, int rdt, size_t row_bytes, const float* x, int ne,
@@ -552,11 +552,13 @@ bool launch_router_logits(hipStream_t s, const uint8_t* router, int rdt, size_t 
         if (rpb == 1 && epb == 2 && ne <= 4096) LAUNCH_RN(2, 4, 1);
         if (rpb == 2 && epb == 2 && ne <= 2048) LAUNCH_RN(2, 4, 2);
         if (rpb == 2 && epb == 2 && ne <= 4096) LAUNCH_RN(2, 8, 2);
-        if (rpb == 4 && epb == 2 && ne <= 4096) LAUNCH_RN(2, 16, 4);
     }
 #undef LAUNCH_RN
     if (nrm.weight) return false;
-    if (rdt == INFR_F32 && (ne & 3) == 0 && gy == passes && rpb == 4 && epb == 8 && ne <= 1024) LAUNCH_RL(8, 4, 4);
+    if (rdt == INFR_F32 && (ne & 3) == 0 && gy == passes && rpb == 4) {
+        if (epb == 2 && ne <= 4096) LAUNCH_RL(2, 16, 4);
+        if (epb == 8 && ne <= 1024) LAUNCH_RL(8, 4, 4);
+    }
     switch (epb) {
         case 8: LAUNCH_RL(8);
         case 4: LAUNCH_RL(4);
