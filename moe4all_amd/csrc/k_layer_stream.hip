@@ -1,4 +1,4 @@
-// Single-token Op::MoeFfn as ONE launch in which the expert weights are requested before the routing is known.
+// Op::MoeFfn of one, two, four or eight token rows as ONE launch in which the expert weights are requested before the routing is known.
 //
 // What the reference fixes for this op is the routing (ids in rank order, routing weights, bit for bit:
 // crates/infr-cpu/src/lib.rs:3684-3716 for the logits' summation order, :3746-3861 for gating, selection and
@@ -12,10 +12,11 @@
 // rounding), the workgroups that hold an expert outside the set compute the missing one late; a record's tag carries
 // the expert it belongs to, so a consumer can never take the product of a wrong guess for the one it waits for.
 //
-// Work split.  256 workgroups of 8 wavefronts in 8 groups of 32 (group = blockIdx & 7; consecutive workgroups go to
-// consecutive XCDs, so a group shares an L2).  Group g computes one expert of the set: workgroup m of the group the
-// features [m * nff / 32, +nff / 32) of gate and up, then the output rows [m * ne / 32, +ne / 32) of down.  An
-// always-on expert folded into the op is spread over all 256 workgroups (features [b * nff / 256, ..), rows
+// Work split.  256 workgroups of 8 wavefronts; of R token rows each has 256 / R of them, whole XCDs (consecutive workgroups go to
+// consecutive XCDs).  A row's workgroups form 8 groups of 32 / R that each share an XCD's L2, or, with four experts per token (one
+// row), 4 groups of 64 on two XCDs.  Group g computes one expert of the set: workgroup m of its M the features
+// [m * nff / M, +nff / M) of gate and up, then the output rows [m * ne / M, +ne / M) of down.  An
+// always-on expert folded into the op is spread over all workgroups of the row (256 for one row: features [b * nff / 256, ..), rows
 // [b * ne / 256, ..)); it needs no routing, so its rows are the first bytes requested.  Wavefront 0 is the router
 // (exact chains, exact routing, check of the guess), wavefronts 1..7 stream weights: each keeps a ring of items
 // (a gate row and an up row, or a group of down rows) in flight, finishes the oldest and requests the one D places

@@ -1,6 +1,6 @@
-// The streaming single-launch kernel of Op::MoeFfn (one, two or four token rows in one launch) and its launcher
-// template: included by the two translation units that instantiate it (k_layer_stream.hip: any shape;
-// k_layer_stream_shapes.hip: the benchmark shapes with their sizes as compile-time constants).
+// The streaming single-launch kernel of Op::MoeFfn (one, two, four or eight token rows in one launch) and its launcher
+// template: included by the translation units that instantiate it (k_layer_stream.hip: any shape;
+// k_layer_stream_shapes.hip and k_layer_stream_shapes_other.hip: the benchmark shapes with their sizes as compile-time constants).
 #pragma once
 
 #include "device_common.h"
@@ -254,9 +254,9 @@ __global__ __launch_bounds__(kThreads) void moe_layer_stream(MoeLayerParams q) {
     constexpr int NS = kHalf ? 1 : NSP, n_expert = kHalf ? 32 : 64 * NSP;   // experts per lane; all of them
     const int n_gather = gather_waves(nff);
     const bool shared = p.sh_gate != nullptr;
-    // One, two or four token rows per launch: a row takes 8 / rows of the XCDs (workgroups are dealt to the XCDs in turn,
+    // One, two, four or eight token rows per launch: a row takes 8 / rows of the XCDs (workgroups are dealt to the XCDs in turn,
     // so workgroup b sits on XCD b & 7 up to a rotation), its eight groups of mpg = 32 / rows members each lie on one XCD
-    // as before, and everything below happens per row among the row's 256 / rows workgroups.
+    // (KR = 4: four groups of 64, on two), and everything below happens per row among the row's 256 / rows workgroups.
     const int b = blockIdx.x;
     const int n_rows = ROWS ? ROWS : p.rows, xpr = 8 / n_rows, bpr = kBlocks / n_rows, mpg = bpr / KR;
     const int xcd = b & 7, jx = b >> 3;
@@ -672,7 +672,7 @@ __global__ __launch_bounds__(kThreads) void moe_layer_stream(MoeLayerParams q) {
             if (wave == 3) STAMP(7);
             if (wave == 1) STAMP(21);
             if (wave == 7) STAMP(22);
-            // ---- hand-over of the group's activations: six (or four) wavefronts gather a share each and turn it into cells
+            // ---- hand-over of the group's activations: four to six wavefronts gather a share each and turn it into cells
             bool superseded = false;
             if (sw < n_gather) {
                 const int st = gather_activations<KR == 4 ? 9 : 4>(q.xh + (size_t)g * nff + sw * chunk, chunk, seq_tag | (uint32_t)e_cur,
@@ -883,8 +883,17 @@ bool launch_stream(hipStream_t s, const MoeLayerParams& q, size_t lds) {
 
 }  // namespace
 
-// The instantiations with compile-time sizes (k_layer_stream_shapes.hip).  *taken: one of them matches the shape; the
-// return value is then that of the launch (true without launching when `launch` is false).
+// The instantiations with compile-time sizes (k_layer_stream_shapes.hip, k_layer_stream_shapes_other.hip).  *taken: one of them matches
+// the shape; the return value is then that of the launch (true without launching when `launch` is false).
 bool launch_stream_fixed(hipStream_t s, const MoeLayerParams& q, const StreamShape& sh, bool launch, bool* taken);
+bool launch_stream_fixed_other(hipStream_t s, const MoeLayerParams& q, const StreamShape& sh, bool launch, bool* taken);
+// One of them, without and with the token rows' RmsNorm folded in.
+#define INFR_STREAM_AT_N(FGt, FDt, DGv, DDv, EPTv, NSPv, NEv, NFFv, ROWSv, NORMv)                                             \
+    if (sh.dg == DGv && sh.dd == DDv && sh.ept == EPTv && sh.nsp == NSPv && p.ne == NEv && p.nff == NFFv && p.rows == ROWSv && \
+        norm == NORMv)                                                                                                       \
+        return launch ? launch_stream<FGt, FDt, DGv, DDv, EPTv, NSPv, NEv, NFFv, ROWSv, NORMv>(s, q, sh.lds) : true;
+#define INFR_STREAM_AT(FGt, FDt, DGv, DDv, EPTv, NSPv, NEv, NFFv, ROWSv)   \
+    INFR_STREAM_AT_N(FGt, FDt, DGv, DDv, EPTv, NSPv, NEv, NFFv, ROWSv, 0) \
+    INFR_STREAM_AT_N(FGt, FDt, DGv, DDv, EPTv, NSPv, NEv, NFFv, ROWSv, 1)
 
 }  // namespace infr
