@@ -43,7 +43,7 @@ inline void lds_limit(const void* kernel, int bytes, std::atomic<uint32_t>& done
         ::infr::lds_limit((const void*)kernel, (bytes), lds_limit_done_);   \
     } while (0)
 
-// An Op::RmsNorm of up to 31 token rows folded into the logits kernel: x are the raw rows, every
+// An Op::RmsNorm folded into the logits kernel (router_logits_can_norm: which): x are the raw rows, every
 // block normalises its rows while staging and the first block of a row also stores it normalised to xn_out.
 struct RouterNorm {
     const float* weight = nullptr;   // [ne]

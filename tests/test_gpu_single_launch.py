@@ -704,7 +704,7 @@ FOLDED = "rms_norm_router_logits"
 
 
 @pytest.mark.parametrize("rows,ne,E,K,nff,gdt,ddt,name", [
-    # two rows to a workgroup of the logits (whole and ragged shares of 256 loads), four; rows behind the last whole workgroup
+    # one row and one expert to a workgroup of the logits, but for 31 rows: two of each, and a row behind the last whole workgroup
     (2, 2048, 8, 2, 256, H.Q4K, H.Q6K, FOLDED), (31, 2048, 32, 2, 256, H.Q8_0, H.Q8_0, FOLDED), (3, 2080, 7, 2, 64, H.Q8_0, H.Q8_0, FOLDED),
     (6, 1024, 32, 8, 512, H.Q8_0, H.Q8_0, FOLDED), (5, 2880, 9, 3, 64, H.Q8_0, H.Q8_0, FOLDED), (2, 4096, 8, 2, 256, H.Q4K, H.Q6K, FOLDED), (7, 4096, 8, 2, 256, H.Q4K, H.Q6K, FOLDED),
     # the whole sublayer in one launch
