@@ -985,3 +985,72 @@ def test_rms_norm_of_rows_whose_mean_square_is_subnormal(be, rows, ne, E, K, nff
     x64 = x.astype(np.float64)
     want = x64 / np.sqrt((x64 ** 2).mean(axis=1, keepdims=True)) * nw
     assert (np.abs(normed.reshape(rows, ne) - want) <= np.abs(want) * 2.0 ** -17).all()
+
+
+@pytest.mark.parametrize("gated", [False, True])
+@pytest.mark.parametrize("rows,ne,E,nff", [(1, 2048, 128, 768), (2, 2048, 128, 768), (3, 2048, 128, 768), (5, 2048, 64, 256), (4, 4096, 256, 1536)])
+def test_rms_norm_of_several_rows_beside_an_always_on_expert(rows, ne, E, nff, gated):
+    """The sublayer with an always-on expert on its three paths, the norm folded into the single launch (not beside a gated one, whose gate
+    logit needs the row earlier) or into the logits of three: every pass, each with another x, has the bits of one launch per op."""
+    K, T, gd, dd = 8, M.TensorDesc, DType.Q4K, DType.Q6K
+    rng = np.random.default_rng(rows + nff)
+    passes = [(rng.standard_normal((rows, ne)) * s).astype(np.float32) for s in (1.0, 4.0)]
+    f32 = dict(nw=rng.uniform(0.5, 1.5, ne), router=rng.standard_normal((E, ne)) * 0.02, wq=rng.standard_normal((1, ne)) * 0.02)
+    outs, names = {}, {}
+    for plain in (False, True):
+        b = M.Backend(0, disable_op_fusion=plain, disable_single_launch_moe=plain)
+        try:
+            g, bind, bufs = M.Graph(), M.Bindings(), []
+
+            def bound(tid, buf):
+                bufs.append(buf)
+                bind.bind(tid, buf)
+                return tid
+
+            def bank(dims, dt, seed):
+                n = int(np.prod(dims))
+                tid = bound(g.weight(T(dims, dt)), b.alloc_uninit(M.backend.bytes_for(dt, n)))
+                synth.weights_device(b, bufs[-1], dt, seed, n)
+                return tid
+            xi = bound(g.input(T([rows, ne], DType.F32)), b.buffer_from(passes[0]))
+            x_buf = bufs[-1]
+            nw, rt, wq = (bound(g.weight(T(list(v.shape), DType.F32)), b.buffer_from(v.astype(np.float32))) for v in f32.values())
+            gt, ut, dt = bank([E, nff, ne], gd, 1), bank([E, nff, ne], gd, 2), bank([E, ne, nff], dd, 3)
+            sg, su, sd = bank([nff, ne], gd, 4), bank([nff, ne], gd, 5), bank([ne, nff], dd, 6)
+            y = bound(g.output(T([rows, ne], DType.F32)), b.alloc(rows * ne * 4))
+            y_buf = bufs[-1]
+            t = lambda n: g.internal(T([rows, n], DType.F32))  # noqa: E731
+            h, moe, tg, tu, ta, ts, sub, tq = t(ne), t(ne), t(nff), t(nff), t(nff), t(ne), t(ne), t(1)
+            g.rms_norm(x=xi, weight=nw, dst=h, rows=rows, dim=ne, eps=1e-6)
+            g.moe_ffn(x=h, router=rt, gate_exps=gt, up_exps=ut, down_exps=dt, dst=moe, ne=ne, n_expert=E, n_used=K, n_ff_exp=nff)
+            if gated:
+                g.linear(x=h, weight=wq, dst=tq, m=rows, in_f=ne, out_f=1)
+            g.linear(x=h, weight=sg, dst=tg, m=rows, in_f=ne, out_f=nff)
+            g.linear(x=h, weight=su, dst=tu, m=rows, in_f=ne, out_f=nff)
+            g.gated_act(gate=tg, up=tu, dst=ta, rows=rows, nff=nff)
+            g.linear(x=ta, weight=sd, dst=ts, m=rows, in_f=nff, out_f=ne)
+            if gated:
+                g.moe_shared_expert_add(moe=moe, shexp=ts, gate=tq, dst=sub, rows=rows, n=ne)
+            else:
+                g.add(a=moe, b=ts, dst=sub, n=rows * ne)
+            g.add(a=xi, b=sub, dst=y, n=rows * ne)
+            plan = b.compile(g)
+            b.prof_enable(True)
+            outs[plain] = []
+            for x in passes:
+                b.upload(x_buf, x)
+                b.execute(plan, bind)
+                outs[plain].append(b.download(y_buf, rows * ne * 4, np.float32).copy())
+            names[plain] = set(b.prof_read())
+            for buf in bufs:
+                buf.free()
+            plan.free()
+        finally:
+            b.close()
+    if rows in (3, 5):
+        assert FOLDED in names[False] and "rms_norm" not in names[False] and "moe_layer_shared" not in names[False], names
+    else:
+        assert names[False] == {"moe_layer_shared"} | ({"rms_norm", "linear"} if gated else set()), names
+    assert {"rms_norm", "linear", "gated_act", "add"} <= names[True]
+    assert all(np.array_equal(bits(a), bits(c)) for a, c in zip(outs[False], outs[True]))
+    assert not np.array_equal(outs[True][0], outs[True][1])
